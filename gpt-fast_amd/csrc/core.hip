@@ -203,70 +203,276 @@ extern "C" int gfa_add_rmsnorm(float* res, const void* y, const float* w, void* 
 }
 
 // --------------------------------------------------------------------------------------
-// float32 matrix product: out[m, n] (+)= sum_k a[m, k] * w[n, k]
-// 64x64 tile per workgroup of 256 threads, 4x4 outputs per thread, k in steps of 16 through
-// shared memory.  Each output is one fused-multiply-add chain over k = 0..K-1 in order.
-#define GF_BM 64
-#define GF_BN 64
-#define GF_BK 16
-__global__ __launch_bounds__(256) void gemm_f32_kernel(
-        const float* __restrict__ a, const float* __restrict__ w, float* __restrict__ out,
-        int M, int N, int K, int lda, int ldo, int accumulate) {
-    __shared__ float As[GF_BK][GF_BM + 4];
-    __shared__ float Ws[GF_BK][GF_BN + 4];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int m0 = blockIdx.y * GF_BM, n0 = blockIdx.x * GF_BN;
-    float acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+// float32 matrix products: out[b][m, n] (+)= sum_k a[b][m, k] * w[b][n, k], element (m, k) of a[b] at
+// a + b sab + m sam + k, element (n, k) of w[b] at w + b swb + n swn + k swk, element (m, n) of out[b] at
+// out + b sob + m som + n.
+//
+// v_mfma_f32_16x16x4_f32: true float32 products and sums, at the vector units' peak rate but without
+// their operand traffic.  The four waves of a workgroup take the same 16 MT x 16 NT tile and every
+// fourth block of 32 k each, so that even a 16-column tile of one row keeps four waves' loads in flight;
+// a lane's 16-byte loads are four k of one row of a or w and land in operand order (the k within a
+// block are taken in an order that is the same for a and w), so nothing goes through shared memory but
+// the four sums at the end.  An output's sum is therefore four chains, added as (0 + 1) + (2 + 3), whose
+// order depends on K alone: every tile size and every M gives the same bits, and a row's result does not
+// depend on the other rows (a float32 logit is the same however tokens are cut into steps).
+// gf_launch picks the tile.  Measured beside 64 x 64 tiles of vector multiply-adds through shared memory,
+// which this replaces: 1 x 768 x 768 76 -> 5.8 us, 1 x 32,000 x 768 120 -> 29 (3.4 TB/s), 717 x 2,304 x 768
+// 99 -> 44, 717 x 768 x 2,048 274 -> 41, 8 x 28,672 x 4,096 617 -> 116 (4.1 TB/s), 2,048 x 4,096 x 4,096
+// 988 -> 704 (98 of the 155 TFLOP/s that a loop of the instruction alone reaches); few rows are bound by
+// latency and the weights, many by the matrix units.
+typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gf_floatx4_t;
 
-    for (int k0 = 0; k0 < K; k0 += GF_BK) {
+// out's tile at (m0, n0) from the waves' sums, ((0 + 1) + (2 + 3)); lane: four columns of a row
+template <int MT, int NT>
+__device__ __forceinline__ void gf_store(const gf_floatx4_t (*sums)[MT * NT][64], float* __restrict__ out, int M,
+                                         int N, int m0, int n0, long long som, int accumulate) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool quad = som % 4 == 0 && (uintptr_t)out % 16 == 0;
+    for (int t = wave; t < MT * NT; t += 4) {
+        const gf_floatx4_t v = (sums[0][t][lane] + sums[1][t][lane]) + (sums[2][t][lane] + sums[3][t][lane]);
+        const int m = m0 + 16 * (t / NT) + (lane & 15), n = n0 + 16 * (t % NT) + 4 * (lane >> 4);
+        if (m >= M || n >= N) continue;
+        float* o = out + (size_t)m * som + n;
+        if (quad && n + 4 <= N) {
+            gf_floatx4_t* o4 = (gf_floatx4_t*)o;
+            *o4 = accumulate ? *o4 + v : v;
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int e = threadIdx.x + i * 256;
-            const int r = e >> 4, c = e & 15;
-            const int k = k0 + c;
-            const int m = m0 + r, n = n0 + r;
-            As[c][r] = (m < M && k < K) ? a[(size_t)m * lda + k] : 0.f;
-            Ws[c][r] = (n < N && k < K) ? w[(size_t)n * K + k] : 0.f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < GF_BK; ++kk) {
-            float av[4], wv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) av[i] = As[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) wv[j] = Ws[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], wv[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty * 4 + i;
-        if (m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (n >= N) continue;
-            float* o = out + (size_t)m * ldo + n;
-            *o = accumulate ? (*o + acc[i][j]) : acc[i][j];
+            for (int q = 0; q < 4; ++q)
+                if (n + q < N) o[q] = accumulate ? o[q] + v[q] : v[q];
         }
     }
 }
 
+template <int MT, int NT, bool WIDE>
+__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(
+        const float* __restrict__ a, const float* __restrict__ w, float* __restrict__ out,
+        int M, int N, int K, long long sab, long long sam, long long swb, long long swn,
+        long long swk, long long sob, long long som, int accumulate) {
+    constexpr int AHEAD = MT * NT == 1 ? 4 : MT * NT <= 4 ? 2 : 1;   // blocks asked for ahead
+    __shared__ gf_floatx4_t sums[4][MT * NT][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = lane & 15, lg = lane >> 4;
+    const int m0 = blockIdx.y * (16 * MT), n0 = blockIdx.x * (16 * NT);
+    a += (size_t)blockIdx.z * sab;
+    w += (size_t)blockIdx.z * swb;
+    out += (size_t)blockIdx.z * sob;
+    const float *ar[MT], *wr[NT];                  // rows beyond the last read it again, never stored
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int m = m0 + 16 * i + li;
+        ar[i] = a + (size_t)(m < M ? m : M - 1) * sam;
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int n = n0 + 16 * j + li;
+        wr[j] = w + (size_t)(n < N ? n : N - 1) * swn;
+    }
+    gf_floatx4_t acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
+
+    struct Block {
+        gf_floatx4_t a[2][MT], w[2][NT];
+    };
+    // the lane's elements of block b (its k: 32 b + 16 h + 4 lg + 0..3); zero beyond K.  Every load is made,
+    // at a place that is there: loads under a condition would not stay in flight
+    auto load = [&](int b, Block& r) {
+        const bool whole = 32 * b + 32 <= K;       // the same for the whole wave
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int k = 32 * b + 16 * h + 4 * lg;
+            if (WIDE) {
+                const int at = k < K ? k : 0;      // K is a multiple of four
+#pragma unroll
+                for (int i = 0; i < MT; ++i) r.a[h][i] = *(const gf_floatx4_t*)(ar[i] + at);
+#pragma unroll
+                for (int j = 0; j < NT; ++j) r.w[h][j] = *(const gf_floatx4_t*)(wr[j] + at);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int at = k + q < K ? k + q : 0;
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) r.a[h][i][q] = ar[i][at];
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) r.w[h][j][q] = wr[j][(size_t)at * swk];
+                }
+            }
+            if (!whole) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (k + q >= K) {
+#pragma unroll
+                        for (int i = 0; i < MT; ++i) r.a[h][i][q] = 0.f;
+#pragma unroll
+                        for (int j = 0; j < NT; ++j) r.w[h][j][q] = 0.f;
+                    }
+            }
+        }
+    };
+    auto multiply = [&](const Block& r) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)   // transposed: a lane ends with four columns of a row
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.w[h][j][q], r.a[h][i][q],
+                                                                         acc[i][j], 0, 0, 0);
+    };
+    const int blocks = (K + 31) / 32;
+    Block ring[AHEAD + 1];
+    if (blocks > 0) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) load(wave + 4 * u, ring[u]);
+    }
+    for (int b = wave; b < blocks; b += 4 * (AHEAD + 1)) {
+#pragma unroll
+        for (int u = 0; u <= AHEAD; ++u) {
+            if (b + 4 * u >= blocks) break;
+            load(b + 4 * (u + AHEAD), ring[(u + AHEAD) % (AHEAD + 1)]);
+            multiply(ring[u]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) sums[wave][i * NT + j][lane] = acc[i][j];
+    __syncthreads();
+    gf_store<MT, NT>(sums, out, M, N, m0, n0, som, accumulate);
+}
+
+// The same arithmetic for many rows (16-byte loads only): a 64 x 64 tile whose waves copy their blocks
+// through shared memory of their own (no barrier while K is walked).  A load instruction then takes eight
+// rows of 128 bytes, whole lines, where the operand order above takes sixteen rows of 64, which the compute
+// unit's cache looks up piece by piece: 2,048 x 4,096 x 4,096 took 1,155 us without it.
+#define GS_PITCH 144                              // bytes per staged row of 32 k: 128 + pad against conflicts
+__global__ __launch_bounds__(256, 2) void gemm_f32_staged_kernel(
+        const float* __restrict__ a, const float* __restrict__ w, float* __restrict__ out,
+        int M, int N, int K, long long sab, long long sam, long long swb, long long swn,
+        long long sob, long long som, int accumulate) {
+    __shared__ __attribute__((aligned(16))) char lds[4 * 128 * GS_PITCH];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = lane & 15, lg = lane >> 4;
+    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
+    a += (size_t)blockIdx.z * sab;
+    w += (size_t)blockIdx.z * swb;
+    out += (size_t)blockIdx.z * sob;
+    const int row = lane >> 3, chunk = lane & 7;   // of eight rows, their 16-byte chunks
+    const float *ar[8], *wr[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int m = m0 + 8 * i + row, n = n0 + 8 * i + row;
+        ar[i] = a + (size_t)(m < M ? m : M - 1) * sam;
+        wr[i] = w + (size_t)(n < N ? n : N - 1) * swn;
+    }
+    gf_floatx4_t acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
+    gf_floatx4_t av[8], wv[8];
+    auto load = [&](int b) {
+        const int k = 32 * b + 4 * chunk, at = k < K ? k : 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            av[i] = *(const gf_floatx4_t*)(ar[i] + at);
+            wv[i] = *(const gf_floatx4_t*)(wr[i] + at);
+        }
+        if (32 * b + 32 > K && k >= K) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) av[i] = wv[i] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+    char* as = lds + wave * 128 * GS_PITCH;
+    char* ws = as + 64 * GS_PITCH;
+    const int put = row * GS_PITCH + chunk * 16, get = li * GS_PITCH + lg * 16;
+    const int blocks = (K + 31) / 32;
+    if (wave < blocks) load(wave);
+    for (int b = wave; b < blocks; b += 4) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            *(gf_floatx4_t*)(as + put + 8 * i * GS_PITCH) = av[i];
+            *(gf_floatx4_t*)(ws + put + 8 * i * GS_PITCH) = wv[i];
+        }
+        if (b + 4 < blocks) load(b + 4);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            gf_floatx4_t af[4], wf[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                af[i] = *(const gf_floatx4_t*)(as + get + 16 * i * GS_PITCH + 64 * h);
+                wf[i] = *(const gf_floatx4_t*)(ws + get + 16 * i * GS_PITCH + 64 * h);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[j][q], af[i][q], acc[i][j], 0, 0, 0);
+        }
+    }
+    __syncthreads();
+    gf_floatx4_t (*sums)[16][64] = (gf_floatx4_t (*)[16][64])lds;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sums[wave][i * 4 + j][lane] = acc[i][j];
+    __syncthreads();
+    gf_store<4, 4>(sums, out, M, N, m0, n0, som, accumulate);
+}
+
+// Up to 16 rows: one 16 x 16 tile a workgroup, which spreads the weights over the most waves.  More rows:
+// 64 x 64 where these tiles are at least 100 (717 x 768 x 2,048, 144 of them: 41 us, as 32 x 32 54 us), else
+// 32 x 32; without 16-byte loads there is no staged kernel, and the unstaged one needs more tiles to win.
+template <bool WIDE>
+static int gf_launch(const float* a, const float* w, float* out, int B, int M, int N, int K,
+                     long long sab, long long sam, long long swb, long long swn, long long swk,
+                     long long sob, long long som, int accumulate, hipStream_t stream) {
+#define GF_GO(MT, NT) do { \
+        if ((M + 16 * MT - 1) / (16 * MT) > 65535 || B > 65535) return (int)hipErrorInvalidValue; \
+        const dim3 grid((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT), B); \
+        gemm_f32_kernel<MT, NT, WIDE><<<grid, 256, 0, stream>>>(a, w, out, M, N, K, sab, sam, swb, swn, \
+                                                                swk, sob, som, accumulate); \
+        return GFA_LAUNCH_RESULT(); \
+    } while (0)
+    const long long big = (long long)((M + 63) / 64) * ((N + 63) / 64) * B;
+    if (M <= 16) GF_GO(1, 1);
+    if (big < (WIDE ? 100 : 384)) GF_GO(2, 2);
+    if (!WIDE) GF_GO(4, 4);
+    if ((M + 63) / 64 > 65535 || B > 65535) return (int)hipErrorInvalidValue;
+    const dim3 grid((N + 63) / 64, (M + 63) / 64, B);
+    gemm_f32_staged_kernel<<<grid, 256, 0, stream>>>(a, w, out, M, N, K, sab, sam, swb, swn, sob, som, accumulate);
+    return GFA_LAUNCH_RESULT();
+#undef GF_GO
+}
+
+static int gf_product(const float* a, const float* w, float* out, int B, int M, int N, int K,
+                      long long sab, long long sam, long long swb, long long swn, long long swk,
+                      long long sob, long long som, int accumulate, hipStream_t stream) {
+    if (B <= 0 || M <= 0 || N <= 0) return 0;
+    // 16-byte loads: whole groups of four k, at addresses that are multiples of 16
+    const bool wide = swk == 1 && K % 4 == 0 && sam % 4 == 0 && swn % 4 == 0 && sab % 4 == 0 && swb % 4 == 0 &&
+                      (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0;
+    return (wide ? gf_launch<true> : gf_launch<false>)(a, w, out, B, M, N, K, sab, sam, swb, swn, swk, sob,
+                                                       som, accumulate, stream);
+}
+
 extern "C" int gfa_gemm_f32(const float* a, const float* w, float* out, int M, int N, int K,
                             int lda, int ldo, int accumulate, hipStream_t stream) {
-    if (M <= 0 || N <= 0) return 0;
-    dim3 grid((N + GF_BN - 1) / GF_BN, (M + GF_BM - 1) / GF_BM);
-    gemm_f32_kernel<<<grid, 256, 0, stream>>>(a, w, out, M, N, K, lda, ldo, accumulate);
-    return GFA_LAUNCH_RESULT();
+    return gf_product(a, w, out, 1, M, N, K, 0, lda, 0, K, 1, 0, ldo, accumulate, stream);
+}
+
+extern "C" int gfa_gemm_f32_strided(const float* a, const float* w, float* out, int B, int M, int N,
+                                    int K, long long sab, long long sam, long long swb,
+                                    long long swn, long long swk, long long sob, long long som,
+                                    hipStream_t stream) {
+    return gf_product(a, w, out, B, M, N, K, sab, sam, swb, swn, swk, sob, som, 0, stream);
 }
 
 // --------------------------------------------------------------------------------------
@@ -955,77 +1161,6 @@ __global__ void add_bias_kernel(float* __restrict__ res, const float* __restrict
 extern "C" int gfa_add_bias(float* res, const float* bias, int n_rows, int dim, hipStream_t stream) {
     if (n_rows <= 0) return 0;
     add_bias_kernel<<<n_rows, 256, 0, stream>>>(res, bias, dim);
-    return GFA_LAUNCH_RESULT();
-}
-
-// --------------------------------------------------------------------------------------
-// A batch of float32 products with strides: for every b < B
-//     out[b][m, n] = sum_k a[b][m, k] * w[b][n, k]
-// with element (m, k) of a[b] at a + b sab + m sam + k (unit stride along k), element (n, k)
-// of w[b] at w + b swb + n swn + k swk, element (m, n) of out[b] at out + b sob + m som + n.
-// The same tiles and the same chain of fused multiply-adds per output as gemm_f32_kernel.
-__global__ __launch_bounds__(256) void gemm_f32_strided_kernel(
-        const float* __restrict__ a, const float* __restrict__ w, float* __restrict__ out,
-        int M, int N, int K, long long sab, long long sam, long long swb, long long swn,
-        long long swk, long long sob, long long som) {
-    __shared__ float As[GF_BK][GF_BM + 4];
-    __shared__ float Ws[GF_BK][GF_BN + 4];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int m0 = blockIdx.y * GF_BM, n0 = blockIdx.x * GF_BN;
-    a += (size_t)blockIdx.z * sab;
-    w += (size_t)blockIdx.z * swb;
-    out += (size_t)blockIdx.z * sob;
-    float acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-    for (int k0 = 0; k0 < K; k0 += GF_BK) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int e = threadIdx.x + i * 256;
-            const int r = e >> 4, c = e & 15;
-            const int k = k0 + c;
-            const int m = m0 + r, n = n0 + r;
-            As[c][r] = (m < M && k < K) ? a[(size_t)m * sam + k] : 0.f;
-            Ws[c][r] = (n < N && k < K) ? w[(size_t)n * swn + (size_t)k * swk] : 0.f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < GF_BK; ++kk) {
-            float av[4], wv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) av[i] = As[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) wv[j] = Ws[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], wv[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty * 4 + i;
-        if (m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx * 4 + j;
-            if (n < N) out[(size_t)m * som + n] = acc[i][j];
-        }
-    }
-}
-
-extern "C" int gfa_gemm_f32_strided(const float* a, const float* w, float* out, int B, int M, int N,
-                                    int K, long long sab, long long sam, long long swb,
-                                    long long swn, long long swk, long long sob, long long som,
-                                    hipStream_t stream) {
-    if (B <= 0 || M <= 0 || N <= 0) return 0;
-    if (B > 65535 || (M + GF_BM - 1) / GF_BM > 65535) return (int)hipErrorInvalidValue;
-    dim3 grid((N + GF_BN - 1) / GF_BN, (M + GF_BM - 1) / GF_BM, B);
-    gemm_f32_strided_kernel<<<grid, 256, 0, stream>>>(a, w, out, M, N, K, sab, sam, swb, swn, swk,
-                                                      sob, som);
     return GFA_LAUNCH_RESULT();
 }
 

@@ -2,7 +2,7 @@
 reference's linears (model.py:110, 174-175, 222-224), with the epilogues the blocks need.
 
 float32 engine: the library's own float32 kernel, for every shape (a true 32-bit
-product; one fused-multiply-add chain per output).
+product; an output's order of additions depends on the inner size alone).
 
 bfloat16 engine, by the rows of x: up to 16, hand-written kernels that stream the weights
 once (csrc/gemm_bf16.hip; up to 24 rows inside a layer's chain where a matrix has no

@@ -89,6 +89,27 @@ def test_gemm_f32(M, N, K_):
     close(res, keep.double() + ref, 1e-5)
 
 
+@pytest.mark.parametrize("N,K_", [(1, 1), (17, 31), (64, 33), (130, 128), (100, 164), (7000, 60)])
+def test_gemm_f32_is_the_same_in_every_tile(N, K_):
+    """Every number of rows (each tile size, whole and ragged), rows at odd addresses and the
+    batched form with its own strides give a row the same bits; against float64 within the rounding
+    of sums of K terms, each of which adds at most half a unit of 2^-23."""
+    torch.manual_seed(4)
+    a = torch.randn(520, K_, device=DEV)
+    w = torch.randn(N, K_, device=DEV)
+    ref = a.double() @ w.double().T
+    most = a.abs().double() @ w.abs().double().T
+    whole = K().gemm_f32(a, w)
+    assert bool(((whole.double() - ref).abs() <= most * (K_ + 4) * 2.0 ** -24).all())
+    for M in (1, 15, 16, 17, 33, 64, 65, 300):
+        assert torch.equal(K().gemm_f32(a[:M], w), whole[:M]), M
+    odd = torch.empty(40, K_ + 1, device=DEV)[:, 1:].copy_(a[:40])
+    assert torch.equal(K().gemm_f32(odd, w), whole[:40])
+    out = torch.empty(2, 40, N, device=DEV)
+    K().gemm_f32_batched(a[:80].view(2, 40, K_), w.t().contiguous().t()[None].expand(2, N, K_), out)
+    assert torch.equal(out.view(80, N), whole[:80])
+
+
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 9, 16, 17, 20, 22, 24, 33, 64])
 @pytest.mark.parametrize("N,K_", [(40, 64), (136, 200), (1000, 328), (96, 4096), (77, 75)])
 def test_skinny_bf16(M, N, K_):
