@@ -763,6 +763,109 @@ __global__ __launch_bounds__(AG_THREADS) void attention_generic_kernel(
     }
 }
 
+// The same for float32 heads of a multiple of 16 (the float32 engine's attention): one workgroup per (token,
+// head), whose four waves take every fourth page each with a running maximum of their own, a key per lane
+// for the scores and an element (or HD / 64) per lane for the values, both in 16-byte loads that do not
+// depend on each other; the waves' results are merged in their order.  What bounds a single-token step is
+// the chain of loads, scores, maximum and values of a page: one page per wave at up to 256 keys, where the
+// kernel above walks all keys' values one after the other: four requests of the 110M shape, 20 to 200 tokens
+// and then 12 steps, 21.4 -> 12.7 ms with it.
+// A row's result depends on its position and window alone.  HD: head size rounded up to 64.
+template <int HD>
+__global__ __launch_bounds__(256) void attention_f32_kernel(
+        const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
+        const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, const int* __restrict__ table,
+        int table_stride, float* __restrict__ out, int H, int Hkv, int hd, float scale, int window) {
+    constexpr int PER = HD / 64;
+    __shared__ __attribute__((aligned(16))) float qs[HD];
+    __shared__ __attribute__((aligned(16))) float ps[4][GFA_PAGE];
+    __shared__ float merged[4][HD + 2];
+    const int n = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int g = h / (H / Hkv);
+    const int pos = tok_pos[n];
+    const int* pages = table + (size_t)tok_seq[n] * table_stride;
+    const int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
+    for (int d = threadIdx.x; d < hd; d += 256) qs[d] = q[((size_t)n * H + h) * hd + d];
+    __syncthreads();
+    float m = -INFINITY, l = 0.f, acc[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) acc[i] = 0.f;
+    // by the page's own index, so that a window's first page does not move a key to another wave
+    const int first = lo / GFA_PAGE;
+    for (int page = first + ((wave - first) & 3); page * GFA_PAGE <= pos; page += 4) {
+        const size_t region = cache_region(pages[page], g, Hkv, hd);
+        const int key = page * GFA_PAGE + lane;
+        const float* kr = k_pages + region + (lane >> 5) * 32 * hd + key_slot(lane & 31) * 8;
+        float dot0 = 0.f, dot1 = 0.f;
+#pragma unroll 8
+        for (int c = 0; c < hd / 8; ++c) {
+            const float4 a = *(const float4*)(kr + c * 256), b = *(const float4*)(kr + c * 256 + 4);
+            const float4 x = *(const float4*)(qs + c * 8), y = *(const float4*)(qs + c * 8 + 4);
+            dot0 = fmaf(a.w, x.w, fmaf(a.z, x.z, fmaf(a.y, x.y, fmaf(a.x, x.x, dot0))));
+            dot1 = fmaf(b.w, y.w, fmaf(b.z, y.z, fmaf(b.y, y.y, fmaf(b.x, y.x, dot1))));
+        }
+        const bool seen = key >= lo && key <= pos;
+        const float s = seen ? (dot0 + dot1) * scale : -INFINITY;
+        const float m_new = fmaxf(m, wave_max(s));
+        const bool any = m_new != -INFINITY;               // no number to scale by otherwise
+        const float alpha = any ? expf(m - m_new) : 1.f;
+        const float p = seen && any ? expf(s - m_new) : 0.f;
+        l = l * alpha + wave_sum(p);
+        m = m_new;
+        ps[wave][lane] = p;                                // read by this wave alone
+        __builtin_amdgcn_wave_barrier();
+        const bool whole = page * GFA_PAGE >= lo && page * GFA_PAGE + GFA_PAGE - 1 <= pos;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int d = lane + 64 * i;
+            if (d >= hd) continue;
+            const float* vr = v_pages + region + (d >> 4) * 1024 + (d & 15) * 8;
+            float sum = acc[i] * alpha;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {                  // keys 8 c .. + 7
+                float4 a = *(const float4*)(vr + c * 128), b = *(const float4*)(vr + c * 128 + 4);
+                if (!whole) {                              // slots that hold no seen key are not numbers to use
+                    const int k0 = page * GFA_PAGE + 8 * c;
+                    if (k0 + 0 < lo || k0 + 0 > pos) a.x = 0.f;
+                    if (k0 + 1 < lo || k0 + 1 > pos) a.y = 0.f;
+                    if (k0 + 2 < lo || k0 + 2 > pos) a.z = 0.f;
+                    if (k0 + 3 < lo || k0 + 3 > pos) a.w = 0.f;
+                    if (k0 + 4 < lo || k0 + 4 > pos) b.x = 0.f;
+                    if (k0 + 5 < lo || k0 + 5 > pos) b.y = 0.f;
+                    if (k0 + 6 < lo || k0 + 6 > pos) b.z = 0.f;
+                    if (k0 + 7 < lo || k0 + 7 > pos) b.w = 0.f;
+                }
+                const float4 x = *(const float4*)(ps[wave] + 8 * c), y = *(const float4*)(ps[wave] + 8 * c + 4);
+                sum = fmaf(a.w, x.w, fmaf(a.z, x.z, fmaf(a.y, x.y, fmaf(a.x, x.x, sum))));
+                sum = fmaf(b.w, y.w, fmaf(b.z, y.z, fmaf(b.y, y.y, fmaf(b.x, y.x, sum))));
+            }
+            acc[i] = sum;
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) merged[wave][lane + 64 * i] = acc[i];
+    if (lane == 0) {
+        merged[wave][HD] = m;
+        merged[wave][HD + 1] = l;
+    }
+    __syncthreads();
+    float top = merged[0][HD];
+    for (int w = 1; w < 4; ++w) top = fmaxf(top, merged[w][HD]);
+    float total = 0.f, part[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        part[w] = merged[w][HD] == -INFINITY ? 0.f : expf(merged[w][HD] - top);
+        total = fmaf(merged[w][HD + 1], part[w], total);
+    }
+    for (int d = threadIdx.x; d < hd; d += 256) {
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) v = fmaf(merged[w][d], part[w], v);
+        out[((size_t)n * H + h) * hd + d] = v / total;
+    }
+}
+
 extern "C" int gfa_attention_generic(const void* q, const void* k_pages, const void* v_pages,
                                      const int* tok_seq, const int* tok_pos, const int* table,
                                      int table_stride, void* out, int n_tokens, int H, int Hkv,
@@ -771,6 +874,16 @@ extern "C" int gfa_attention_generic(const void* q, const void* k_pages, const v
     if (n_tokens <= 0) return 0;
     if (hd > AG_THREADS * AG_MAX_PER_THREAD || H > 65535) return (int)hipErrorInvalidValue;
     dim3 grid(n_tokens, H);
+    // 16-byte loads of the cache's operand order need it to begin at such an address
+    if (!is_bf16 && hd % 16 == 0 && hd <= 256 && (uintptr_t)k_pages % 16 == 0 && (uintptr_t)v_pages % 16 == 0) {
+#define AF_GO(HD) attention_f32_kernel<HD><<<grid, 256, 0, stream>>>((const float*)q, (const float*)k_pages, \
+        (const float*)v_pages, tok_seq, tok_pos, table, table_stride, (float*)out, H, Hkv, hd, scale, window)
+        if (hd <= 64) AF_GO(64);
+        else if (hd <= 128) AF_GO(128);
+        else AF_GO(256);
+#undef AF_GO
+        return GFA_LAUNCH_RESULT();
+    }
     const size_t shmem = (size_t)(hd + AG_THREADS + 16) * sizeof(float);
     if (is_bf16)
         attention_generic_kernel<bf16_t><<<grid, AG_THREADS, shmem, stream>>>(
