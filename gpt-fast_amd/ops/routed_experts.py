@@ -256,13 +256,15 @@ def expert_tiles(offsets: torch.Tensor, n_experts: int, pairs: int) -> torch.Ten
 
 
 def expert_tile_product(x: torch.Tensor, order: Optional[torch.Tensor], top: int, w: torch.Tensor,
-                        offsets: torch.Tensor, tiles: torch.Tensor, pairs: int,
+                        offsets: torch.Tensor, tiles: Optional[torch.Tensor], pairs: int,
                         activation: Optional[str] = None, gated: bool = False,
                         limit: Optional[float] = None) -> torch.Tensor:
     """bfloat16 [pairs, F]: row p of expert e is ``act(W[e] x[r])``, r = ``order[p] // top`` (or p itself
     without ``order``); ``gated``: W is [E, 2 F, K] and the row ``act(W_gate x) * (W_up x)``, or the
-    clamped gate.  Rows that belong to no expert of ``tiles`` are not written.  Operands as for
-    :func:`grouped_rows`; nothing is read on the host."""
+    clamped gate.  Rows that belong to no expert are not written.  Operands as for
+    :func:`grouped_rows`; nothing is read on the host.  Inner sizes of whole pieces of 64 and F of whole
+    16 bytes take the kernel that finds its tiles in ``offsets``; other sizes take one that needs
+    ``tiles`` (:func:`expert_tiles`; None: made here)."""
     require_device(x, order, w, offsets, tiles)
     require_contiguous(x=x, order=order, w=w, offsets=offsets, tiles=tiles)
     if not grouped_rows_take(x, w):
@@ -270,8 +272,8 @@ def expert_tile_product(x: torch.Tensor, order: Optional[torch.Tensor], top: int
     E, N, K = w.shape
     if gated and N % 2:
         raise KernelError("expert_tile_product: gated experts have an even number of rows")
-    if offsets.dtype != torch.int32 or offsets.numel() < E + 1 or tiles.dtype != torch.int32 or tiles.dim() != 2 \
-            or tiles.shape[1] != 2:
+    if offsets.dtype != torch.int32 or offsets.numel() < E + 1 or (tiles is not None and (
+            tiles.dtype != torch.int32 or tiles.dim() != 2 or tiles.shape[1] != 2)):
         raise KernelError(f"expert_tile_product: offsets int32 [>= {E + 1}], tiles int32 [T, 2]")
     if order is not None and (order.dtype != torch.int32 or order.numel() < pairs or pairs > x.shape[0] * top):
         raise KernelError("expert_tile_product: order must be int32 and name every pair")
@@ -285,8 +287,15 @@ def expert_tile_product(x: torch.Tensor, order: Optional[torch.Tensor], top: int
     F = N // 2 if gated else N
     out = torch.empty((pairs, F), dtype=torch.bfloat16, device=x.device)
     mode = 3 if clamped else (2 if gated else (1 if activation is not None else 0))
+    act = 0 if clamped or activation is None else ACTIVATIONS[activation]
+    if K % 64 == 0 and F % 8 == 0 and 0 < N * K * 2 < 1 << 32:
+        check(library("routed_experts").gfa_expert_rows_product(
+            ptr(x), ptr(order), _i(max(1, top)), ptr(w), ptr(offsets), _i(E), _i(pairs), ptr(out), _i(F), _i(K),
+            _i(mode), _i(act), _f(limit or 0.0), stream_handle()), "expert_tile_product")
+        return out
+    if tiles is None:
+        tiles = expert_tiles(offsets, E, pairs)
     check(library("routed_experts").gfa_expert_tile_product(
         ptr(x), ptr(order), _i(max(1, top)), ptr(w), ptr(offsets), ptr(tiles), _i(tiles.shape[0]), ptr(out), _i(F),
-        _i(K), _i(mode), _i(0 if clamped or activation is None else ACTIVATIONS[activation]), _f(limit or 0.0),
-        stream_handle()), "expert_tile_product")
+        _i(K), _i(mode), _i(act), _f(limit or 0.0), stream_handle()), "expert_tile_product")
     return out

@@ -287,6 +287,48 @@ def test_tiles_of_the_experts_rows(E, D, Fh, counts):
             assert rel_err(got[lo:lo + c], rows[lo:lo + c].double() @ w[e].double().T) < 1e-2
 
 
+@pytest.mark.parametrize("E,D,Fh,counts", [(3, 64, 8, [1, 0, 70]), (70, 128, 24, [3] * 69 + [30]),
+                                           (4, 192, 136, [40, 64, 0, 65]), (2, 512, 128, [127, 129]),
+                                           (3, 4096, 264, [1, 257, 300]), (5, 576, 72, [0, 511, 0, 1, 256])])
+def test_the_experts_rows_in_tiles_of_whole_pieces(E, D, Fh, counts):
+    """Inner sizes of one, two and many pieces, columns that end inside a tile, more experts than lanes,
+    shares at the edges of 64, 128 and 256 rows, and each of the three tiles that the average share picks;
+    against the same bfloat16 operands in float64.  The result is rounded to bfloat16 once, which moves a
+    value by at most 2^-8 of itself (eight bits of significand), after sums of D float32 products (2^-24
+    each)."""
+    from gpt_fast_amd.ops import routed_experts as RE
+    g = torch.Generator().manual_seed(D + E)
+    top, n = 2, (sum(counts) + 5 + 1) // 2
+    pairs = n * top
+    ids = torch.tensor([e for e, c in enumerate(counts) for _ in range(c)] + [E] * (pairs - sum(counts)), dtype=torch.int32)
+    chosen = ids[torch.randperm(pairs, generator=g)].view(n, top).to(DEV)
+    offsets, order, place = RE.expert_order(chosen, E + 1)
+    x = torch.randn(n, D, generator=g).bfloat16()
+    w = (torch.randn(E, 2 * Fh, D, generator=g) * 0.3).bfloat16()
+    xs = x.double()[(order.cpu() // top).long()]
+    f = {None: lambda v: v, "silu": P.silu, "gelu": torch.nn.functional.gelu, "gelu_tanh": P.gelu_tanh}
+    for act, gated, limit in ((None, False, None), ("silu", False, None), ("gelu", False, None),
+                              ("gelu_tanh", False, None), ("silu", True, None), ("gelu_tanh", True, None),
+                              ("clamped_swish", True, 0.9)):
+        got = RE.expert_tile_product(x.to(DEV), order, top, w.to(DEV), offsets, None, pairs, act, gated, limit)
+        for e, c in enumerate(counts):
+            lo = sum(counts[:e])
+            z = xs[lo:lo + c] @ w[e].double().T
+            if act == "clamped_swish":
+                a, u = z[:, :Fh].clamp(max=limit), z[:, Fh:].clamp(-limit, limit)
+                z = a * torch.sigmoid(1.702 * a) * (u + 1)
+            else:
+                z = f[act](z[:, :Fh]) * z[:, Fh:] if gated else f[act](z)
+            if c:
+                assert rel_err(got[lo:lo + c].double().cpu(), z) < 2.0 ** -8, (act, gated, e)
+    rows = torch.randn(pairs, D, generator=g).bfloat16()
+    got = RE.expert_tile_product(rows.to(DEV), None, 1, w.to(DEV), offsets, None, pairs).double().cpu()
+    for e, c in enumerate(counts):
+        lo = sum(counts[:e])
+        if c:
+            assert rel_err(got[lo:lo + c], rows[lo:lo + c].double() @ w[e].double().T) < 2.0 ** -8
+
+
 def test_the_correction_moves_the_choice_and_not_the_weights():
     part, rt, w, mlp = _mixture(4, 2, 2, 64, 32, 1.0, None, "float32")
     part.correction.copy_(torch.tensor([0.0, 0.0, 0.0, 0.0, 5.0, 5.0]))     # both identity experts, always
