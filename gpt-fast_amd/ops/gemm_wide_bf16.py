@@ -64,11 +64,11 @@ def sum_store(part: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
 
 
 def sum_add_norm(residual: torch.Tensor, part: torch.Tensor, norm_w: Optional[torch.Tensor] = None,
-                 eps: float = 0.0) -> Optional[torch.Tensor]:
+                 eps: float = 0.0, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """residual += the slices added in order; with ``norm_w`` also returns the RMS norm of
-    the new rows in bfloat16."""
+    the new rows in bfloat16 (``out``: where they go)."""
     S, M, N = part.shape
-    require_device(residual, part, norm_w)
+    require_device(residual, part, norm_w, out)
     if residual.shape != (M, N) or residual.dtype != torch.float32 or not residual.is_contiguous():
         raise KernelError("sum_add_norm: residual must be contiguous float32 [M, N]")
     if N % 4 or N > 16384:
@@ -77,7 +77,9 @@ def sum_add_norm(residual: torch.Tensor, part: torch.Tensor, norm_w: Optional[to
     if norm_w is not None:
         if norm_w.dtype != torch.float32 or norm_w.numel() != N or not norm_w.is_contiguous():
             raise KernelError("sum_add_norm: one float32 norm weight per column")
-        xn = torch.empty((M, N), dtype=torch.bfloat16, device=residual.device)
+        xn = out if out is not None else torch.empty((M, N), dtype=torch.bfloat16, device=residual.device)
+        if xn.shape != (M, N) or xn.dtype != torch.bfloat16 or not xn.is_contiguous():
+            raise KernelError("sum_add_norm: out must be contiguous bfloat16 [M, N]")
     check(library("gemm_wide_bf16").gfa_wide_sum_add_norm(
         ptr(residual), ptr(part), _i(S), _i(M), _i(N), ptr(norm_w), ptr(xn), ctypes.c_float(eps),
         stream_handle()), "sum_add_norm")

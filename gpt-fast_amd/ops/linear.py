@@ -102,6 +102,25 @@ def _library_slices(M: int, N: int, K_: int, device) -> int:
     return S
 
 
+def _whole_rounds(M: int, N: int, K_: int, device) -> int:
+    """Rows that a product of the vendor library should take first, the others in a second one; 0: all at
+    once.  Its best kernels make 256 x 256 tiles, one to a compute unit; where these columns divide the
+    units, ``round`` rows fill the chip exactly, and for some numbers of rows beyond whole rounds the library
+    picks kernels that take far longer than its own two products for the whole rounds and the rest
+    (N = 4,096, K = 14,336, round 4,096, with the sum and norm behind it: 4,200 rows 750 us as one product,
+    427 as two; 5,500: 877, 525; 6,001: 586, 567; 7,491: 1,046, 683; 9,000: 1,203, 830).  Nothing is gained where
+    the rest nearly fills a round itself (8,000 rows: 697, 700; K = 4,096, 7,491 rows: 239, 256), sooner with
+    a short inner size (K = 4,096, 6,500 rows: 228, 220).  Measured for N of 2,048, 4,096 and 8,192, K >= N."""
+    cus = _compute_units(device)
+    if N % 256 or not 8 <= N // 256 <= 32 or cus % (N // 256) or K_ < N:
+        return 0
+    per_round = 256 * (cus // (N // 256))
+    rest = M % per_round
+    if M <= per_round or rest == 0 or rest * 20 >= per_round * (18 if K_ >= 2 * N else 13):
+        return 0
+    return M - rest
+
+
 def _library_partial_sums(x: torch.Tensor, w: torch.Tensor, S: int) -> torch.Tensor:
     """float32 [S, M, N]: x W^T over each of S equal slices of the inner size, as one batched
     product of the vendor library over views of x and w (nothing is copied)."""
@@ -193,6 +212,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         if S > 1:
             rows = SlicedRows(_library_partial_sums(x, w, S), out_dtype)
             return rows if may_stay_sliced else rows.rows()
+        first = _whole_rounds(M, w.shape[0], x.shape[1], x.device)
+        if first:
+            out = torch.empty((M, w.shape[0]), dtype=x.dtype, device=x.device)
+            torch.matmul(x[:first], w.t(), out=out[:first])
+            torch.matmul(x[first:], w.t(), out=out[first:])
+            return out
     return torch.matmul(x, w.t())
 
 
@@ -219,12 +244,28 @@ def linear_into(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, then_n
             return _wide().product_into(x, w, residual, weight, eps)
         if x.shape[0] > _wide().MAX_ROWS and w.shape[0] % 4 == 0 and w.shape[0] <= 16384 \
                 and x.is_contiguous() and w.is_contiguous():
-            S = _library_slices(x.shape[0], w.shape[0], x.shape[1], x.device)
-            if S > 1:
-                return _wide().sum_add_norm(residual, _library_partial_sums(x, w, S), weight, eps)
+            first = _whole_rounds(x.shape[0], w.shape[0], x.shape[1], x.device)
+            if first:
+                out = torch.empty(residual.shape, dtype=torch.bfloat16, device=x.device) if form is not None else None
+                for lo, hi in ((0, first), (first, x.shape[0])):
+                    _library_into(x[lo:hi], w, residual[lo:hi], weight, eps, None if out is None else out[lo:hi])
+                return out
+            return _library_into(x, w, residual, weight, eps)
         if form is not None:
             return K.add_rmsnorm(residual, torch.matmul(x, w.t()), weight, eps)
     _linear_into(x, w, residual)
+    return None
+
+
+def _library_into(x, w, residual, weight, eps, out=None):
+    """residual += x W^T through the vendor library, in slices of the inner size where that is faster; with the
+    next norm's ``weight`` its rows (into ``out`` if given), else None."""
+    S = _library_slices(x.shape[0], w.shape[0], x.shape[1], x.device)
+    if S > 1:
+        return _wide().sum_add_norm(residual, _library_partial_sums(x, w, S), weight, eps, out)
+    if weight is not None:
+        return K.add_rmsnorm(residual, torch.matmul(x, w.t()), weight, eps, out)
+    K.add_into(residual, torch.matmul(x, w.t()))
     return None
 
 

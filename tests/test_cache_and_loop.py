@@ -531,6 +531,12 @@ def test_dispatch_thresholds_follow_the_number_of_compute_units():
         assert L._library_slices(2048, 4096, 14336, "fake64") == 1
         assert L._library_slices(512, 4096, 4096, "fake256") == 4
         assert L._library_slices(300, 200, 96, "fake256") == 1     # a short inner size is never cut
+        assert [L._whole_rounds(M, 4096, 14336, "fake256") for M in (4096, 4097, 7491, 8000, 8192, 9000)] \
+            == [0, 4096, 4096, 0, 0, 8192]
+        assert [L._whole_rounds(M, 4096, 4096, "fake256") for M in (6500, 7491)] == [4096, 0]
+        assert L._whole_rounds(2100, 8192, 8192, "fake256") == 2048
+        assert L._whole_rounds(7491, 28672, 4096, "fake256") == 0     # its columns do not divide the units
+        assert L._whole_rounds(7491, 6144, 4096, "fake256") == 0
     finally:
         del L._units["fake256"], L._units["fake64"]
 

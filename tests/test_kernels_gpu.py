@@ -110,6 +110,36 @@ def test_gemm_f32_is_the_same_in_every_tile(N, K_):
     assert torch.equal(out.view(80, N), whole[:80])
 
 
+@pytest.mark.parametrize("M", [2049, 2148, 3000])
+def test_products_of_whole_rounds_and_the_rest(M):
+    """Rows beyond a whole round of the chip go through a second product (of one row, of few and of many):
+    the sum, the next norm and the plain product against float32 over the same operands, whose bfloat16
+    results are rounded once (2^-8 of a value at most)."""
+    from gpt_fast_amd.ops import linear as L
+    torch.manual_seed(M)
+    N = K_ = 8192
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert L._whole_rounds(M, N, K_, torch.device(DEV)) == 2048
+    x = bf(torch.randn(M, K_, device=DEV))
+    w = bf(torch.randn(N, K_, device=DEV) * 0.02)
+    ref = x.float() @ w.float().t()
+    close(L.linear(x, w), ref, 2.0 ** -8)
+
+    class Norm:
+        w = 1 + 0.1 * torch.randn(N, device=DEV)
+
+        def row_and_column_form(self):
+            return self.w, 1e-5
+    res = torch.randn(M, N, device=DEV)
+    want = res + ref
+    rows = L.linear_into(x, w, res, Norm())
+    close(res, want, 2.0 ** -8)
+    close(rows, want * torch.rsqrt((want ** 2).mean(-1, keepdim=True) + 1e-5) * Norm.w, 2.0 ** -7)
+    res = torch.zeros(M, N, device=DEV)
+    assert L.linear_into(x, w, res) is None
+    close(res, ref, 2.0 ** -8)
+
+
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 9, 16, 17, 20, 22, 24, 33, 64])
 @pytest.mark.parametrize("N,K_", [(40, 64), (136, 200), (1000, 328), (96, 4096), (77, 75)])
 def test_skinny_bf16(M, N, K_):
