@@ -648,6 +648,154 @@ __global__ __launch_bounds__(256) void rope_cache_sliced_bf16x8_kernel(
     }
 }
 
+// Both for prompts.  The first `qk_blocks` rows of the grid rotate and store q and k, RC_TOKENS tokens per
+// workgroup, so that all its threads work out angles.  The others write values: in a page these lie as groups
+// of eight keys per dim, so where the eight tokens of a group are all there one thread takes eight dims of
+// them and stores 16 bytes per dim; other tokens' values leave element by element.  As 2-byte stores, a token
+// at a time, the values took more than half of the kernel: neighbouring tokens' workgroups run on different
+// XCDs, which then all write the same lines.  Heads as in the 8B shape, before and now: 401 tokens 7.3 -> 6.3 us,
+// 2,048 21.5 -> 15.9 (50 MB), 7,491 65 -> 42, six prompts of 2,696 tokens together 26.2 -> 18.5; two slices of
+// 640 12.4 -> 11.1, of 2,048 30.4 -> 27.3.
+template <bool SLICED>
+__device__ __forceinline__ void rope_eight(const void* __restrict__ qkv, int S, size_t slice, size_t at, float (&v)[8]) {
+    if (SLICED) {
+        const float* src = (const float*)qkv + at;
+        const float4 a = *(const float4*)src, b = *(const float4*)(src + 4);
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+        for (int s = 1; s < S; ++s) {
+            const float4 c = *(const float4*)(src + s * slice), d = *(const float4*)(src + s * slice + 4);
+            v[0] += c.x; v[1] += c.y; v[2] += c.z; v[3] += c.w; v[4] += d.x; v[5] += d.y; v[6] += d.z; v[7] += d.w;
+        }
+    } else {
+        const uint4 u = *(const uint4*)((const bf16_t*)qkv + at);
+        const uint32_t* w = (const uint32_t*)&u;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            v[2 * p] = __uint_as_float(w[p] << 16);
+            v[2 * p + 1] = __uint_as_float(w[p] & 0xffff0000u);
+        }
+    }
+}
+__device__ __forceinline__ uint4 rope_pack(const float (&v)[8]) {      // exact for what was bfloat16 before
+    uint32_t o[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) o[p] = (uint32_t)float_to_bf16(v[2 * p]) | ((uint32_t)float_to_bf16(v[2 * p + 1]) << 16);
+    return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+#define RC_TOKENS 4
+#define RC_VALUE_TOKENS 2
+template <bool SLICED>
+__global__ __launch_bounds__(256) void rope_cache_rows_kernel(
+        const void* __restrict__ qkv, int S, size_t slice, bf16_t* __restrict__ q_out,
+        bf16_t* __restrict__ k_pages, bf16_t* __restrict__ v_pages, const float* __restrict__ freqs,
+        const int* __restrict__ tok_seq, const int* __restrict__ tok_pos,
+        const int* __restrict__ table, int table_stride, int n_tokens, int H, int Hkv, int hd, int rot, int qk_blocks) {
+    const int per_head = hd / 8;
+    const size_t width = (size_t)(H + 2 * Hkv) * hd;
+    if ((int)blockIdx.y >= qk_blocks) {
+        const int v_chunks = Hkv * per_head;
+        const int teams = v_chunks < 256 ? 256 / v_chunks : 1;   // groups of threads that take tokens of their own
+        const int team = threadIdx.x / (v_chunks < 256 ? v_chunks : 256);
+        if (team >= teams) return;
+        const int block = (blockIdx.x * (gridDim.y - qk_blocks) + blockIdx.y - qk_blocks) * RC_VALUE_TOKENS;
+        for (int n = block + team; n < block + RC_VALUE_TOKENS && n < n_tokens; n += teams) {
+            const int pos = tok_pos[n], seq = tok_seq[n];
+            // a group of eight keys that is there whole is its first token's
+            const int first = n - pos % 8;
+            bool whole = first >= 0 && first + 7 < n_tokens && hd % 16 == 0 && (uintptr_t)v_pages % 16 == 0;
+            for (int t = 0; whole && t < 8; ++t)
+                whole = tok_seq[first + t] == seq && tok_pos[first + t] == pos - pos % 8 + t;
+            if (whole && n != first) continue;
+            const int page = table[(size_t)seq * table_stride + pos / GFA_PAGE], off = pos % GFA_PAGE;
+            for (int c = threadIdx.x - team * v_chunks; c < v_chunks; c += 256) {
+                const int g = c / per_head, d0 = (c - g * per_head) * 8;
+                const size_t at = (size_t)n * width + (size_t)(H + Hkv + g) * hd + d0;
+                if (whole) {
+                    uint4 row[8];
+#pragma unroll
+                    for (int t = 0; t < 8; ++t) {
+                        float v[8];
+                        rope_eight<SLICED>(qkv, S, slice, at + t * width, v);
+                        row[t] = rope_pack(v);
+                    }
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        uint32_t o[4];
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) {
+                            const uint32_t lo = ((const uint32_t*)&row[2 * t])[j / 2], hi = ((const uint32_t*)&row[2 * t + 1])[j / 2];
+                            o[t] = j % 2 ? (lo >> 16) | (hi & 0xffff0000u) : (lo & 0xffffu) | (hi << 16);
+                        }
+                        *(uint4*)(v_pages + value_elem(page, g, d0 + j, off, Hkv, hd)) = make_uint4(o[0], o[1], o[2], o[3]);
+                    }
+                } else {
+                    float v[8];
+                    rope_eight<SLICED>(qkv, S, slice, at, v);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        v_pages[value_elem(page, g, d0 + j, off, Hkv, hd)] = float_to_bf16(v[j]);
+                }
+            }
+        }
+        return;
+    }
+    const int n0 = blockIdx.x * RC_TOKENS;
+    const int qk_chunks = (H + Hkv) * per_head;
+    const int c = blockIdx.y * 256 + threadIdx.x;
+    extern __shared__ float cs[];                          // [RC_TOKENS][rot / 2][2]
+    for (int i = threadIdx.x; i < RC_TOKENS * (rot / 2); i += 256) {
+        const int t = i / (rot / 2);
+        const int n = n0 + t < n_tokens ? n0 + t : n_tokens - 1;
+        sincosf((float)tok_pos[n] * freqs[i - t * (rot / 2)], &cs[2 * i + 1], &cs[2 * i]);
+    }
+    __syncthreads();
+    if (c >= qk_chunks) return;
+    const int head = c / per_head, d0 = (c - head * per_head) * 8;
+    float v[RC_TOKENS][8];
+#pragma unroll
+    for (int t = 0; t < RC_TOKENS; ++t)
+        rope_eight<SLICED>(qkv, S, slice, (size_t)(n0 + t < n_tokens ? n0 + t : n_tokens - 1) * width + (size_t)head * hd + d0, v[t]);
+#pragma unroll
+    for (int t = 0; t < RC_TOKENS; ++t) {
+        const int n = n0 + t;
+        if (n >= n_tokens) break;
+        if (d0 < rot) {
+            const float* at = cs + t * rot + d0;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const float a = v[t][2 * p], b = v[t][2 * p + 1], c_ = at[2 * p], s_ = at[2 * p + 1];
+                v[t][2 * p] = fmaf(a, c_, -(b * s_));
+                v[t][2 * p + 1] = fmaf(b, c_, a * s_);
+            }
+        }
+        if (head < H) {
+            *(uint4*)(q_out + ((size_t)n * H + head) * hd + d0) = rope_pack(v[t]);
+        } else if (k_pages) {                              // one chunk of 8 dims
+            const int pos = tok_pos[n], page = table[(size_t)tok_seq[n] * table_stride + pos / GFA_PAGE];
+            *(uint4*)(k_pages + key_elem(page, head - H, pos % GFA_PAGE, d0, Hkv, hd)) = rope_pack(v[t]);
+        }
+    }
+}
+
+// From this many tokens on the kernel above is the faster one (300 tokens: 7.2 against 6.4 us, two slices of 512:
+// 10.1 against 9.4).
+static bool rope_cache_prompt(int n_tokens, bool sliced) { return n_tokens >= (sliced ? 640 : 400); }
+
+template <bool SLICED>
+static int rope_cache_launch(const void* qkv, int S, size_t slice, void* q_out, void* k_pages, void* v_pages,
+                             const float* freqs, const int* tok_seq, const int* tok_pos, const int* table,
+                             int table_stride, int n_tokens, int H, int Hkv, int hd, int rot, hipStream_t stream) {
+    const int qk_blocks = ((H + Hkv) * (hd / 8) + 255) / 256, columns = (n_tokens + RC_TOKENS - 1) / RC_TOKENS;
+    // rows of the grid for the values: every column takes RC_VALUE_TOKENS tokens in each of them
+    const int v_blocks = v_pages ? ((n_tokens + RC_VALUE_TOKENS - 1) / RC_VALUE_TOKENS + columns - 1) / columns : 0;
+    rope_cache_rows_kernel<SLICED><<<dim3(columns, qk_blocks + v_blocks), 256,
+                                     RC_TOKENS * (rot > 0 ? rot : 2) * sizeof(float), stream>>>(
+        qkv, S, slice, (bf16_t*)q_out, (bf16_t*)k_pages, (bf16_t*)v_pages, freqs, tok_seq, tok_pos, table,
+        table_stride, n_tokens, H, Hkv, hd, rot, qk_blocks);
+    return GFA_LAUNCH_RESULT();
+}
+
 // part [S, n_tokens, (H + 2 Hkv) * hd] float; interleaved pairs, hd and rot multiples of 8.
 extern "C" int gfa_rope_cache_write_sliced(const float* part, int S, void* q_out, void* k_pages,
                                            void* v_pages, const float* freqs, const int* tok_seq,
@@ -657,8 +805,11 @@ extern "C" int gfa_rope_cache_write_sliced(const float* part, int S, void* q_out
     if (n_tokens <= 0) return 0;
     if (S <= 0 || hd % 8 != 0 || rot % 8 != 0 || rot > hd || (rot > 0 && !freqs))
         return (int)hipErrorInvalidValue;
-    const dim3 grid(n_tokens, ((H + 2 * Hkv) * (hd / 8) + 255) / 256);
     const size_t slice = (size_t)n_tokens * (H + 2 * Hkv) * hd;
+    if (rope_cache_prompt(n_tokens, true))
+        return rope_cache_launch<true>(part, S, slice, q_out, k_pages, v_pages, freqs, tok_seq, tok_pos, table,
+                                       table_stride, n_tokens, H, Hkv, hd, rot, stream);
+    const dim3 grid(n_tokens, ((H + 2 * Hkv) * (hd / 8) + 255) / 256);
     rope_cache_sliced_bf16x8_kernel<<<grid, 256, (size_t)(rot > 0 ? rot : 2) * sizeof(float), stream>>>(
         part, S, slice, (bf16_t*)q_out, (bf16_t*)k_pages, (bf16_t*)v_pages, freqs, tok_seq, tok_pos,
         table, table_stride, H, Hkv, hd, rot);
@@ -672,6 +823,9 @@ extern "C" int gfa_rope_cache_write(const void* qkv, void* q_out, void* k_pages,
                                     hipStream_t stream) {
     if (n_tokens <= 0) return 0;
     if (is_bf16 && layout == 0 && hd % 8 == 0 && rot % 8 == 0) {
+        if (rope_cache_prompt(n_tokens, false))
+            return rope_cache_launch<false>(qkv, 1, 0, q_out, k_pages, v_pages, freqs, tok_seq, tok_pos, table,
+                                            table_stride, n_tokens, H, Hkv, hd, rot, stream);
         const dim3 grid8(n_tokens, ((H + 2 * Hkv) * (hd / 8) + 255) / 256);
         rope_cache_bf16x8_kernel<<<grid8, 256, (size_t)(rot > 0 ? rot : 2) * sizeof(float), stream>>>(
             (const bf16_t*)qkv, (bf16_t*)q_out, (bf16_t*)k_pages, (bf16_t*)v_pages, freqs, tok_seq,

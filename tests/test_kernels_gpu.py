@@ -110,6 +110,44 @@ def test_gemm_f32_is_the_same_in_every_tile(N, K_):
     assert torch.equal(out.view(80, N), whole[:80])
 
 
+@pytest.mark.parametrize("H,G,hd,rot", [(8, 2, 128, 128), (4, 4, 64, 32), (3, 1, 24, 8), (2, 1, 80, 80),
+                                        (20, 20, 128, 128)])
+@pytest.mark.parametrize("lens,starts", [((401,), (0,)), ((3, 5, 640, 17, 8), (61, 7, 3, 0, 56)), ((9,) * 80, range(80))])
+def test_rotation_and_cache_write_of_many_tokens(H, G, hd, rot, lens, starts):
+    """The kernel of prompts against the one of few tokens (the same rows in steps of at most 160): whole
+    groups of eight keys, groups that begin or end inside a step, neighbouring sequences.  Values are
+    copies; rotated elements may differ by one rounding of the two products' sum (2^-7 of the value, or of
+    what cancels: the pair's larger element)."""
+    g = torch.Generator().manual_seed(hd + H)
+    n, B, W = sum(lens), len(lens), (max(l + s for l, s in zip(lens, starts)) + 63) // 64
+    table = torch.randperm(B * W, generator=g).int().view(B, W).to(DEV)
+    seq = torch.cat([torch.full((l,), b) for b, l in enumerate(lens)]).int().to(DEV)
+    pos = torch.cat([torch.arange(s, s + l) for s, l in zip(starts, lens)]).int().to(DEV)
+    freqs = (10000.0 ** (-torch.arange(rot // 2) * 2.0 / rot)).to(DEV)
+    width = (H + 2 * G) * hd
+    qkv, part = bf(torch.randn(n, width, generator=g)).to(DEV), torch.randn(2, n, width, generator=g).to(DEV)
+
+    def run(cuts, sliced):
+        pages = [torch.zeros(B * W, G, 64, hd, device=DEV, dtype=torch.bfloat16),
+                 torch.zeros(B * W, G, hd, 64, device=DEV, dtype=torch.bfloat16)]
+        qs = []
+        for a, b in zip(cuts, cuts[1:]):
+            maps = (freqs, seq[a:b].contiguous(), pos[a:b].contiguous(), table, *pages, H, G, hd, rot)
+            qs.append(K().rope_cache_write_sliced(part[:, a:b].contiguous(), *maps) if sliced
+                      else K().rope_cache_write(qkv[a:b].contiguous(), *maps, 0))
+        return [torch.cat(qs), *pages]
+    few = list(range(0, n, 160)) + [n]
+    for sliced in (False, True):
+        if sliced and n < 640:
+            continue
+        (q1, k1, v1), (q2, k2, v2) = run([0, n], sliced), run(few, sliced)
+        assert torch.equal(v1, v2)
+        most = float(qkv.abs().max() if not sliced else part.sum(0).abs().max())
+        for a, b in ((q1, q2), (k1, k2)):
+            assert float((a.float() - b.float()).abs().max()) <= 2.0 ** -7 * most
+            assert float((a != b).float().mean()) < 0.05
+
+
 @pytest.mark.parametrize("M", [2049, 2148, 3000])
 def test_products_of_whole_rounds_and_the_rest(M):
     """Rows beyond a whole round of the chip go through a second product (of one row, of few and of many):
