@@ -19,6 +19,8 @@ from typing import Optional
 
 import torch
 
+from . import gemm_bf16, gemm_wide_bf16
+from . import gemm_tiled_bf16 as T
 from . import kernels as K
 from .library import KernelError
 
@@ -47,17 +49,12 @@ def _own_gate_is_faster(M: int, inner: int, K_: int, device) -> bool:
     wins by 5-7 us up to 48 rows (inner 14336: 46-52 us against 52-59), and at more rows only
     where every compute unit has a workgroup and a half or more (inner 28672: 173 against 192
     us at 64 rows, while inner 14336 loses 55 to 51)."""
-    if K_ % 8 or not 16 < M <= _wide().MAX_ROWS:
+    if K_ % 8 or not 16 < M <= gemm_wide_bf16.MAX_ROWS:
         return False
     wgs, cus = (inner + 63) // 64, _compute_units(device)
     if wgs * 5 < cus * 4:
         return False
     return M <= 48 or wgs * 2 >= cus * 3
-
-
-def _fast():
-    from . import gemm_bf16
-    return gemm_bf16
 
 
 # From this many rows on (up to 64), a product reads its weights from a second copy kept in the
@@ -71,7 +68,6 @@ TILED_FROM_ROWS = 17
 
 def _tiled_for(rows: int, w: torch.Tensor, gate: bool = False):
     """The tiled form of ``w`` if a product of this many rows should use it, else None."""
-    from . import gemm_tiled_bf16 as T
     if rows < TILED_FROM_ROWS or not T.takes(rows, w.shape[1]) or w.dtype != torch.bfloat16:
         return None
     return T.tiled_of(w, gate)
@@ -180,7 +176,7 @@ class SlicedRows:
 
     def rows(self) -> torch.Tensor:
         """[M, N] in the product's type: the slices added in order."""
-        return _wide().sum_store(self.part, self.dtype)
+        return gemm_wide_bf16.sum_store(self.part, self.dtype)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None,
@@ -189,25 +185,24 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
     ``may_stay_sliced``: the caller also takes a :class:`SlicedRows`."""
     out_dtype = out_dtype or x.dtype
     if isinstance(x, HalfNormed):
-        return _fast().skinny_after_chain(x.xg, x.ssq, x.eps, w, out_dtype=out_dtype)
+        return gemm_bf16.skinny_after_chain(x.xg, x.ssq, x.eps, w, out_dtype=out_dtype)
     if x.dtype == torch.float32:
         if out_dtype != torch.float32:
             raise KernelError("a float32 product has a float32 result")
         return K.gemm_f32(x, w)
     M = x.shape[0]
     if M <= SKINNY_MAX_ROWS:
-        return _fast().skinny(x, w, out_dtype=out_dtype)
+        return gemm_bf16.skinny(x, w, out_dtype=out_dtype)
     # the kernel that adds a sliced product's partial sums stores four columns at a time
     t = _tiled_for(M, w) if out_dtype == torch.float32 or w.shape[0] % 4 == 0 else None
     if t is not None:
-        from . import gemm_tiled_bf16 as T
         if out_dtype == torch.float32:
             return T.product_f32(x, t)
         rows = SlicedRows(T.partial_sums(x, t), out_dtype)
         return rows if may_stay_sliced else rows.rows()
     if out_dtype == torch.float32:
-        return _fast().wide_f32_out(x, w)
-    if M > _wide().MAX_ROWS and w.shape[0] % 4 == 0 and x.is_contiguous() and w.is_contiguous():
+        return gemm_bf16.wide_f32_out(x, w)
+    if M > gemm_wide_bf16.MAX_ROWS and w.shape[0] % 4 == 0 and x.is_contiguous() and w.is_contiguous():
         S = _library_slices(M, w.shape[0], x.shape[1], x.device)
         if S > 1:
             rows = SlicedRows(_library_partial_sums(x, w, S), out_dtype)
@@ -232,17 +227,16 @@ def linear_into(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor, then_n
     form = getattr(then_norm, "row_and_column_form", None)
     if _chains(x.shape[0], x.dtype, w, then_norm, takes_halves):
         weight, eps = form()
-        xg, ssq = _fast().skinny_into_chain(x, w, residual, weight)
+        xg, ssq = gemm_bf16.skinny_into_chain(x, w, residual, weight)
         return HalfNormed(xg, ssq, eps)
     if x.dtype == torch.bfloat16 and x.shape[0] > SKINNY_MAX_ROWS:
         weight, eps = form() if form is not None else (None, 0.0)
         t = _tiled_for(x.shape[0], w) if w.shape[0] % 4 == 0 and w.shape[0] <= 16384 else None
         if t is not None:
-            from . import gemm_tiled_bf16 as T
-            return _wide().sum_add_norm(residual, T.partial_sums(x, t), weight, eps)
+            return gemm_wide_bf16.sum_add_norm(residual, T.partial_sums(x, t), weight, eps)
         if _sliced_is_faster(x.shape[0], w.shape[0], x.shape[1]):
-            return _wide().product_into(x, w, residual, weight, eps)
-        if x.shape[0] > _wide().MAX_ROWS and w.shape[0] % 4 == 0 and w.shape[0] <= 16384 \
+            return gemm_wide_bf16.product_into(x, w, residual, weight, eps)
+        if x.shape[0] > gemm_wide_bf16.MAX_ROWS and w.shape[0] % 4 == 0 and w.shape[0] <= 16384 \
                 and x.is_contiguous() and w.is_contiguous():
             first = _whole_rounds(x.shape[0], w.shape[0], x.shape[1], x.device)
             if first:
@@ -262,7 +256,7 @@ def _library_into(x, w, residual, weight, eps, out=None):
     next norm's ``weight`` its rows (into ``out`` if given), else None."""
     S = _library_slices(x.shape[0], w.shape[0], x.shape[1], x.device)
     if S > 1:
-        return _wide().sum_add_norm(residual, _library_partial_sums(x, w, S), weight, eps, out)
+        return gemm_wide_bf16.sum_add_norm(residual, _library_partial_sums(x, w, S), weight, eps, out)
     if weight is not None:
         return K.add_rmsnorm(residual, torch.matmul(x, w.t()), weight, eps, out)
     K.add_into(residual, torch.matmul(x, w.t()))
@@ -275,9 +269,9 @@ def linear_terms(x: torch.Tensor, w: torch.Tensor):
     product for these rows leaves."""
     if x.dtype == torch.float32 or x.shape[0] <= SKINNY_MAX_ROWS:
         return linear(x, w, out_dtype=torch.float32)
-    if x.shape[0] <= _wide().MAX_ROWS and w.shape[0] % 4 == 0 and _tiled_for(x.shape[0], w) is None \
+    if x.shape[0] <= gemm_wide_bf16.MAX_ROWS and w.shape[0] % 4 == 0 and _tiled_for(x.shape[0], w) is None \
             and _sliced_is_faster(x.shape[0], w.shape[0], x.shape[1]):
-        return _wide().partial_sums(x, w)
+        return gemm_wide_bf16.partial_sums(x, w)
     rows = linear(x, w, may_stay_sliced=True)
     return rows.part if isinstance(rows, SlicedRows) else rows
 
@@ -293,27 +287,22 @@ def _chains(rows: int, dtype, w, then_norm, takes_halves: bool) -> bool:
     ``then_norm`` for a reader that takes it in halves."""
     return (takes_halves and dtype == torch.bfloat16
             and getattr(then_norm, "row_and_column_form", None) is not None
-            and _fast().can_chain_norm(rows, w.shape[0], w.shape[1])
+            and gemm_bf16.can_chain_norm(rows, w.shape[0], w.shape[1])
             and _tiled_for(rows, w) is None)        # with the second copy, 17..24 rows go there
-
-
-def _wide():
-    from . import gemm_wide_bf16
-    return gemm_wide_bf16
 
 
 def _sliced_is_faster(M: int, N: int, K_: int) -> bool:
     """17..64 rows times a matrix with few rows and a long inner size (the feed-forward's
     second product): the hand-written kernel cuts K into slices over many workgroups where
     the vendor library runs few; measured faster from an inner size of twice the width."""
-    return M <= _wide().MAX_ROWS and K_ % 8 == 0 and N % 4 == 0 and N <= 16384 and K_ >= 2 * N
+    return M <= gemm_wide_bf16.MAX_ROWS and K_ % 8 == 0 and N % 4 == 0 and N <= 16384 and K_ >= 2 * N
 
 
 def _linear_into(x, w, residual):
     if x.dtype == torch.float32:
         return K.gemm_f32(x, w, out=residual, accumulate=True)
     if x.shape[0] <= SKINNY_MAX_ROWS:
-        return _fast().skinny(x, w, residual=residual)
+        return gemm_bf16.skinny(x, w, residual=residual)
     return K.add_into(residual, torch.matmul(x, w.t()))
 
 
@@ -334,20 +323,19 @@ def gated_linear(x: torch.Tensor, w13: torch.Tensor, activation: str = "silu",
             return K.gate_mul_sums(linear(x, w13, out_dtype=torch.float32), activation, limit)
         return K.gate_mul(linear(x, w13), activation, limit=limit)
     if isinstance(x, HalfNormed):
-        return _fast().skinny_after_chain_gated(x.xg, x.ssq, x.eps, w13, activation=activation)
+        return gemm_bf16.skinny_after_chain_gated(x.xg, x.ssq, x.eps, w13, activation=activation)
     if x.dtype == torch.float32:
         return K.gate_mul(K.gemm_f32(x, w13), activation)
     if x.shape[0] <= SKINNY_MAX_ROWS:
-        return _fast().skinny_gated(x, w13, activation=activation)
+        return gemm_bf16.skinny_gated(x, w13, activation=activation)
     if activation != "silu":
         # beyond sixteen rows only silu has kernels with the gate in their epilogue
         return K.gate_mul(linear(x, w13), activation)
     t = _tiled_for(x.shape[0], w13, gate=True) if w13.shape[0] % 2 == 0 else None
     if t is not None:
-        from . import gemm_tiled_bf16 as T
         return T.product_gated(x, t)
     if w13.shape[0] % 2 == 0 and _own_gate_is_faster(x.shape[0], w13.shape[0] // 2, x.shape[1], x.device):
-        return _wide().product_gated(x, w13)
+        return gemm_wide_bf16.product_gated(x, w13)
     return K.silu_mul(torch.matmul(x, w13.t()))
 
 
@@ -359,7 +347,7 @@ def gated_into(x, w13: torch.Tensor, w2: torch.Tensor, residual: torch.Tensor, t
     in (``gemm_bf16.ChunkedRows``)."""
     if isinstance(x, HalfNormed) and activation != "clamped_swish" \
             and _chains(x.shape[0], x.dtype, w2, then_norm, takes_halves):
-        h = _fast().skinny_after_chain_gated(x.xg, x.ssq, x.eps, w13, chunked=True,
+        h = gemm_bf16.skinny_after_chain_gated(x.xg, x.ssq, x.eps, w13, chunked=True,
                                              activation=activation)
     else:
         h = gated_linear(x, w13, activation, limit)
@@ -380,7 +368,7 @@ def qkv_rope_store(x, wqkv, freqs, tok_seq, tok_pos, table, k_pages, v_pages, n_
     """q [M, H, hd] of normed rows ``x`` (a tensor or a :class:`HalfNormed`) through the fused
     projection / rotation / cache-write kernel."""
     if isinstance(x, HalfNormed):
-        return _fast().qkv_rope_store(x.xg, wqkv, freqs, tok_seq, tok_pos, table, k_pages, v_pages,
+        return gemm_bf16.qkv_rope_store(x.xg, wqkv, freqs, tok_seq, tok_pos, table, k_pages, v_pages,
                                       n_heads, n_kv_heads, head_dim, rotary_dim, ssq=x.ssq, eps=x.eps)
-    return _fast().qkv_rope_store(x, wqkv, freqs, tok_seq, tok_pos, table, k_pages, v_pages,
+    return gemm_bf16.qkv_rope_store(x, wqkv, freqs, tok_seq, tok_pos, table, k_pages, v_pages,
                                   n_heads, n_kv_heads, head_dim, rotary_dim)
