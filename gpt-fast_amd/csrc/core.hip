@@ -779,8 +779,10 @@ __global__ __launch_bounds__(256) void rope_cache_rows_kernel(
 }
 
 // From this many tokens on the kernel above is the faster one (300 tokens: 7.2 against 6.4 us, two slices of 512:
-// 10.1 against 9.4).
-static bool rope_cache_prompt(int n_tokens, bool sliced) { return n_tokens >= (sliced ? 640 : 400); }
+// 10.1 against 9.4), where the angles of its tokens fit into shared memory.
+static bool rope_cache_prompt(int n_tokens, int rot, bool sliced) {
+    return n_tokens >= (sliced ? 640 : 400) && RC_TOKENS * rot * sizeof(float) <= 32 * 1024;
+}
 
 template <bool SLICED>
 static int rope_cache_launch(const void* qkv, int S, size_t slice, void* q_out, void* k_pages, void* v_pages,
@@ -806,7 +808,7 @@ extern "C" int gfa_rope_cache_write_sliced(const float* part, int S, void* q_out
     if (S <= 0 || hd % 8 != 0 || rot % 8 != 0 || rot > hd || (rot > 0 && !freqs))
         return (int)hipErrorInvalidValue;
     const size_t slice = (size_t)n_tokens * (H + 2 * Hkv) * hd;
-    if (rope_cache_prompt(n_tokens, true))
+    if (rope_cache_prompt(n_tokens, rot, true))
         return rope_cache_launch<true>(part, S, slice, q_out, k_pages, v_pages, freqs, tok_seq, tok_pos, table,
                                        table_stride, n_tokens, H, Hkv, hd, rot, stream);
     const dim3 grid(n_tokens, ((H + 2 * Hkv) * (hd / 8) + 255) / 256);
@@ -823,7 +825,7 @@ extern "C" int gfa_rope_cache_write(const void* qkv, void* q_out, void* k_pages,
                                     hipStream_t stream) {
     if (n_tokens <= 0) return 0;
     if (is_bf16 && layout == 0 && hd % 8 == 0 && rot % 8 == 0) {
-        if (rope_cache_prompt(n_tokens, false))
+        if (rope_cache_prompt(n_tokens, rot, false))
             return rope_cache_launch<false>(qkv, 1, 0, q_out, k_pages, v_pages, freqs, tok_seq, tok_pos, table,
                                             table_stride, n_tokens, H, Hkv, hd, rot, stream);
         const dim3 grid8(n_tokens, ((H + 2 * Hkv) * (hd / 8) + 255) / 256);
