@@ -1,4 +1,5 @@
-// The tile kernel of products with many rows: out = x W^T in bfloat16 with float32 sums.
+// The tile kernel of the experts' products with many rows: out = x W[e]^T in bfloat16 with float32 sums, the
+// rows of x being sorted by expert.
 //
 // A workgroup of four waves makes a tile of 64 TM rows of x by 64 TN rows of W, each wave a quarter
 // (32 TM x 32 TN) with v_mfma_f32_32x32x16_bf16, formed transposed (A = W, B = x) so that a lane ends with
@@ -9,15 +10,14 @@
 // row so that operand reads have no bank conflicts.
 //
 // What bounds it is the path into a compute unit, not the arithmetic: at 256 x 256 a piece takes 2,048
-// cycles of the matrix units and 64 KB of copies.  Hence, measured on 2,048 x 28,672 x 4,096 and, in
-// brackets, 2,048 x 4,096 x 14,336 (128 tiles):
+// cycles of the matrix units and 64 KB of copies.  Hence:
 //  * operands of the next 16 k are read between the products of this one, one read per two products, and
 //    the one barrier of a piece stands before its last 16 k, so that nothing waits behind it;
 //  * copies are spread over three of a piece's four steps instead of issued in a burst (a burst fills the
 //    address unit and holds the products up);
-//  * lines are asked for two pieces before they are copied, each by one of the workgroups of an XCD that
-//    share them (one dword of 64 lines per instruction, into shared memory that nobody reads), so that the
-//    copies themselves find them in that XCD's cache: 440 -> 412 us [311 -> 241].
+//  * in the tiles that fill a compute unit by themselves, lines are asked for two pieces before they are
+//    copied (one dword of 64 lines per instruction, into shared memory that nobody reads), those of x by one of
+//    the workgroups of an XCD that share them, so that the copies find them in that XCD's cache.
 // The copies are written in asm because the compiler takes any operand read to depend on every copy in
 // flight and waits for all of them; they have no output registers, and the waits below count them.
 #pragma once
@@ -33,8 +33,8 @@ union PtFrag {
 };
 
 enum PtMode {
-    PT_ROWS = 0,        // bfloat16 rows [M, N] of the sums, or of act(sum)
-    PT_GATE = 1,        // W: F gate rows, then F up rows; bfloat16 [M, F] of act(gate) * up
+    PT_ROWS = 0,        // bfloat16 rows [pairs, F] of the sums, or of act(sum)
+    PT_GATE = 1,        // W: F gate rows, then F up rows; bfloat16 [pairs, F] of act(gate) * up
 };
 
 // act < 0: none; 0 silu, 1 gelu (tanh form), 3 gelu (exact); as a gate also 2: a sigmoid(1.702 a) (b + 1) of
@@ -43,12 +43,11 @@ struct PtArgs {
     const bf16_t* x;
     const bf16_t* w;
     void* out;
-    int M, N, K;                        // N: rows of W (PT_GATE: 2 F); K: a multiple of 64
-    int n_begin, n_end;                 // the columns of out that this launch makes
+    int F, K;                           // columns of out, a multiple of 8; a multiple of 64
     int act;
     float limit;
-    // experts: rows offsets[e] .. offsets[e + 1] - 1 are those of expert e, row p being row order[p] / top of x (or
-    // p), W [E, N, K]; tiles of rows do not cross experts
+    // rows offsets[e] .. offsets[e + 1] - 1 are those of expert e, row p being row order[p] / top of x (or p),
+    // W [E, F or 2 F, K]; tiles of rows do not cross experts
     const int* order;
     const int* offsets;
     int top, E;
@@ -152,7 +151,7 @@ __device__ __forceinline__ void pt_find_tile(const int* __restrict__ offsets, in
 #define PT_WAVES 4
 #define PT_AS3(p) ((__attribute__((address_space(3))) void*)(p))
 
-template <int TM, int TN, int MODE, bool EXPERT>
+template <int TM, int TN, int MODE>
 __global__ __launch_bounds__(PT_WAVES * 64, (TM + TN) * 64 * 256 <= 79 * 1024 ? 2 : 1)
 void prompt_tile_kernel(const PtArgs g) {
     constexpr int BM = 64 * TM, BN = 64 * TN;
@@ -161,12 +160,12 @@ void prompt_tile_kernel(const PtArgs g) {
     // asking ahead pays where no second workgroup shares the compute unit (1,777 tokens of 32 experts, W 3,584 x
     // 4,096: tiles of 256 x 256 374 -> 368 us, 256 x 128 409 -> 384, but 128 x 128 368 -> 432)
     constexpr bool ASK = (BM + BN) * 256 > 80 * 1024;
-    constexpr int G = EXPERT ? 4 : 8;                            // row tiles that share columns of W at a time
+    constexpr int G = 4;                                         // row tiles that run through the columns together
     __shared__ __attribute__((aligned(1024))) char lds[2 * BUF + PT_WAVES * 256];
 
-    const int F = MODE == PT_GATE ? g.N / 2 : g.N;               // columns of out
+    const int F = g.F, N = MODE == PT_GATE ? 2 * F : F;          // columns of out, rows of an expert's W
     constexpr int CN = MODE == PT_GATE ? BN / 2 : BN;            // columns of out that a tile makes
-    const int mt = EXPERT ? pt_row_tiles<BM>(g.offsets, g.E) : (g.M + BM - 1) / BM, nt = (g.n_end - g.n_begin + CN - 1) / CN;
+    const int mt = pt_row_tiles<BM>(g.offsets, g.E), nt = (F + CN - 1) / CN;
     // the workgroups of one XCD (every eighth) take consecutive tiles
     const int total = mt * nt, per = (total + 7) / 8;
     const int work = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
@@ -178,34 +177,32 @@ void prompt_tile_kernel(const PtArgs g) {
     const int K = g.K;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wr = wave & 1, wc = wave >> 1;
-    int m0 = bm * BM, m1 = g.M, e = 0;
-    if (EXPERT) pt_find_tile<BM>(g.offsets, g.E, bm, e, m0, m1);
-    const int n0 = g.n_begin + bn * CN, n1 = g.n_end;
-    const bf16_t* we = g.w + (size_t)e * g.N * K;
+    int m0 = 0, m1 = 0, e = 0;
+    pt_find_tile<BM>(g.offsets, g.E, bm, e, m0, m1);
+    const int n0 = bn * CN;
+    const bf16_t* we = g.w + (size_t)e * N * K;
     // row of x and row of W that row r of the tile stands for; beyond the last one it again, never stored
     auto x_row = [&](int r) {
         const int m = m0 + r < m1 ? m0 + r : m1 - 1;
-        return EXPERT && g.order ? g.order[m] / g.top : m;
+        return g.order ? g.order[m] / g.top : m;
     };
     auto w_row = [&](int r) {
-        if (MODE != PT_GATE) return n0 + r < n1 ? n0 + r : n1 - 1;
+        if (MODE != PT_GATE) return n0 + r < F ? n0 + r : F - 1;
         const int n = n0 + (r >> 6) * 32 + (r & 31);             // 32 gate rows, then the same up rows
-        return (n < n1 ? n : n1 - 1) + ((r >> 5) & 1) * F;
+        return (n < F ? n : F - 1) + ((r >> 5) & 1) * F;
     };
 #define PT_SWIZZLE(r) (((r) >> 1) & 7)
     const int T = K / 64;                                        // pieces
     // experts begin at different pieces: their matrices are often a power of two apart, and walked in step from
     // the first piece they meet in the same memory channels (32 experts of 4,096 x 4,096, 40 tokens: 266 -> 190 us)
-    const int turn = EXPERT ? (e * 8) % T : 0;
-    const char* xp[EXPERT ? UX : 1];
-    uint32_t xo[EXPERT ? 1 : UX], wo[UW];
+    const int turn = (e * 8) % T;
+    const char* xp[UX];
+    uint32_t wo[UW];
 #pragma unroll
     for (int i = 0; i < UX; ++i) {
         const int r = (wave + PT_WAVES * i) * 8 + (lane >> 3), c = (lane & 7) ^ PT_SWIZZLE(r);
-        if (EXPERT) xp[EXPERT ? i : 0] = (const char*)(g.x + (size_t)x_row(r) * K) + c * 16;
-        else xo[EXPERT ? 0 : i] = (uint32_t)(x_row(r) - m0) * (uint32_t)(K * 2) + c * 16;
+        xp[i] = (const char*)(g.x + (size_t)x_row(r) * K) + c * 16;
     }
-    const char* xbase = (const char*)(g.x + (size_t)m0 * K);
     const int wfirst = MODE == PT_GATE ? 0 : n0;
 #pragma unroll
     for (int i = 0; i < UW; ++i) {
@@ -214,15 +211,13 @@ void prompt_tile_kernel(const PtArgs g) {
     }
     const char* wbase = (const char*)(we + (size_t)wfirst * K);
 
-    // the line (of the pieces to come) that this lane asks for: its share of the rows of W that this XCD's
-    // workgroups of the same columns read, then of the rows of x that those of the same rows read
+    // the line (of the pieces to come) that this lane asks for: one of the tile's rows of W, or its share of the
+    // rows of x that this XCD's workgroups of the same rows read
     const char* line = nullptr;
     if (ASK) {
-        const int sw = EXPERT ? 1 : group_rows >= 8 ? 8 : group_rows >= 4 ? 4 : group_rows >= 2 ? 2 : 1;
-        const int lw = BN / PT_WAVES / sw;
-        const int lx = BM / PT_WAVES / 4 < 64 - lw ? BM / PT_WAVES / 4 : 64 - lw;
+        constexpr int lw = BN / PT_WAVES, lx = BM / PT_WAVES / 4 < 64 - lw ? BM / PT_WAVES / 4 : 64 - lw;
         const int l = lane < lw + lx ? lane : 0;
-        const bf16_t* row = l < lw ? we + (size_t)w_row((bm % sw) * (BN / sw) + wave * lw + l) * K
+        const bf16_t* row = l < lw ? we + (size_t)w_row(wave * lw + l) * K
                                    : g.x + (size_t)x_row((bn & 3) * (BM / 4) + wave * (BM / 16) + (l - lw)) * K;
         line = (const char*)row;
     }
@@ -233,13 +228,12 @@ void prompt_tile_kernel(const PtArgs g) {
         const uint32_t to = __builtin_amdgcn_readfirstlane(lds_at + (b) * BUF + (X ? 0 : XB) + \
                             (wave + PT_WAVES * (X ? (i) : (i) - UX)) * 1024); \
         const size_t at = (size_t)(uint32_t)__builtin_amdgcn_readfirstlane((t) + turn < T ? (t) + turn : (t) + turn - T) * 128; \
-        if (X && EXPERT) \
+        if (X) \
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" \
-                         :: "s"(to), "v"(xp[X && EXPERT ? (i) : 0] + at) : "memory", "m0"); \
+                         :: "s"(to), "v"(xp[X ? (i) : 0] + at) : "memory", "m0"); \
         else \
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" \
-                         :: "s"(to), "v"(X ? xo[X && !EXPERT ? (i) : 0] : wo[X ? 0 : (i) - UX]), \
-                            "s"((X ? xbase : wbase) + at) : "memory", "m0"); \
+                         :: "s"(to), "v"(wo[X ? 0 : (i) - UX]), "s"(wbase + at) : "memory", "m0"); \
     } while (0)
 #define PT_ASK(t) do { if (ASK) { \
         const int piece = ((t) < T ? (t) : T - 1) + turn; \
@@ -340,7 +334,7 @@ void prompt_tile_kernel(const PtArgs g) {
             } else {
                 pt_act(z, g.act);
             }
-            if (m < m1 && n < n1) {                              // n_begin, n_end and F are multiples of eight
+            if (m < m1 && n < F) {                               // F is a multiple of eight
                 const uint4 v = make_uint4((uint32_t)float_to_bf16(z[0]) | ((uint32_t)float_to_bf16(z[1]) << 16),
                                            (uint32_t)float_to_bf16(z[2]) | ((uint32_t)float_to_bf16(z[3]) << 16),
                                            (uint32_t)float_to_bf16(z[4]) | ((uint32_t)float_to_bf16(z[5]) << 16),

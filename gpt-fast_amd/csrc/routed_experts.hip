@@ -877,17 +877,17 @@ extern "C" int gfa_expert_tile_product(const void* x, const int* order, int top,
     return GFA_LAUNCH_RESULT();
 }
 
-// The same product for inner sizes of whole pieces of 64 and rows of out of whole 16 bytes, by the tile kernel
-// of prompt_tile.h, which finds its tiles in `offsets` itself.
+// The same product for inner sizes of whole pieces of 64 and rows of out of whole 16 bytes, by the tile kernel of
+// prompt_tile.h, which finds its tiles in `offsets` itself; the kernel above serves the other sizes.
 template <int TM, int TN>
 static int expert_rows_launch(const PtArgs& a, int mode, int pairs, hipStream_t stream) {
     const int cols = mode >= 2 ? 32 * TN : 64 * TN;
     const long long row_tiles = pairs / (64 * TM) + (a.E < pairs ? a.E : pairs);       // at most
-    const long long total = row_tiles * ((a.n_end + cols - 1) / cols);
+    const long long total = row_tiles * ((a.F + cols - 1) / cols);
     if (total > 0x7ffffff0LL) return (int)hipErrorInvalidValue;
     const unsigned grid = (unsigned)((total + 7) / 8 * 8);
-    if (mode >= 2) prompt_tile_kernel<TM, TN, PT_GATE, true><<<grid, 256, 0, stream>>>(a);
-    else prompt_tile_kernel<TM, TN, PT_ROWS, true><<<grid, 256, 0, stream>>>(a);
+    if (mode >= 2) prompt_tile_kernel<TM, TN, PT_GATE><<<grid, 256, 0, stream>>>(a);
+    else prompt_tile_kernel<TM, TN, PT_ROWS><<<grid, 256, 0, stream>>>(a);
     return GFA_LAUNCH_RESULT();
 }
 
@@ -896,7 +896,7 @@ extern "C" int gfa_expert_rows_product(const void* x, const int* order, int top,
                                        int act, float limit, hipStream_t stream) {
     if (pairs <= 0) return 0;
     const long long matrix = (long long)(mode >= 2 ? 2 : 1) * F * K * 2;
-    if (E <= 0 || F <= 0 || F % 8 || K <= 0 || K % 64 || top <= 0 || mode < 0 || mode > 3 ||
+    if (E <= 0 || E > 8192 || F <= 0 || F % 8 || K <= 0 || K % 64 || top <= 0 || mode < 0 || mode > 3 ||
         (act != 0 && act != 1 && act != 3) || matrix > 0xffffffffLL || (uintptr_t)x % 16 || (uintptr_t)w % 16 ||
         (uintptr_t)out % 16)
         return (int)hipErrorInvalidValue;
@@ -904,11 +904,8 @@ extern "C" int gfa_expert_rows_product(const void* x, const int* order, int top,
     a.x = (const bf16_t*)x;
     a.w = (const bf16_t*)w;
     a.out = out;
-    a.M = pairs;
-    a.N = mode >= 2 ? 2 * F : F;
+    a.F = F;
     a.K = K;
-    a.n_begin = 0;
-    a.n_end = F;
     a.act = mode == 0 ? -1 : mode == 3 ? 2 : act;
     a.limit = limit;
     a.order = order;
