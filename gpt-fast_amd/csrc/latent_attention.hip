@@ -16,10 +16,13 @@
 #include "common.h"
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 la_bf16x8_t;
+typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 la_bf16x2_t;
+typedef __attribute__((__vector_size__(2 * sizeof(float)))) float la_floatx2_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float la_floatx4_t;
 union LAFrag {
     uint4 u;
     bf16_t e[8];
+    la_bf16x2_t p[4];
     la_bf16x8_t v;
 };
 
@@ -50,24 +53,27 @@ __device__ __forceinline__ float la_sum_lane_groups(float v) {
 template <int NT, int DK, int DVT>
 __device__ __forceinline__ void la_copy(const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
                                         int page, int bi, int hd, int vd, char* kbuf, char* vbuf) {
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    // addresses are a scalar part and 16 bytes a lane, made anew for every block: kept over the loop they took
+    // the registers of the products
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
     const char* ks = (const char*)(k_pages + cache_region(page, 0, 1, hd)) + (size_t)(bi & 1) * 64 * hd;
     const char* vs = (const char*)(v_pages + cache_region(page, 0, 1, vd)) + (size_t)(bi & 1) * 1024;
 #pragma unroll
     for (int i = 0; i < (DK * 128 + NT - 1) / NT; ++i) {
-        const int u = tid + i * NT;
-        if (u < 4 * hd)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(ks + (size_t)u * 16),
-                                             (__attribute__((address_space(3))) void*)(kbuf + wave * 1024 + i * NT * 16),
-                                             16, 0, 0);
+        const int u = wave * 64 + i * NT;
+        if (lane < 4 * hd - u)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(ks + (size_t)u * 16 + lane * 16),
+                                             (__attribute__((address_space(3))) void*)(kbuf + u * 16), 16, 0, 0);
     }
 #pragma unroll
     for (int i = 0; i < (DVT * 64 + NT - 1) / NT; ++i) {
-        const int u = tid + i * NT;
+        const int u = wave * 64 + i * NT;                        // vd / 16 pieces of 64
         if (u < 4 * vd)
             __builtin_amdgcn_global_load_lds(
-                (const __attribute__((address_space(1))) void*)(vs + (size_t)(u >> 6) * 2048 + (u & 63) * 16),
-                (__attribute__((address_space(3))) void*)(vbuf + wave * 1024 + i * NT * 16), 16, 0, 0);
+                (const __attribute__((address_space(1))) void*)(vs + (size_t)(u >> 6) * 2048 + lane * 16),
+                (__attribute__((address_space(3))) void*)(vbuf + u * 16), 16, 0, 0);
     }
 }
 
@@ -79,9 +85,11 @@ __device__ __forceinline__ void la_landed(int bi, int last, int vd, char* vbuf) 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     const int ok = last - bi * 32;                     // keys 0 .. ok of the block count
     if (ok >= 31) return;
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
 #pragma unroll
     for (int i = 0; i < (DVT * 64 + NT - 1) / NT; ++i) {
-        const int u = threadIdx.x + i * NT, first = ((u >> 4) & 3) * 8;
+        const int u = tid + i * NT, first = ((u >> 4) & 3) * 8;
         if (u < 4 * vd && first + 7 > ok) {
             LAFrag f;
             f.u = *(const uint4*)(vbuf + (size_t)u * 16);
@@ -115,9 +123,11 @@ struct LATile {
         l = 0.f;
     }
 
-    // FULL: hd and vd are exactly the sizes of the template
+    // FULL: hd and vd are the sizes of the template, or the buffers are zero behind them; whole: every row of the
+    // wave sees the whole block
     template <bool FULL>
-    __device__ __forceinline__ void block(int bi, const char* kt, const char* vt, int hd, int vd, float scale_log2) {
+    __device__ __forceinline__ void block(int bi, const char* kt, const char* vt, int hd, int vd, float scale_log2,
+                                          bool whole = false) {
         const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
         const int chunks = hd >> 3, vtiles = vd >> 4;
         la_floatx4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
@@ -138,7 +148,8 @@ struct LATile {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int j = key0 + e;
-            sv[e] = (j <= pos && j >= lo) ? sv[e] * scale_log2 : -INFINITY;
+            sv[e] *= scale_log2;
+            if (!whole) sv[e] = (j <= pos && j >= lo) ? sv[e] : -INFINITY;
             mx = fmaxf(mx, sv[e]);
         }
         mx = la_max_lane_groups(mx);
@@ -154,10 +165,11 @@ struct LATile {
         const float ref = m == -INFINITY ? 0.f : m;
         LAFrag pf;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float p = exp2f(sv[e] - ref);
-            l += p;
-            pf.e[e] = float_to_bf16(p);
+        for (int e = 0; e < 8; e += 2) {
+            const la_floatx2_t p = {exp2f(sv[e] - ref), exp2f(sv[e + 1] - ref)};
+            l += p[0];
+            l += p[1];
+            pf.p[e / 2] = __builtin_convertvector(p, la_bf16x2_t);
         }
         const char* vl = vt + lane * 16;
 #pragma unroll
@@ -178,8 +190,16 @@ __device__ __forceinline__ void la_store4(bf16_t* dst, float a, float b, float c
 // Prompts and portions: eight waves, a tile of sixteen rows each; one workgroup per 128 rows of a
 // sequence, those with the most keys first.  The copies of the next block run while this one is
 // multiplied; one barrier a block.  grid (tiles of 128 rows, 1, sequences).
+//
+// At a latent of 512 a wave's queries and O^T are 200 of its 256 registers.  The buffers' ends beyond hd and vd are
+// zeroed once, so that one form serves every size up to the template's: a choice per read instead took registers
+// that were not there, and reading them back from scratch in the loop waited for the copies in flight as well.
+// Microseconds before and now (32 heads, 1,777 tokens): 512 / 512 325 -> 178, 576 / 512 204 -> 175; 16 heads 192 / 128
+// 78 -> 71, 320 / 256 107 -> 98.  What is left is the blocks' way out of shared memory (every wave reads all of a
+// block, 544 KB per block and compute unit at 576 / 512) and the softmax between the products; tiles of 32 rows
+// shared by two waves, which read half as much, took 198, 208, 92 and 114 for the exchange of their sums.
 #define LA_WAVES 8
-template <int DK, int DVT, bool FULL>
+template <int DK, int DVT>
 __global__ __launch_bounds__(LA_WAVES * 64, 2) void latent_prompt_kernel(
         const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages,
         const int* __restrict__ q_start, const int* __restrict__ start_pos, const int* __restrict__ table,
@@ -213,15 +233,22 @@ __global__ __launch_bounds__(LA_WAVES * 64, 2) void latent_prompt_kernel(
     const int w_end = row0 + 16 < rows_total ? row0 + 16 : rows_total;
     const int w_lo = row0 < rows_total ? first_seen(spos + row0 / s.H) >> 5 : 0;
     const int w_hi = row0 < rows_total ? (spos + (w_end - 1) / s.H) >> 5 : -1;
+    // of those, the ones that all its rows see whole
+    const int w_all = (first_seen(spos + (w_end - 1) / s.H) + 31) >> 5, w_whole = ((spos + row0 / s.H + 1) >> 5) - 1;
 
     la_copy<NT, DK, DVT>(k_pages, v_pages, pages[b_lo >> 1], b_lo, s.hd, s.vd, kb0, vb0);
+    for (int u = 4 * s.hd + threadIdx.x; u < DK * 128; u += NT)
+        *(uint4*)(kb0 + u * 16) = *(uint4*)(kb1 + u * 16) = make_uint4(0, 0, 0, 0);
+    for (int u = 4 * s.vd + threadIdx.x; u < DVT * 64; u += NT)
+        *(uint4*)(vb0 + u * 16) = *(uint4*)(vb1 + u * 16) = make_uint4(0, 0, 0, 0);
 #define LA_STEP(B, K, V, KN, VN)                                                                        \
     {                                                                                                   \
         la_landed<NT, DVT>(B, wg_last, s.vd, V);                                                        \
         __syncthreads();               /* block B is whole, and nobody reads the other buffers any more */ \
         if ((B) + 1 <= b_hi)                                                                            \
             la_copy<NT, DK, DVT>(k_pages, v_pages, pages[((B) + 1) >> 1], (B) + 1, s.hd, s.vd, KN, VN); \
-        if ((B) >= w_lo && (B) <= w_hi) t.template block<FULL>(B, K, V, s.hd, s.vd, s.scale_log2);      \
+        if ((B) >= w_lo && (B) <= w_hi) t.template block<true>(B, K, V, s.hd, s.vd, s.scale_log2,       \
+                                                                 (B) >= w_all && (B) <= w_whole);       \
     }
     for (int b = b_lo; b <= b_hi; b += 2) {
         LA_STEP(b, kb0, vb0, kb1, vb1)
@@ -235,7 +262,7 @@ __global__ __launch_bounds__(LA_WAVES * 64, 2) void latent_prompt_kernel(
     bf16_t* orow = out + (size_t)(q0 + tok) * s.o_tok + (size_t)head * s.o_head;
 #pragma unroll
     for (int dt = 0; dt < DVT; ++dt)
-        if (FULL || dt * 16 < s.vd)
+        if (dt * 16 < s.vd)
             la_store4(orow + dt * 16 + lg * 4, t.o[dt][0] * inv, t.o[dt][1] * inv, t.o[dt][2] * inv, t.o[dt][3] * inv);
 }
 
@@ -391,16 +418,22 @@ extern "C" int gfa_latent_attention(const void* q, const void* k_pages, const vo
     LAShape s{H, hd, vd, q_tok, q_head, o_tok, o_head, table_stride, window, scale * 1.4426950408889634f, gate, gate_tok};
     const dim3 step_grid(parts, (H + 63) / 64, n_seqs);
     const dim3 prompt_grid((unsigned)(((long long)max_q_len * H + LA_WAVES * 16 - 1) / (LA_WAVES * 16)), 1, n_seqs);
-#define LA_GO(DK, DVT, FULL) do {                                                                          \
-        if (max_q_len == 1)                                                                                \
-            latent_step_kernel<DK, DVT, FULL><<<step_grid, 256, 0, stream>>>(                              \
-                (const bf16_t*)q, (const bf16_t*)k_pages, (const bf16_t*)v_pages, q_start, start_pos, table, \
-                (bf16_t*)out, part_ml, part_o, parts, s);                                                  \
-        else                                                                                               \
-            latent_prompt_kernel<DK, DVT, FULL><<<prompt_grid, LA_WAVES * 64, 0, stream>>>(                \
-                (const bf16_t*)q, (const bf16_t*)k_pages, (const bf16_t*)v_pages, q_start, start_pos, table, \
-                (bf16_t*)out, s);                                                                          \
-    } while (0)
+    if (max_q_len > 1) {
+#define LA_GO(DK, DVT)                                                                                     \
+        latent_prompt_kernel<DK, DVT><<<prompt_grid, LA_WAVES * 64, 0, stream>>>(                          \
+            (const bf16_t*)q, (const bf16_t*)k_pages, (const bf16_t*)v_pages, q_start, start_pos, table,   \
+            (bf16_t*)out, s)
+        if (hd <= 192 && vd <= 128) LA_GO(6, 8);
+        else if (hd <= 320 && vd <= 256) LA_GO(10, 16);
+        else if (hd <= 512) LA_GO(16, 32);
+        else LA_GO(18, 32);
+#undef LA_GO
+        return GFA_LAUNCH_RESULT();
+    }
+#define LA_GO(DK, DVT, FULL)                                                                               \
+    latent_step_kernel<DK, DVT, FULL><<<step_grid, 256, 0, stream>>>(                                      \
+        (const bf16_t*)q, (const bf16_t*)k_pages, (const bf16_t*)v_pages, q_start, start_pos, table,       \
+        (bf16_t*)out, part_ml, part_o, parts, s)
     if (hd == 576 && vd == 512) LA_GO(18, 32, true);
     else if (hd <= 192 && vd <= 128) LA_GO(6, 8, false);
     else if (hd <= 320 && vd <= 256) LA_GO(10, 16, false);

@@ -449,6 +449,42 @@ def test_the_attention_gates_its_heads_and_finds_a_key_that_stands_out(dtype, to
             assert rel_err(got.permute(1, 0, 2), want) < tol, (lens, starts, n_parts)
 
 
+@pytest.mark.parametrize("H,hd,vd", [(3, 8, 16), (3, 192, 128), (5, 200, 128), (2, 192, 144), (2, 320, 256), (3, 328, 16),
+                                     (4, 512, 512), (2, 520, 496), (3, 576, 16), (1, 8, 512)])
+def test_prompts_at_the_edges_of_the_sizes_one_form_serves(H, hd, vd):
+    """Keys and values as large as a form takes, one step larger, and far smaller on one side, with and without a
+    window; two sequences that end inside a tile and a block, pool beyond their ends not a number.  q, k, v are exact; the
+    weights are rounded to bfloat16 (2^-9 of each at most) and so is the result (2^-9 of it), which together with
+    float32 sums stays below 2^-7 of the largest value."""
+    from gpt_fast_amd.ops import latent_attention as LA
+    from gpt_fast_amd.ops import scored_attention as SA
+    g = torch.Generator().manual_seed(hd + vd)
+    lens, starts, dtype = [70, 9], [33, 0], torch.bfloat16
+    total = [s + l for s, l in zip(starts, lens)]
+    n_pages, tables, table, _, _, _ = _table_and_positions(total, [0] * len(total))
+    ks = [torch.randn(t, hd, generator=g, dtype=F).to(dtype).double() for t in total]
+    vs = [torch.randn(t, vd, generator=g, dtype=F).to(dtype).double() for t in total]
+    q = torch.randn(H, sum(lens), hd, generator=g, dtype=F).to(dtype)
+    k_pages = torch.full((n_pages + 1, 1, 64, hd), float("nan"), dtype=dtype, device=DEV)
+    v_pages = torch.full((n_pages + 1, 1, vd, 64), float("nan"), dtype=dtype, device=DEV)
+    rows = torch.cat([torch.cat([torch.zeros(t, hd, dtype=F), k, v], 1) for t, k, v in zip(total, ks, vs)])
+    SA.unit_heads_store(_f32(rows), None, _ints([b for b, t in enumerate(total) for _ in range(t)]),
+                        _ints([i for t in total for i in range(t)]), table, k_pages, v_pages, 1, 1, hd, vd, None, dtype)
+    tok_seq = _ints([b for b, l in enumerate(lens) for _ in range(l)])
+    tok_pos = _ints([s + i for s, l in zip(starts, lens) for i in range(l)])
+    step = (_ints([0, lens[0], sum(lens)]), _ints(starts), len(lens), max(lens))
+    for window in (0, 40):
+        want, at = torch.zeros(H, sum(lens), vd, dtype=F), 0
+        for b, l in enumerate(lens):
+            for i in range(l):
+                end = starts[b] + i + 1
+                seen = slice(max(0, end - window) if window else 0, end)
+                want[:, at] = torch.softmax(q[:, at].double() @ ks[b][seen].T * 0.1, -1) @ vs[b][seen]
+                at += 1
+        got = LA.attention(q.to(DEV), k_pages, v_pages, tok_seq, tok_pos, table, 0.1, step, window=window)
+        assert rel_err(got, want) < 2.0 ** -7, window
+
+
 @pytest.mark.parametrize("window", [1, 31, 32, 33, 64, 100])
 @pytest.mark.parametrize("H,hd,vd", [(5, 72, 64), (32, 576, 512)])
 def test_one_shared_kv_head_with_a_window(H, hd, vd, window):
