@@ -538,7 +538,17 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(
     }
 }
 
-// The same for bfloat16 with interleaved pairs, eight elements (four pairs) per thread:
+// (a, b) <- (a c - b s, b c + a s) of pair p of eight elements.  Which of the two products is rounded before it is
+// added is written out, because compilers choose it by what surrounds the expression: a key has to have the same
+// bits whether its prompt comes whole (rope_cache_rows_kernel) or in portions of few tokens.
+template <bool SLICED>
+__device__ __forceinline__ void rope_turn(float& a, float& b, float c, float s, int p) {
+    const float x = SLICED || p % 2 == 0 ? fmaf(a, c, -(b * s)) : fmaf(-b, s, a * c);
+    b = SLICED ? fmaf(b, c, a * s) : fmaf(a, s, b * c);
+    a = x;
+}
+
+// The rotation and cache write for bfloat16 with interleaved pairs, eight elements (four pairs) per thread:
 // 16-byte loads and stores for q and k.  Needs hd and rot to be multiples of 8.
 __global__ __launch_bounds__(256) void rope_cache_bf16x8_kernel(
         const bf16_t* __restrict__ qkv, bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_pages,
@@ -567,10 +577,10 @@ __global__ __launch_bounds__(256) void rope_cache_bf16x8_kernel(
         if (d0 < rot) {
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
-                const float a = bf16_to_float(in.e[2 * p]), b = bf16_to_float(in.e[2 * p + 1]);
-                const float c_ = cs[d0 + 2 * p], s_ = cs[d0 + 2 * p + 1];
-                out.e[2 * p] = float_to_bf16(a * c_ - b * s_);
-                out.e[2 * p + 1] = float_to_bf16(b * c_ + a * s_);
+                float a = bf16_to_float(in.e[2 * p]), b = bf16_to_float(in.e[2 * p + 1]);
+                rope_turn<false>(a, b, cs[d0 + 2 * p], cs[d0 + 2 * p + 1], p);
+                out.e[2 * p] = float_to_bf16(a);
+                out.e[2 * p + 1] = float_to_bf16(b);
             }
         } else {
             out.u = in.u;
@@ -627,10 +637,9 @@ __global__ __launch_bounds__(256) void rope_cache_sliced_bf16x8_kernel(
         if (d0 < rot) {
 #pragma unroll
             for (int p = 0; p < 4; ++p) {
-                const float a = v[2 * p], b = v[2 * p + 1];
-                const float c_ = cs[d0 + 2 * p], s_ = cs[d0 + 2 * p + 1];
-                out.e[2 * p] = float_to_bf16(a * c_ - b * s_);
-                out.e[2 * p + 1] = float_to_bf16(b * c_ + a * s_);
+                rope_turn<true>(v[2 * p], v[2 * p + 1], cs[d0 + 2 * p], cs[d0 + 2 * p + 1], p);
+                out.e[2 * p] = float_to_bf16(v[2 * p]);
+                out.e[2 * p + 1] = float_to_bf16(v[2 * p + 1]);
             }
         } else {
 #pragma unroll
@@ -656,6 +665,7 @@ __global__ __launch_bounds__(256) void rope_cache_sliced_bf16x8_kernel(
 // XCDs, which then all write the same lines.  Heads as in the 8B shape, before and now: 401 tokens 7.3 -> 6.3 us,
 // 2,048 21.5 -> 15.9 (50 MB), 7,491 65 -> 42, six prompts of 2,696 tokens together 26.2 -> 18.5; two slices of
 // 640 12.4 -> 11.1, of 2,048 30.4 -> 27.3.
+// eight elements of a row at `at`: the slices added in order (SLICED), or the bfloat16 values as floats
 template <bool SLICED>
 __device__ __forceinline__ void rope_eight(const void* __restrict__ qkv, int S, size_t slice, size_t at, float (&v)[8]) {
     if (SLICED) {
@@ -676,11 +686,19 @@ __device__ __forceinline__ void rope_eight(const void* __restrict__ qkv, int S, 
         }
     }
 }
-__device__ __forceinline__ uint4 rope_pack(const float (&v)[8]) {      // exact for what was bfloat16 before
+__device__ __forceinline__ uint4 rope_pack(const float (&v)[8]) {
     uint32_t o[4];
 #pragma unroll
     for (int p = 0; p < 4; ++p) o[p] = (uint32_t)float_to_bf16(v[2 * p]) | ((uint32_t)float_to_bf16(v[2 * p + 1]) << 16);
     return make_uint4(o[0], o[1], o[2], o[3]);
+}
+// the same eight as bfloat16; what was bfloat16 before is copied bit by bit
+template <bool SLICED>
+__device__ __forceinline__ uint4 rope_copy(const void* __restrict__ qkv, int S, size_t slice, size_t at) {
+    if (!SLICED) return *(const uint4*)((const bf16_t*)qkv + at);
+    float v[8];
+    rope_eight<SLICED>(qkv, S, slice, at, v);
+    return rope_pack(v);
 }
 
 #define RC_TOKENS 4
@@ -714,11 +732,7 @@ __global__ __launch_bounds__(256) void rope_cache_rows_kernel(
                 if (whole) {
                     uint4 row[8];
 #pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        float v[8];
-                        rope_eight<SLICED>(qkv, S, slice, at + t * width, v);
-                        row[t] = rope_pack(v);
-                    }
+                    for (int t = 0; t < 8; ++t) row[t] = rope_copy<SLICED>(qkv, S, slice, at + t * width);
 #pragma unroll
                     for (int j = 0; j < 8; ++j) {
                         uint32_t o[4];
@@ -730,11 +744,10 @@ __global__ __launch_bounds__(256) void rope_cache_rows_kernel(
                         *(uint4*)(v_pages + value_elem(page, g, d0 + j, off, Hkv, hd)) = make_uint4(o[0], o[1], o[2], o[3]);
                     }
                 } else {
-                    float v[8];
-                    rope_eight<SLICED>(qkv, S, slice, at, v);
+                    const uint4 row = rope_copy<SLICED>(qkv, S, slice, at);
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
-                        v_pages[value_elem(page, g, d0 + j, off, Hkv, hd)] = float_to_bf16(v[j]);
+                        v_pages[value_elem(page, g, d0 + j, off, Hkv, hd)] = (bf16_t)(((const uint32_t*)&row)[j / 2] >> (j % 2 * 16));
                 }
             }
         }
@@ -752,10 +765,14 @@ __global__ __launch_bounds__(256) void rope_cache_rows_kernel(
     __syncthreads();
     if (c >= qk_chunks) return;
     const int head = c / per_head, d0 = (c - head * per_head) * 8;
+    uint4 row[RC_TOKENS];
     float v[RC_TOKENS][8];
 #pragma unroll
-    for (int t = 0; t < RC_TOKENS; ++t)
-        rope_eight<SLICED>(qkv, S, slice, (size_t)(n0 + t < n_tokens ? n0 + t : n_tokens - 1) * width + (size_t)head * hd + d0, v[t]);
+    for (int t = 0; t < RC_TOKENS; ++t) {
+        const size_t at = (size_t)(n0 + t < n_tokens ? n0 + t : n_tokens - 1) * width + (size_t)head * hd + d0;
+        if (d0 < rot) rope_eight<SLICED>(qkv, S, slice, at, v[t]);
+        else row[t] = rope_copy<SLICED>(qkv, S, slice, at);
+    }
 #pragma unroll
     for (int t = 0; t < RC_TOKENS; ++t) {
         const int n = n0 + t;
@@ -763,17 +780,14 @@ __global__ __launch_bounds__(256) void rope_cache_rows_kernel(
         if (d0 < rot) {
             const float* at = cs + t * rot + d0;
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const float a = v[t][2 * p], b = v[t][2 * p + 1], c_ = at[2 * p], s_ = at[2 * p + 1];
-                v[t][2 * p] = fmaf(a, c_, -(b * s_));
-                v[t][2 * p + 1] = fmaf(b, c_, a * s_);
-            }
+            for (int p = 0; p < 4; ++p) rope_turn<SLICED>(v[t][2 * p], v[t][2 * p + 1], at[2 * p], at[2 * p + 1], p);
+            row[t] = rope_pack(v[t]);
         }
         if (head < H) {
-            *(uint4*)(q_out + ((size_t)n * H + head) * hd + d0) = rope_pack(v[t]);
+            *(uint4*)(q_out + ((size_t)n * H + head) * hd + d0) = row[t];
         } else if (k_pages) {                              // one chunk of 8 dims
             const int pos = tok_pos[n], page = table[(size_t)tok_seq[n] * table_stride + pos / GFA_PAGE];
-            *(uint4*)(k_pages + key_elem(page, head - H, pos % GFA_PAGE, d0, Hkv, hd)) = rope_pack(v[t]);
+            *(uint4*)(k_pages + key_elem(page, head - H, pos % GFA_PAGE, d0, Hkv, hd)) = row[t];
         }
     }
 }

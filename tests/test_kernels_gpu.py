@@ -115,9 +115,8 @@ def test_gemm_f32_is_the_same_in_every_tile(N, K_):
 @pytest.mark.parametrize("lens,starts", [((401,), (0,)), ((3, 5, 640, 17, 8), (61, 7, 3, 0, 56)), ((9,) * 80, range(80))])
 def test_rotation_and_cache_write_of_many_tokens(H, G, hd, rot, lens, starts):
     """The kernel of prompts against the one of few tokens (the same rows in steps of at most 160): whole
-    groups of eight keys, groups that begin or end inside a step, neighbouring sequences.  Values are
-    copies; rotated elements may differ by one rounding of the two products' sum (2^-7 of the value, or of
-    what cancels: the pair's larger element)."""
+    groups of eight keys, groups that begin or end inside a step, neighbouring sequences.  The same bits, those
+    of values that are no number among them: a key may not depend on how its prompt is cut into steps."""
     g = torch.Generator().manual_seed(hd + H)
     n, B, W = sum(lens), len(lens), (max(l + s for l, s in zip(lens, starts)) + 63) // 64
     table = torch.randperm(B * W, generator=g).int().view(B, W).to(DEV)
@@ -126,6 +125,7 @@ def test_rotation_and_cache_write_of_many_tokens(H, G, hd, rot, lens, starts):
     freqs = (10000.0 ** (-torch.arange(rot // 2) * 2.0 / rot)).to(DEV)
     width = (H + 2 * G) * hd
     qkv, part = bf(torch.randn(n, width, generator=g)).to(DEV), torch.randn(2, n, width, generator=g).to(DEV)
+    qkv.view(torch.int16)[::3, (H + G) * hd::5] = 0x7f81
 
     def run(cuts, sliced):
         pages = [torch.zeros(B * W, G, 64, hd, device=DEV, dtype=torch.bfloat16),
@@ -140,12 +140,8 @@ def test_rotation_and_cache_write_of_many_tokens(H, G, hd, rot, lens, starts):
     for sliced in (False, True):
         if sliced and n < 640:
             continue
-        (q1, k1, v1), (q2, k2, v2) = run([0, n], sliced), run(few, sliced)
-        assert torch.equal(v1, v2)
-        most = float(qkv.abs().max() if not sliced else part.sum(0).abs().max())
-        for a, b in ((q1, q2), (k1, k2)):
-            assert float((a.float() - b.float()).abs().max()) <= 2.0 ** -7 * most
-            assert float((a != b).float().mean()) < 0.05
+        for whole, portions in zip(run([0, n], sliced), run(few, sliced)):
+            assert torch.equal(whole.view(torch.int16), portions.view(torch.int16))
 
 
 @pytest.mark.parametrize("M", [2049, 2148, 3000])
