@@ -1,6 +1,9 @@
 """The cache's bookkeeping and the generation loop's decisions.  No GPU: the cache is
 built on CPU tensors and the loop is driven by a scripted stepper."""
+import os
 import random
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -585,3 +588,16 @@ def test_residual_stream_runs_what_was_put_off_before_any_read():
     plain = torch.zeros(1, 2)
     add_late(plain, finish("g"))                          # a plain tensor: at once
     assert log[-1] == ("g", None, False) and float(plain.sum()) == 2
+
+
+def test_the_package_imports_with_a_torch_that_was_built_without_a_gpu():
+    """Such a torch has no functions for devices' streams in its C module."""
+    code = ("import sys; sys.path.insert(0, %r)\n"
+            "import torch\n"
+            "for name in [n for n in dir(torch._C) if n.startswith('_cuda_')]:\n"
+            "    if name not in ('_cuda_getDeviceCount',):\n"
+            "        delattr(torch._C, name)\n"
+            "import gpt_fast_amd as gfa\n"
+            "print(gfa.find_preset('stories110M')[1].hidden_size)\n") % os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    got = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert got.returncode == 0 and got.stdout.strip() == "768", got.stderr
