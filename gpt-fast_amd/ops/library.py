@@ -47,8 +47,8 @@ def stream_handle() -> ctypes.c_void_p:
     (a prompt of 32 tokens and one token after it on a 12-layer model of 768 columns, 130
     launches: 2.58 ms of host time with it, 1.99 without)."""
     global _raw_stream, _current_device
-    if _raw_stream is None:
-        stream = torch.cuda.current_stream()
+    if _raw_stream is None or not torch.cuda.is_initialized():
+        stream = torch.cuda.current_stream()   # starts the device, or says why it cannot (a forked process)
         if not hasattr(torch._C, "_cuda_getCurrentRawStream") or not hasattr(torch._C, "_cuda_getDevice"):
             return ctypes.c_void_p(stream.cuda_stream)
         _current_device, _raw_stream = torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream

@@ -601,3 +601,17 @@ def test_the_package_imports_with_a_torch_that_was_built_without_a_gpu():
             "print(gfa.find_preset('stories110M')[1].hidden_size)\n") % os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
     got = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
     assert got.returncode == 0 and got.stdout.strip() == "768", got.stderr
+
+
+def test_a_launch_where_the_device_may_not_be_used_is_refused_by_torch(monkeypatch):
+    """A process forked from one that uses the device has its tensors but may not use them: torch says so."""
+    from gpt_fast_amd.ops import library
+
+    def refuse():
+        raise RuntimeError("forked")
+    monkeypatch.setattr(library, "_raw_stream", lambda device: 5)
+    monkeypatch.setattr(library, "_current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: False)
+    monkeypatch.setattr(torch.cuda, "current_stream", refuse)
+    with pytest.raises(RuntimeError, match="forked"):
+        library.stream_handle()
