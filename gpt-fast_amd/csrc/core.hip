@@ -977,9 +977,11 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
         const bool seen = key >= lo && key <= pos;
         const float s = seen ? (dot0 + dot1) * scale : -INFINITY;
         const float m_new = fmaxf(m, wave_max(s));
-        const bool any = m_new != -INFINITY;               // no number to scale by otherwise
-        const float alpha = any ? expf(m - m_new) : 1.f;
-        const float p = seen && any ? expf(s - m_new) : 0.f;
+        // scores that are no number do not count in a maximum: where there is nothing else the reference is 0, and
+        // their weights, and with them the row, are no number either
+        const float ref = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = m_new == -INFINITY ? 1.f : expf(m - m_new);
+        const float p = seen ? expf(s - ref) : 0.f;
         l = l * alpha + wave_sum(p);
         m = m_new;
         ps[wave][lane] = p;                                // read by this wave alone

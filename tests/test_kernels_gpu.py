@@ -144,6 +144,27 @@ def test_rotation_and_cache_write_of_many_tokens(H, G, hd, rot, lens, starts):
             assert torch.equal(whole.view(torch.int16), portions.view(torch.int16))
 
 
+@pytest.mark.parametrize("hd", [16, 64, 128, 256, 24])
+@pytest.mark.parametrize("first,last", [(64, 64), (64, 127), (0, 63), (70, 70), (0, 299)])
+def test_a_seen_key_that_is_no_number_reaches_the_row(hd, first, last):
+    """Keys first .. last are no numbers, alone in what a page holds for a token, among others, everywhere: every
+    token that sees one of them has a row that is no number, the others do not notice."""
+    g = torch.Generator().manual_seed(hd)
+    n, H, G, W, window = 300, 2, 1, 5, 80
+    seq = torch.zeros(n, dtype=torch.int32, device=DEV)
+    pos = torch.arange(n, dtype=torch.int32, device=DEV)
+    table = torch.randperm(W, generator=g).int().view(1, W).to(DEV)
+    qkv = torch.randn(n, (H + 2 * G) * hd, generator=g)
+    qkv[first:last + 1, H * hd:(H + G) * hd] = float("nan")
+    pages = [torch.full((W, G, 64, hd), float("nan"), device=DEV), torch.full((W, G, hd, 64), float("nan"), device=DEV)]
+    q = K().rope_cache_write(qkv.to(DEV), None, seq, pos, table, *pages, H, G, hd, 0, 0)
+    for w in (0, window):
+        out = K().attention_generic(q, *pages, seq, pos, table, hd ** -0.5, w).cpu()
+        t = torch.arange(n)
+        sees = (t >= first) & ((t - w < last) if w else torch.ones(n, dtype=torch.bool))
+        assert torch.equal(out.isnan(), sees[:, None, None].expand_as(out)), w
+
+
 @pytest.mark.parametrize("M", [2049, 2148, 3000])
 def test_products_of_whole_rounds_and_the_rest(M):
     """Rows beyond a whole round of the chip go through a second product (of one row, of few and of many):
