@@ -53,48 +53,40 @@ struct PtArgs {
     int top, E;
 };
 
-// The activations in float32 with the exponential and reciprocal instructions (each within a unit of the last
-// place), which the library forms would spend several times the arithmetic on.
-__device__ __forceinline__ float pt_sigmoid(float z) {
-    return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
+// The activations of all kernels of the experts, so that a value does not depend on how many rows share its step.
+// The gate of clamped experts: a <- min(a, limit), b <- b clamped to -limit .. limit, a sigmoid(1.702 a) (b + 1)
+__device__ __forceinline__ float re_clamped_pair(float a, float b, float limit) {
+    a = fminf(a, limit);
+    b = fminf(fmaxf(b, -limit), limit);
+    return a / (1.f + expf(-1.702f * a)) * (b + 1.f);
 }
-// z Phi(z) with Phi(-|z|) = exp(-z^2 / 2) g(t), t = 1 / (1 + 0.3 |z| / sqrt 2): g / t is smooth in t, and the
-// polynomial is its least relative deviation (2.1e-8) on 0 <= |z| / sqrt 2 <= 12, fitted to scipy's erfcx.  Against
-// 0.5 z (1 + erff(z / sqrt 2)) it keeps its relative error (9e-7 at most down to z = -4) where that cancels.
-__device__ __forceinline__ float pt_gelu(float z) {
-    const float t = __builtin_amdgcn_rcpf(fmaf(0.3f * 0.7071067811865476f, fabsf(z), 1.f));
-    float g = -0.12925273180007935f;
-    g = fmaf(g, t, 0.48429954051971436f);
-    g = fmaf(g, t, -0.5097681879997253f);
-    g = fmaf(g, t, 0.5449625253677368f);
-    g = fmaf(g, t, -0.09282324463129044f);
-    g = fmaf(g, t, 0.2141803354024887f);
-    g = fmaf(g, t, 0.1485215127468109f);
-    g = fmaf(g, t, 0.1706908941268921f);
-    g = fmaf(g, t, 0.16918934881687164f);
-    const float tail = 0.5f * g * t * __builtin_amdgcn_exp2f(-0.7213475204444817f * z * z);
-    return z * (z < 0.f ? tail : 1.f - tail);
+
+// 0 silu, 1 gelu (tanh form), 3 gelu (exact); the numbers of ops.kernels.ACTIVATIONS
+__device__ __forceinline__ float re_activation(float z, int act) {
+    if (act == 0) return z / (1.f + expf(-z));
+    if (act == 1) return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+    return 0.5f * z * (1.f + erff(z * 0.7071067811865476f));
 }
-// act of eight values; the branch is the same for the whole launch
+
+// act of eight values, once for the whole launch.  (With the exponential and reciprocal instructions in place of the
+// library's forms a product of 222 rows for each of 32 experts, 4,096 -> 2 x 3,584, took 606 us and not 623, but
+// silu's error grew with its argument, from 1.2e-7 of the value to 3.5e-6 at -60.)
 __device__ __forceinline__ void pt_act(float (&z)[8], int act) {
     if (act == 0) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) z[i] *= pt_sigmoid(z[i]);
-    } else if (act == 1) {       // z / (1 + exp(-2 y)) is 0.5 z (1 + tanh y)
+        for (int i = 0; i < 8; ++i) z[i] = re_activation(z[i], 0);
+    } else if (act == 1) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) z[i] *= pt_sigmoid(1.5957691216057308f * (z[i] + 0.044715f * z[i] * z[i] * z[i]));
+        for (int i = 0; i < 8; ++i) z[i] = re_activation(z[i], 1);
     } else if (act == 3) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) z[i] = pt_gelu(z[i]);
+        for (int i = 0; i < 8; ++i) z[i] = re_activation(z[i], 3);
     }
 }
-__device__ __forceinline__ void pt_gate(float (&a)[8], float (&b)[8], int act, float limit) {
+__device__ __forceinline__ void pt_gate(float (&a)[8], const float (&b)[8], int act, float limit) {
     if (act == 2) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float z = fminf(a[i], limit);
-            a[i] = z * pt_sigmoid(1.702f * z) * (fminf(fmaxf(b[i], -limit), limit) + 1.f);
-        }
+        for (int i = 0; i < 8; ++i) a[i] = re_clamped_pair(a[i], b[i], limit);
         return;
     }
     pt_act(a, act);
@@ -322,6 +314,7 @@ void prompt_tile_kernel(const PtArgs g) {
         for (int u = lane; u < 32 * UNITS; u += 64) {
             const int row = u / UNITS, unit = u % UNITS;
             const int m = m0 + (wr * TM + j) * 32 + row, n = c0 + unit * 8;
+            if (m >= m1 || n >= F) continue;                     // F is a multiple of eight
             const char* from = mine + row * PITCH + (MODE == PT_GATE ? (unit / 4) * 256 + (unit % 4) * 32 : unit * 32);
             float z[8];
             *(pt_floatx4_t*)z = *(const pt_floatx4_t*)from;
@@ -334,13 +327,11 @@ void prompt_tile_kernel(const PtArgs g) {
             } else {
                 pt_act(z, g.act);
             }
-            if (m < m1 && n < F) {                               // F is a multiple of eight
-                const uint4 v = make_uint4((uint32_t)float_to_bf16(z[0]) | ((uint32_t)float_to_bf16(z[1]) << 16),
-                                           (uint32_t)float_to_bf16(z[2]) | ((uint32_t)float_to_bf16(z[3]) << 16),
-                                           (uint32_t)float_to_bf16(z[4]) | ((uint32_t)float_to_bf16(z[5]) << 16),
-                                           (uint32_t)float_to_bf16(z[6]) | ((uint32_t)float_to_bf16(z[7]) << 16));
-                *(uint4*)((bf16_t*)g.out + (size_t)m * F + n) = v;
-            }
+            *(uint4*)((bf16_t*)g.out + (size_t)m * F + n) =
+                make_uint4((uint32_t)float_to_bf16(z[0]) | ((uint32_t)float_to_bf16(z[1]) << 16),
+                           (uint32_t)float_to_bf16(z[2]) | ((uint32_t)float_to_bf16(z[3]) << 16),
+                           (uint32_t)float_to_bf16(z[4]) | ((uint32_t)float_to_bf16(z[5]) << 16),
+                           (uint32_t)float_to_bf16(z[6]) | ((uint32_t)float_to_bf16(z[7]) << 16));
         }
         __builtin_amdgcn_wave_barrier();
     }

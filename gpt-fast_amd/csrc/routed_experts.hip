@@ -149,20 +149,6 @@ extern "C" int gfa_route(const float* z, long long z_stride, int n_tokens, int E
     return GFA_LAUNCH_RESULT();
 }
 
-// the gate of clamped experts: a <- min(a, limit), b <- b clamped to -limit .. limit, a sigmoid(1.702 a) (b + 1)
-__device__ __forceinline__ float re_clamped_pair(float a, float b, float limit) {
-    a = fminf(a, limit);
-    b = fminf(fmaxf(b, -limit), limit);
-    return a / (1.f + expf(-1.702f * a)) * (b + 1.f);
-}
-
-// 0 silu, 1 gelu (tanh form), 3 gelu (exact); the numbers of ops.kernels.ACTIVATIONS
-__device__ __forceinline__ float re_activation(float z, int act) {
-    if (act == 0) return z / (1.f + expf(-z));
-    if (act == 1) return 0.5f * z * (1.f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-    return 0.5f * z * (1.f + erff(z * 0.7071067811865476f));
-}
-
 template <typename T> struct Vec8;
 template <> struct Vec8<bf16_t> {
     static __device__ __forceinline__ void load(const bf16_t* p, float* f) {

@@ -329,6 +329,33 @@ def test_the_experts_rows_in_tiles_of_whole_pieces(E, D, Fh, counts):
             assert rel_err(got[lo:lo + c], rows[lo:lo + c].double() @ w[e].double().T) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("act,gated,limit", [("silu", False, None), ("gelu", False, None), ("gelu_tanh", False, None),
+                                             ("silu", True, None), ("gelu_tanh", True, None), ("clamped_swish", True, 7.0)])
+def test_an_experts_activation_is_the_same_in_every_kernel(act, gated, limit):
+    """Sums that are exact (one product each), over the range in which the activations are not the identity or
+    zero, a thousand bfloat16 numbers and the ends of the range of float: rows of an inner size of whole pieces, of one that
+    takes the other kernel, and of few pairs have the same bits."""
+    from gpt_fast_amd.ops import routed_experts as RE
+    z = torch.cat([torch.linspace(-95.0, 95.0, 1000), torch.tensor([-88.0, -87.5, -3e38, 3e38, 0.0, -0.0])]).bfloat16()
+    z = z[:len(z) // 8 * 8]
+    Fh, n = z.numel(), 40
+    offsets, order, _ = RE.expert_order(torch.zeros(n, 1, dtype=torch.int32, device=DEV), 1)
+    got = []
+    for K_ in (64, 8):
+        w = torch.zeros(1, 2 * Fh if gated else Fh, K_)
+        w[0, :Fh, 0] = z.float()
+        if gated:
+            w[0, Fh:, 0] = 0.75
+        x = torch.zeros(n, K_)
+        x[:, 0] = 1.0
+        operands = x.bfloat16().to(DEV), order, 1, w.bfloat16().to(DEV), offsets
+        got.append(RE.expert_tile_product(*operands, None, n, act, gated, limit))
+        if not gated and act in RE.EXPERT_ACTIVATIONS:
+            got.append(RE.grouped_rows(*operands, act, n))
+    for other in got[1:]:
+        assert torch.equal(got[0].view(torch.int16), other.view(torch.int16))
+
+
 def test_the_correction_moves_the_choice_and_not_the_weights():
     part, rt, w, mlp = _mixture(4, 2, 2, 64, 32, 1.0, None, "float32")
     part.correction.copy_(torch.tensor([0.0, 0.0, 0.0, 0.0, 5.0, 5.0]))     # both identity experts, always
