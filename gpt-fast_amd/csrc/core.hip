@@ -215,7 +215,7 @@ extern "C" int gfa_add_rmsnorm(float* res, const void* y, const float* w, void* 
 // the four sums at the end.  An output's sum is therefore four chains, added as (0 + 1) + (2 + 3), whose
 // order depends on K alone: every tile size and every M gives the same bits, and a row's result does not
 // depend on the other rows (a float32 logit is the same however tokens are cut into steps).
-// gf_launch picks the tile.  Measured beside 64 x 64 tiles of vector multiply-adds through shared memory,
+// gf_product picks the tile.  Measured beside 64 x 64 tiles of vector multiply-adds through shared memory,
 // which this replaces: 1 x 768 x 768 76 -> 5.8 us, 1 x 32,000 x 768 120 -> 29 (3.4 TB/s), 717 x 2,304 x 768
 // 99 -> 44, 717 x 768 x 2,048 274 -> 41, 8 x 28,672 x 4,096 617 -> 116 (4.1 TB/s), 2,048 x 4,096 x 4,096
 // 988 -> 704 (98 of the 155 TFLOP/s that a loop of the instruction alone reaches); few rows are bound by
@@ -346,14 +346,22 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(
     gf_store<MT, NT>(sums, out, M, N, m0, n0, som, accumulate);
 }
 
-// The same arithmetic for many rows (16-byte loads only): a 64 x 64 tile whose waves copy their blocks
-// through shared memory of their own (no barrier while K is walked).  A load instruction then takes eight
-// rows of 128 bytes, whole lines, where the operand order above takes sixteen rows of 64, which the compute
-// unit's cache looks up piece by piece: 2,048 x 4,096 x 4,096 took 1,155 us without it.
+// How the staged kernel gets a row's 32 k of a block: in 16-byte loads at multiples of 16, in 16-byte loads at any
+// float, or as elements `swk` apart, where the lanes take neighbouring rows (those of a matrix that lies transposed).
+enum GfLoads { GF_WIDE, GF_ALONG, GF_ACROSS };
+typedef gf_floatx4_t gf_loose4_t __attribute__((aligned(4)));
+
+// The same arithmetic for many rows: a 64 x 64 tile whose waves copy their blocks through shared memory of their
+// own (no barrier while K is walked).  A load instruction then takes whole lines, eight rows of 128 bytes (across:
+// 64 rows of one k), where the operand order above takes sixteen rows of 64 bytes, which the compute unit's cache
+// looks up piece by piece: 2,048 x 4,096 x 4,096 took 1,155 us without it, 2,048 x 4,096 x 1,022 (rows at odd
+// addresses) 616 against 168 now and 261 in vector multiply-adds, 32 x 1,000 x 512 x 128 with the second operand
+// transposed, as latent attention has it, 161 against 65 and 98.
 #define GS_PITCH 144                              // bytes per staged row of 32 k: 128 + pad against conflicts
+template <GfLoads AL, GfLoads WL>
 __global__ __launch_bounds__(256, 2) void gemm_f32_staged_kernel(
         const float* __restrict__ a, const float* __restrict__ w, float* __restrict__ out,
-        int M, int N, int K, long long sab, long long sam, long long swb, long long swn,
+        int M, int N, int K, long long sab, long long sam, long long swb, long long swn, long long swk,
         long long sob, long long som, int accumulate) {
     __shared__ __attribute__((aligned(16))) char lds[4 * 128 * GS_PITCH];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -363,12 +371,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_staged_kernel(
     w += (size_t)blockIdx.z * swb;
     out += (size_t)blockIdx.z * sob;
     const int row = lane >> 3, chunk = lane & 7;   // of eight rows, their 16-byte chunks
-    const float *ar[8], *wr[8];
+    const float *ar[8], *wr[WL == GF_ACROSS ? 1 : 8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const int m = m0 + 8 * i + row, n = n0 + 8 * i + row;
+        const int m = m0 + 8 * i + row, n = n0 + (WL == GF_ACROSS ? lane : 8 * i + row);
         ar[i] = a + (size_t)(m < M ? m : M - 1) * sam;
-        wr[i] = w + (size_t)(n < N ? n : N - 1) * swn;
+        if (WL != GF_ACROSS || i == 0) wr[i] = w + (size_t)(n < N ? n : N - 1) * swn;
     }
     gf_floatx4_t acc[4][4];
 #pragma unroll
@@ -377,15 +385,38 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_staged_kernel(
         for (int j = 0; j < 4; ++j) acc[i][j] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
     gf_floatx4_t av[8], wv[8];
     auto load = [&](int b) {
-        const int k = 32 * b + 4 * chunk, at = k < K ? k : 0;
+        const bool whole = 32 * b + 32 <= K;       // the same for the whole wave
+        const int k = 32 * b + 4 * chunk;
+        // eight times four k, the row's first ones again beyond K
+        auto eight = [&](auto row_of, auto k_of, GfLoads how, gf_floatx4_t (&v)[8]) {
+            if (how == GF_ALONG && whole) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            av[i] = *(const gf_floatx4_t*)(ar[i] + at);
-            wv[i] = *(const gf_floatx4_t*)(wr[i] + at);
-        }
-        if (32 * b + 32 > K && k >= K) {
+                for (int i = 0; i < 8; ++i) v[i] = *(const gf_loose4_t*)(row_of(i) + k_of(i));
+                return;
+            }
 #pragma unroll
-            for (int i = 0; i < 8; ++i) av[i] = wv[i] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < 8; ++i) {
+                if (how == GF_WIDE) {
+                    v[i] = *(const gf_floatx4_t*)(row_of(i) + (k_of(i) < K ? k_of(i) : 0));
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int at = k_of(i) + q < K ? k_of(i) + q : 0;
+                        v[i][q] = how == GF_ACROSS ? row_of(i)[(size_t)at * swk] : row_of(i)[at];
+                    }
+                }
+            }
+        };
+        eight([&](int i) { return ar[i]; }, [&](int) { return k; }, AL, av);
+        eight([&](int i) { return wr[WL == GF_ACROSS ? 0 : i]; }, [&](int i) { return WL == GF_ACROSS ? 32 * b + 4 * i : k; }, WL, wv);
+        if (!whole) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (k + q >= K) av[i][q] = 0.f;
+                    if ((WL == GF_ACROSS ? 32 * b + 4 * i : k) + q >= K) wv[i][q] = 0.f;
+                }
         }
     };
     char* as = lds + wave * 128 * GS_PITCH;
@@ -397,7 +428,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_staged_kernel(
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             *(gf_floatx4_t*)(as + put + 8 * i * GS_PITCH) = av[i];
-            *(gf_floatx4_t*)(ws + put + 8 * i * GS_PITCH) = wv[i];
+            *(gf_floatx4_t*)(ws + (WL == GF_ACROSS ? lane * GS_PITCH + 16 * i : put + 8 * i * GS_PITCH)) = wv[i];
         }
         if (b + 4 < blocks) load(b + 4);
 #pragma unroll
@@ -429,38 +460,33 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_staged_kernel(
 
 // Up to 16 rows: one 16 x 16 tile a workgroup, which spreads the weights over the most waves.  More rows:
 // 64 x 64 where these tiles are at least 100 (717 x 768 x 2,048, 144 of them: 41 us, as 32 x 32 54 us), else
-// 32 x 32; without 16-byte loads there is no staged kernel, and the unstaged one needs more tiles to win.
-template <bool WIDE>
-static int gf_launch(const float* a, const float* w, float* out, int B, int M, int N, int K,
-                     long long sab, long long sam, long long swb, long long swn, long long swk,
-                     long long sob, long long som, int accumulate, hipStream_t stream) {
-#define GF_GO(MT, NT) do { \
-        if ((M + 16 * MT - 1) / (16 * MT) > 65535 || B > 65535) return (int)hipErrorInvalidValue; \
-        const dim3 grid((N + 16 * NT - 1) / (16 * NT), (M + 16 * MT - 1) / (16 * MT), B); \
-        gemm_f32_kernel<MT, NT, WIDE><<<grid, 256, 0, stream>>>(a, w, out, M, N, K, sab, sam, swb, swn, \
-                                                                swk, sob, som, accumulate); \
-        return GFA_LAUNCH_RESULT(); \
-    } while (0)
-    const long long big = (long long)((M + 63) / 64) * ((N + 63) / 64) * B;
-    if (M <= 16) GF_GO(1, 1);
-    if (big < (WIDE ? 100 : 384)) GF_GO(2, 2);
-    if (!WIDE) GF_GO(4, 4);
-    if ((M + 63) / 64 > 65535 || B > 65535) return (int)hipErrorInvalidValue;
-    const dim3 grid((N + 63) / 64, (M + 63) / 64, B);
-    gemm_f32_staged_kernel<<<grid, 256, 0, stream>>>(a, w, out, M, N, K, sab, sam, swb, swn, sob, som, accumulate);
-    return GFA_LAUNCH_RESULT();
-#undef GF_GO
-}
-
+// 32 x 32.
 static int gf_product(const float* a, const float* w, float* out, int B, int M, int N, int K,
                       long long sab, long long sam, long long swb, long long swn, long long swk,
                       long long sob, long long som, int accumulate, hipStream_t stream) {
     if (B <= 0 || M <= 0 || N <= 0) return 0;
     // 16-byte loads: whole groups of four k, at addresses that are multiples of 16
-    const bool wide = swk == 1 && K % 4 == 0 && sam % 4 == 0 && swn % 4 == 0 && sab % 4 == 0 && swb % 4 == 0 &&
-                      (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0;
-    return (wide ? gf_launch<true> : gf_launch<false>)(a, w, out, B, M, N, K, sab, sam, swb, swn, swk, sob,
-                                                       som, accumulate, stream);
+    const bool a_wide = K % 4 == 0 && sam % 4 == 0 && sab % 4 == 0 && (uintptr_t)a % 16 == 0;
+    const bool w_wide = swk == 1 && K % 4 == 0 && swn % 4 == 0 && swb % 4 == 0 && (uintptr_t)w % 16 == 0;
+    const int tile = M <= 16 ? 16 : (long long)((M + 63) / 64) * ((N + 63) / 64) * B < 100 ? 32 : 64;
+    if ((M + tile - 1) / tile > 65535 || B > 65535) return (int)hipErrorInvalidValue;
+    const dim3 grid((N + tile - 1) / tile, (M + tile - 1) / tile, B);
+#define GF_GO(...) __VA_ARGS__<<<grid, 256, 0, stream>>>(a, w, out, M, N, K, sab, sam, swb, swn, swk, sob, som, accumulate)
+    if (tile == 16) {
+        if (a_wide && w_wide) GF_GO(gemm_f32_kernel<1, 1, true>);
+        else GF_GO(gemm_f32_kernel<1, 1, false>);
+    } else if (tile == 32) {
+        if (a_wide && w_wide) GF_GO(gemm_f32_kernel<2, 2, true>);
+        else GF_GO(gemm_f32_kernel<2, 2, false>);
+    } else if (swk != 1) {
+        if (a_wide) GF_GO(gemm_f32_staged_kernel<GF_WIDE, GF_ACROSS>);
+        else GF_GO(gemm_f32_staged_kernel<GF_ALONG, GF_ACROSS>);
+    } else {
+        if (a_wide && w_wide) GF_GO(gemm_f32_staged_kernel<GF_WIDE, GF_WIDE>);
+        else GF_GO(gemm_f32_staged_kernel<GF_ALONG, GF_ALONG>);
+    }
+#undef GF_GO
+    return GFA_LAUNCH_RESULT();
 }
 
 extern "C" int gfa_gemm_f32(const float* a, const float* w, float* out, int M, int N, int K,

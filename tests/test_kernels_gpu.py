@@ -144,6 +144,38 @@ def test_rotation_and_cache_write_of_many_tokens(H, G, hd, rot, lens, starts):
             assert torch.equal(whole.view(torch.int16), portions.view(torch.int16))
 
 
+@pytest.mark.parametrize("B,M,N,K_", [(1, 200, 1700, 1), (8, 200, 1000, 45), (3, 257, 1601, 64), (2, 640, 660, 130),
+                                      (32, 130, 129, 36), (1, 130, 2200, 31), (5, 300, 520, 200)])
+def test_float_products_of_many_rows_whose_operands_lie_otherwise(B, M, N, K_):
+    """Tiles of 64 x 64 (at least 100 of them, ragged on both sides) without 16-byte loads: rows at odd addresses, a
+    transposed second operand beside aligned and odd rows, one with strides on both sides, a sum into what is there.
+    A row has the bits of the same row in a product of few rows (16 x 16 and 32 x 32 tiles) over operands that lie
+    plainly; against float64 within the rounding of sums of K terms, each of which adds at most half a unit of 2^-23."""
+    assert (M + 63) // 64 * ((N + 63) // 64) * B >= 100
+    g = torch.Generator().manual_seed(M + N)
+    a = torch.randn(B, M, K_, generator=g).to(DEV)
+    w = torch.randn(B, N, K_, generator=g).to(DEV)
+    ref, most = a.double() @ w.double().mT.contiguous(), a.abs().double() @ w.abs().double().mT.contiguous()
+    few = torch.cat([torch.stack([K().gemm_f32(a[b, :17].contiguous(), w[b]) for b in range(B)]),
+                     torch.stack([K().gemm_f32(a[b, 17:33].contiguous(), w[b]) for b in range(B)])], 1)
+    odd = torch.empty(B, M, K_ + 1, device=DEV)[:, :, 1:].copy_(a)
+    heads = torch.empty(M, B, K_, device=DEV).transpose(0, 1).copy_(a)
+    across = w.mT.contiguous().mT
+    apart = torch.empty(B, N, K_, 2, device=DEV)[..., 0].copy_(w)
+    first = None
+    for x, y in ((a, w), (odd, w), (a, across), (odd, across), (heads, across), (a, apart), (heads, apart)):
+        out = K().gemm_f32_batched(x, y, torch.full((B, M, N), float("nan"), device=DEV))
+        if first is None:
+            first = out
+            assert bool(((out.double() - ref).abs() <= most * (K_ + 4) * 2.0 ** -24).all())
+            assert torch.equal(out[:, :33], few)
+        assert torch.equal(out, first)
+    for b in range(B if M * N > 60 * 64 * 64 else 0):
+        res = first[b].clone()
+        K().gemm_f32(odd[b], w[b], out=res, accumulate=True)
+        assert torch.equal(res, first[b] + first[b])
+
+
 @pytest.mark.parametrize("hd", [16, 64, 128, 256, 24])
 @pytest.mark.parametrize("first,last", [(64, 64), (64, 127), (0, 63), (70, 70), (0, 299)])
 def test_a_seen_key_that_is_no_number_reaches_the_row(hd, first, last):
