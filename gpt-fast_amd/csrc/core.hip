@@ -818,10 +818,17 @@ __global__ __launch_bounds__(256) void rope_cache_rows_kernel(
     }
 }
 
-// From this many tokens on the kernel above is the faster one (300 tokens: 7.2 against 6.4 us, two slices of 512:
-// 10.1 against 9.4), where the angles of its tokens fit into shared memory.
-static bool rope_cache_prompt(int n_tokens, int rot, bool sliced) {
-    return n_tokens >= (sliced ? 640 : 400) && RC_TOKENS * rot * sizeof(float) <= 32 * 1024;
+// The kernel above wins by its stores of values, where these are many and whole groups of eight keys are the rule:
+// by the values of a step and the tokens per sequence on average (rows of the page table).  Microseconds of the kernel of
+// few tokens and of this one, values of a token in brackets: 401 tokens (256) 3.3, 4.4; 700 (768) 7.3, 6.0;
+// 2,048 (256) 7.1, 5.6; 500 sequences of one (1,024) 7.3, 8.3; 32 of 32 (512) 8.5, 9.1; 20 of 48 (1,024) 12.0, 10.1.
+// Two slices: 6,001 (256) 30.1, 32.3; 700 (1,024) 17.7, 18.7; 2,048 (768) 18.5, 13.6; 20 of 100 (1,024) 39.4,
+// 40.5.  The angles of its tokens have to fit into shared memory.
+static bool rope_cache_prompt(int n_tokens, int n_seqs, int values, int rot, bool sliced) {
+    const long long stored = (long long)n_tokens * values;
+    return (sliced ? values >= 512 && stored >= 1 << 20 && n_tokens >= 128LL * n_seqs
+                   : stored >= (values >= 512 ? 300 << 10 : 1 << 19) && n_tokens >= 48LL * n_seqs) &&
+           RC_TOKENS * rot * sizeof(float) <= 32 * 1024;
 }
 
 template <bool SLICED>
@@ -842,13 +849,13 @@ static int rope_cache_launch(const void* qkv, int S, size_t slice, void* q_out, 
 extern "C" int gfa_rope_cache_write_sliced(const float* part, int S, void* q_out, void* k_pages,
                                            void* v_pages, const float* freqs, const int* tok_seq,
                                            const int* tok_pos, const int* table, int table_stride,
-                                           int n_tokens, int H, int Hkv, int hd, int rot,
+                                           int n_seqs, int n_tokens, int H, int Hkv, int hd, int rot,
                                            hipStream_t stream) {
     if (n_tokens <= 0) return 0;
     if (S <= 0 || hd % 8 != 0 || rot % 8 != 0 || rot > hd || (rot > 0 && !freqs))
         return (int)hipErrorInvalidValue;
     const size_t slice = (size_t)n_tokens * (H + 2 * Hkv) * hd;
-    if (rope_cache_prompt(n_tokens, rot, true))
+    if (rope_cache_prompt(n_tokens, n_seqs, v_pages ? Hkv * hd : 0, rot, true))
         return rope_cache_launch<true>(part, S, slice, q_out, k_pages, v_pages, freqs, tok_seq, tok_pos, table,
                                        table_stride, n_tokens, H, Hkv, hd, rot, stream);
     const dim3 grid(n_tokens, ((H + 2 * Hkv) * (hd / 8) + 255) / 256);
@@ -860,12 +867,12 @@ extern "C" int gfa_rope_cache_write_sliced(const float* part, int S, void* q_out
 
 extern "C" int gfa_rope_cache_write(const void* qkv, void* q_out, void* k_pages, void* v_pages,
                                     const float* freqs, const int* tok_seq, const int* tok_pos,
-                                    const int* table, int table_stride, int n_tokens, int H,
+                                    const int* table, int table_stride, int n_seqs, int n_tokens, int H,
                                     int Hkv, int hd, int rot, int layout, int is_bf16,
                                     hipStream_t stream) {
     if (n_tokens <= 0) return 0;
     if (is_bf16 && layout == 0 && hd % 8 == 0 && rot % 8 == 0) {
-        if (rope_cache_prompt(n_tokens, rot, false))
+        if (rope_cache_prompt(n_tokens, n_seqs, v_pages ? Hkv * hd : 0, rot, false))
             return rope_cache_launch<false>(qkv, 1, 0, q_out, k_pages, v_pages, freqs, tok_seq, tok_pos, table,
                                             table_stride, n_tokens, H, Hkv, hd, rot, stream);
         const dim3 grid8(n_tokens, ((H + 2 * Hkv) * (hd / 8) + 255) / 256);

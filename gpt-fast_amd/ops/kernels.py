@@ -233,7 +233,7 @@ def rope_cache_write(qkv: torch.Tensor, freqs: Optional[torch.Tensor], tok_seq, 
         raise KernelError("rope: q_out has the wrong size or dtype")
     check(library("core").gfa_rope_cache_write(
         ptr(qkv), ptr(q_out), ptr(k_pages), ptr(v_pages), ptr(freqs), ptr(tok_seq), ptr(tok_pos),
-        ptr(table), _i(table.shape[1]), _i(n), _i(n_heads), _i(n_kv_heads), _i(head_dim),
+        ptr(table), _i(table.shape[1]), _i(table.shape[0]), _i(n), _i(n_heads), _i(n_kv_heads), _i(head_dim),
         _i(rotary_dim), _i(layout), _i(_is_bf16(qkv)), stream_handle()), "rope_cache_write")
     return q_out
 
@@ -267,7 +267,7 @@ def rope_cache_write_sliced(part: torch.Tensor, freqs: Optional[torch.Tensor], t
     q_out = torch.empty((n, n_heads, head_dim), dtype=torch.bfloat16, device=part.device)
     check(library("core").gfa_rope_cache_write_sliced(
         ptr(part), _i(S), ptr(q_out), ptr(k_pages), ptr(v_pages), ptr(freqs), ptr(tok_seq),
-        ptr(tok_pos), ptr(table), _i(table.shape[1]), _i(n), _i(n_heads), _i(n_kv_heads),
+        ptr(tok_pos), ptr(table), _i(table.shape[1]), _i(table.shape[0]), _i(n), _i(n_heads), _i(n_kv_heads),
         _i(head_dim), _i(rotary_dim), stream_handle()), "rope_cache_write_sliced")
     return q_out
 

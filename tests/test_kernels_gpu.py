@@ -110,11 +110,13 @@ def test_gemm_f32_is_the_same_in_every_tile(N, K_):
     assert torch.equal(out.view(80, N), whole[:80])
 
 
-@pytest.mark.parametrize("H,G,hd,rot", [(8, 2, 128, 128), (4, 4, 64, 32), (3, 1, 24, 8), (2, 1, 80, 80),
-                                        (20, 20, 128, 128)])
-@pytest.mark.parametrize("lens,starts", [((401,), (0,)), ((3, 5, 640, 17, 8), (61, 7, 3, 0, 56)), ((9,) * 80, range(80))])
+@pytest.mark.parametrize("H,G,hd,rot,lens,starts", [
+    (*heads, *tokens) for heads in ((8, 2, 128, 128), (4, 4, 64, 32), (3, 1, 24, 8), (2, 1, 80, 80), (20, 20, 128, 128))
+    for tokens in (((401,), (0,)), ((3, 5, 640, 17, 8), (61, 7, 3, 0, 56)), ((9,) * 80, range(80)))] + [
+    (8, 2, 128, 128, (3, 5, 2100, 17), (61, 7, 3, 0)), (4, 4, 64, 32, (9, 2100, 44), (50, 3, 64)),
+    (3, 1, 24, 8, (22000, 3), (0, 5)), (2, 1, 80, 80, (61, 6600, 9), (3, 1, 60)), (9, 8, 64, 64, (2100, 7), (6, 0))])
 def test_rotation_and_cache_write_of_many_tokens(H, G, hd, rot, lens, starts):
-    """The kernel of prompts against the one of few tokens (the same rows in steps of at most 160): whole
+    """The kernel of prompts against the one of few tokens (the same rows in steps of at most 100): whole
     groups of eight keys, groups that begin or end inside a step, neighbouring sequences.  The same bits, those
     of values that are no number among them: a key may not depend on how its prompt is cut into steps."""
     g = torch.Generator().manual_seed(hd + H)
@@ -136,7 +138,7 @@ def test_rotation_and_cache_write_of_many_tokens(H, G, hd, rot, lens, starts):
             qs.append(K().rope_cache_write_sliced(part[:, a:b].contiguous(), *maps) if sliced
                       else K().rope_cache_write(qkv[a:b].contiguous(), *maps, 0))
         return [torch.cat(qs), *pages]
-    few = list(range(0, n, 160)) + [n]
+    few = list(range(0, n, 100)) + [n]
     for sliced in (False, True):
         if sliced and n < 640:
             continue
