@@ -144,7 +144,7 @@ __device__ __forceinline__ void pt_find_tile(const int* __restrict__ offsets, in
 #define PT_AS3(p) ((__attribute__((address_space(3))) void*)(p))
 
 template <int TM, int TN, int MODE>
-__global__ __launch_bounds__(PT_WAVES * 64, (TM + TN) * 64 * 256 <= 79 * 1024 ? 2 : 1)
+__global__ __launch_bounds__(PT_WAVES * 64, (TM + TN) * 64 * 256 <= 80 * 1024 ? 2 : 1)
 void prompt_tile_kernel(const PtArgs g) {
     constexpr int BM = 64 * TM, BN = 64 * TN;
     constexpr int UX = BM / 32, UW = BN / 32, U = UX + UW;       // 1 KB copies (8 rows) of a wave and piece
@@ -153,7 +153,7 @@ void prompt_tile_kernel(const PtArgs g) {
     // 4,096: tiles of 256 x 256 374 -> 368 us, 256 x 128 409 -> 384, but 128 x 128 368 -> 432)
     constexpr bool ASK = (BM + BN) * 256 > 80 * 1024;
     constexpr int G = 4;                                         // row tiles that run through the columns together
-    __shared__ __attribute__((aligned(1024))) char lds[2 * BUF + PT_WAVES * 256];
+    __shared__ __attribute__((aligned(1024))) char lds[2 * BUF + (ASK ? PT_WAVES * 256 : 0)];
 
     const int F = g.F, N = MODE == PT_GATE ? 2 * F : F;          // columns of out, rows of an expert's W
     constexpr int CN = MODE == PT_GATE ? BN / 2 : BN;            // columns of out that a tile makes
