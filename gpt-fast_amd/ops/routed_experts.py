@@ -255,6 +255,14 @@ def expert_tiles(offsets: torch.Tensor, n_experts: int, pairs: int) -> torch.Ten
     return tiles
 
 
+def takes_tile_list(w: torch.Tensor, gated: bool = False) -> bool:
+    """Whether :func:`expert_tile_product` with these experts takes the kernel that needs the list of
+    :func:`expert_tiles`: inner sizes that are no whole pieces of 64, results of no whole 16 bytes, matrices of
+    4 GiB and more."""
+    N, K = w.shape[1:]
+    return K % 64 != 0 or (N // 2 if gated else N) % 8 != 0 or not 0 < N * K * 2 < 1 << 32
+
+
 def expert_tile_product(x: torch.Tensor, order: Optional[torch.Tensor], top: int, w: torch.Tensor,
                         offsets: torch.Tensor, tiles: Optional[torch.Tensor], pairs: int,
                         activation: Optional[str] = None, gated: bool = False,
@@ -262,9 +270,8 @@ def expert_tile_product(x: torch.Tensor, order: Optional[torch.Tensor], top: int
     """bfloat16 [pairs, F]: row p of expert e is ``act(W[e] x[r])``, r = ``order[p] // top`` (or p itself
     without ``order``); ``gated``: W is [E, 2 F, K] and the row ``act(W_gate x) * (W_up x)``, or the
     clamped gate.  Rows that belong to no expert are not written.  Operands as for
-    :func:`grouped_rows`; nothing is read on the host.  Inner sizes of whole pieces of 64 and F of whole
-    16 bytes take the kernel that finds its tiles in ``offsets``; other sizes take one that needs
-    ``tiles`` (:func:`expert_tiles`; None: made here)."""
+    :func:`grouped_rows`; nothing is read on the host.  Where :func:`takes_tile_list`
+    says so it needs ``tiles`` (:func:`expert_tiles`; None: made here), else it finds them in ``offsets``."""
     require_device(x, order, w, offsets, tiles)
     require_contiguous(x=x, order=order, w=w, offsets=offsets, tiles=tiles)
     if not grouped_rows_take(x, w):
@@ -288,7 +295,7 @@ def expert_tile_product(x: torch.Tensor, order: Optional[torch.Tensor], top: int
     out = torch.empty((pairs, F), dtype=torch.bfloat16, device=x.device)
     mode = 3 if clamped else (2 if gated else (1 if activation is not None else 0))
     act = 0 if clamped or activation is None else ACTIVATIONS[activation]
-    if K % 64 == 0 and F % 8 == 0 and 0 < N * K * 2 < 1 << 32:
+    if not takes_tile_list(w, gated):
         check(library("routed_experts").gfa_expert_rows_product(
             ptr(x), ptr(order), _i(max(1, top)), ptr(w), ptr(offsets), _i(E), _i(pairs), ptr(out), _i(F), _i(K),
             _i(mode), _i(act), _f(limit or 0.0), stream_handle()), "expert_tile_product")

@@ -143,9 +143,12 @@ class RoutedExperts(Part):
                                        gated=s.gated, limit=s.limit)
         offsets, order, place = RE.expert_order(chosen, self.n_choices)
         if RE.grouped_rows_take(x, self.w_up) and s.hidden % 8 == 0:
-            hs = RE.expert_tile_product(x, order, s.top, self.w_up, offsets, None, n * s.top, s.activation,
+            # one list of tiles for both products, if one of them needs it
+            listed = RE.takes_tile_list(self.w_up, s.gated) or RE.takes_tile_list(self.w_down)
+            tiles = RE.expert_tiles(offsets, s.n_experts, n * s.top) if listed else None
+            hs = RE.expert_tile_product(x, order, s.top, self.w_up, offsets, tiles, n * s.top, s.activation,
                                         s.gated, s.limit)
-            ys = RE.expert_tile_product(hs, None, 1, self.w_down, offsets, None, n * s.top)
+            ys = RE.expert_tile_product(hs, None, 1, self.w_down, offsets, tiles, n * s.top)
             return RE.combine_pairs(ys, place, weights, out=y, identity=identity)
         bounds = offsets.cpu().tolist()                         # the host learns the experts' shares
         most = max(bounds[e + 1] - bounds[e] for e in range(s.n_experts))

@@ -356,6 +356,19 @@ def test_an_experts_activation_is_the_same_in_every_kernel(act, gated, limit):
         assert torch.equal(got[0].view(torch.int16), other.view(torch.int16))
 
 
+@pytest.mark.parametrize("D,Fh,lists", [(96, 40, 1), (64, 72, 1), (72, 64, 1), (64, 64, 0)])
+def test_a_layer_makes_one_list_of_tiles_for_both_products_or_none(monkeypatch, D, Fh, lists):
+    """By inner sizes that are whole pieces of 64 or not, for either product."""
+    from gpt_fast_amd.ops import routed_experts as RE
+    part, rt, w, mlp = _mixture(5, 0, 2, D, Fh, 0.8, None, "bfloat16")
+    made, make = [], RE.expert_tiles
+    monkeypatch.setattr(RE, "expert_tiles", lambda *a: made.append(a) or make(*a))
+    x = torch.randn(90, D, device=DEV).bfloat16()
+    want = P.mixture(w, "", mlp, x.double().cpu())
+    assert rel_err(part.forward_rows(x, None), want) < 5e-2
+    assert len(made) == lists
+
+
 def test_the_correction_moves_the_choice_and_not_the_weights():
     part, rt, w, mlp = _mixture(4, 2, 2, 64, 32, 1.0, None, "float32")
     part.correction.copy_(torch.tensor([0.0, 0.0, 0.0, 0.0, 5.0, 5.0]))     # both identity experts, always
