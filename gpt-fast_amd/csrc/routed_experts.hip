@@ -864,7 +864,8 @@ extern "C" int gfa_expert_tile_product(const void* x, const int* order, int top,
 }
 
 // The same product for inner sizes of whole pieces of 64 and rows of out of whole 16 bytes, by the tile kernel of
-// prompt_tile.h, which finds its tiles in `offsets` itself; the kernel above serves the other sizes.
+// prompt_tile.h, which finds its tiles in `offsets` itself.  The caller chooses between it and the kernel above, and
+// its tile.
 template <int TM, int TN>
 static int expert_rows_launch(const PtArgs& a, int mode, int pairs, hipStream_t stream) {
     const int cols = mode >= 2 ? 32 * TN : 64 * TN;
@@ -877,14 +878,15 @@ static int expert_rows_launch(const PtArgs& a, int mode, int pairs, hipStream_t 
     return GFA_LAUNCH_RESULT();
 }
 
+// tile: 1, 2, 4 for tiles of 64 x 256, 128 x 128 and 256 x 256 rows of x and of W.
 extern "C" int gfa_expert_rows_product(const void* x, const int* order, int top, const void* w,
                                        const int* offsets, int E, int pairs, void* out, int F, int K, int mode,
-                                       int act, float limit, hipStream_t stream) {
+                                       int act, float limit, int tile, hipStream_t stream) {
     if (pairs <= 0) return 0;
     const long long matrix = (long long)(mode >= 2 ? 2 : 1) * F * K * 2;
     if (E <= 0 || E > 8192 || F <= 0 || F % 8 || K <= 0 || K % 64 || top <= 0 || mode < 0 || mode > 3 ||
-        (act != 0 && act != 1 && act != 3) || matrix > 0xffffffffLL || (uintptr_t)x % 16 || (uintptr_t)w % 16 ||
-        (uintptr_t)out % 16)
+        (act != 0 && act != 1 && act != 3) || (tile != 1 && tile != 2 && tile != 4) || matrix > 0xffffffffLL ||
+        (uintptr_t)x % 16 || (uintptr_t)w % 16 || (uintptr_t)out % 16)
         return (int)hipErrorInvalidValue;
     PtArgs a{};
     a.x = (const bf16_t*)x;
@@ -898,12 +900,7 @@ extern "C" int gfa_expert_rows_product(const void* x, const int* order, int top,
     a.offsets = offsets;
     a.top = top;
     a.E = E;
-    // By the rows an expert has on average.  Microseconds of both products of 32 experts (4,096 -> 3,584 -> 4,096;
-    // in brackets gated, 4,096 -> 2 x 2,048 -> 4,096) with tiles of 64 x 256, 128 x 128 and 256 x 256 rows and
-    // columns, and by expert_tile_kernel:
-    //   5 rows: 341, -, -; 436 (284, -, -; 411)         62 rows: 493, 384, -; 477 (401, 315, -; 424)
-    //   222 rows: 1,106, 768, 723; 830 (928, 665, 563; 664)
-    if (pairs < 40LL * E) return expert_rows_launch<1, 4>(a, mode, pairs, stream);
-    if (pairs < 128LL * E) return expert_rows_launch<2, 2>(a, mode, pairs, stream);
+    if (tile == 1) return expert_rows_launch<1, 4>(a, mode, pairs, stream);
+    if (tile == 2) return expert_rows_launch<2, 2>(a, mode, pairs, stream);
     return expert_rows_launch<4, 4>(a, mode, pairs, stream);
 }

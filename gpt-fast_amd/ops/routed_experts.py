@@ -1,11 +1,14 @@
 """Python faces of csrc/routed_experts.hip: the router's choice per token and the products of
 the chosen experts.  Shape checks on the host, then the launch."""
 import ctypes
+import functools
+import math
 from typing import Optional
 
 import torch
 
 from .kernels import ACTIVATIONS, check_gate_limit
+from .linear import _compute_units
 from .library import KernelError, check, library, ptr, require_contiguous, require_device, stream_handle
 
 _i, _f, _ll = ctypes.c_int, ctypes.c_float, ctypes.c_longlong
@@ -255,12 +258,70 @@ def expert_tiles(offsets: torch.Tensor, n_experts: int, pairs: int) -> torch.Ten
     return tiles
 
 
-def takes_tile_list(w: torch.Tensor, gated: bool = False) -> bool:
+def _tiles(pairs: int, n_experts: int, rows: int, F: int, columns: int) -> float:
+    """Tiles of ``rows`` x ``columns`` that the experts' products have on average, their shares of the pairs spread
+    evenly from half to one and a half of the mean."""
+    mean = pairs / n_experts
+    of_one = sum(min(1.0, 1.5 - rows * k / mean) for k in range(math.ceil(1.5 * mean / rows)))
+    return of_one * min(n_experts, pairs) * ((F + columns - 1) // columns)
+
+
+@functools.lru_cache(maxsize=4096)
+def rows_tile(n_experts: int, pairs: int, F: int, K: int, mode: int, units: int) -> int:
+    """Which kernel makes the experts' products of ``pairs`` rows of K into rows of F on ``units`` compute units
+    (``mode`` 0: the sums, 1: an activation of them, 2: a gated one): 1, 2 or 4 for the tile kernel
+    (csrc/prompt_tile.h) with tiles of 64 x 256, 128 x 128 or 256 x 256 rows of x and of W, 0 for the older one
+    (``expert_tile_kernel``, which needs :func:`expert_tiles`).
+
+    The rows of an expert are known on the device alone; on the host there is their mean.  A round of the chip is one
+    tile 4 to a unit, two of tile 1 or 2, three of the older kernel's.  Microseconds, n x m being n experts of m rows
+    on average:
+
+    * From 36 rows on shares above 64 become frequent, whose matrices the 64 x 256 tile reads twice: 64 x 34,
+      1,280 -> 2,048 tile 1 68, tile 2 76; 32 x 39, 3,584 -> 4,096 219, 179.  Below, where its workgroups
+      are fewer than the units, tile 2 has twice as many: 8 x 10, 4,096 -> 2 x 2,048 74, 68.
+    * Where tile 2 does not need a second round it is the best: 8 x 400, 1,024 -> 2 x 512 older 23, tile 2 19, tile 4
+      38; 8 x 170, 4,096 -> 2 x 2,048 101, 90, 109, but x 222, beyond the round, 131, 143, 114.
+    * Up to K = 1,024 a tile is over so soon that its first loads and its last stores show; over some rounds the older
+      kernel, three to a unit, hides them best: 64 x 62, 1,024 -> 2 x 1,024 69, tile 2 77; 128 x 62, 768 -> 2,048 100,
+      110; 256 x 140, 512 -> 2 x 1,024 207, 253.  Over fewer it is not worth the list (3 to 8 us): 64 x 62, 768 ->
+      2,048 64, 58; 128 x 127, 512 -> 2 x 256 37, 31.  Sums alone of K = 1,024: 128 x 222, 1,024 -> 4,096 older 473,
+      tile 4 475; x 400 724, 686.
+    * 256 x 256 tiles read each operand half as often, from about 120 rows on: 32 x 127, 4,096 -> 2 x 2,048 tile 2
+      306, tile 4 277; x 90 267, 272; with a round that they just fill, sooner: 16 x 100, 4,096 -> 4,096 167, 136.  A
+      second or third round that they hardly need costs more than that: 16 x 190 183, 222; x 300 259, 228;
+      128 x 260, 2,048 -> 1,024 278, 316."""
+    gated = mode == 2
+    if pairs < 36 * n_experts:
+        columns = 128 if gated else 256
+        return 1 if min(n_experts, pairs) * ((F + columns - 1) // columns) >= units else 2
+    small = _tiles(pairs, n_experts, 128, F, 64 if gated else 128)
+    if small <= 2 * units:
+        return 2
+    if K <= 1024:
+        if mode == 0 and K == 1024 and pairs >= 400 * n_experts:
+            return 4
+        return 0 if small >= min(8, 4096 / K) * units else 2
+    rounds = _tiles(pairs, n_experts, 256, F, 128 if gated else 256) / units
+    if 1.0 < rounds < 3.1 and 0.0 < rounds % 1.0 < 0.35:
+        return 2
+    return 4 if pairs >= 120 * n_experts or rounds <= 1.0 else 2
+
+
+def _tile_of(w: torch.Tensor, mode: int, pairs: int) -> int:
+    """:func:`rows_tile` where the tile kernel takes these experts (inner sizes of whole pieces of 64, results of
+    whole 16 bytes, matrices below 4 GiB), else 0."""
+    E, N, K = w.shape
+    F = N // 2 if mode == 2 else N
+    if K % 64 != 0 or F % 8 != 0 or not 0 < N * K * 2 < 1 << 32:
+        return 0
+    return rows_tile(E, pairs, F, K, mode, _compute_units(w.device))
+
+
+def takes_tile_list(w: torch.Tensor, activation: Optional[str], gated: bool, pairs: int) -> bool:
     """Whether :func:`expert_tile_product` with these experts takes the kernel that needs the list of
-    :func:`expert_tiles`: inner sizes that are no whole pieces of 64, results of no whole 16 bytes, matrices of
-    4 GiB and more."""
-    N, K = w.shape[1:]
-    return K % 64 != 0 or (N // 2 if gated else N) % 8 != 0 or not 0 < N * K * 2 < 1 << 32
+    :func:`expert_tiles`."""
+    return _tile_of(w, 2 if gated else int(activation is not None), pairs) == 0
 
 
 def expert_tile_product(x: torch.Tensor, order: Optional[torch.Tensor], top: int, w: torch.Tensor,
@@ -295,10 +356,11 @@ def expert_tile_product(x: torch.Tensor, order: Optional[torch.Tensor], top: int
     out = torch.empty((pairs, F), dtype=torch.bfloat16, device=x.device)
     mode = 3 if clamped else (2 if gated else (1 if activation is not None else 0))
     act = 0 if clamped or activation is None else ACTIVATIONS[activation]
-    if not takes_tile_list(w, gated):
+    tile = _tile_of(w, min(mode, 2), pairs)
+    if tile:
         check(library("routed_experts").gfa_expert_rows_product(
             ptr(x), ptr(order), _i(max(1, top)), ptr(w), ptr(offsets), _i(E), _i(pairs), ptr(out), _i(F), _i(K),
-            _i(mode), _i(act), _f(limit or 0.0), stream_handle()), "expert_tile_product")
+            _i(mode), _i(act), _f(limit or 0.0), _i(tile), stream_handle()), "expert_tile_product")
         return out
     if tiles is None:
         tiles = expert_tiles(offsets, E, pairs)

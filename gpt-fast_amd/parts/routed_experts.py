@@ -144,11 +144,13 @@ class RoutedExperts(Part):
         offsets, order, place = RE.expert_order(chosen, self.n_choices)
         if RE.grouped_rows_take(x, self.w_up) and s.hidden % 8 == 0:
             # one list of tiles for both products, if one of them needs it
-            listed = RE.takes_tile_list(self.w_up, s.gated) or RE.takes_tile_list(self.w_down)
-            tiles = RE.expert_tiles(offsets, s.n_experts, n * s.top) if listed else None
-            hs = RE.expert_tile_product(x, order, s.top, self.w_up, offsets, tiles, n * s.top, s.activation,
+            pairs = n * s.top
+            listed = RE.takes_tile_list(self.w_up, s.activation, s.gated, pairs) or \
+                RE.takes_tile_list(self.w_down, None, False, pairs)
+            tiles = RE.expert_tiles(offsets, s.n_experts, pairs) if listed else None
+            hs = RE.expert_tile_product(x, order, s.top, self.w_up, offsets, tiles, pairs, s.activation,
                                         s.gated, s.limit)
-            ys = RE.expert_tile_product(hs, None, 1, self.w_down, offsets, tiles, n * s.top)
+            ys = RE.expert_tile_product(hs, None, 1, self.w_down, offsets, tiles, pairs)
             return RE.combine_pairs(ys, place, weights, out=y, identity=identity)
         bounds = offsets.cpu().tolist()                         # the host learns the experts' shares
         most = max(bounds[e + 1] - bounds[e] for e in range(s.n_experts))

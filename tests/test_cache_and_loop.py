@@ -544,6 +544,21 @@ def test_dispatch_thresholds_follow_the_number_of_compute_units():
         del L._units["fake256"], L._units["fake64"]
 
 
+def test_the_kernel_of_the_experts_rows_goes_by_their_sizes_and_the_chip():
+    """0: the older kernel, 1, 2, 4: tiles of 64 x 256, 128 x 128, 256 x 256."""
+    from gpt_fast_amd.ops.routed_experts import rows_tile
+
+    def tiles(E, F, K, mode, means, units=256):
+        return [rows_tile(E, int(m * E), F, K, mode, units) for m in means]
+    assert tiles(32, 3584, 4096, 1, (0.5, 1, 35, 36, 119, 120, 800)) == [2, 1, 1, 2, 2, 4, 4]
+    assert tiles(8, 2048, 4096, 2, (1, 35, 36, 170, 222)) == [2, 2, 2, 2, 4]      # a round of tiles of 128 x 128
+    assert tiles(8, 512, 1024, 2, (1, 129, 400, 800)) == [2, 2, 2, 2]
+    assert tiles(128, 2048, 768, 0, (1, 35, 36, 400)) == [1, 1, 0, 0]
+    assert tiles(128, 256, 512, 2, (127, 400)) == [2, 2] and tiles(128, 256, 512, 2, (400,), units=64) == [0]
+    assert tiles(128, 4096, 1024, 0, (399, 400)) == [0, 4] and tiles(128, 4096, 1024, 1, (400,)) == [0]
+    assert tiles(16, 4096, 4096, 0, (85, 100, 160, 190, 300)) == [2, 4, 4, 2, 4]     # one round, a little more
+
+
 def test_residual_stream_runs_what_was_put_off_before_any_read():
     """The stream holds at most one part's last kernels back; every read - the rows of a norm
     or the tensor itself - runs them first, telling them the norm that reads (only if all

@@ -290,14 +290,16 @@ def test_tiles_of_the_experts_rows(E, D, Fh, counts):
 @pytest.mark.parametrize("E,D,Fh,counts", [(3, 64, 8, [1, 0, 70]), (70, 128, 24, [3] * 69 + [30]),
                                            (4, 192, 136, [40, 64, 0, 65]), (2, 512, 128, [127, 129]),
                                            (3, 4096, 264, [1, 257, 300]), (5, 576, 72, [0, 511, 0, 1, 256])])
-def test_the_experts_rows_in_tiles_of_whole_pieces(E, D, Fh, counts):
+@pytest.mark.parametrize("tile", [1, 2, 4])
+def test_the_experts_rows_in_tiles_of_whole_pieces(monkeypatch, E, D, Fh, counts, tile):
     """Inner sizes of one, two and many pieces, columns that end inside a tile, more experts than lanes,
-    shares at the edges of 64, 128 and 256 rows, and each of the three tiles that the average share picks;
+    shares at the edges of 64, 128 and 256 rows, and each of the three tiles;
     against the same bfloat16 operands in float64.  The result is rounded to bfloat16 once, which moves a
     value by at most 2^-8 of itself (eight bits of significand), after sums of D float32 products (2^-24
     each)."""
     from gpt_fast_amd.ops import routed_experts as RE
     g = torch.Generator().manual_seed(D + E)
+    monkeypatch.setattr(RE, "rows_tile", lambda *sizes: tile)
     top, n = 2, (sum(counts) + 5 + 1) // 2
     pairs = n * top
     ids = torch.tensor([e for e, c in enumerate(counts) for _ in range(c)] + [E] * (pairs - sum(counts)), dtype=torch.int32)
