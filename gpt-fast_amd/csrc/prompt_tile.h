@@ -15,9 +15,9 @@
 //    the one barrier of a piece stands before its last 16 k, so that nothing waits behind it;
 //  * copies are spread over three of a piece's four steps instead of issued in a burst (a burst fills the
 //    address unit and holds the products up);
-//  * in the tiles that fill a compute unit by themselves, lines are asked for two pieces before they are
-//    copied (one dword of 64 lines per instruction, into shared memory that nobody reads), those of x by one of
-//    the workgroups of an XCD that share them, so that the copies find them in that XCD's cache.
+//  * in the tile that fills a compute unit by itself, the lines of W are asked for two pieces before they are
+//    copied (one dword of 64 lines per instruction, into shared memory that nobody reads), so that the copies find
+//    them in the XCD's cache.
 // The copies are written in asm because the compiler takes any operand read to depend on every copy in
 // flight and waits for all of them; they have no output registers, and the waits below count them.
 #pragma once
@@ -203,15 +203,11 @@ void prompt_tile_kernel(const PtArgs g) {
     }
     const char* wbase = (const char*)(we + (size_t)wfirst * K);
 
-    // the line (of the pieces to come) that this lane asks for: one of the tile's rows of W, or its share of the
-    // rows of x that this XCD's workgroups of the same rows read
+    // the line (of the pieces to come) that this lane asks for: one of the tile's rows of W
     const char* line = nullptr;
     if (ASK) {
-        constexpr int lw = BN / PT_WAVES, lx = BM / PT_WAVES / 4 < 64 - lw ? BM / PT_WAVES / 4 : 64 - lw;
-        const int l = lane < lw + lx ? lane : 0;
-        const bf16_t* row = l < lw ? we + (size_t)w_row(wave * lw + l) * K
-                                   : g.x + (size_t)x_row((bn & 3) * (BM / 4) + wave * (BM / 16) + (l - lw)) * K;
-        line = (const char*)row;
+        static_assert(BN / PT_WAVES <= 64, "a lane asks for one line");
+        line = (const char*)(we + (size_t)w_row(wave * (BN / PT_WAVES) + lane % (BN / PT_WAVES)) * K);
     }
     const uint32_t lds_at = (uint32_t)(uintptr_t)PT_AS3(lds);
     // copy i of the wave (x first) of piece t into buffer b
