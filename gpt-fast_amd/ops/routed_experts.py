@@ -289,8 +289,8 @@ def rows_tile(n_experts: int, pairs: int, F: int, K: int, mode: int, units: int)
       tile 4 475; x 400 724, 686.
     * 256 x 256 tiles read each operand half as often, from about 120 rows on: 32 x 127, 4,096 -> 2 x 2,048 tile 2
       306, tile 4 277; x 90 267, 272; with a round that they just fill, sooner: 16 x 100, 4,096 -> 4,096 167, 136.  A
-      second or third round that they hardly need costs more than that: 16 x 190 183, 222; x 300 259, 228;
-      128 x 260, 2,048 -> 1,024 278, 316."""
+      second or third round that they hardly need costs more than that: 16 x 190 183, 222; x 222 233, 224; x
+      300 259, 228; 64 x 222, 2,048 -> 1,024 137, 155."""
     gated = mode == 2
     if pairs < 36 * n_experts:
         columns = 128 if gated else 256
@@ -303,7 +303,7 @@ def rows_tile(n_experts: int, pairs: int, F: int, K: int, mode: int, units: int)
             return 4
         return 0 if small >= min(8, 4096 / K) * units else 2
     rounds = _tiles(pairs, n_experts, 256, F, 128 if gated else 256) / units
-    if 1.0 < rounds < 3.1 and 0.0 < rounds % 1.0 < 0.35:
+    if 1.0 < rounds < 3.1 and 0.0 < rounds % 1.0 < (0.35 if K <= 2048 else 0.3):
         return 2
     return 4 if pairs >= 120 * n_experts or rounds <= 1.0 else 2
 

@@ -556,7 +556,8 @@ def test_the_kernel_of_the_experts_rows_goes_by_their_sizes_and_the_chip():
     assert tiles(128, 2048, 768, 0, (1, 35, 36, 400)) == [1, 1, 0, 0]
     assert tiles(128, 256, 512, 2, (127, 400)) == [2, 2] and tiles(128, 256, 512, 2, (400,), units=64) == [0]
     assert tiles(128, 4096, 1024, 0, (399, 400)) == [0, 4] and tiles(128, 4096, 1024, 1, (400,)) == [0]
-    assert tiles(16, 4096, 4096, 0, (85, 100, 160, 190, 300)) == [2, 4, 4, 2, 4]     # one round, a little more
+    assert tiles(16, 4096, 4096, 0, (85, 100, 160, 190, 222, 300)) == [2, 4, 4, 2, 4, 4]     # one round, a little more
+    assert tiles(64, 1024, 2048, 1, (160, 190, 222)) == [4, 2, 2]
 
 
 def test_residual_stream_runs_what_was_put_off_before_any_read():
