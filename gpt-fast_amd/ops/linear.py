@@ -207,7 +207,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         if S > 1:
             rows = SlicedRows(_library_partial_sums(x, w, S), out_dtype)
             return rows if may_stay_sliced else rows.rows()
-        first = _whole_rounds(M, w.shape[0], x.shape[1], x.device)
+        # a product into a given tensor has no gradient
+        recorded = torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)
+        first = 0 if recorded else _whole_rounds(M, w.shape[0], x.shape[1], x.device)
         if first:
             out = torch.empty((M, w.shape[0]), dtype=x.dtype, device=x.device)
             torch.matmul(x[:first], w.t(), out=out[:first])

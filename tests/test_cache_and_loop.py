@@ -544,6 +544,28 @@ def test_dispatch_thresholds_follow_the_number_of_compute_units():
         del L._units["fake256"], L._units["fake64"]
 
 
+def test_a_product_in_whole_rounds_keeps_its_gradient():
+    """Rows beyond a whole round of a chip of eight units: with a gradient, the product's own; without, the same rows
+    but for the rounding to bfloat16 (2^-8 of a value) of sums in another order."""
+    from gpt_fast_amd.ops import linear as L
+    device = torch.device("cpu")
+    g = torch.Generator().manual_seed(1)
+    x, w = (torch.randn(n, 2048, generator=g).bfloat16() for n in (300, 2048))
+    L._units[device] = 8
+    try:
+        assert L._whole_rounds(300, 2048, 2048, device) == 256
+        plain = L.linear(x, w)
+        w.requires_grad_(True)
+        rows = L.linear(x, w)
+        rows.float().sum().backward()
+    finally:
+        del L._units[device]
+    assert float((plain.float() - rows.detach().float()).abs().max()) <= 2.0 ** -7 * float(rows.abs().max())
+    got, w.grad = w.grad, None
+    torch.matmul(x, w.t()).float().sum().backward()
+    assert torch.equal(got, w.grad)
+
+
 def test_the_kernel_of_the_experts_rows_goes_by_their_sizes_and_the_chip():
     """0: the older kernel, 1, 2, 4: tiles of 64 x 256, 128 x 128, 256 x 256."""
     from gpt_fast_amd.ops.routed_experts import rows_tile
