@@ -102,17 +102,26 @@ def _whole_rounds(M: int, N: int, K_: int, device) -> int:
     """Rows that a product of the vendor library should take first, the others in a second one; 0: all at
     once.  Its best kernels make 256 x 256 tiles, one to a compute unit; where these columns divide the
     units, ``round`` rows fill the chip exactly, and for some numbers of rows beyond whole rounds the library
-    picks kernels that take far longer than its own two products for the whole rounds and the rest
-    (N = 4,096, K = 14,336, round 4,096, with the sum and norm behind it: 4,200 rows 750 us as one product,
-    427 as two; 5,500: 877, 525; 6,001: 586, 567; 7,491: 1,046, 683; 9,000: 1,203, 830).  Nothing is gained where
-    the rest nearly fills a round itself (8,000 rows: 697, 700; K = 4,096, 7,491 rows: 239, 256), sooner with
-    a short inner size (K = 4,096, 6,500 rows: 228, 220).  Measured for N of 2,048, 4,096 and 8,192, K >= N."""
+    picks kernels that take far longer than its own two products for the whole rounds and the rest.  Microseconds as
+    one product and as two, with the sum and norm behind it:
+
+    * N = 4,096, K = 14,336 (round 4,096): 4,097 rows 757, 356; 4,160 756, 356; 4,396 798, 383; 5,120 485, 452; 6,144
+      560, 538; 7,372 1,053, 705; 8,193 1,086, 691; 10,240 1,206, 868.  8,000 rows, whose rest nearly fills a round
+      itself: 697, 700.
+    * N = 2,048, K = 5,632 (8,192): 8,193 328, 187; 8,492 223, 199; 13,107 312, 312, but 14,745 326, 344: where K is
+      below 3 N the rest may be less of a round.
+    * N = K = 4,096 (4,096): 4,097 173, 146; 5,120 180, 185; 6,553 231, 233; 8,193 370, 283; 10,240 451, 359.
+    * N = K = 2,048 (8,192): 8,193 109, 106; 8,492 110, 111; 10,240 122, 133; 12,288 141, 152: products so short that
+      two norms instead of one show.
+
+    Measured for N of 2,048, 4,096 and 8,192, K >= N, rests from one row on."""
     cus = _compute_units(device)
     if N % 256 or not 8 <= N // 256 <= 32 or cus % (N // 256) or K_ < N:
         return 0
     per_round = 256 * (cus // (N // 256))
     rest = M % per_round
-    if M <= per_round or rest == 0 or rest * 20 >= per_round * (18 if K_ >= 2 * N else 13):
+    most = 18 if K_ >= 3 * N else 13 if K_ >= 2 * N or N >= 4096 else 5      # twentieths of a round
+    if M <= per_round or rest == 0 or rest * 20 >= per_round * most:
         return 0
     return M - rest
 

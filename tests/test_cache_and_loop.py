@@ -538,6 +538,8 @@ def test_dispatch_thresholds_follow_the_number_of_compute_units():
             == [0, 4096, 4096, 0, 0, 8192]
         assert [L._whole_rounds(M, 4096, 4096, "fake256") for M in (6500, 7491)] == [4096, 0]
         assert L._whole_rounds(2100, 8192, 8192, "fake256") == 2048
+        assert [L._whole_rounds(M, 2048, 5632, "fake256") for M in (13107, 14745)] == [8192, 0]
+        assert [L._whole_rounds(M, 2048, 2048, "fake256") for M in (8193, 10239, 10240, 12288)] == [8192, 8192, 0, 0]
         assert L._whole_rounds(7491, 28672, 4096, "fake256") == 0     # its columns do not divide the units
         assert L._whole_rounds(7491, 6144, 4096, "fake256") == 0
     finally:
