@@ -449,7 +449,8 @@ def test_the_attention_gates_its_heads_and_finds_a_key_that_stands_out(dtype, to
             assert rel_err(got.permute(1, 0, 2), want) < tol, (lens, starts, n_parts)
 
 
-@pytest.mark.parametrize("H,hd,vd", [(3, 8, 16), (3, 192, 128), (5, 200, 128), (2, 192, 144), (2, 320, 256), (3, 328, 16),
+@pytest.mark.parametrize("H,hd,vd", [(3, 8, 16), (3, 192, 128), (5, 200, 128), (2, 192, 144), (2, 256, 128), (3, 264, 128),
+                                     (2, 192, 192), (3, 200, 192), (2, 192, 208), (2, 320, 256), (3, 328, 16),
                                      (4, 512, 512), (2, 520, 496), (3, 576, 16), (1, 8, 512)])
 def test_prompts_at_the_edges_of_the_sizes_one_form_serves(H, hd, vd):
     """Keys and values as large as a form takes, one step larger, and far smaller on one side, with and without a
