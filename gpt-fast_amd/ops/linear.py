@@ -18,6 +18,7 @@ float32 everywhere.
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
 
 from . import gemm_bf16, gemm_wide_bf16
 from . import gemm_tiled_bf16 as T
@@ -126,6 +127,21 @@ def _whole_rounds(M: int, N: int, K_: int, device) -> int:
     return M - rest
 
 
+def _computed_only(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether torch has no more to do with a product of these than to compute it.  Its products into a given tensor
+    have no gradient, no forward derivative and no form mapped over a dimension, and autocast leaves them alone."""
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad) or torch.is_autocast_enabled(x.device.type):
+        return False
+    try:
+        for t in (x, w):
+            t.untyped_storage()            # tensors of vmap and of torch.func's derivatives have none
+            if forward_ad.unpack_dual(t).tangent is not None:
+                return False
+    except RuntimeError:
+        return False
+    return True
+
+
 def _library_partial_sums(x: torch.Tensor, w: torch.Tensor, S: int) -> torch.Tensor:
     """float32 [S, M, N]: x W^T over each of S equal slices of the inner size, as one batched
     product of the vendor library over views of x and w (nothing is copied)."""
@@ -216,9 +232,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = 
         if S > 1:
             rows = SlicedRows(_library_partial_sums(x, w, S), out_dtype)
             return rows if may_stay_sliced else rows.rows()
-        # a product into a given tensor has no gradient
-        recorded = torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)
-        first = 0 if recorded else _whole_rounds(M, w.shape[0], x.shape[1], x.device)
+        first = _whole_rounds(M, w.shape[0], x.shape[1], x.device)
+        if first and not _computed_only(x, w):
+            first = 0
         if first:
             out = torch.empty((M, w.shape[0]), dtype=x.dtype, device=x.device)
             torch.matmul(x[:first], w.t(), out=out[:first])

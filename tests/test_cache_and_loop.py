@@ -546,23 +546,35 @@ def test_dispatch_thresholds_follow_the_number_of_compute_units():
         del L._units["fake256"], L._units["fake64"]
 
 
-def test_a_product_in_whole_rounds_keeps_its_gradient():
-    """Rows beyond a whole round of a chip of eight units: with a gradient, the product's own; without, the same rows
-    but for the rounding to bfloat16 (2^-8 of a value) of sums in another order."""
+def test_a_product_in_whole_rounds_is_still_differentiated_mapped_and_cast():
+    """Rows beyond a whole round of a chip of eight units.  By itself the product has the rows of the single one
+    but for the rounding to bfloat16 (2^-8 of a value) of sums in another order; with a gradient, a forward derivative,
+    under a map over either operand and under autocast it is torch's own."""
+    from torch.autograd import forward_ad
     from gpt_fast_amd.ops import linear as L
     device = torch.device("cpu")
     g = torch.Generator().manual_seed(1)
-    x, w = (torch.randn(n, 2048, generator=g).bfloat16() for n in (300, 2048))
+    x, t, w = (torch.randn(n, 2048, generator=g).bfloat16() for n in (300, 300, 2048))
+    want = torch.matmul(x, w.t())
     L._units[device] = 8
     try:
         assert L._whole_rounds(300, 2048, 2048, device) == 256
         plain = L.linear(x, w)
+        assert torch.equal(torch.vmap(lambda a: L.linear(a, w))(torch.stack([x, t]))[0], want)
+        assert torch.equal(torch.vmap(lambda a: L.linear(x, a))(torch.stack([w, w]))[1], want)
+        assert torch.equal(torch.func.jvp(lambda a: L.linear(a, w), (x,), (t,))[1], torch.matmul(t, w.t()))
+        with torch.no_grad(), forward_ad.dual_level():
+            dual = L.linear(forward_ad.make_dual(x, t), w)
+            assert torch.equal(forward_ad.unpack_dual(dual).tangent, torch.matmul(t, w.t()))
+        with torch.autocast("cpu", torch.float16):
+            assert L.linear(x, w).dtype == torch.float16
         w.requires_grad_(True)
         rows = L.linear(x, w)
         rows.float().sum().backward()
     finally:
         del L._units[device]
-    assert float((plain.float() - rows.detach().float()).abs().max()) <= 2.0 ** -7 * float(rows.abs().max())
+    assert float((plain.float() - want.float()).abs().max()) <= 2.0 ** -7 * float(want.abs().max())
+    assert torch.equal(rows.detach(), want)
     got, w.grad = w.grad, None
     torch.matmul(x, w.t()).float().sum().backward()
     assert torch.equal(got, w.grad)
