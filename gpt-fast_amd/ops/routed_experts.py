@@ -287,10 +287,14 @@ def rows_tile(n_experts: int, pairs: int, F: int, K: int, mode: int, units: int)
       110; 256 x 140, 512 -> 2 x 1,024 207, 253.  Over fewer it is not worth the list (3 to 8 us): 64 x 62, 768 ->
       2,048 64, 58; 128 x 127, 512 -> 2 x 256 37, 31.  Sums alone of K = 1,024: 128 x 222, 1,024 -> 4,096 older 473,
       tile 4 475; x 400 724, 686.
-    * 256 x 256 tiles read each operand half as often, from about 120 rows on: 32 x 127, 4,096 -> 2 x 2,048 tile 2
-      306, tile 4 277; x 90 267, 272; with a round that they just fill, sooner: 16 x 100, 4,096 -> 4,096 167, 136.  A
-      second or third round that they hardly need costs more than that: 16 x 190 183, 222; x 222 233, 224; x
-      300 259, 228; 64 x 222, 2,048 -> 1,024 137, 155."""
+    * 256 x 256 tiles read each operand half as often, but a router that prefers some experts leaves many of them
+      nearly empty.  Both products of 32 experts, 4,096 -> 2 x 2,048 -> 4,096, as the routers of random weights of two
+      designs choose, older, tile 2, tile 4: x 112 451, 473, 521 and 460, 447, 524; x 128 474, 490, 528 and 507, 510,
+      546; x 162 525, 539, 536 and 572, 553, 544; x 181 552, 586, 541 and 591, 579, 551; x 256 682, 671, 670 and 758,
+      744, 677.  4,096 -> 3,584 -> 4,096, each: x 128 286, 284, 310; x 181 343, 337, 349; x 225 388, 377, 384.  With
+      even shares they win sooner (the first: x 128 616, 550, 510; x 160 685, 640, 524).  A second or third round that
+      they hardly need costs more than that: 16 x 190, 4,096 -> 4,096 tile 2 183, tile 4 222; x 222 233, 224; x 300
+      259, 228; 64 x 222, 2,048 -> 1,024 137, 155."""
     gated = mode == 2
     if pairs < 36 * n_experts:
         columns = 128 if gated else 256
@@ -305,7 +309,7 @@ def rows_tile(n_experts: int, pairs: int, F: int, K: int, mode: int, units: int)
     rounds = _tiles(pairs, n_experts, 256, F, 128 if gated else 256) / units
     if 1.0 < rounds < 3.1 and 0.0 < rounds % 1.0 < (0.35 if K <= 2048 else 0.3):
         return 2
-    return 4 if pairs >= 120 * n_experts or rounds <= 1.0 else 2
+    return 4 if pairs >= 160 * n_experts else 2
 
 
 def _tile_of(w: torch.Tensor, mode: int, pairs: int) -> int:

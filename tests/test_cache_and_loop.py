@@ -586,13 +586,13 @@ def test_the_kernel_of_the_experts_rows_goes_by_their_sizes_and_the_chip():
 
     def tiles(E, F, K, mode, means, units=256):
         return [rows_tile(E, int(m * E), F, K, mode, units) for m in means]
-    assert tiles(32, 3584, 4096, 1, (0.5, 1, 35, 36, 119, 120, 800)) == [2, 1, 1, 2, 2, 4, 4]
+    assert tiles(32, 3584, 4096, 1, (0.5, 1, 35, 36, 159, 160, 800)) == [2, 1, 1, 2, 2, 4, 4]
     assert tiles(8, 2048, 4096, 2, (1, 35, 36, 170, 222)) == [2, 2, 2, 2, 4]      # a round of tiles of 128 x 128
     assert tiles(8, 512, 1024, 2, (1, 129, 400, 800)) == [2, 2, 2, 2]
     assert tiles(128, 2048, 768, 0, (1, 35, 36, 400)) == [1, 1, 0, 0]
     assert tiles(128, 256, 512, 2, (127, 400)) == [2, 2] and tiles(128, 256, 512, 2, (400,), units=64) == [0]
     assert tiles(128, 4096, 1024, 0, (399, 400)) == [0, 4] and tiles(128, 4096, 1024, 1, (400,)) == [0]
-    assert tiles(16, 4096, 4096, 0, (85, 100, 160, 190, 222, 300)) == [2, 4, 4, 2, 4, 4]     # one round, a little more
+    assert tiles(16, 4096, 4096, 0, (85, 100, 160, 190, 222, 300)) == [2, 2, 4, 2, 4, 4]     # one round, a little more
     assert tiles(64, 1024, 2048, 1, (160, 190, 222)) == [4, 2, 2]
 
 
