@@ -663,7 +663,16 @@ def test_a_launch_where_the_device_may_not_be_used_is_refused_by_torch(monkeypat
         raise RuntimeError("forked")
     monkeypatch.setattr(library, "_raw_stream", lambda device: 5)
     monkeypatch.setattr(library, "_current_device", lambda: 0)
-    monkeypatch.setattr(torch.cuda, "is_initialized", lambda: False)
     monkeypatch.setattr(torch.cuda, "current_stream", refuse)
-    with pytest.raises(RuntimeError, match="forked"):
-        library.stream_handle()
+    assert library.stream_handle().value == 5
+    child = os.fork()
+    if child == 0:
+        refused = 1
+        try:
+            library.stream_handle()
+        except RuntimeError as e:
+            refused = 0 if str(e) == "forked" else 2
+        finally:
+            os._exit(refused)
+    assert os.waitstatus_to_exitcode(os.waitpid(child, 0)[1]) == 0
+    assert library.stream_handle().value == 5
