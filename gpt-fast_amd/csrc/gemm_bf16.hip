@@ -934,3 +934,110 @@ extern "C" int gfa_skinny_bf16(const void* x, const void* w, void* out, int M, i
     }
     return (int)hipErrorInvalidValue;
 }
+
+// --------------------------------------------------------------------------------------
+// Whole decoder layers over a few rows: for every layer the five launches that the entries above and
+// those of attention_bf16.hip make one at a time, with the same arguments, so the same bits.  What this
+// saves is the host's time between them: a step of twelve layers, 65 launches, is 0.35 ms of GPU work at 768
+// columns, and making each launch from Python, with its checks and its output tensors, took the
+// host 1.0 ms.
+
+// One layer's tensors; norm_next: the weights of the norm before the layer behind it, or null.
+struct FewRowLayer {
+    const void *wqkv, *wo, *w13, *w2;
+    const float *norm_ffn, *norm_next;
+    void *k_pages, *v_pages;
+    const int* table;
+};
+
+// What all layers share.  The rows of the first layer's norm are x0: plain [M, D], or with ssq0 [t0,
+// gfa_share_rows(M)] in the two halves of gfa_skinny_into_chain_bf16.
+struct FewRowStep {
+    const void* x0;
+    const float* ssq0;
+    float* residual;                      // [M, D], updated in place
+    const float* freqs;
+    const int *tok_seq, *tok_pos, *q_start, *start_pos;
+    void* work;                           // gfa_few_row_work_bytes
+    // gfa_attention_bf16 and gfa_attention_tiled_bf16, which another library holds
+    int (*attend)(const void*, const void*, const void*, const int*, const int*, const int*, int, void*, float*, float*,
+                  int, int, int, int, int, float, int, int, int, int, int, int, int, hipStream_t);
+    int (*attend_tiled)(const void*, const void*, const void*, const int*, const int*, const int*, int, void*, int, int,
+                        int, int, int, float, int, int, int, hipStream_t);
+    int t0, M, D, I, H, Hkv, hd, rot, table_stride, n_seqs, window, gate_mode;
+    int rows_tiled;                       // (token, head) rows per kv head for attend_tiled, 0: attend
+    int row_tiles, n_waves, max_tiles, n_splits, one_token_each;
+    float eps_mixer, eps_ffn, scale;
+};
+
+struct FewRowWork {
+    size_t q, y, xa, sa, h, xb, sb, po, pml, bytes;
+    FewRowWork(int M, int D, int I, int H, int hd, int splits) {
+        const size_t pad = gfa_share_rows(M), heads = (size_t)H * hd, records = gfa_skinny_workgroups(2, M, D);
+        size_t at = 0;
+        auto take = [&](size_t n) { const size_t o = at; at += (n + 255) / 256 * 256; return o; };
+        q = take((size_t)M * heads * 2);
+        y = take(pad * heads * 2);
+        xa = take(pad * D * 2);
+        sa = take(records * pad * 4);
+        h = take(pad * (size_t)I * 2);
+        xb = take(pad * D * 2);
+        sb = take(records * pad * 4);
+        po = take(splits > 1 ? (size_t)splits * M * heads * 4 : 0);
+        pml = take(splits > 1 ? (size_t)splits * M * H * 2 * 4 : 0);
+        bytes = at;
+    }
+};
+
+extern "C" long gfa_few_row_work_bytes(int M, int D, int I, int H, int hd, int splits) {
+    return (long)FewRowWork(M, D, I, H, hd, splits).bytes;
+}
+
+extern "C" int gfa_few_row_layers_bf16(const FewRowLayer* layers, int n_layers, const FewRowStep* step,
+                                       hipStream_t stream) {
+    const FewRowStep& s = *step;
+    if (n_layers <= 0 || s.M <= 0 || s.M > 16 || s.D <= 0 || s.D % 8 || s.I <= 0 || s.I % 8 || s.hd <= 0 || s.hd % 16 ||
+        s.n_splits < 1 || (s.rows_tiled ? !s.attend_tiled : !s.attend))
+        return (int)hipErrorInvalidValue;
+    const FewRowWork at(s.M, s.D, s.I, s.H, s.hd, s.n_splits);
+    char* w = (char*)s.work;
+    const int records = gfa_skinny_workgroups(2, s.M, s.D), inner = s.H * s.hd;
+    // one token for each sequence and a group that fits one tile: the heads' results stay chunked
+    const int chunked = !s.rows_tiled && s.one_token_each && s.max_tiles == 1;
+    const void* x = s.x0;
+    const float* ssq = s.ssq0;
+    int shares = s.t0, rc = 0;
+    for (int l = 0; l < n_layers && rc == 0; ++l) {
+        const FewRowLayer& L = layers[l];
+        rc = gfa_qkv_rope_store_bf16(x, ssq, shares, s.eps_mixer, L.wqkv, w + at.q, L.k_pages, L.v_pages, s.freqs, s.tok_seq,
+                                     s.tok_pos, L.table, s.table_stride, s.M, s.D, s.H, s.Hkv, s.hd, s.rot, stream);
+        if (rc) break;
+        if (s.rows_tiled)
+            rc = s.attend_tiled(w + at.q, L.k_pages, L.v_pages, s.q_start, s.start_pos, L.table, s.table_stride, w + at.y,
+                                s.M, s.n_seqs, s.H, s.Hkv, s.hd, s.scale, s.window, s.rows_tiled, 0, stream);
+        else
+            rc = s.attend(w + at.q, L.k_pages, L.v_pages, s.q_start, s.start_pos, L.table, s.table_stride, w + at.y,
+                          (float*)(w + at.po), (float*)(w + at.pml), s.M, s.n_seqs, s.H, s.Hkv, s.hd, s.scale, s.window,
+                          s.row_tiles, s.n_waves, s.max_tiles, s.n_splits, s.one_token_each, chunked, stream);
+        if (rc) break;
+        rc = gfa_skinny_into_chain_bf16(w + at.y, chunked, L.wo, s.residual, s.M, s.D, inner, L.norm_ffn, w + at.xa,
+                                        (float*)(w + at.sa), stream);
+        if (rc) break;
+        const bool last = L.norm_next == nullptr;          // nothing takes halves: plain rows, as for any product
+        rc = gfa_skinny_after_chain_bf16(w + at.xa, (const float*)(w + at.sa), records, s.eps_ffn, L.w13, w + at.h, s.M, s.I,
+                                         s.D, s.I, s.gate_mode, s.I, !last, stream);
+        if (rc) break;
+        if (!last) {
+            rc = gfa_skinny_into_chain_bf16(w + at.h, 1, L.w2, s.residual, s.M, s.D, s.I, L.norm_next, w + at.xb,
+                                            (float*)(w + at.sb), stream);
+        } else if (s.M > 1) {
+            rc = gfa_skinny_mfma_bf16(w + at.h, L.w2, s.residual, s.M, s.D, s.I, s.D, 2, 0, stream);
+        } else {
+            rc = gfa_skinny_bf16(w + at.h, L.w2, s.residual, s.M, s.D, s.I, s.D, 2, 0, stream);
+        }
+        x = w + at.xb;
+        ssq = (const float*)(w + at.sb);
+        shares = records;
+    }
+    return rc;
+}

@@ -1,0 +1,75 @@
+"""Runs of plain decoder layers whose few-row steps are launched by one native call."""
+from ..ops import few_row_layers as F
+from ..ops.linear import HalfNormed
+from .attention import Attention
+from .block import PreNormBlock
+from .feed_forward import GatedFeedForward
+from .norm import RMSNorm
+from .position import RotaryPosition
+
+
+def _plain_layer(block) -> bool:
+    """Pre-norm attention with interleaved rotation, then a gated feed-forward, root-mean-square norms before
+    both: the layers whose few-row steps ops.few_row_layers launches."""
+    if type(block) is not PreNormBlock or type(block.mixer) is not Attention \
+            or type(block.feed_forward) is not GatedFeedForward:
+        return False
+    f, p = block.feed_forward.spec, block.mixer.position
+    return (isinstance(block.mixer_norm, RMSNorm) and isinstance(block.feed_forward_norm, RMSNorm)
+            and type(p) is RotaryPosition and p.spec.layout == "interleaved"
+            and f.activation in F.GATE_MODES and f.limit is None)
+
+
+def _alike(a, b) -> bool:
+    return (a.mixer.spec == b.mixer.spec and a.feed_forward.spec == b.feed_forward.spec
+            and a.mixer_norm.spec.eps == b.mixer_norm.spec.eps
+            and a.feed_forward_norm.spec.eps == b.feed_forward_norm.spec.eps)
+
+
+class FewRowRuns:
+    """For every run of a plan's order, where the plain layers of one shape that begin with it end.  None
+    where the layer behind them would take its norm in halves from their last product
+    (``ops.linear.HalfNormed``): the native call ends in plain sums, and a norm kernel more per
+    run of layers costs a recorded step what the call saves an eager one."""
+
+    def __init__(self, plan, blocks, runtime):
+        order = plan.order
+        self.blocks = [blocks[run.layer] for run in order]
+        self.ends = [0] * len(order)
+        if runtime.is_float32 or plan.streams is not None:
+            return
+        for n in reversed(range(len(order))):
+            if not _plain_layer(self.blocks[n]) or order[n].cache_from is not None:
+                continue
+            behind = n + 1
+            if behind == len(order) or getattr(order[behind], "enter", None) is not None \
+                    or not getattr(self.blocks[behind], "takes_prepared", False):
+                self.ends[n] = behind
+                continue
+            if self.ends[behind] and _alike(self.blocks[n], self.blocks[behind]):
+                self.ends[n] = self.ends[behind]
+
+    def take(self, n: int, stream, batch, cache) -> int:
+        """Run the plain layers from run ``n`` on over the stream, if this step's rows are few enough;
+        the number of runs taken (0: none)."""
+        end = self.ends[n]
+        if not end or not 0 < batch.n_tokens <= F.MAX_ROWS:
+            return 0
+        first = self.blocks[n]
+        m, f = first.mixer.spec, first.feed_forward.spec
+        entries = cache.entries[n:end]
+        if not F.takes(batch.n_tokens, m.dim, f.hidden, m.n_heads, m.n_kv_heads, m.head_dim, m.position.rotary_dim) \
+                or any(not e.writes for e in entries) \
+                or len({batch.table(e.group_id).shape for e in entries}) != 1:
+            return 0
+        x = stream.normed(first.mixer_norm, reader=first.mixer)
+        layers = []
+        for i, (block, e) in enumerate(zip(self.blocks[n:end], entries)):
+            behind = None if n + i + 1 == end else self.blocks[n + i + 1].mixer_norm.weight
+            layers.append(F.Layer(block.mixer.wqkv, block.mixer.wo, block.feed_forward.w13, block.feed_forward.w2,
+                                  block.feed_forward_norm.weight, behind, e.k_pages, e.v_pages, batch.table(e.group_id)))
+        F.run_layers(layers, (x.xg, x.ssq) if isinstance(x, HalfNormed) else x, stream.tensor,
+                     first.mixer.position.freqs, m.position.rotary_dim, batch, m.n_heads, m.n_kv_heads, m.head_dim,
+                     first.mixer.window, first.mixer_norm.spec.eps, first.feed_forward_norm.spec.eps, first.mixer.scale,
+                     f.activation)
+        return end - n

@@ -10,6 +10,7 @@ from ..ops import streams as ST
 from .base import (BLOCKS, INPUT_ADDS, NORMS, POSITIONS, STREAM_STEPS, Param, ResidualStream, Runtime,
                    check_bound)
 from .block import StreamRead
+from .few_rows import FewRowRuns
 
 
 class DecoderModel:
@@ -27,6 +28,7 @@ class DecoderModel:
         self.plan = plan
         self.rt = runtime
         self.blocks = [BLOCKS.build(_Arranged(layer), runtime) for layer in plan.layers]
+        self.few_rows = FewRowRuns(plan, self.blocks, runtime)
         self.final_norm = NORMS.build(plan.final_norm, runtime)
         # what reads the stream last: the final norm, over the sum of the streams if there are several
         self.final_read = self.final_norm if plan.streams is None else \
@@ -212,10 +214,17 @@ class DecoderModel:
         if self.enter_steps:
             embedded = residual if getattr(plan.order[0], "enter", None) is not None \
                 else residual.clone()
+        taken = 0                                        # runs before this one are done
         for n, run in enumerate(plan.order):                              # model.py:142-143
+            if n < taken:
+                continue
             if getattr(run, "enter", None) is not None:
                 stream = ResidualStream(self.enter_steps[run.enter].forward(
                     stream.tensor, embedded, batch))
+            if self.tap is None:
+                taken = n + self.few_rows.take(n, stream, batch, cache)
+                if taken > n:
+                    continue
             block = self.blocks[run.layer]
             block.forward(stream if getattr(block, "takes_stream", False) else stream.tensor,
                           batch, cache.entries[n])
