@@ -7,7 +7,7 @@
 // produce one output element depends only on that element's own inputs (its row, its
 // position), never on the number of rows or on the other sequences of the launch, so a
 // float32 result is the same however the tokens were cut into steps or batched.
-#include "common.h"
+#include "few_row_layers.h"
 
 // --------------------------------------------------------------------------------------
 // embedding gather: out[n, :] = float(table[tokens[n], :])          (model.py:140)
@@ -974,12 +974,16 @@ __global__ __launch_bounds__(AG_THREADS) void attention_generic_kernel(
 // kernel above walks all keys' values one after the other: four requests of the 110M shape, 20 to 200 tokens
 // and then 12 steps, 21.4 -> 12.7 ms with it.
 // A row's result depends on its position and window alone.  HD: head size rounded up to 64.
+// Head sizes up to 64 (EARLY): a wave's next page is asked for, keys and values at once, before anything waits - the
+// first one beside the query, not behind it: 11.01 -> 10.61 ms for the same requests (with the products of
+// normed_gemm_f32_kernel); larger heads do not hold a page in registers.
 template <int HD>
 __global__ __launch_bounds__(256) void attention_f32_kernel(
         const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
         const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, const int* __restrict__ table,
         int table_stride, float* __restrict__ out, int H, int Hkv, int hd, float scale, int window) {
     constexpr int PER = HD / 64;
+    constexpr bool EARLY = HD == 64;
     __shared__ __attribute__((aligned(16))) float qs[HD];
     __shared__ __attribute__((aligned(16))) float ps[4][GFA_PAGE];
     __shared__ float merged[4][HD + 2];
@@ -988,24 +992,51 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
     const int pos = tok_pos[n];
     const int* pages = table + (size_t)tok_seq[n] * table_stride;
     const int lo = (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
+    // by the page's own index, so that a window's first page does not move a key to another wave
+    const int first = lo / GFA_PAGE;
+    int page = first + ((wave - first) & 3);
+    float4 ke[EARLY ? 16 : 1], ve[EARLY ? 16 : 1];
+    auto ask = [&](int p) {                                // lanes beyond the head and pages beyond the last: others again
+        const int there = p * GFA_PAGE <= pos ? p : pos / GFA_PAGE;
+        const size_t region = cache_region(pages[there], g, Hkv, hd);
+        const float* kr = k_pages + region + (lane >> 5) * 32 * hd + key_slot(lane & 31) * 8;
+        const int d = lane < hd ? lane : 0;
+        const float* vr = v_pages + region + (d >> 4) * 1024 + (d & 15) * 8;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            const float* at = kr + (c * 8 < hd ? c : 0) * 256;
+            ke[EARLY ? 2 * c : 0] = *(const float4*)at;
+            ke[EARLY ? 2 * c + 1 : 0] = *(const float4*)(at + 4);
+        }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            ve[EARLY ? 2 * c : 0] = *(const float4*)(vr + c * 128);
+            ve[EARLY ? 2 * c + 1 : 0] = *(const float4*)(vr + c * 128 + 4);
+        }
+    };
+    if (EARLY) ask(page);
     for (int d = threadIdx.x; d < hd; d += 256) qs[d] = q[((size_t)n * H + h) * hd + d];
     __syncthreads();
     float m = -INFINITY, l = 0.f, acc[PER];
 #pragma unroll
     for (int i = 0; i < PER; ++i) acc[i] = 0.f;
-    // by the page's own index, so that a window's first page does not move a key to another wave
-    const int first = lo / GFA_PAGE;
-    for (int page = first + ((wave - first) & 3); page * GFA_PAGE <= pos; page += 4) {
+    for (; page * GFA_PAGE <= pos; page += 4) {
         const size_t region = cache_region(pages[page], g, Hkv, hd);
         const int key = page * GFA_PAGE + lane;
         const float* kr = k_pages + region + (lane >> 5) * 32 * hd + key_slot(lane & 31) * 8;
         float dot0 = 0.f, dot1 = 0.f;
-#pragma unroll 8
-        for (int c = 0; c < hd / 8; ++c) {
-            const float4 a = *(const float4*)(kr + c * 256), b = *(const float4*)(kr + c * 256 + 4);
+        auto chunk = [&](int c, const float4& a, const float4& b) {
             const float4 x = *(const float4*)(qs + c * 8), y = *(const float4*)(qs + c * 8 + 4);
             dot0 = fmaf(a.w, x.w, fmaf(a.z, x.z, fmaf(a.y, x.y, fmaf(a.x, x.x, dot0))));
             dot1 = fmaf(b.w, y.w, fmaf(b.z, y.z, fmaf(b.y, y.y, fmaf(b.x, y.x, dot1))));
+        };
+        if (EARLY) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+                if (c * 8 < hd) chunk(c, ke[EARLY ? 2 * c : 0], ke[EARLY ? 2 * c + 1 : 0]);
+        } else {
+#pragma unroll 8
+            for (int c = 0; c < hd / 8; ++c) chunk(c, *(const float4*)(kr + c * 256), *(const float4*)(kr + c * 256 + 4));
         }
         const bool seen = key >= lo && key <= pos;
         const float s = seen ? (dot0 + dot1) * scale : -INFINITY;
@@ -1028,7 +1059,8 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
             float sum = acc[i] * alpha;
 #pragma unroll
             for (int c = 0; c < 8; ++c) {                  // keys 8 c .. + 7
-                float4 a = *(const float4*)(vr + c * 128), b = *(const float4*)(vr + c * 128 + 4);
+                float4 a = EARLY ? ve[EARLY ? 2 * c : 0] : *(const float4*)(vr + c * 128);
+                float4 b = EARLY ? ve[EARLY ? 2 * c + 1 : 0] : *(const float4*)(vr + c * 128 + 4);
                 if (!whole) {                              // slots that hold no seen key are not numbers to use
                     const int k0 = page * GFA_PAGE + 8 * c;
                     if (k0 + 0 < lo || k0 + 0 > pos) a.x = 0.f;
@@ -1047,6 +1079,7 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
             acc[i] = sum;
         }
         __builtin_amdgcn_wave_barrier();
+        if (EARLY && (page + 4) * GFA_PAGE <= pos) ask(page + 4);
     }
 #pragma unroll
     for (int i = 0; i < PER; ++i) merged[wave][lane + 64 * i] = acc[i];
@@ -1180,6 +1213,215 @@ extern "C" int gfa_gate_mul(const void* gu, void* out, int n_rows, int I, int ac
 extern "C" int gfa_silu_mul(const void* gu, void* out, int n_rows, int I, int is_bf16,
                             hipStream_t stream) {
     return launch_gate_mul<0>(gu, out, n_rows, I, is_bf16, 0.f, stream);
+}
+
+// --------------------------------------------------------------------------------------
+// Few rows in float32: a norm, the product behind it and what follows that in one kernel, for the two products
+// of a layer that read a norm.  out = act(n Wg^T) * (n Wu^T) with the gate's act (EPI 0 silu, 1 gelu's tanh form,
+// w = rows of Wg, then of Wu), or q, k, v = n W^T rotated and stored (EPI 2, interleaved pairs, as
+// rope_cache_kernel); n = x * rsqrt(mean(x^2) + eps) * g.
+//
+// What bounds a layer of few rows is its chain of kernels, 5 to 10 us each whatever they do: a norm 5, the rotation
+// 5.5, the gate 5 beside products of 7 to 10 (four rows, 768 columns).  Every workgroup reads all of x
+// anyway, so each works the rows' factors out for itself, while its first weights are on the way: five kernels a
+// layer and not nine, four requests of 20 to 200 tokens and then 12 steps on 12 layers of 768 columns 12.5 -> 11.0 ms.
+//
+// The same bits as rmsnorm_vec_kernel, gemm_f32_kernel and the kernels behind them: the squares are added by as
+// many lanes and in the order of that norm kernel's (256 or 1,024 threads by the width), the products as four chains of
+// every fourth 32 k.  K a multiple of 4 up to 4,096, M <= 16, 16-byte aligned rows.
+struct NormedEpilogue {
+    float* out;                           // EPI 0, 1: [M, N]
+    float *q, *k_pages, *v_pages;         // EPI 2
+    const float* freqs;
+    const int *tok_seq, *tok_pos, *table;
+    int table_stride, H, Hkv, hd, rot;
+};
+
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void normed_gemm_f32_kernel(
+        const float* __restrict__ x, const float* __restrict__ g, const float* __restrict__ w, int M, int N, int K,
+        float eps, NormedEpilogue e) {
+    constexpr int AHEAD = 3;                       // the whole step with 2, 3, 4 blocks: 10.60, 10.57, 10.68 ms
+    __shared__ gf_floatx4_t sums[4][64];
+    __shared__ float squares[16][16], factor[16];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int li = lane & 15, lg = lane >> 4;
+    const int n0 = blockIdx.x * (EPI == 2 ? 16 : 8);
+    const float* xr = x + (size_t)(li < M ? li : M - 1) * K;     // rows beyond the last read it again, never stored
+    // a gate's tile: eight rows of Wg and the same eight of Wu, which keeps as many workgroups at work as sixteen
+    // columns of a plain product (four rows, 768 -> 2 x 2,048: 9 us; two tiles each in half as many, 11)
+    const int wn = n0 + (EPI == 2 ? li : li & 7);
+    const float* wr = w + (size_t)((wn < N ? wn : N - 1) + (EPI != 2 && li >= 8 ? N : 0)) * K;
+    struct Block {
+        gf_floatx4_t a[2], g[2], w[2];
+    };
+    auto place = [&](int b, int h) {               // the lane's k of block b; the row's first ones again beyond K
+        const int k = 32 * b + 16 * h + 4 * lg;
+        return k < K ? k : 0;
+    };
+    auto load = [&](int b, Block& r) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            r.w[h] = *(const gf_floatx4_t*)(wr + place(b, h));
+            r.a[h] = *(const gf_floatx4_t*)(xr + place(b, h));
+            r.g[h] = *(const gf_floatx4_t*)(g + place(b, h));
+        }
+    };
+    const int blocks = (K + 31) / 32;
+    Block ring[AHEAD + 1];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) load(wave + 4 * u, ring[u]);
+
+    // 64 lanes at a time of the norm kernel's threads
+    const int groups = K <= 1024 ? 4 : 16, n4 = K >> 2;
+    for (int group = wave; group < groups; group += 4) {
+        const int at = group * 64 + lane;
+#pragma unroll 4
+        for (int m = 0; m < M; ++m) {
+            const float4 v = at < n4 ? ((const float4*)(x + (size_t)m * K))[at] : make_float4(0.f, 0.f, 0.f, 0.f);
+            float ss = 0.f;
+            ss = fmaf(v.x, v.x, ss);
+            ss = fmaf(v.y, v.y, ss);
+            ss = fmaf(v.z, v.z, ss);
+            ss = fmaf(v.w, v.w, ss);
+            ss = wave_sum(ss);
+            if (lane == 0) squares[m][group] = ss;
+        }
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < M) {
+        float ss = 0.f;
+        for (int i = 0; i < groups; ++i) ss += squares[threadIdx.x][i];
+        factor[threadIdx.x] = rsqrtf(ss / (float)K + eps);
+    }
+    __syncthreads();
+    const float rs = factor[li < M ? li : M - 1];
+    gf_floatx4_t acc = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
+    for (int b = wave; b < blocks; b += 4 * (AHEAD + 1)) {
+#pragma unroll
+        for (int u = 0; u <= AHEAD; ++u) {
+            const int at = b + 4 * u;
+            if (at >= blocks) break;
+            load(at + 4 * AHEAD, ring[(u + AHEAD) % (AHEAD + 1)]);
+            Block& r = ring[u];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) r.a[h][q] = r.a[h][q] * rs * r.g[h][q];
+            if (32 * at + 32 > K) {                // the same for the whole wave: zero beyond K
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (32 * at + 16 * h + 4 * lg >= K) {
+                        r.a[h] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
+                        r.w[h] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
+                    }
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(r.w[h][q], r.a[h][q], acc, 0, 0, 0);
+        }
+    }
+    sums[wave][lane] = acc;
+    __syncthreads();
+    if (wave != 0) return;
+    const gf_floatx4_t v = (sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane]);
+    float up[4];
+    if (EPI != 2) {                                // lanes 32 .. 63 hold the sums of Wu
+#pragma unroll
+        for (int q = 0; q < 4; ++q) up[q] = __shfl_xor(v[q], 32, GFA_WAVE);
+    }
+    const int m = li, n = n0 + 4 * lg;             // four columns of a row
+    if (m >= M || n >= N) return;
+    if (EPI != 2) {
+        if (lg >= 2) return;
+        float* o = e.out + (size_t)m * N + n;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (n + q < N) o[q] = gate_pair<EPI == 1 ? 1 : 0>(v[q], up[q], 0.f);
+        return;
+    }
+    const int hd = e.hd, head = n / hd, d = n - head * hd;       // hd is a multiple of 16: the columns of one head
+    const int pos = e.tok_pos[m], off = pos % GFA_PAGE;
+    float r[4] = {v[0], v[1], v[2], v[3]};
+    if (head < e.H + e.Hkv) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+            if (d + 2 * p < e.rot) {
+                float s, c;
+                sincosf((float)pos * e.freqs[(d + 2 * p) >> 1], &s, &c);
+                const float a = r[2 * p], b = r[2 * p + 1];
+                r[2 * p] = a * c - b * s;
+                r[2 * p + 1] = b * c + a * s;
+            }
+    }
+    if (head < e.H) {
+        *(float4*)(e.q + ((size_t)m * e.H + head) * hd + d) = make_float4(r[0], r[1], r[2], r[3]);
+        return;
+    }
+    const int page = e.table[(size_t)e.tok_seq[m] * e.table_stride + pos / GFA_PAGE];
+    if (head < e.H + e.Hkv) {
+        float* k = e.k_pages + cache_region(page, head - e.H, e.Hkv, hd);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) k[key_offset(off, d + q, hd)] = r[q];
+    } else {
+        float* vp = e.v_pages + cache_region(page, head - e.H - e.Hkv, e.Hkv, hd);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) vp[value_offset(d + q, off, hd)] = r[q];
+    }
+}
+
+static size_t few_row_up(size_t n) { return (n + 255) / 256 * 256; }
+
+extern "C" long gfa_few_row_work_bytes_f32(int M, int I, int H, int hd) {
+    return (long)(2 * few_row_up((size_t)M * H * hd * 4) + few_row_up((size_t)M * I * 4));
+}
+
+// The layers' launches, five a layer.
+extern "C" int gfa_few_row_layers_f32(const FewRowLayer* layers, int n_layers, const FewRowStep* step, hipStream_t stream) {
+    const FewRowStep& s = *step;
+    const int inner = s.H * s.hd;
+    if (n_layers <= 0 || s.M <= 0 || s.M > 16 || s.D <= 0 || s.D % 4 || s.D > 4096 || s.I <= 0 || s.I % 4 || s.hd <= 0 ||
+        s.hd % 16 || s.hd > 256 || s.rot % 2 || s.rot > s.hd || (s.gate_mode != 0 && s.gate_mode != 1) ||
+        (uintptr_t)s.residual % 16 || (uintptr_t)s.work % 16)
+        return (int)hipErrorInvalidValue;
+    float* q = (float*)s.work;
+    float* y = (float*)((char*)q + few_row_up((size_t)s.M * inner * 4));
+    float* h = (float*)((char*)y + few_row_up((size_t)s.M * inner * 4));
+    const int n_qkv = (s.H + 2 * s.Hkv) * s.hd;
+    int rc = 0;
+    for (int l = 0; l < n_layers && rc == 0; ++l) {
+        const FewRowLayer& L = layers[l];
+        if ((uintptr_t)L.wqkv % 16 || (uintptr_t)L.w13 % 16 || (uintptr_t)L.norm_mixer % 16 || (uintptr_t)L.norm_ffn % 16)
+            return (int)hipErrorInvalidValue;
+        NormedEpilogue e = {};
+        e.q = q;
+        e.k_pages = (float*)L.k_pages;
+        e.v_pages = (float*)L.v_pages;
+        e.freqs = s.freqs;
+        e.tok_seq = s.tok_seq;
+        e.tok_pos = s.tok_pos;
+        e.table = L.table;
+        e.table_stride = s.table_stride;
+        e.H = s.H; e.Hkv = s.Hkv; e.hd = s.hd; e.rot = s.rot;
+        normed_gemm_f32_kernel<2><<<n_qkv / 16, 256, 0, stream>>>(s.residual, L.norm_mixer, (const float*)L.wqkv, s.M, n_qkv,
+                                                                  s.D, s.eps_mixer, e);
+        rc = gfa_attention_generic(q, L.k_pages, L.v_pages, s.tok_seq, s.tok_pos, L.table, s.table_stride, y, s.M, s.H,
+                                   s.Hkv, s.hd, s.scale, s.window, 0, stream);
+        if (rc) break;
+        rc = gfa_gemm_f32(y, (const float*)L.wo, s.residual, s.M, s.D, inner, inner, s.D, 1, stream);
+        if (rc) break;
+        e.out = h;
+        if (s.gate_mode == 0)
+            normed_gemm_f32_kernel<0><<<(s.I + 7) / 8, 256, 0, stream>>>(s.residual, L.norm_ffn, (const float*)L.w13, s.M,
+                                                                           s.I, s.D, s.eps_ffn, e);
+        else
+            normed_gemm_f32_kernel<1><<<(s.I + 7) / 8, 256, 0, stream>>>(s.residual, L.norm_ffn, (const float*)L.w13, s.M,
+                                                                           s.I, s.D, s.eps_ffn, e);
+        rc = gfa_gemm_f32(h, (const float*)L.w2, s.residual, s.M, s.D, s.I, s.I, s.D, 1, stream);
+    }
+    return rc;
 }
 
 // --------------------------------------------------------------------------------------

@@ -13,7 +13,7 @@
 // Epilogues (MODE): 0 store bfloat16, 1 store float, 2 add into a float matrix (the
 // residual stream), 3 gate: out[m, n] = silu(x W[n]) * (x W[n + gate_rows]) in bfloat16
 // (the reference's feed-forward, model.py:227), 6 the same gate with the tanh form of gelu.
-#include "common.h"
+#include "few_row_layers.h"
 
 typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2_t;
 
@@ -942,34 +942,6 @@ extern "C" int gfa_skinny_bf16(const void* x, const void* w, void* out, int M, i
 // columns, and making each launch from Python, with its checks and its output tensors, took the
 // host 1.0 ms.
 
-// One layer's tensors; norm_next: the weights of the norm before the layer behind it, or null.
-struct FewRowLayer {
-    const void *wqkv, *wo, *w13, *w2;
-    const float *norm_ffn, *norm_next;
-    void *k_pages, *v_pages;
-    const int* table;
-};
-
-// What all layers share.  The rows of the first layer's norm are x0: plain [M, D], or with ssq0 [t0,
-// gfa_share_rows(M)] in the two halves of gfa_skinny_into_chain_bf16.
-struct FewRowStep {
-    const void* x0;
-    const float* ssq0;
-    float* residual;                      // [M, D], updated in place
-    const float* freqs;
-    const int *tok_seq, *tok_pos, *q_start, *start_pos;
-    void* work;                           // gfa_few_row_work_bytes
-    // gfa_attention_bf16 and gfa_attention_tiled_bf16, which another library holds
-    int (*attend)(const void*, const void*, const void*, const int*, const int*, const int*, int, void*, float*, float*,
-                  int, int, int, int, int, float, int, int, int, int, int, int, int, hipStream_t);
-    int (*attend_tiled)(const void*, const void*, const void*, const int*, const int*, const int*, int, void*, int, int,
-                        int, int, int, float, int, int, int, hipStream_t);
-    int t0, M, D, I, H, Hkv, hd, rot, table_stride, n_seqs, window, gate_mode;
-    int rows_tiled;                       // (token, head) rows per kv head for attend_tiled, 0: attend
-    int row_tiles, n_waves, max_tiles, n_splits, one_token_each;
-    float eps_mixer, eps_ffn, scale;
-};
-
 struct FewRowWork {
     size_t q, y, xa, sa, h, xb, sb, po, pml, bytes;
     FewRowWork(int M, int D, int I, int H, int hd, int splits) {
@@ -1023,12 +995,12 @@ extern "C" int gfa_few_row_layers_bf16(const FewRowLayer* layers, int n_layers, 
         rc = gfa_skinny_into_chain_bf16(w + at.y, chunked, L.wo, s.residual, s.M, s.D, inner, L.norm_ffn, w + at.xa,
                                         (float*)(w + at.sa), stream);
         if (rc) break;
-        const bool last = L.norm_next == nullptr;          // nothing takes halves: plain rows, as for any product
+        const bool last = l + 1 == n_layers;               // nothing takes halves: plain rows, as for any product
         rc = gfa_skinny_after_chain_bf16(w + at.xa, (const float*)(w + at.sa), records, s.eps_ffn, L.w13, w + at.h, s.M, s.I,
                                          s.D, s.I, s.gate_mode, s.I, !last, stream);
         if (rc) break;
         if (!last) {
-            rc = gfa_skinny_into_chain_bf16(w + at.h, 1, L.w2, s.residual, s.M, s.D, s.I, L.norm_next, w + at.xb,
+            rc = gfa_skinny_into_chain_bf16(w + at.h, 1, L.w2, s.residual, s.M, s.D, s.I, layers[l + 1].norm_mixer, w + at.xb,
                                             (float*)(w + at.sb), stream);
         } else if (s.M > 1) {
             rc = gfa_skinny_mfma_bf16(w + at.h, L.w2, s.residual, s.M, s.D, s.I, s.D, 2, 0, stream);

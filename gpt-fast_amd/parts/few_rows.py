@@ -1,4 +1,6 @@
 """Runs of plain decoder layers whose few-row steps are launched by one native call."""
+import torch
+
 from ..ops import few_row_layers as F
 from ..ops.linear import HalfNormed
 from .attention import Attention
@@ -28,7 +30,7 @@ def _alike(a, b) -> bool:
 
 class FewRowRuns:
     """For every run of a plan's order, where the plain layers of one shape that begin with it end.  None
-    where the layer behind them would take its norm in halves from their last product
+    (bfloat16) where the layer behind them would take its norm in halves from their last product
     (``ops.linear.HalfNormed``): the native call ends in plain sums, and a norm kernel more per
     run of layers costs a recorded step what the call saves an eager one."""
 
@@ -36,18 +38,22 @@ class FewRowRuns:
         order = plan.order
         self.blocks = [blocks[run.layer] for run in order]
         self.ends = [0] * len(order)
-        if runtime.is_float32 or plan.streams is not None:
+        self.dtype = runtime.dtype
+        if plan.streams is not None:
             return
         for n in reversed(range(len(order))):
             if not _plain_layer(self.blocks[n]) or order[n].cache_from is not None:
                 continue
             behind = n + 1
             if behind == len(order) or getattr(order[behind], "enter", None) is not None \
-                    or not getattr(self.blocks[behind], "takes_prepared", False):
+                    or runtime.is_float32 and not self._joins(n, behind) or not getattr(self.blocks[behind], "takes_prepared", False):
                 self.ends[n] = behind
                 continue
-            if self.ends[behind] and _alike(self.blocks[n], self.blocks[behind]):
+            if self._joins(n, behind):
                 self.ends[n] = self.ends[behind]
+
+    def _joins(self, n: int, behind: int) -> bool:
+        return bool(self.ends[behind]) and _alike(self.blocks[n], self.blocks[behind])
 
     def take(self, n: int, stream, batch, cache) -> int:
         """Run the plain layers from run ``n`` on over the stream, if this step's rows are few enough;
@@ -58,17 +64,21 @@ class FewRowRuns:
         first = self.blocks[n]
         m, f = first.mixer.spec, first.feed_forward.spec
         entries = cache.entries[n:end]
-        if not F.takes(batch.n_tokens, m.dim, f.hidden, m.n_heads, m.n_kv_heads, m.head_dim, m.position.rotary_dim) \
+        if not F.takes(batch.n_tokens, m.dim, f.hidden, m.n_heads, m.n_kv_heads, m.head_dim, m.position.rotary_dim,
+                       self.dtype) \
                 or any(not e.writes for e in entries) \
                 or len({batch.table(e.group_id).shape for e in entries}) != 1:
             return 0
-        x = stream.normed(first.mixer_norm, reader=first.mixer)
-        layers = []
-        for i, (block, e) in enumerate(zip(self.blocks[n:end], entries)):
-            behind = None if n + i + 1 == end else self.blocks[n + i + 1].mixer_norm.weight
-            layers.append(F.Layer(block.mixer.wqkv, block.mixer.wo, block.feed_forward.w13, block.feed_forward.w2,
-                                  block.feed_forward_norm.weight, behind, e.k_pages, e.v_pages, batch.table(e.group_id)))
-        F.run_layers(layers, (x.xg, x.ssq) if isinstance(x, HalfNormed) else x, stream.tensor,
+        layers = [F.Layer(b.mixer.wqkv, b.mixer.wo, b.feed_forward.w13, b.feed_forward.w2, b.mixer_norm.weight,
+                          b.feed_forward_norm.weight, e.k_pages, e.v_pages, batch.table(e.group_id))
+                  for b, e in zip(self.blocks[n:end], entries)]
+        x = None                                         # in float32 the first product makes its norm itself
+        if self.dtype == torch.bfloat16:
+            x = stream.normed(first.mixer_norm, reader=first.mixer)
+            x = (x.xg, x.ssq) if isinstance(x, HalfNormed) else x
+        elif not F.aligned(layers):
+            return 0
+        F.run_layers(layers, x, stream.tensor,
                      first.mixer.position.freqs, m.position.rotary_dim, batch, m.n_heads, m.n_kv_heads, m.head_dim,
                      first.mixer.window, first.mixer_norm.spec.eps, first.feed_forward_norm.spec.eps, first.mixer.scale,
                      f.activation)

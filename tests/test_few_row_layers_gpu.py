@@ -9,10 +9,11 @@ pytestmark = pytest.mark.gpu
 
 # head sizes 16, 48, 128, 256; one to twenty query heads of a group; widths that are no multiple of 16
 SHAPES = {"16": (64, 4, 4, 16, 176, 3), "48": (200, 10, 5, 48, 328, 2), "128": (256, 16, 1, 128, 400, 2),
-          "256": (128, 2, 1, 256, 264, 2), "20 heads": (128, 20, 1, 32, 256, 1)}
+          "256": (128, 2, 1, 256, 264, 2), "20 heads": (128, 20, 1, 32, 256, 1),
+          "1032": (1032, 4, 4, 64, 1104, 2), "4096": (4096, 4, 1, 64, 40, 2)}
 
 
-def _engine(tmp_path, shape):
+def _engine(tmp_path, shape, dtype="bfloat16"):
     import gpt_fast_amd as gfa
     hidden, heads, kv_heads, head_dim, inner, layers = SHAPES[shape]
     config = {"architectures": ["LlamaForCausalLM"], "model_type": "llama", "hidden_size": hidden,
@@ -21,17 +22,19 @@ def _engine(tmp_path, shape):
               "max_position_embeddings": 4096, "rope_theta": 10000.0, "rms_norm_eps": 1e-5,
               "rope_scaling": None, "tie_word_embeddings": False}
     arch = gfa.config.registry.architecture_of(config)
-    gfa.write_random_model(str(tmp_path), arch, arch.read_config(config), seed=5, dtype="bfloat16", std=0.05)
-    return gfa.Engine.from_folder(str(tmp_path), dtype="bfloat16", device="cuda:0", max_tokens=16384)
+    gfa.write_random_model(str(tmp_path), arch, arch.read_config(config), seed=5, dtype=dtype, std=0.05)
+    return gfa.Engine.from_folder(str(tmp_path), dtype=dtype, device="cuda:0", max_tokens=16384)
 
 
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 @pytest.mark.parametrize("shape", SHAPES, ids=str)
-def test_one_call_launches_what_the_layers_launch(tmp_path, shape, monkeypatch):
+def test_one_call_launches_what_the_layers_launch(tmp_path, shape, dtype, monkeypatch):
+    """float32: the norms, the rotation and the gate are worked out inside the products, to the same bits."""
     import gpt_fast_amd as gfa
     from gpt_fast_amd.ops import few_row_layers as F
     calls, run = [], F.run_layers
     monkeypatch.setattr(F, "run_layers", lambda layers, *a, **k: (calls.append(len(layers)), run(layers, *a, **k))[1])
-    engine = _engine(tmp_path, shape)
+    engine = _engine(tmp_path, shape, dtype)
     ends = list(engine.model.few_rows.ends)
     assert ends == [SHAPES[shape][5]] * SHAPES[shape][5]
     # held tokens, then the tokens of the step: one each (a context that is split among them), a short prompt, both
