@@ -413,11 +413,55 @@ __global__ void combine_pairs_kernel(const T* __restrict__ ys, const int* __rest
     }
 }
 
+// The same sums for whole groups of eight elements in 16-byte accesses, without identity experts.  What bounds
+// it is its bytes; an element a lane took 54 us for 1,777 rows of four bfloat16 pairs, 4,096 wide.
+template <typename T>
+__global__ __launch_bounds__(256) void combine_pairs_vec_kernel(const T* __restrict__ ys, const int* __restrict__ place,
+                                                                const float* __restrict__ weights, float* __restrict__ y,
+                                                                int top, int D, int accumulate, size_t groups) {
+    const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
+    if (i >= groups) return;
+    const int per_row = D >> 3;
+    const size_t n = i / per_row;
+    const int d = (int)(i - n * per_row) * 8;
+    float acc[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) acc[q] = 0.f;
+#pragma unroll 4
+    for (int k = 0; k < top; ++k) {
+        const size_t p = n * top + k;
+        const float wk = weights[p];
+        float v[8];
+        Vec8<T>::load(ys + (size_t)place[p] * D + d, v);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) acc[q] = fmaf(wk, v[q], acc[q]);
+    }
+    float4* o = (float4*)(y + n * D + d);
+    float4 a = make_float4(acc[0], acc[1], acc[2], acc[3]), b = make_float4(acc[4], acc[5], acc[6], acc[7]);
+    if (accumulate) {
+        const float4 u = o[0], w = o[1];
+        a = make_float4(u.x + a.x, u.y + a.y, u.z + a.z, u.w + a.w);
+        b = make_float4(w.x + b.x, w.y + b.y, w.z + b.z, w.w + b.w);
+    }
+    o[0] = a;
+    o[1] = b;
+}
+
 extern "C" int gfa_combine_pairs(const void* ys, const int* place, const float* weights, const int* chosen,
                                  int E, const void* x, int x_bf16, float* y, int n_tokens, int top, int D,
                                  int accumulate, int is_bf16, hipStream_t stream) {
     if (n_tokens <= 0) return 0;
     if (chosen && !x) return (int)hipErrorInvalidValue;
+    if (!chosen && D % 8 == 0 && (uintptr_t)ys % 16 == 0 && (uintptr_t)y % 16 == 0) {
+        const size_t groups = (size_t)n_tokens * (D / 8), blocks = (groups + 255) / 256;
+        if (blocks < (1u << 31)) {
+            if (is_bf16)
+                combine_pairs_vec_kernel<bf16_t><<<(unsigned)blocks, 256, 0, stream>>>((const bf16_t*)ys, place, weights, y, top, D, accumulate, groups);
+            else
+                combine_pairs_vec_kernel<float><<<(unsigned)blocks, 256, 0, stream>>>((const float*)ys, place, weights, y, top, D, accumulate, groups);
+            return GFA_LAUNCH_RESULT();
+        }
+    }
     // few tokens: a row's elements are spread over several workgroups
     int parts = (D + 255) / 256;
     if (parts > 32) parts = 32;
@@ -446,11 +490,17 @@ extern "C" int gfa_combine_pairs(const void* ys, const int* place, const float* 
 // tile of its own into the operand layout of v_mfma_f32_16x16x32_bf16, DEPTH pieces ahead.  XD (up to
 // 16 rows, for steps of very few tokens, where few experts have rows at all and the chip is not
 // full): no shared x and no barriers while K is walked; a lane reads its own operand pieces of
-// x from memory, four pieces ahead like W; the workgroup's four waves take the same 16 columns
+// x from memory, as far ahead as W; the workgroup's four waves take the same 16 columns
 // and a quarter of K each, and the first adds their sums in the waves' order (four times the
 // workgroups).  A
-// row of x meets only its own lanes of the operand and K is walked in the same order whatever
-// the step holds, so a pair's result does not depend on the other pairs.  act < 0: the float
+// row of x meets only its own lanes of the operand and K is walked in an order that the expert and the
+// tile alone decide, so a pair's result does not depend on the other pairs.
+// What bounds it is the stream of the chosen experts' matrices.  Barriers that wait for shared memory alone keep
+// DEPTH pieces of W under way, and tiles begin at different pieces: decode steps of 16, 24 and 56 rows with
+// 32 experts of 2 x 4,096 x 3,584 (whole requests) 57.5 -> 55.5, 61.2 -> 58.6, 75.5 -> 73.0 ms; of 2, 4 and 12
+// rows with gated ones of 3 x 4,096 x 2,048 25.7 -> 24.5, 37.8 -> 36.2, 43.9 -> 40.6.  DEPTH: at 16 rows four pieces
+// 55.5, two 56.8, eight 57.0; at 17 to 32 rows two 58.6, four 60.9; above four 72.9, two 73.2;
+// XD one 36.2, two 36.6, four 37.9 (more waves share a compute unit).  act < 0: the float
 // sums are stored; else act(sum) as bfloat16.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 re_bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float re_floatx4_t;
@@ -469,6 +519,7 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
         const bf16_t* __restrict__ x, const int* __restrict__ order, int top,
         const bf16_t* __restrict__ w, const int* __restrict__ offsets, void* __restrict__ out,
         int N, int K, int act) {
+    static_assert(XD || DEPTH % 2 == 0, "x alternates between two buffers");
     constexpr int NT = GR_NW * 64;
     constexpr int XBYTES = CT * 16 * GR_PITCH;
     constexpr int XPER = CT;                               // CT * 16 rows of 16 pieces over 256 threads
@@ -476,13 +527,19 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
     const int e = blockIdx.y;
     const int lo = offsets[e], hi = offsets[e + 1];
     if (hi <= lo) return;                                  // the same for every thread of the workgroup
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int fi = lane & 15, fg = lane >> 4;
     const int lrow = lane >> 4, lchunk = lane & 15;
     char* stage = gr_smem + (XD ? 0 : 2 * XBYTES) + wave * GR_TILE;
     const int n0w = XD ? blockIdx.x * 16 : (blockIdx.x * GR_NW + wave) * 16;
     const int T = (K + GR_SUBK - 1) / GR_SUBK;
     const bf16_t* we = w + (size_t)e * N * K;
+    // The pieces that this workgroup (XD: the wave) walks, and the one that it begins with: rows of a matrix are
+    // often a power of two apart, and tiles that walk them in step meet in the same memory channels.
+    const int per_wave = XD ? (T + GR_NW - 1) / GR_NW : T;
+    const int t_lo = XD ? wave * per_wave : 0, t_hi = t_lo + per_wave < T ? t_lo + per_wave : T;
+    const int turn = t_hi > t_lo ? (blockIdx.x * 3 + e * 5) % (t_hi - t_lo) : 0;
+    auto piece = [&](int t) { return t + turn < t_hi ? t + turn : t + turn - (t_hi - t_lo); };
     const bf16_t* wsrc[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -513,14 +570,16 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
         uint4 xd[XD ? DEPTH : 1][4];
         const bf16_t* xrow = nullptr;
         if (XD && fi < M) xrow = x + (size_t)(order ? order[m0 + fi] / top : m0 + fi) * K + fg * 8;
-        auto load_xd = [&](int t, uint4 (&regs)[4]) {
+        auto load_xd = [&](int at, uint4 (&regs)[4]) {
+            const int t = piece(at);
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const bool ok = xrow != nullptr && t * GR_SUBK + s * 32 + fg * 8 < K;
                 regs[s] = ok ? *(const uint4*)(xrow + (size_t)t * GR_SUBK + s * 32) : make_uint4(0, 0, 0, 0);
             }
         };
-        auto load_w = [&](int t, uint4 (&regs)[4]) {
+        auto load_w = [&](int at, uint4 (&regs)[4]) {
+            const int t = piece(at);
             const bool ok = t * GR_SUBK + lchunk * 8 < K;
 #pragma unroll
             for (int j = 0; j < 4; ++j)
@@ -531,7 +590,8 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
             for (int j = 0; j < 4; ++j)
                 *(uint4*)(stage + (lrow + 4 * j) * GR_PITCH + lchunk * 16) = regs[j];
         };
-        auto load_x = [&](int t) {
+        auto load_x = [&](int at) {
+            const int t = piece(at);
 #pragma unroll
             for (int i = 0; i < XPER; ++i) {
                 const int c = threadIdx.x + i * NT;
@@ -565,9 +625,6 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
         if (XD) {
             // no shared x, no barriers while K is walked: the workgroup's waves take the same 16
             // columns and a quarter of K each; their sums are added in the waves' order
-            const int per_wave = (T + GR_NW - 1) / GR_NW;
-            const int t_lo = wave * per_wave;
-            const int t_hi = (t_lo + per_wave < T) ? t_lo + per_wave : T;
 #pragma unroll
             for (int u = 0; u < DEPTH; ++u)
                 if (t_lo + u < t_hi) {
@@ -609,13 +666,13 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
             }
             __syncthreads();                               // before the next chunk's sums
         } else {
-        __syncthreads();                                   // the chunk before has been multiplied
+        lds_barrier();                                     // the chunk before has been multiplied
         load_x(0);
 #pragma unroll
         for (int u = 0; u < DEPTH; ++u)
             if (u < T) load_w(u, wr[u]);
         store_x(0);
-        __syncthreads();
+        lds_barrier();
         // piece t: x in buffer t & 1, W in wr[t % DEPTH], asked for DEPTH pieces ahead
         for (int t = 0; t < T; t += DEPTH) {
 #pragma unroll
@@ -627,7 +684,7 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
                 if (tt + DEPTH < T) load_w(tt + DEPTH, wr[u]);
                 multiply(u & 1);
                 if (tt + 1 < T) store_x((u + 1) & 1);
-                __syncthreads();
+                lds_barrier();                             // the pieces of W asked for stay under way
             }
         }
         }
@@ -665,10 +722,10 @@ extern "C" int gfa_grouped_rows(const void* x, const int* order, int top, const 
     grouped_rows_kernel<CTV, DV, XDV><<<(XDV ? grid_direct : grid), GR_NW * 64,                   \
         (XDV ? GR_NW * 64 * 4 * sizeof(float) : 2 * CTV * 16 * GR_PITCH) + GR_NW * GR_TILE, stream>>>( \
         (const bf16_t*)x, order, top, (const bf16_t*)w, offsets, out, N, K, act)
-    if (rows_at_most <= 16 && x_direct) GFA_LAUNCH_GROUPED(1, 4, true);
-    else if (rows_at_most <= 16) GFA_LAUNCH_GROUPED(1, 2, false);
+    if (rows_at_most <= 16 && x_direct) GFA_LAUNCH_GROUPED(1, 1, true);
+    else if (rows_at_most <= 16) GFA_LAUNCH_GROUPED(1, 4, false);
     else if (rows_at_most <= 32) GFA_LAUNCH_GROUPED(2, 2, false);
-    else GFA_LAUNCH_GROUPED(4, 2, false);
+    else GFA_LAUNCH_GROUPED(4, 4, false);
 #undef GFA_LAUNCH_GROUPED
     return GFA_LAUNCH_RESULT();
 }
