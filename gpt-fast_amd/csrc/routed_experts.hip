@@ -28,17 +28,19 @@
 // group's score is the sum of its `group_top` largest c (1: its largest), the experts of the
 // groups that are not kept count as minus infinity (c can be negative), and the `top`
 // largest c are chosen; the WEIGHTS are the chosen experts' s over their sum.
-__global__ __launch_bounds__(64) void route_kernel(
-        const float* __restrict__ z, long long z_stride, int E, int top, int groups, int keep,
-        float weight_eps, int scoring, const float* __restrict__ correction, int group_top,
-        int* __restrict__ chosen, float* __restrict__ weights) {
-    extern __shared__ float re_lds[];            // s [E], c [E], group scores [groups], allowed [groups]
-    float* s = re_lds;
+// The exchanges go through shared memory of the wave's own (re_lds), whose accesses are in order.  Lane k < top
+// ends with the k-th choice and its weight.
+__device__ __forceinline__ void re_own_exchange() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ void route_token(
+        const float* __restrict__ zr, int E, int top, int groups, int keep, float weight_eps, int scoring,
+        const float* __restrict__ correction, int group_top, float* re_lds, int lane, int& choice, float& weight) {
+    float* s = re_lds;                           // s [E], c [E], group scores [groups], allowed [groups]
     float* c = s + E;
     float* gscore = c + E;
     int* allowed = (int*)(gscore + groups);
-    const int lane = threadIdx.x, n = blockIdx.x;
-    const float* zr = z + (size_t)n * z_stride;
     if (scoring == 0) {
         float mx = -INFINITY;
         for (int e = lane; e < E; e += 64) mx = fmaxf(mx, zr[e]);
@@ -56,7 +58,7 @@ __global__ __launch_bounds__(64) void route_kernel(
         for (int e = lane; e < E; e += 64) s[e] = 1.f / (1.f + expf(-zr[e]));
     }
     for (int e = lane; e < E; e += 64) c[e] = s[e] + (correction ? correction[e] : 0.f);
-    __syncthreads();
+    re_own_exchange();
     const int per = E / groups;
     const bool choose_groups = keep < groups;           // else every group stays
     for (int g = lane; choose_groups && g < groups; g += 64) {
@@ -79,14 +81,14 @@ __global__ __launch_bounds__(64) void route_kernel(
         }
         gscore[g] = total;
     }
-    __syncthreads();
+    re_own_exchange();
     for (int g = lane; choose_groups && g < groups; g += 64) {
         int better = 0;
         for (int o = 0; o < groups; ++o)
             better += (gscore[o] > gscore[g] || (gscore[o] == gscore[g] && o < g)) ? 1 : 0;
         allowed[g] = better < keep;
     }
-    __syncthreads();
+    re_own_exchange();
     // the lane's experts that can still be chosen; minus infinity marks one that cannot
     float mine[RE_MAX_PER_LANE];
 #pragma unroll
@@ -129,11 +131,82 @@ __global__ __launch_bounds__(64) void route_kernel(
         }
     }
     const float norm = 1.f / (total + weight_eps);
+    choice = e_k;
+    weight = w_k * norm;
+}
+
+__global__ __launch_bounds__(64) void route_kernel(
+        const float* __restrict__ z, long long z_stride, int E, int top, int groups, int keep,
+        float weight_eps, int scoring, const float* __restrict__ correction, int group_top,
+        int* __restrict__ chosen, float* __restrict__ weights) {
+    extern __shared__ float re_lds[];
+    const int lane = threadIdx.x, n = blockIdx.x;
+    int choice;
+    float weight;
+    route_token(z + (size_t)n * z_stride, E, top, groups, keep, weight_eps, scoring, correction, group_top, re_lds, lane,
+                choice, weight);
     if (lane < top) {
-        chosen[(size_t)n * top + lane] = e_k;
-        weights[(size_t)n * top + lane] = w_k * norm;
+        chosen[(size_t)n * top + lane] = choice;
+        weights[(size_t)n * top + lane] = weight;
     }
 }
+
+// Up to sixteen tokens, a wave each in one workgroup: their choices, and the pairs in the order of their experts
+// (expert_order_kernel) without a launch of its own.
+#define RO_TOKENS 16
+__global__ __launch_bounds__(RO_TOKENS * 64) void route_order_kernel(
+        const float* __restrict__ z, long long z_stride, int n_tokens, int E, int top, int groups, int keep,
+        float weight_eps, int scoring, const float* __restrict__ correction, int group_top,
+        int* __restrict__ chosen, float* __restrict__ weights, int* __restrict__ offsets, int* __restrict__ order,
+        int* __restrict__ place) {
+    extern __shared__ float re_lds[];            // per wave as above; then start [E + 1], cursor [E]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    int* start = (int*)(re_lds + (size_t)waves * (2 * E + 2 * groups));
+    int* cursor = start + E + 1;
+    for (int e = threadIdx.x; e <= E; e += blockDim.x) start[e] = 0;
+    int choice = 0;
+    float weight = 0.f;
+    const bool pair = wave < n_tokens && lane < top;
+    if (wave < n_tokens)
+        route_token(z + (size_t)wave * z_stride, E, top, groups, keep, weight_eps, scoring, correction, group_top,
+                    re_lds + (size_t)wave * (2 * E + 2 * groups), lane, choice, weight);
+    const int p = wave * top + lane;
+    if (pair) {
+        chosen[p] = choice;
+        weights[p] = weight;
+    }
+    __syncthreads();
+    if (pair) atomicAdd(&start[choice + 1], 1);
+    __syncthreads();
+    if (wave == 0) {                             // running sums, 64 experts at a time
+        int before = 0;
+        for (int first = 0; first < E; first += 64) {
+            const int e = first + lane;
+            int sum = e < E ? start[e + 1] : 0;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int other = __shfl_up(sum, o, 64);
+                if (lane >= o) sum += other;
+            }
+            sum += before;
+            if (e < E) {
+                start[e + 1] = sum;
+                offsets[e + 1] = sum;
+            }
+            before = __shfl(sum, 63, 64);
+        }
+        if (lane == 0) offsets[0] = 0;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < E; e += blockDim.x) cursor[e] = start[e];
+    __syncthreads();
+    if (pair) {
+        const int at = atomicAdd(&cursor[choice], 1);
+        order[at] = p;
+        place[p] = at;
+    }
+}
+
 
 extern "C" int gfa_route(const float* z, long long z_stride, int n_tokens, int E, int top, int groups,
                          int keep, float weight_eps, int scoring, const float* correction,
@@ -146,6 +219,19 @@ extern "C" int gfa_route(const float* z, long long z_stride, int n_tokens, int E
     const size_t shmem = sizeof(float) * (size_t)(2 * E + 2 * groups);
     route_kernel<<<n_tokens, 64, shmem, stream>>>(z, z_stride, E, top, groups, keep, weight_eps,
                                                    scoring, correction, group_top, chosen, weights);
+    return GFA_LAUNCH_RESULT();
+}
+
+extern "C" int gfa_route_order(const float* z, long long z_stride, int n_tokens, int E, int top, int groups,
+                               int keep, float weight_eps, int scoring, const float* correction, int group_top,
+                               int* chosen, float* weights, int* offsets, int* order, int* place, hipStream_t stream) {
+    const size_t shmem = sizeof(float) * ((size_t)n_tokens * (2 * E + 2 * groups) + 2 * E + 1);
+    if (n_tokens <= 0 || n_tokens > RO_TOKENS || E <= 0 || E > 64 * RE_MAX_PER_LANE || groups <= 0 || E % groups ||
+            keep < 1 || keep > groups || top < 1 || top > 64 || top > keep * (E / groups) || (scoring != 0 && scoring != 1) ||
+            group_top < 1 || group_top > RE_MAX_GROUP_TOP || shmem > 65536)
+        return (int)hipErrorInvalidValue;
+    route_order_kernel<<<1, n_tokens * 64, shmem, stream>>>(z, z_stride, n_tokens, E, top, groups, keep, weight_eps, scoring,
+                                                            correction, group_top, chosen, weights, offsets, order, place);
     return GFA_LAUNCH_RESULT();
 }
 
@@ -393,13 +479,19 @@ extern "C" int gfa_padded_places(const int* place, const int* chosen, const int*
 }
 
 // y[n, :] (+)= sum_k weight[n, k] ys[place[n top + k], :], in the order of the choice; with `chosen`,
-// a pair whose expert is E or more adds weight * x[n, :] instead
+// a pair whose expert is E or more adds weight * x[n, :] instead.  With `gate`, what is there already
+// is multiplied by sigmoid(gate[n * gate_stride]) first (a shared expert's result and its gate).
+__device__ __forceinline__ float re_row_gate(const float* gate, long long gate_stride, size_t n) {
+    return gate ? 1.f / (1.f + expf(-gate[n * gate_stride])) : 1.f;
+}
 template <typename T, typename X>
 __global__ void combine_pairs_kernel(const T* __restrict__ ys, const int* __restrict__ place,
                                      const float* __restrict__ weights, const int* __restrict__ chosen,
                                      int E, const X* __restrict__ x, float* __restrict__ y,
-                                     int top, int D, int accumulate) {
+                                     int top, int D, int accumulate, const float* __restrict__ gate,
+                                     long long gate_stride) {
     const int n = blockIdx.x;
+    const float there = re_row_gate(gate, gate_stride, n);
     for (int d = blockIdx.y * blockDim.x + threadIdx.x; d < D; d += gridDim.y * blockDim.x) {
         float acc = 0.f;
         for (int k = 0; k < top; ++k) {
@@ -409,7 +501,7 @@ __global__ void combine_pairs_kernel(const T* __restrict__ ys, const int* __rest
             acc = fmaf(weights[p], v, acc);
         }
         float* o = y + (size_t)n * D + d;
-        *o = accumulate ? *o + acc : acc;
+        *o = accumulate ? *o * there + acc : acc;
     }
 }
 
@@ -418,7 +510,8 @@ __global__ void combine_pairs_kernel(const T* __restrict__ ys, const int* __rest
 template <typename T>
 __global__ __launch_bounds__(256) void combine_pairs_vec_kernel(const T* __restrict__ ys, const int* __restrict__ place,
                                                                 const float* __restrict__ weights, float* __restrict__ y,
-                                                                int top, int D, int accumulate, size_t groups) {
+                                                                int top, int D, int accumulate, size_t groups,
+                                                                const float* __restrict__ gate, long long gate_stride) {
     const size_t i = blockIdx.x * (size_t)256 + threadIdx.x;
     if (i >= groups) return;
     const int per_row = D >> 3;
@@ -440,8 +533,9 @@ __global__ __launch_bounds__(256) void combine_pairs_vec_kernel(const T* __restr
     float4 a = make_float4(acc[0], acc[1], acc[2], acc[3]), b = make_float4(acc[4], acc[5], acc[6], acc[7]);
     if (accumulate) {
         const float4 u = o[0], w = o[1];
-        a = make_float4(u.x + a.x, u.y + a.y, u.z + a.z, u.w + a.w);
-        b = make_float4(w.x + b.x, w.y + b.y, w.z + b.z, w.w + b.w);
+        const float there = re_row_gate(gate, gate_stride, n);
+        a = make_float4(u.x * there + a.x, u.y * there + a.y, u.z * there + a.z, u.w * there + a.w);
+        b = make_float4(w.x * there + b.x, w.y * there + b.y, w.z * there + b.z, w.w * there + b.w);
     }
     o[0] = a;
     o[1] = b;
@@ -449,16 +543,17 @@ __global__ __launch_bounds__(256) void combine_pairs_vec_kernel(const T* __restr
 
 extern "C" int gfa_combine_pairs(const void* ys, const int* place, const float* weights, const int* chosen,
                                  int E, const void* x, int x_bf16, float* y, int n_tokens, int top, int D,
-                                 int accumulate, int is_bf16, hipStream_t stream) {
+                                 int accumulate, const float* gate, long long gate_stride, int is_bf16,
+                                 hipStream_t stream) {
     if (n_tokens <= 0) return 0;
     if (chosen && !x) return (int)hipErrorInvalidValue;
     if (!chosen && D % 8 == 0 && (uintptr_t)ys % 16 == 0 && (uintptr_t)y % 16 == 0) {
         const size_t groups = (size_t)n_tokens * (D / 8), blocks = (groups + 255) / 256;
         if (blocks < (1u << 31)) {
             if (is_bf16)
-                combine_pairs_vec_kernel<bf16_t><<<(unsigned)blocks, 256, 0, stream>>>((const bf16_t*)ys, place, weights, y, top, D, accumulate, groups);
+                combine_pairs_vec_kernel<bf16_t><<<(unsigned)blocks, 256, 0, stream>>>((const bf16_t*)ys, place, weights, y, top, D, accumulate, groups, gate, gate_stride);
             else
-                combine_pairs_vec_kernel<float><<<(unsigned)blocks, 256, 0, stream>>>((const float*)ys, place, weights, y, top, D, accumulate, groups);
+                combine_pairs_vec_kernel<float><<<(unsigned)blocks, 256, 0, stream>>>((const float*)ys, place, weights, y, top, D, accumulate, groups, gate, gate_stride);
             return GFA_LAUNCH_RESULT();
         }
     }
@@ -468,7 +563,7 @@ extern "C" int gfa_combine_pairs(const void* ys, const int* place, const float* 
     if (n_tokens >= 1024) parts = 1;
     dim3 grid(n_tokens, parts);
 #define CP_GO(T, X) combine_pairs_kernel<T, X><<<grid, 256, 0, stream>>>( \
-        (const T*)ys, place, weights, chosen, E, (const X*)x, y, top, D, accumulate)
+        (const T*)ys, place, weights, chosen, E, (const X*)x, y, top, D, accumulate, gate, gate_stride)
     if (is_bf16 && x_bf16) CP_GO(bf16_t, bf16_t);
     else if (is_bf16) CP_GO(bf16_t, float);
     else if (x_bf16) CP_GO(float, bf16_t);
@@ -514,11 +609,11 @@ union ReFrag {
 #define GR_TILE (16 * GR_PITCH)
 #define GR_NW 4                               // waves per workgroup: 64 columns
 
-template <int CT, int DEPTH, bool XD>
+template <int CT, int DEPTH, bool XD, bool GATED>
 __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
         const bf16_t* __restrict__ x, const int* __restrict__ order, int top,
         const bf16_t* __restrict__ w, const int* __restrict__ offsets, void* __restrict__ out,
-        int N, int K, int act) {
+        int N, int K, int act, float limit) {
     static_assert(XD || DEPTH % 2 == 0, "x alternates between two buffers");
     constexpr int NT = GR_NW * 64;
     constexpr int XBYTES = CT * 16 * GR_PITCH;
@@ -532,6 +627,7 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
     const int lrow = lane >> 4, lchunk = lane & 15;
     char* stage = gr_smem + (XD ? 0 : 2 * XBYTES) + wave * GR_TILE;
     const int n0w = XD ? blockIdx.x * 16 : (blockIdx.x * GR_NW + wave) * 16;
+    const int F = N / 2;                                   // GATED: columns of out
     const int T = (K + GR_SUBK - 1) / GR_SUBK;
     const bf16_t* we = w + (size_t)e * N * K;
     // The pieces that this workgroup (XD: the wave) walks, and the one that it begins with: rows of a matrix are
@@ -543,8 +639,10 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
     const bf16_t* wsrc[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        int n = n0w + lrow + 4 * j;
-        if (n >= N) n = N - 1;                             // read again, never stored
+        const int r = lrow + 4 * j;
+        int n = GATED ? n0w / 2 + (r & 7) : n0w + r;
+        if (n >= (GATED ? F : N)) n = (GATED ? F : N) - 1; // read again, never stored
+        if (GATED && r >= 8) n += F;
         wsrc[j] = we + (size_t)n * K + lchunk * 8;
     }
 
@@ -695,6 +793,17 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
             for (int ct = 0; ct < CT; ++ct) {
                 const int m = ct * 16 + fi;
                 if (m >= M) continue;
+                if (GATED) {                               // lanes 32 .. 63 hold the sums of the up rows
+                    const int n = n0w / 2 + (fg & 1) * 4;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float a = acc[ct][j], up = __shfl_xor(a, 32, GFA_WAVE);
+                        if (fg < 2 && n + j < F)
+                            ((bf16_t*)out)[(size_t)(m0 + m) * F + n + j] = float_to_bf16(
+                                act == 2 ? re_clamped_pair(a, up, limit) : re_activation(a, act) * up);
+                    }
+                    continue;
+                }
                 const int n = n0w + fg * 4;
                 const size_t at = (size_t)(m0 + m) * N + n;
 #pragma unroll
@@ -710,22 +819,32 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
 }
 
 // out [pairs, N] from x (rows by order / top, or by place) and W [E, N, K]; rows_at_most: the
-// most rows one expert can have (the step's tokens), which sizes the tiles of x.
+// most rows one expert can have (the step's tokens), which sizes the tiles of x.  gated: W holds N / 2 gate
+// rows, then as many up rows, and out is bfloat16 [pairs, N / 2] of act(gate) * up (act 2: the clamped
+// gate); a tile of 16 rows of W is eight of either.
 extern "C" int gfa_grouped_rows(const void* x, const int* order, int top, const void* w,
                                 const int* offsets, void* out, int E, int N, int K, int act,
-                                int rows_at_most, int x_direct, hipStream_t stream) {
+                                int rows_at_most, int x_direct, int gated, float limit, hipStream_t stream) {
+    if (gated && (N % 2 || act < 0 || act > 2)) return (int)hipErrorInvalidValue;
     if (E <= 0 || N <= 0 || K <= 0 || K % 8 || top <= 0 || E > 65535) return (int)hipErrorInvalidValue;
-    if (act >= 0 && act != 0 && act != 1 && act != 3) return (int)hipErrorInvalidValue;
-    dim3 grid((N + GR_NW * 16 - 1) / (GR_NW * 16), E);
-    dim3 grid_direct((N + 15) / 16, E);
-#define GFA_LAUNCH_GROUPED(CTV, DV, XDV)                                                          \
-    grouped_rows_kernel<CTV, DV, XDV><<<(XDV ? grid_direct : grid), GR_NW * 64,                   \
+    if (!gated && act >= 0 && act != 0 && act != 1 && act != 3) return (int)hipErrorInvalidValue;
+    const int tiles = gated ? (N / 2 + 7) / 8 : (N + 15) / 16;
+    dim3 grid((tiles + GR_NW - 1) / GR_NW, E);
+    dim3 grid_direct(tiles, E);
+#define GFA_LAUNCH_GROUPED_G(CTV, DV, XDV, GV)                                                    \
+    grouped_rows_kernel<CTV, DV, XDV, GV><<<(XDV ? grid_direct : grid), GR_NW * 64,               \
         (XDV ? GR_NW * 64 * 4 * sizeof(float) : 2 * CTV * 16 * GR_PITCH) + GR_NW * GR_TILE, stream>>>( \
-        (const bf16_t*)x, order, top, (const bf16_t*)w, offsets, out, N, K, act)
+        (const bf16_t*)x, order, top, (const bf16_t*)w, offsets, out, N, K, act, limit)
+#define GFA_LAUNCH_GROUPED(CTV, DV, XDV)                                                          \
+    do {                                                                                          \
+        if (gated) GFA_LAUNCH_GROUPED_G(CTV, DV, XDV, true);                                      \
+        else GFA_LAUNCH_GROUPED_G(CTV, DV, XDV, false);                                           \
+    } while (0)
     if (rows_at_most <= 16 && x_direct) GFA_LAUNCH_GROUPED(1, 1, true);
     else if (rows_at_most <= 16) GFA_LAUNCH_GROUPED(1, 4, false);
     else if (rows_at_most <= 32) GFA_LAUNCH_GROUPED(2, 2, false);
     else GFA_LAUNCH_GROUPED(4, 4, false);
+#undef GFA_LAUNCH_GROUPED_G
 #undef GFA_LAUNCH_GROUPED
     return GFA_LAUNCH_RESULT();
 }

@@ -7,7 +7,7 @@ from typing import Optional
 
 import torch
 
-from .kernels import ACTIVATIONS, check_gate_limit
+from .kernels import ACTIVATIONS, GATE_ACTIVATIONS, check_gate_limit
 from .linear import _compute_units
 from .library import KernelError, check, library, ptr, require_contiguous, require_device, stream_handle
 
@@ -34,14 +34,16 @@ MAX_GROUP_TOP = 8
 
 
 def route(z: torch.Tensor, n_experts: int, top: int, groups: int, keep: int, weight_eps: float,
-          scoring: str = "softmax", correction: Optional[torch.Tensor] = None, group_top: int = 1):
+          scoring: str = "softmax", correction: Optional[torch.Tensor] = None, group_top: int = 1,
+          ordered: bool = False):
     """(chosen int32 [N, top], weights float32 [N, top]) from router logits z float32
     [N, >= n_experts] (a view of wider rows is allowed): scores s = softmax over the experts, or
     sigmoid of each (``scoring``); the choice is made on s + ``correction`` (float32
     [n_experts]; None: on s): the ``keep`` best of ``groups`` equal groups of neighbours by the
     sum of their ``group_top`` largest choice scores (1: by their largest), of their experts
     the ``top`` with the largest choice scores in falling order; each weighted by its s over
-    the chosen experts' s summed, plus ``weight_eps``."""
+    the chosen experts' s summed, plus ``weight_eps``.  ``ordered`` (where :func:`orders_with_route`): a third
+    result, what :func:`expert_order` makes of the choice, from the same launch."""
     require_device(z, correction)
     require_contiguous(correction=correction)
     if z.dtype != torch.float32 or z.dim() != 2 or z.shape[1] < n_experts or z.stride(1) != 1:
@@ -58,11 +60,28 @@ def route(z: torch.Tensor, n_experts: int, top: int, groups: int, keep: int, wei
     n = z.shape[0]
     chosen = torch.empty((n, top), dtype=torch.int32, device=z.device)
     weights = torch.empty((n, top), dtype=torch.float32, device=z.device)
+    if ordered:
+        if not orders_with_route(n, n_experts, groups):
+            raise KernelError(f"route: {n} tokens of {n_experts} experts are not ordered in the same launch")
+        lists = (torch.empty(n_experts + 1, dtype=torch.int32, device=z.device),
+                 torch.empty(n * top, dtype=torch.int32, device=z.device),
+                 torch.empty(n * top, dtype=torch.int32, device=z.device))
+        check(library("routed_experts").gfa_route_order(
+            ptr(z), _ll(z.stride(0)), _i(n), _i(n_experts), _i(top), _i(groups), _i(keep), _f(weight_eps),
+            _i(ROUTER_SCORINGS[scoring]), ptr(correction), _i(group_top), ptr(chosen), ptr(weights),
+            *(ptr(t) for t in lists), stream_handle()), "route_order")
+        return chosen, weights, lists
     check(library("routed_experts").gfa_route(ptr(z), _ll(z.stride(0)), _i(n), _i(n_experts), _i(top),
                                               _i(groups), _i(keep), _f(weight_eps),
                                               _i(ROUTER_SCORINGS[scoring]), ptr(correction), _i(group_top),
                                               ptr(chosen), ptr(weights), stream_handle()), "route")
     return chosen, weights
+
+
+def orders_with_route(n_tokens: int, n_experts: int, groups: int) -> bool:
+    """Whether :func:`route` can put the pairs in the order of their experts in the same launch: up to sixteen tokens,
+    a wave each in one workgroup, whose scores fit its shared memory."""
+    return 0 < n_tokens <= 16 and 4 * (n_tokens * 2 * (n_experts + groups) + 2 * n_experts + 1) <= 65536
 
 
 def _check_experts(x, w_up, w_down, chosen, weights, gated=False):
@@ -172,9 +191,11 @@ def padded_places(place: torch.Tensor, chosen: torch.Tensor, offsets: torch.Tens
 
 
 def combine_pairs(ys: torch.Tensor, place: torch.Tensor, weights: torch.Tensor,
-                  out: Optional[torch.Tensor] = None, identity=None) -> torch.Tensor:
+                  out: Optional[torch.Tensor] = None, identity=None,
+                  gate: Optional[torch.Tensor] = None) -> torch.Tensor:
     """float32 [N, D] (+)= sum_k weights[n, k] ys[place[n top + k]], in the order of k; every
-    place must be a row of ys (the caller's to know).  ``identity`` = (chosen int32 [N, top],
+    place must be a row of ys (the caller's to know).  ``gate`` (float32 [N, >= 1], first column read): ``out`` is
+    multiplied by sigmoid(gate[n, 0]) before the sums are added to it.  ``identity`` = (chosen int32 [N, top],
     number of experts, x [N, D]): a pair whose expert's index is that number or more adds
     ``weights[n, k] x[n]`` instead, and its place is not looked at."""
     chosen, n_experts, x = identity if identity is not None else (None, 0, None)
@@ -188,6 +209,10 @@ def combine_pairs(ys: torch.Tensor, place: torch.Tensor, weights: torch.Tensor,
                                  or tuple(x.shape) != (n, D)):
         raise KernelError("combine_pairs: identity needs chosen int32 [N, top] and x [N, D]")
     accumulate = out is not None
+    if gate is not None:
+        require_device(gate)
+        if not accumulate or gate.dtype != torch.float32 or gate.dim() != 2 or gate.shape[0] != n or gate.shape[1] < 1:
+            raise KernelError("combine_pairs: a gate is float32 [N, >= 1] and multiplies rows given as out")
     if out is None:
         out = torch.empty((n, D), dtype=torch.float32, device=ys.device)
     elif tuple(out.shape) != (n, D) or out.dtype != torch.float32:
@@ -195,7 +220,8 @@ def combine_pairs(ys: torch.Tensor, place: torch.Tensor, weights: torch.Tensor,
     check(library("routed_experts").gfa_combine_pairs(ptr(ys), ptr(place), ptr(weights), ptr(chosen),
                                                       _i(n_experts), ptr(x),
                                                       _i(0 if x is None else _is_bf16(x)), ptr(out), _i(n),
-                                                      _i(top), _i(D), _i(int(accumulate)),
+                                                      _i(top), _i(D), _i(int(accumulate)), ptr(gate),
+                                                      _ll(0 if gate is None else gate.stride(0)),
                                                       _i(_is_bf16(ys)), stream_handle()), "combine_pairs")
     return out
 
@@ -209,10 +235,13 @@ def grouped_rows_take(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def grouped_rows(x: torch.Tensor, order: Optional[torch.Tensor], top: int, w: torch.Tensor,
-                 offsets: torch.Tensor, activation: Optional[str], rows_at_most: int) -> torch.Tensor:
+                 offsets: torch.Tensor, activation: Optional[str], rows_at_most: int, gated: bool = False,
+                 limit: Optional[float] = None) -> torch.Tensor:
     """[P, N]: row ``offsets[e] + i`` is ``W[e] x[r]`` for expert e's i-th pair, r = the pair's
     token ``order[.] // top`` (or, without ``order``, the row at the same place of x, which then
-    has P rows).  With an activation the result is act(.) in bfloat16, else the float32 sums.
+    has P rows).  With an activation the result is act(.) in bfloat16, else the float32 sums; ``gated``: W holds
+    the gate rows, then as many up rows, and the result is bfloat16 [P, N / 2] of act(gate) * up, or of the clamped
+    gate with its ``limit``.
     x bfloat16 [rows, K], W bfloat16 [E, N, K], offsets int32 [E + 1] as :func:`expert_order`
     gives them; ``rows_at_most``: the most pairs one expert can have.  One pass over each
     expert's matrix whatever the number of its rows; nothing is read on the host."""
@@ -229,14 +258,20 @@ def grouped_rows(x: torch.Tensor, order: Optional[torch.Tensor], top: int, w: to
         P = order.numel()
     else:
         P, top = x.shape[0], 1
-    if activation is not None and activation not in EXPERT_ACTIVATIONS:
+    if gated:
+        if activation not in GATE_ACTIVATIONS or N % 2:
+            raise KernelError(f"grouped_rows: gate activation '{activation}' of {N} rows: {sorted(GATE_ACTIVATIONS)}")
+        act, limit = GATE_ACTIVATIONS[activation], check_gate_limit(activation, limit)
+    elif activation is not None and activation not in EXPERT_ACTIVATIONS:
         raise KernelError(f"grouped_rows: activation '{activation}': {EXPERT_ACTIVATIONS}")
-    out = torch.empty((P, N), dtype=torch.float32 if activation is None else torch.bfloat16,
+    else:
+        act = -1 if activation is None else ACTIVATIONS[activation]
+    out = torch.empty((P, N // 2 if gated else N), dtype=torch.float32 if activation is None else torch.bfloat16,
                       device=x.device)
     check(library("routed_experts").gfa_grouped_rows(
         ptr(x), ptr(order), _i(top), ptr(w), ptr(offsets), ptr(out), _i(E), _i(N), _i(K),
-        _i(-1 if activation is None else ACTIVATIONS[activation]), _i(max(1, int(rows_at_most))),
-        _i(int(rows_at_most <= DIRECT_X_MAX_ROWS)), stream_handle()), "grouped_rows")
+        _i(act), _i(max(1, int(rows_at_most))), _i(int(rows_at_most <= DIRECT_X_MAX_ROWS)), _i(int(gated)),
+        _f(limit or 0.0), stream_handle()), "grouped_rows")
     return out
 
 

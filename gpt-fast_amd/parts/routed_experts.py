@@ -123,22 +123,28 @@ class RoutedExperts(Part):
         per_expert = (self.w_up[0].numel() + self.w_down[0].numel()) * self.w_up.element_size()
         return idle * per_expert
 
-    def _routed(self, x, chosen, weights, y, batch):
+    def _few(self, n: int, batch) -> bool:
+        return n <= PAIRWISE_MAX_ROWS or getattr(batch, "is_decode", False)
+
+    def _grouped(self, x, batch) -> bool:
+        """One pass over each chosen expert's matrices, the pairs in the order of their experts."""
+        return (self._few(x.shape[0], batch) and x.shape[0] >= GROUPED_MIN_ROWS
+                and RE.grouped_rows_take(x, self.w_up) and self.spec.hidden % 8 == 0)
+
+    def _routed(self, x, chosen, weights, y, batch, lists=None, gate=None):
+        """``lists``: the pairs in the order of their experts, if they are there already; ``gate``: what
+        still multiplies y, a column of the router's sums."""
         s = self.spec
         n = x.shape[0]
         identity = (chosen, s.n_experts, x) if s.identity else None
-        few = n <= PAIRWISE_MAX_ROWS or getattr(batch, "is_decode", False)
-        if few and n >= GROUPED_MIN_ROWS and RE.grouped_rows_take(x, self.w_up) and s.hidden % 8 == 0:
-            offsets, order, place = RE.expert_order(chosen, self.n_choices)
-            if s.gated:
-                # the float32 sums of the gate rows and the up rows, then the gate
-                sums = RE.grouped_rows(x, order, s.top, self.w_up, offsets, None, n)
-                h = K.gate_mul_sums(sums, s.activation, s.limit)
-            else:
-                h = RE.grouped_rows(x, order, s.top, self.w_up, offsets, s.activation, n)
+        if self._grouped(x, batch):
+            offsets, order, place = lists if lists is not None else RE.expert_order(chosen, self.n_choices)
+            h = RE.grouped_rows(x, order, s.top, self.w_up, offsets, s.activation, n, s.gated, s.limit)
             ys = RE.grouped_rows(h, None, 1, self.w_down, offsets, None, n)
-            return RE.combine_pairs(ys, place, weights, out=y, identity=identity)
-        if few:
+            return RE.combine_pairs(ys, place, weights, out=y, identity=identity, gate=gate)
+        if self._few(n, batch):
+            if gate is not None:
+                K.scale_rows_sigmoid(y, gate)
             return RE.experts_few_rows(x, self.w_up, self.w_down, chosen, weights, s.activation, out=y,
                                        gated=s.gated, limit=s.limit)
         offsets, order, place = RE.expert_order(chosen, self.n_choices)
@@ -151,7 +157,7 @@ class RoutedExperts(Part):
             hs = RE.expert_tile_product(x, order, s.top, self.w_up, offsets, tiles, pairs, s.activation,
                                         s.gated, s.limit)
             ys = RE.expert_tile_product(hs, None, 1, self.w_down, offsets, tiles, pairs)
-            return RE.combine_pairs(ys, place, weights, out=y, identity=identity)
+            return RE.combine_pairs(ys, place, weights, out=y, identity=identity, gate=gate)
         bounds = offsets.cpu().tolist()                         # the host learns the experts' shares
         most = max(bounds[e + 1] - bounds[e] for e in range(s.n_experts))
         cap = max(1, (most + PAD_ROWS_TO - 1) // PAD_ROWS_TO) * PAD_ROWS_TO
@@ -164,7 +170,7 @@ class RoutedExperts(Part):
             ys = torch.empty((s.n_experts, cap, s.dim), dtype=x.dtype, device=x.device)
             K.gemm_f32_batched(hs, self.w_down, ys)
             return RE.combine_pairs(ys.view(-1, s.dim), RE.padded_places(place, chosen, offsets, cap),
-                                    weights, out=y, identity=identity)
+                                    weights, out=y, identity=identity, gate=gate)
         # (the pairs of identity experts stand behind the others and take part in no product)
         xs = RE.gather_pairs(x, order[:bounds[s.n_experts]], s.top)
         hs = torch.empty((xs.shape[0], self.up_rows), dtype=x.dtype, device=x.device)
@@ -178,7 +184,7 @@ class RoutedExperts(Part):
             a, b = bounds[e], bounds[e + 1]
             if b > a:
                 self._product(hs[a:b], self.w_down[e], ys[a:b])
-        return RE.combine_pairs(ys, place, weights, out=y, identity=identity)
+        return RE.combine_pairs(ys, place, weights, out=y, identity=identity, gate=gate)
 
     def _activated(self, h):
         """The inner rows from the first product's rows [P, F] (or [P, 2 F]: gate, then up)."""
@@ -195,8 +201,10 @@ class RoutedExperts(Part):
         """The feed-forward's output alone, float32 [N, D]."""
         s = self.spec
         z = L.linear(x, self.w_router, out_dtype=torch.float32)
-        chosen, weights = RE.route(z, self.n_choices, s.top, s.n_groups, s.keep_groups, s.weight_eps,
-                                   scoring=s.scoring, correction=self.correction, group_top=s.group_top)
+        ordered = self._grouped(x, batch) and RE.orders_with_route(x.shape[0], self.n_choices, s.n_groups)
+        chosen, weights, *lists = RE.route(z, self.n_choices, s.top, s.n_groups, s.keep_groups, s.weight_eps,
+                                           scoring=s.scoring, correction=self.correction, group_top=s.group_top,
+                                           ordered=ordered)
         self.last_chosen = chosen                  # a replayed step leaves its choice here as well
         y = None
         if s.shared_hidden:
@@ -206,9 +214,9 @@ class RoutedExperts(Part):
                 h = L.linear(x, self.shared_up)
                 K.activate(h, s.activation, out=h)
             y = L.linear(h, self.shared_down, out_dtype=torch.float32)
-            if self.shared_gate:
-                K.scale_rows_sigmoid(y, z[:, self.n_choices:])
-        return self._routed(x, chosen, weights, y, batch)
+        # the shared expert's gate is applied where the experts' results are added to it
+        gate = z[:, self.n_choices:] if self.shared_gate and y is not None else None
+        return self._routed(x, chosen, weights, y, batch, lists[0] if lists else None, gate)
 
     def forward(self, x, batch, residual):
         K.add_into(residual, self.forward_rows(x, batch))

@@ -1,0 +1,77 @@
+"""What the experts' kernels of few-row steps do on their way, against the kernels of its own that each replaces: the
+pairs' order from the router's launch, the gate inside the first product, a shared expert's gate inside the sum."""
+import pytest
+import torch
+
+from util import rel_err
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("n,E,top,groups,keep", [(1, 8, 1, 1, 1), (3, 32, 4, 4, 2), (16, 32, 4, 1, 1), (16, 65, 7, 5, 3),
+                                                 (5, 256, 8, 8, 4), (16, 128, 64, 1, 1)])
+@pytest.mark.parametrize("scoring", ["softmax", "sigmoid"])
+def test_order_from_the_routers_launch(n, E, top, groups, keep, scoring):
+    from gpt_fast_amd.ops import routed_experts as RE
+    torch.manual_seed(n * 1000 + E)
+    z = torch.randn(n, E + 3, device=DEV)[:, :E + 1]
+    correction = torch.randn(E, device=DEV) * 0.1
+    args = dict(scoring=scoring, correction=correction, group_top=2)
+    assert RE.orders_with_route(n, E, groups)
+    want_c, want_w = RE.route(z, E, top, groups, keep, 1e-20, **args)
+    chosen, weights, (offsets, order, place) = RE.route(z, E, top, groups, keep, 1e-20, ordered=True, **args)
+    assert torch.equal(chosen, want_c) and torch.equal(weights, want_w)
+    counts = torch.bincount(chosen.flatten().long(), minlength=E)
+    assert offsets.tolist() == [0] + counts.cumsum(0).tolist()
+    # every pair once, among its expert's places; the order inside an expert is free
+    assert sorted(order.tolist()) == list(range(n * top))
+    assert torch.equal(place[order.long()], torch.arange(n * top, dtype=torch.int32, device=DEV))
+    experts = chosen.flatten()[order.long()]
+    assert torch.equal(experts, experts.sort().values)
+
+
+def test_what_does_not_fit_one_workgroup_is_refused():
+    from gpt_fast_amd.ops import routed_experts as RE
+    from gpt_fast_amd.ops.library import KernelError
+    assert not RE.orders_with_route(17, 8, 1) and not RE.orders_with_route(16, 1024, 1)
+    with pytest.raises(KernelError):
+        RE.route(torch.zeros(17, 8, device=DEV), 8, 2, 1, 1, 0.0, ordered=True)
+
+
+@pytest.mark.parametrize("activation,limit", [("silu", None), ("gelu_tanh", None), ("clamped_swish", 1.5)])
+@pytest.mark.parametrize("n,E,top,F,K", [(1, 4, 2, 8, 64), (2, 6, 2, 40, 136), (7, 3, 2, 100, 520), (16, 5, 3, 72, 1032),
+                                         (30, 4, 2, 64, 256), (60, 3, 1, 136, 264)])
+def test_gate_inside_the_grouped_product(n, E, top, F, K, activation, limit):
+    from gpt_fast_amd.ops import kernels, routed_experts as RE
+    torch.manual_seed(n * 100 + F)
+    x = torch.randn(n, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(E, 2 * F, K, device=DEV) * K ** -0.5).to(torch.bfloat16)
+    chosen = torch.stack([torch.randperm(E)[:top] for _ in range(n)]).to(torch.int32).to(DEV)
+    offsets, order, _ = RE.expert_order(chosen, E)
+    sums = RE.grouped_rows(x, order, top, w, offsets, None, n)
+    want = kernels.gate_mul_sums(sums, activation, limit)
+    got = RE.grouped_rows(x, order, top, w, offsets, activation, n, True, limit)
+    assert got.shape == want.shape and got.dtype == torch.bfloat16
+    # the same sums but for where a tile's rows of W begin to be walked: float32 sums in another order (1e-6 of their
+    # size), which now and then round to the neighbouring bfloat16 (2^-8)
+    assert rel_err(got, want) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("n,top,D,dtype", [(1, 1, 8, torch.float32), (3, 4, 136, torch.bfloat16), (16, 2, 100, torch.float32),
+                                           (1100, 3, 264, torch.bfloat16)])
+def test_sum_of_the_pairs_with_a_gate_on_what_is_there(n, top, D, dtype):
+    from gpt_fast_amd.ops import kernels, routed_experts as RE
+    torch.manual_seed(n + D)
+    ys = torch.randn(n * top, D, device=DEV).to(dtype)
+    place = torch.randperm(n * top, device=DEV).to(torch.int32)
+    weights = torch.rand(n, top, device=DEV)
+    gate = torch.randn(n, 5, device=DEV)[:, 2:]
+    start = torch.randn(n, D, device=DEV)
+    want = start.double() * torch.sigmoid(gate[:, :1].double()) + \
+        (ys.double()[place.long()].view(n, top, D) * weights.double()[:, :, None]).sum(1)
+    got = RE.combine_pairs(ys, place, weights, out=start.clone(), gate=gate)
+    assert rel_err(got, want) < 1e-6                     # top + 2 float32 roundings of 6e-8 each
+    scaled = start.clone()
+    kernels.scale_rows_sigmoid(scaled, gate)
+    assert rel_err(RE.combine_pairs(ys, place, weights, out=scaled), want) < 1e-6
