@@ -1048,7 +1048,7 @@ static int expert_rows_launch(const PtArgs& a, int mode, int pairs, hipStream_t 
     const long long row_tiles = pairs / (64 * TM) + (a.E < pairs ? a.E : pairs);       // at most
     const long long total = row_tiles * ((a.F + cols - 1) / cols);
     if (total > 0x7ffffff0LL) return (int)hipErrorInvalidValue;
-    const unsigned grid = (unsigned)((total + 7) / 8 * 8);
+    const unsigned grid = (unsigned)((total + 8 * PT_RUN - 1) / (8 * PT_RUN) * (8 * PT_RUN));
     if (mode >= 2) prompt_tile_kernel<TM, TN, PT_GATE><<<grid, 256, 0, stream>>>(a);
     else prompt_tile_kernel<TM, TN, PT_ROWS><<<grid, 256, 0, stream>>>(a);
     return GFA_LAUNCH_RESULT();

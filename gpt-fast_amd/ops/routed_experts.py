@@ -302,11 +302,31 @@ def _tiles(pairs: int, n_experts: int, rows: int, F: int, columns: int) -> float
 
 
 @functools.lru_cache(maxsize=4096)
+def tall_tiles_win(n_experts: int, pairs: int, F: int, K: int, mode: int, units: int) -> bool:
+    """Whether 256 x 256 tiles, which read each operand half as often and are only as high as their rows (steps of 64),
+    make the products of :func:`rows_tile`'s arguments fastest.  Microseconds, shares spread as exp(0.4 normal), tiles of
+    128 x 128 and these: 32 experts, 4,096 -> 3,584, x 40 rows 192, 192; x 64 202, 211; x 100 256, 222; x 140 302, 247;
+    x 222 385, 338; x 450 616, 504; 64 of them, 4,096 -> 2 x 2,048, x 64 506, 434; x 180 779, 601; 128, 2,048 ->
+    4,096, x 64 461, 467; x 140 639, 571.  Not where 128 x 128 tiles need no second round (8, 4,096 -> 3,584, x 222 94,
+    119), nor where these need one for little (16, 4,096 -> 3,584, x 222 179, 210, 1.18 rounds; x 300 250, 228, 1.44;
+    16, 2,048 -> 4,096, x 180 96, 101, 1.08; x 222 125, 109, 1.35).  Up to K = 1,024 it is either by some percent."""
+    if K <= 1024 or pairs < 64 * n_experts:
+        return False
+    gated = mode == 2
+    if _tiles(pairs, n_experts, 128, F, 64 if gated else 128) <= 2 * units:
+        return False
+    return not 1.0 < _tiles(pairs, n_experts, 256, F, 128 if gated else 256) / units < 1.3
+
+
+@functools.lru_cache(maxsize=4096)
 def rows_tile(n_experts: int, pairs: int, F: int, K: int, mode: int, units: int) -> int:
     """Which kernel makes the experts' products of ``pairs`` rows of K into rows of F on ``units`` compute units
     (``mode`` 0: the sums, 1: an activation of them, 2: a gated one): 1, 2 or 4 for the tile kernel
     (csrc/prompt_tile.h) with tiles of 64 x 256, 128 x 128 or 256 x 256 rows of x and of W, 0 for the older one
     (``expert_tile_kernel``, which needs :func:`expert_tiles`).
+
+    Asked where :func:`tall_tiles_win` does not say so; its measurements of tile 4 are of tiles that are 256 high
+    whatever their rows.
 
     The rows of an expert are known on the device alone; on the host there is their mean.  A round of the chip is one
     tile 4 to a unit, two of tile 1 or 2, three of the older kernel's.  Microseconds, n x m being n experts of m rows
@@ -348,13 +368,14 @@ def rows_tile(n_experts: int, pairs: int, F: int, K: int, mode: int, units: int)
 
 
 def _tile_of(w: torch.Tensor, mode: int, pairs: int) -> int:
-    """:func:`rows_tile` where the tile kernel takes these experts (inner sizes of whole pieces of 64, results of
+    """:func:`tall_tiles_win`, then :func:`rows_tile`, where the tile kernel takes these experts (inner sizes of whole pieces of 64, results of
     whole 16 bytes, matrices below 4 GiB), else 0."""
     E, N, K = w.shape
     F = N // 2 if mode == 2 else N
     if K % 64 != 0 or F % 8 != 0 or not 0 < N * K * 2 < 1 << 32:
         return 0
-    return rows_tile(E, pairs, F, K, mode, _compute_units(w.device))
+    sizes = (E, pairs, F, K, mode, _compute_units(w.device))
+    return 4 if tall_tiles_win(*sizes) else rows_tile(*sizes)
 
 
 def takes_tile_list(w: torch.Tensor, activation: Optional[str], gated: bool, pairs: int) -> bool:

@@ -75,3 +75,28 @@ def test_sum_of_the_pairs_with_a_gate_on_what_is_there(n, top, D, dtype):
     scaled = start.clone()
     kernels.scale_rows_sigmoid(scaled, gate)
     assert rel_err(RE.combine_pairs(ys, place, weights, out=scaled), want) < 1e-6
+
+
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("rows", [[1, 64, 65, 0, 128], [129, 192, 193, 255], [256, 257, 300], [513, 0, 2, 1030]])
+def test_tall_tiles_of_every_height(rows, gated, monkeypatch):
+    """Tiles of 64, 128, 192 and 256 rows: an expert's rows in equal parts, remainders on either side of a step."""
+    from gpt_fast_amd.ops import routed_experts as RE
+    monkeypatch.setattr(RE, "tall_tiles_win", lambda *a: True)
+    torch.manual_seed(sum(rows))
+    E, F, K, n = len(rows), 328, 192, sum(rows)
+    x = torch.randn(n, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(E, (2 if gated else 1) * F, K, device=DEV) * K ** -0.5).to(torch.bfloat16)
+    offsets = torch.tensor([0] + list(torch.tensor(rows).cumsum(0)), dtype=torch.int32, device=DEV)
+    order = torch.randperm(n, device=DEV).to(torch.int32)
+    got = RE.expert_tile_product(x, order, 1, w, offsets, None, n, "silu" if gated else None, gated)
+    assert got.shape == (n, F)
+    for e in range(E):
+        a, b = int(offsets[e]), int(offsets[e + 1])
+        if a == b:
+            continue
+        want = x[order[a:b].long()].double() @ w[e].double().t()
+        if gated:
+            want = torch.nn.functional.silu(want[:, :F]) * want[:, F:]
+        # one rounding to bfloat16 (2^-9 of a value) and float32 sums
+        assert rel_err(got[a:b], want) < 2.0 ** -8, (e, rows[e])
