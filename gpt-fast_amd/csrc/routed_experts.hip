@@ -594,7 +594,8 @@ extern "C" int gfa_combine_pairs(const void* ys, const int* place, const float* 
 // DEPTH pieces of W under way, and tiles begin at different pieces: decode steps of 16, 24 and 56 rows with
 // 32 experts of 2 x 4,096 x 3,584 (whole requests) 57.5 -> 55.5, 61.2 -> 58.6, 75.5 -> 73.0 ms; of 2, 4 and 12
 // rows with gated ones of 3 x 4,096 x 2,048 25.7 -> 24.5, 37.8 -> 36.2, 43.9 -> 40.6.  DEPTH: at 16 rows four pieces
-// 55.5, two 56.8, eight 57.0; at 17 to 32 rows two 58.6, four 60.9; above four 72.9, two 73.2;
+// 55.5, two 56.8, eight 57.0; at 17 to 32 rows two 58.6, four 60.9; above
+// two (64 rows on 32 experts, 4,096 -> 3,584 and back 165 and 155 us; four 179 and 168);
 // XD one 36.2, two 36.6, four 37.9 (more waves share a compute unit).  act < 0: the float
 // sums are stored; else act(sum) as bfloat16.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 re_bf16x8_t;
@@ -634,7 +635,10 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
     // often a power of two apart, and tiles that walk them in step meet in the same memory channels.
     const int per_wave = XD ? (T + GR_NW - 1) / GR_NW : T;
     const int t_lo = XD ? wave * per_wave : 0, t_hi = t_lo + per_wave < T ? t_lo + per_wave : T;
-    const int turn = t_hi > t_lo ? (blockIdx.x * 3 + e * 5) % (t_hi - t_lo) : 0;
+    // Rows of 7,168 bytes (K = 3,584) spread by themselves: 27 experts' product of 4,096 columns 135 us with turns,
+    // 132 without; all 32 145, 141; of 8,192 bytes (3,584 columns) without turns and waiting at barriers 179, now 144.
+    const bool meet = XD || K % 2048 == 0;
+    const int turn = meet && t_hi > t_lo ? (blockIdx.x * 3 + e * 5) % (t_hi - t_lo) : 0;
     auto piece = [&](int t) { return t + turn < t_hi ? t + turn : t + turn - (t_hi - t_lo); };
     const bf16_t* wsrc[4];
 #pragma unroll
@@ -843,7 +847,7 @@ extern "C" int gfa_grouped_rows(const void* x, const int* order, int top, const 
     if (rows_at_most <= 16 && x_direct) GFA_LAUNCH_GROUPED(1, 1, true);
     else if (rows_at_most <= 16) GFA_LAUNCH_GROUPED(1, 4, false);
     else if (rows_at_most <= 32) GFA_LAUNCH_GROUPED(2, 2, false);
-    else GFA_LAUNCH_GROUPED(4, 4, false);
+    else GFA_LAUNCH_GROUPED(4, 2, false);
 #undef GFA_LAUNCH_GROUPED_G
 #undef GFA_LAUNCH_GROUPED
     return GFA_LAUNCH_RESULT();
