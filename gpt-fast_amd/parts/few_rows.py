@@ -6,18 +6,20 @@ from ..ops.linear import HalfNormed
 from .attention import Attention
 from .block import PreNormBlock
 from .feed_forward import GatedFeedForward
-from .norm import RMSNorm
+from .norm import RMSNorm, ScalarRMSNorm
 from .position import RotaryPosition
 
 
 def _plain_layer(block) -> bool:
     """Pre-norm attention with interleaved rotation, then a gated feed-forward, root-mean-square norms before
-    both: the layers whose few-row steps ops.few_row_layers launches."""
+    both: the layers whose few-row steps ops.few_row_layers launches.  Exactly these classes: the call takes their
+    weights and never asks their ``forward``, which a class derived from one may have replaced."""
     if type(block) is not PreNormBlock or type(block.mixer) is not Attention \
             or type(block.feed_forward) is not GatedFeedForward:
         return False
     f, p = block.feed_forward.spec, block.mixer.position
-    return (isinstance(block.mixer_norm, RMSNorm) and isinstance(block.feed_forward_norm, RMSNorm)
+    norms = (RMSNorm, ScalarRMSNorm)                     # both hold a float32 weight per column
+    return (type(block.mixer_norm) in norms and type(block.feed_forward_norm) in norms
             and type(p) is RotaryPosition and p.spec.layout == "interleaved"
             and f.activation in F.GATE_MODES and f.limit is None)
 

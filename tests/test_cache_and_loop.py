@@ -8,6 +8,7 @@ import sys
 import pytest
 import torch
 
+import util
 from gpt_fast_amd.cache.slots import CacheFull, FreeList
 from gpt_fast_amd.cache.store import Cache, KVNeed, StateNeed
 from gpt_fast_amd.engine.batch import BatchLayout, Entry, fill_host
@@ -594,6 +595,41 @@ def test_the_kernel_of_the_experts_rows_goes_by_their_sizes_and_the_chip():
     assert tiles(128, 4096, 1024, 0, (399, 400)) == [0, 4] and tiles(128, 4096, 1024, 1, (400,)) == [0]
     assert tiles(16, 4096, 4096, 0, (85, 100, 160, 190, 222, 300)) == [2, 2, 4, 2, 4, 4]     # one round, a little more
     assert tiles(64, 1024, 2048, 1, (160, 190, 222)) == [4, 2, 2]
+
+
+def test_a_registered_norm_derived_from_the_librarys_is_not_replaced_in_few_row_steps(monkeypatch):
+    """Layers whose few-row steps one native call launches have the library's own norms: the call never asks a norm's
+    ``forward``."""
+    import dataclasses
+    from gpt_fast_amd.architectures.llama import llama_plan
+    from gpt_fast_amd.config.llama import LlamaConfig
+    from gpt_fast_amd.config.spec import NormSpec
+    from gpt_fast_amd.parts import Runtime, register_norm
+    from gpt_fast_amd.parts.base import NORMS
+    from gpt_fast_amd.parts.model import DecoderModel
+    from gpt_fast_amd.parts.norm import RMSNorm
+
+    class Doubled(RMSNorm):
+        def forward(self, residual, rows=None):
+            return 2 * super().forward(residual, rows=rows)
+
+    monkeypatch.setattr(NORMS, "_kinds", dict(NORMS._kinds))
+    register_norm("test_doubled", Doubled)
+    plan = llama_plan(LlamaConfig.from_dict(util.TINY_A))
+    own = NormSpec(64, 1e-5, kind="test_doubled")
+
+    def ends(dtype, **norms):
+        second = dataclasses.replace(plan.layers[1], **norms)
+        changed = dataclasses.replace(plan, layers=[plan.layers[0], second])
+        return DecoderModel(changed, Runtime(dtype, "cpu")).few_rows.ends
+
+    for dtype in (torch.float32, torch.bfloat16):
+        assert ends(dtype) == [2, 2]
+        scalar = NormSpec(64, 1e-5, kind="rms_scalar")
+        assert ends(dtype, mixer_norm=scalar, feed_forward_norm=scalar) == [2, 2]
+        for name in ("mixer_norm", "feed_forward_norm"):
+            # the layer before it may still go alone, but in bfloat16 only where the layer behind takes no halves
+            assert ends(dtype, **{name: own}) == ([1, 0] if dtype == torch.float32 else [0, 0])
 
 
 def test_residual_stream_runs_what_was_put_off_before_any_read():
