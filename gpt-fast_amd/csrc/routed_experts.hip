@@ -580,24 +580,30 @@ extern "C" int gfa_combine_pairs(const void* ys, const int* place, const float* 
 //   row(p) = order[p] / top if order is given (the token of the pair at place p), else p.
 //
 // Grid (column tiles, experts).  A workgroup of an expert without rows ends at once; the others
-// walk K in pieces of 128: the expert's rows of x (up to CT * 16 at a time, gathered) go once
-// per workgroup into LDS, double-buffered; each wave streams 16 rows of W through a padded LDS
-// tile of its own into the operand layout of v_mfma_f32_16x16x32_bf16, DEPTH pieces ahead.  XD (up to
-// 16 rows, for steps of very few tokens, where few experts have rows at all and the chip is not
-// full): no shared x and no barriers while K is walked; a lane reads its own operand pieces of
-// x from memory, as far ahead as W; the workgroup's four waves take the same 16 columns
-// and a quarter of K each, and the first adds their sums in the waves' order (four times the
-// workgroups).  A
-// row of x meets only its own lanes of the operand and K is walked in an order that the expert and the
-// tile alone decide, so a pair's result does not depend on the other pairs.
-// What bounds it is the stream of the chosen experts' matrices.  Barriers that wait for shared memory alone keep
-// DEPTH pieces of W under way, and tiles begin at different pieces: decode steps of 16, 24 and 56 rows with
-// 32 experts of 2 x 4,096 x 3,584 (whole requests) 57.5 -> 55.5, 61.2 -> 58.6, 75.5 -> 73.0 ms; of 2, 4 and 12
-// rows with gated ones of 3 x 4,096 x 2,048 25.7 -> 24.5, 37.8 -> 36.2, 43.9 -> 40.6.  DEPTH: at 16 rows four pieces
-// 55.5, two 56.8, eight 57.0; at 17 to 32 rows two 58.6, four 60.9; above
-// two (64 rows on 32 experts, 4,096 -> 3,584 and back 165 and 155 us; four 179 and 168);
-// XD one 36.2, two 36.6, four 37.9 (more waves share a compute unit).  act < 0: the float
-// sums are stored; else act(sum) as bfloat16.
+// walk K in pieces of 128, each wave through a padded LDS tile of its own into the operand layout of
+// v_mfma_f32_16x16x32_bf16, DEPTH pieces of W ahead.
+// XD, up to 16 rows: a lane reads its own operand pieces of x from memory, as far ahead as W; the workgroup's four
+// waves take the same 16 columns and a quarter of K each, without barriers, and the first adds their sums in the
+// waves' order.  Else the expert's rows of x (up to CT * 16 at a time, gathered) go once per workgroup into LDS,
+// double-buffered, and each wave takes 16 columns; barriers that wait for shared memory alone keep the pieces of W
+// under way.
+// A row of x meets only its own lanes of the operand.  A pair's sums are the same whatever else the step holds, as long as
+// it takes the same form: among steps of up to 16 rows, and among larger ones; the two forms add K up in another order.
+//
+// What bounds it is the stream of the chosen experts' matrices, and the round of the chip that their workgroups end
+// in: how many experts have rows is known on the device alone.  XD's quarter-sized workgroups end in small ones.
+// 32 experts of 4,096 -> 3,584 and back, us, by the experts that have rows, XD against shared x with workgroups of
+// 64 columns and two pieces ahead (five workgroups a unit) or four (three):
+//   16 experts 71 + 70, 81 + 79, 94 + 86; 18 78 + 77, 87 + 83, 98 + 90; 21 91 + 90, 96 + 111, 103 + 96;
+//   23 99 + 98, 124 + 115, 107 + 102; 28 120 + 119, 145 + 127, 145 + 134.
+// Gated ones of 4,096 -> 2 x 2,048, 18 experts: 90, 103, 110; 28: 135, 163, 167.
+// XD takes its pieces in step: beginning elsewhere for each tile cost it 4 to 8 % (18 experts 86 + 80).
+// Shared x: rows of a matrix that are a multiple of 4,096 bytes apart meet in the same memory channels where tiles walk
+// them in step, so tiles begin at different pieces (TURN): 32 experts, 24 to 32 rows, K = 4,096 without turns and waiting
+// for every load at barriers 171 to 178, now 139 to 144; not for K = 3,584, 512, 1,024 and 1,536 (3,584: 141, with
+// turns 145).  DEPTH there: at 17 to 32 rows two pieces, four cost 4 % of a request; above, 64 rows, two 165 + 155,
+// four 179 + 168.
+// act < 0: the float sums are stored; else act(sum) as bfloat16.
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 re_bf16x8_t;
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float re_floatx4_t;
 union ReFrag {
@@ -610,12 +616,14 @@ union ReFrag {
 #define GR_TILE (16 * GR_PITCH)
 #define GR_NW 4                               // waves per workgroup: 64 columns
 
+// Five workgroups of XD fit a unit without the gate (with it the fifth would cost spilled registers: 4,096 ->
+// 2 x 2,048, 18 experts 90 us, 103 with).
 template <int CT, int DEPTH, bool XD, bool GATED>
-__global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
+__global__ __launch_bounds__(GR_NW * 64, XD && DEPTH == 1 && !GATED ? 5 : 1) void grouped_rows_kernel(
         const bf16_t* __restrict__ x, const int* __restrict__ order, int top,
         const bf16_t* __restrict__ w, const int* __restrict__ offsets, void* __restrict__ out,
         int N, int K, int act, float limit) {
-    static_assert(XD || DEPTH % 2 == 0, "x alternates between two buffers");
+    static_assert(XD ? CT == 1 : DEPTH % 2 == 0, "16 rows a lane reads itself; shared x alternates between two buffers");
     constexpr int NT = GR_NW * 64;
     constexpr int XBYTES = CT * 16 * GR_PITCH;
     constexpr int XPER = CT;                               // CT * 16 rows of 16 pieces over 256 threads
@@ -631,15 +639,11 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
     const int F = N / 2;                                   // GATED: columns of out
     const int T = (K + GR_SUBK - 1) / GR_SUBK;
     const bf16_t* we = w + (size_t)e * N * K;
-    // The pieces that this workgroup (XD: the wave) walks, and the one that it begins with: rows of a matrix are
-    // often a power of two apart, and tiles that walk them in step meet in the same memory channels.
-    const int per_wave = XD ? (T + GR_NW - 1) / GR_NW : T;
-    const int t_lo = XD ? wave * per_wave : 0, t_hi = t_lo + per_wave < T ? t_lo + per_wave : T;
-    // Rows of 7,168 bytes (K = 3,584) spread by themselves: 27 experts' product of 4,096 columns 135 us with turns,
-    // 132 without; all 32 145, 141; of 8,192 bytes (3,584 columns) without turns and waiting at barriers 179, now 144.
-    const bool meet = XD || K % 2048 == 0;
-    const int turn = meet && t_hi > t_lo ? (blockIdx.x * 3 + e * 5) % (t_hi - t_lo) : 0;
-    auto piece = [&](int t) { return t + turn < t_hi ? t + turn : t + turn - (t_hi - t_lo); };
+    // XD: the wave's quarter of the pieces; else all of them, beginning with the turn's
+    const int per_wave = (T + GR_NW - 1) / GR_NW;
+    const int t_lo = XD ? wave * per_wave : 0, t_hi = XD && t_lo + per_wave < T ? t_lo + per_wave : T;
+    const int turn = !XD && K % 2048 == 0 ? (blockIdx.x * 3 + e * 5) % T : 0;
+    auto piece = [&](int t) { return XD || t + turn < T ? t + turn : t + turn - T; };
     const bf16_t* wsrc[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -823,12 +827,13 @@ __global__ __launch_bounds__(GR_NW * 64) void grouped_rows_kernel(
 }
 
 // out [pairs, N] from x (rows by order / top, or by place) and W [E, N, K]; rows_at_most: the
-// most rows one expert can have (the step's tokens), which sizes the tiles of x.  gated: W holds N / 2 gate
+// most rows one expert can have (the step's tokens), which chooses the form; depth: pieces ahead of the
+// one of up to 16 rows (1 or 2).  gated: W holds N / 2 gate
 // rows, then as many up rows, and out is bfloat16 [pairs, N / 2] of act(gate) * up (act 2: the clamped
 // gate); a tile of 16 rows of W is eight of either.
 extern "C" int gfa_grouped_rows(const void* x, const int* order, int top, const void* w,
                                 const int* offsets, void* out, int E, int N, int K, int act,
-                                int rows_at_most, int x_direct, int gated, float limit, hipStream_t stream) {
+                                int rows_at_most, int depth, int gated, float limit, hipStream_t stream) {
     if (gated && (N % 2 || act < 0 || act > 2)) return (int)hipErrorInvalidValue;
     if (E <= 0 || N <= 0 || K <= 0 || K % 8 || top <= 0 || E > 65535) return (int)hipErrorInvalidValue;
     if (!gated && act >= 0 && act != 0 && act != 1 && act != 3) return (int)hipErrorInvalidValue;
@@ -844,8 +849,8 @@ extern "C" int gfa_grouped_rows(const void* x, const int* order, int top, const 
         if (gated) GFA_LAUNCH_GROUPED_G(CTV, DV, XDV, true);                                      \
         else GFA_LAUNCH_GROUPED_G(CTV, DV, XDV, false);                                           \
     } while (0)
-    if (rows_at_most <= 16 && x_direct) GFA_LAUNCH_GROUPED(1, 1, true);
-    else if (rows_at_most <= 16) GFA_LAUNCH_GROUPED(1, 4, false);
+    if (rows_at_most <= 16 && depth >= 2) GFA_LAUNCH_GROUPED(1, 2, true);
+    else if (rows_at_most <= 16) GFA_LAUNCH_GROUPED(1, 1, true);
     else if (rows_at_most <= 32) GFA_LAUNCH_GROUPED(2, 2, false);
     else GFA_LAUNCH_GROUPED(4, 2, false);
 #undef GFA_LAUNCH_GROUPED_G

@@ -16,9 +16,6 @@ EXPERT_ACTIVATIONS = ("silu", "gelu_tanh", "gelu")
 CLAMPED_GATE = "clamped_swish"          # of gated experts only: ops.kernels.gate_mul
 MAX_EXPERTS = 1024
 MAX_TOP = 64
-# steps of up to this many tokens take the form of grouped_rows in which every wave reads its
-# own pieces of x (no barriers); more tokens share x through LDS
-DIRECT_X_MAX_ROWS = 4
 
 
 def _is_bf16(t: torch.Tensor) -> int:
@@ -234,6 +231,15 @@ def grouped_rows_take(x: torch.Tensor, w: torch.Tensor) -> bool:
             and w.is_contiguous() and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
+def _pieces_ahead(n_experts: int, pairs: int, rows: int, units: int) -> int:
+    """Pieces of W that a wave of :func:`grouped_rows` has under way at up to 16 rows of x: two where all workgroups that
+    can have work, one per 16 of the ``rows`` of an expert's matrix, are on the chip at once, three to a unit, as the
+    registers of two pieces allow; else one, four or five to a unit.  Microseconds with two and with one: 3,072 -> 512, 12
+    experts with rows 12.4, 14.6; 22 14.8, 16.9; 26, more than fit, 18.9, 17.9; 4,096 -> 1,536, six 15.2, 18.1;
+    1,536 -> 4,096, two 8.9, 9.0; eight 22.2, 19.7; 512 -> 3,072, 39 26.7, 20.3."""
+    return 2 if min(n_experts, pairs) * ((rows + 15) // 16) <= 3 * units else 1
+
+
 def grouped_rows(x: torch.Tensor, order: Optional[torch.Tensor], top: int, w: torch.Tensor,
                  offsets: torch.Tensor, activation: Optional[str], rows_at_most: int, gated: bool = False,
                  limit: Optional[float] = None) -> torch.Tensor:
@@ -270,8 +276,8 @@ def grouped_rows(x: torch.Tensor, order: Optional[torch.Tensor], top: int, w: to
                       device=x.device)
     check(library("routed_experts").gfa_grouped_rows(
         ptr(x), ptr(order), _i(top), ptr(w), ptr(offsets), ptr(out), _i(E), _i(N), _i(K),
-        _i(act), _i(max(1, int(rows_at_most))), _i(int(rows_at_most <= DIRECT_X_MAX_ROWS)), _i(int(gated)),
-        _f(limit or 0.0), stream_handle()), "grouped_rows")
+        _i(act), _i(max(1, int(rows_at_most))), _i(_pieces_ahead(E, P, N, _compute_units(w.device))),
+        _i(int(gated)), _f(limit or 0.0), stream_handle()), "grouped_rows")
     return out
 
 

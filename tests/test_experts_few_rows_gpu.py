@@ -58,6 +58,52 @@ def test_gate_inside_the_grouped_product(n, E, top, F, K, activation, limit):
     assert rel_err(got, want) <= 2.0 ** -8
 
 
+def _pairs(n, E, top, K, N, seed):
+    torch.manual_seed(seed)
+    x = torch.randn(n, K, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(E, N, K, device=DEV) * K ** -0.5).to(torch.bfloat16)
+    return x, w, torch.stack([torch.randperm(E)[:top] for _ in range(n)]).to(torch.int32).to(DEV)
+
+
+# up to 16 rows a wave takes a quarter of K in pieces of 128: quarters without, with unequal and with cut pieces, one
+# piece ahead and two (which of them by the workgroups that a unit gets: few columns and many).  More rows: K whose
+# pieces are walked from the workgroup's own place on (multiples of 2,048), several of these, and others.
+WALKS = [(1, 3, 2, 40, 1032), (2, 8, 4, 24, 136), (4, 24, 4, 1024, 3584), (5, 4, 2, 24, 4096), (9, 16, 6, 2048, 640),
+         (16, 5, 3, 72, 4104), (17, 5, 3, 328, 2048), (30, 6, 2, 200, 4096), (33, 6, 2, 136, 2056), (60, 4, 3, 520, 6144)]
+
+
+@pytest.mark.parametrize("n,E,top,F,K", WALKS)
+def test_grouped_product_from_every_place_of_the_walk(n, E, top, F, K):
+    from gpt_fast_amd.ops import routed_experts as RE
+    x, w, chosen = _pairs(n, E, top, K, 2 * F, n + K)
+    offsets, order, _ = RE.expert_order(chosen, E)
+    sums = RE.grouped_rows(x, order, top, w, offsets, None, n).double()
+    gated = RE.grouped_rows(x, order, top, w, offsets, "silu", n, True)
+    for e in range(E):
+        a, b = int(offsets[e]), int(offsets[e + 1])
+        xs = x[(order[a:b] // top).long()].double()
+        want, size = xs @ w[e].double().t(), xs.abs() @ w[e].double().abs().t()
+        # K / 32 matrix instructions one after the other, of 32 products each: as many float32 roundings of at most the
+        # sum of the products' sizes, and four partial sums
+        assert ((sums[a:b] - want).abs() <= (K / 32 + 36) * 2.0 ** -23 * size).all(), e
+        if b > a:                                        # one rounding to bfloat16 more
+            assert rel_err(gated[a:b], torch.nn.functional.silu(want[:, :F]) * want[:, F:]) < 2.0 ** -8, e
+
+
+@pytest.mark.parametrize("counts", [(16, 1, 3, 4, 9), (60, 17, 32, 33)])
+@pytest.mark.parametrize("K", [1032, 4096])
+def test_a_pairs_sums_are_the_same_among_steps_of_one_form(counts, K):
+    """Up to 16 rows, and more: whatever else the step holds."""
+    from gpt_fast_amd.ops import routed_experts as RE
+    E, top, N = 6, 2, 200
+    x, w, chosen = _pairs(counts[0], E, top, K, N, K)
+    rows = []
+    for n in counts:
+        offsets, order, place = RE.expert_order(chosen[:n], E)
+        rows.append(RE.grouped_rows(x[:n], order, top, w, offsets, None, n)[place.long()])
+        assert torch.equal(rows[-1], rows[0][:n * top]), n
+
+
 @pytest.mark.parametrize("n,top,D,dtype", [(1, 1, 8, torch.float32), (3, 4, 136, torch.bfloat16), (16, 2, 100, torch.float32),
                                            (1100, 3, 264, torch.bfloat16)])
 def test_sum_of_the_pairs_with_a_gate_on_what_is_there(n, top, D, dtype):

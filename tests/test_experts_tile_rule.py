@@ -1,4 +1,4 @@
-"""Where the experts' products take tiles of 256 x 256 that are as high as their rows."""
+"""Which form the experts' products take, by their sizes and the chip."""
 
 
 def test_tall_tiles_by_rows_rounds_and_inner_size():
@@ -13,3 +13,10 @@ def test_tall_tiles_by_rows_rounds_and_inner_size():
     assert wins(128, 4096, 1024, 0, (100, 400)) == [False, False]
     # a gated product's tiles make half the columns
     assert wins(16, 2048, 4096, 2, (100,)) == wins(16, 4096, 4096, 0, (100,)) == [True]
+
+
+def test_two_pieces_ahead_where_every_workgroup_that_can_have_work_is_on_the_chip():
+    from gpt_fast_amd.ops.routed_experts import _pieces_ahead
+    # 32 tiles of 16 rows: 24 experts on 256 units, whether the experts or the pairs are fewer
+    assert [_pieces_ahead(E, P, 512, 256) for E, P in ((24, 99), (25, 99), (64, 24), (64, 25))] == [2, 1, 2, 1]
+    assert [_pieces_ahead(1, 1, rows, 1) for rows in (1, 48, 49)] == [2, 2, 1]
