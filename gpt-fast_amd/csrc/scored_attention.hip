@@ -874,31 +874,45 @@ __global__ __launch_bounds__(SA_THREADS) void whole_norm_store_kernel(
     }
 }
 
-// The same for rows of up to 4,096 VPT elements in whole groups of four (heads of a multiple of 8): the row is read
-// once, in 16-byte loads, and both sums come out of one exchange.  A chain of latencies: with 256 threads, an element
-// at a time, 16 rows of 6,832 took 15.5 us and 1,777 rows 32.
-#define WN_THREADS 1024
-template <typename T, int VPT>
-__global__ __launch_bounds__(WN_THREADS) void whole_norm_store_vec_kernel(
+// The same for rows of up to 4 C NT elements in whole groups of four (heads of a multiple of 8): the row is read
+// once, in 16-byte loads, both sums come out of one exchange, and queries and keys are stored four at a time.  A few
+// rows are a chain of latencies, many are bound by their accesses.  us, the kernel above, this one with each
+// element stored by itself, and as it is (bfloat16, values the keys): rows of 5,120, 16 of them 9.8, 5.6, 4.5; 1,777 26.3,
+// 30.9, 22.4; 4,096 63, 75, 51; rows of 1,536, 16 5.3, 4.1, 3.4; 4,096 19.0, 33.7, 15.7; of 14,336, 4,096 172, 183, 118.
+// C and NT go by the width alone, so a row's sums do not depend on how many rows there are.
+template <typename T> __device__ __forceinline__ void wn_store4(T* to, float a, float b, float c, float d);
+template <> __device__ __forceinline__ void wn_store4<float>(float* to, float a, float b, float c, float d) {
+    *(float4*)to = make_float4(a, b, c, d);
+}
+template <> __device__ __forceinline__ void wn_store4<bf16_t>(bf16_t* to, float a, float b, float c, float d) {
+    *(uint2*)to = make_uint2((uint32_t)float_to_bf16(a) | (uint32_t)float_to_bf16(b) << 16,
+                             (uint32_t)float_to_bf16(c) | (uint32_t)float_to_bf16(d) << 16);
+}
+template <typename T, int NT, int C>
+__global__ __launch_bounds__(NT) void whole_norm_store_vec_kernel(
         const float* __restrict__ proj, int row_width, const float* __restrict__ bias,
         const float* __restrict__ wq, const float* __restrict__ wk, T* __restrict__ q_out,
         T* __restrict__ k_pages, T* __restrict__ v_pages, const int* __restrict__ tok_seq,
         const int* __restrict__ tok_pos, const int* __restrict__ table, int table_stride, int H,
         int G, int d, int dv, float eps, float temp_coef, int temp_every, int values_are_keys) {
-    __shared__ float sums[2][WN_THREADS / GFA_WAVE];
+    __shared__ float sums[2][NT / GFA_WAVE];
     const int n = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int nq = H * d, nk = G * d, width = nq + nk + (values_are_keys ? 0 : G * dv);
     const float* row = proj + (size_t)n * row_width;
     const int pos = tok_pos[n];
-    float x[VPT][4];
+    float x[C][4];
     float sq = 0.f, sk = 0.f;
 #pragma unroll
-    for (int j = 0; j < VPT; ++j) {
-        const int e = (threadIdx.x + j * WN_THREADS) * 4;
+    for (int j = 0; j < C; ++j) {
+        const int e = (threadIdx.x + j * NT) * 4;
         const bool there = e < width;
         const float4 v = *(const float4*)(row + (there ? e : 0));
         const float4 b = bias ? *(const float4*)(bias + (there ? e : 0)) : make_float4(0.f, 0.f, 0.f, 0.f);
         x[j][0] = v.x + b.x; x[j][1] = v.y + b.y; x[j][2] = v.z + b.z; x[j][3] = v.w + b.w;
+    }
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+        const int e = (threadIdx.x + j * NT) * 4;
         const float ss = fmaf(x[j][0], x[j][0], fmaf(x[j][1], x[j][1], fmaf(x[j][2], x[j][2], x[j][3] * x[j][3])));
         if (e < nq) sq += ss;
         else if (e < nq + nk) sk += ss;
@@ -914,7 +928,7 @@ __global__ __launch_bounds__(WN_THREADS) void whole_norm_store_vec_kernel(
         __syncthreads();
         sq = sk = 0.f;
 #pragma unroll
-        for (int w = 0; w < WN_THREADS / GFA_WAVE; ++w) {
+        for (int w = 0; w < NT / GFA_WAVE; ++w) {
             sq += sums[0][w];
             sk += sums[1][w];
         }
@@ -926,22 +940,23 @@ __global__ __launch_bounds__(WN_THREADS) void whole_norm_store_vec_kernel(
     if (k_pages) page = table[(size_t)tok_seq[n] * table_stride + pos / GFA_PAGE];
     const int slot = pos % GFA_PAGE;
 #pragma unroll
-    for (int j = 0; j < VPT; ++j) {
-        const int e = (threadIdx.x + j * WN_THREADS) * 4;
+    for (int j = 0; j < C; ++j) {
+        const int e = (threadIdx.x + j * NT) * 4;
         if (e >= width) break;
         if (e < nq) {
-            T* to = q_out + (size_t)n * nq + e;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) store_from_float(to + q, x[j][q] * rq * (eps >= 0.f ? wq[e + q] : 1.f));
+            const float4 w = eps >= 0.f ? *(const float4*)(wq + e) : make_float4(1.f, 1.f, 1.f, 1.f);
+            wn_store4(q_out + (size_t)n * nq + e, x[j][0] * rq * w.x, x[j][1] * rq * w.y, x[j][2] * rq * w.z,
+                      x[j][3] * rq * w.w);
         } else if (!k_pages) {
             break;
         } else if (e < nq + nk) {
             const int at = e - nq, g = at / d, i = at - g * d;
-            T* to = k_pages + key_elem(page, g, slot, i, G, d);   // four elements of a chunk of eight
+            const float4 w = eps >= 0.f ? *(const float4*)(wk + at) : make_float4(1.f, 1.f, 1.f, 1.f);
+            wn_store4(k_pages + key_elem(page, g, slot, i, G, d),    // four elements of a chunk of eight
+                      x[j][0] * rk * w.x, x[j][1] * rk * w.y, x[j][2] * rk * w.z, x[j][3] * rk * w.w);
+            if (values_are_keys) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                store_from_float(to + q, x[j][q] * rk * (eps >= 0.f ? wk[at + q] : 1.f));
-                if (values_are_keys) store_from_float(v_pages + value_elem(page, g, i + q, slot, G, dv), x[j][q]);
+                for (int q = 0; q < 4; ++q) store_from_float(v_pages + value_elem(page, g, i + q, slot, G, dv), x[j][q]);
             }
         } else {
             const int at = e - nq - nk, g = at / dv, i = at - g * dv;
@@ -961,15 +976,18 @@ extern "C" int gfa_whole_norm_store(const float* proj, int row_width, const floa
     if ((values_are_keys && dv != d) || (eps >= 0.f && (!wq || !wk)) || temp_every < 0)
         return (int)hipErrorInvalidValue;
     const int width = (H + G) * d + (values_are_keys ? 0 : G * dv);
-    if (d % 8 == 0 && dv % 4 == 0 && row_width % 4 == 0 && width <= 4 * 4 * WN_THREADS && (uintptr_t)proj % 16 == 0 &&
-        (uintptr_t)bias % 16 == 0) {
-#define WN_GO(T, VPT) whole_norm_store_vec_kernel<T, VPT><<<n_tokens, WN_THREADS, 0, stream>>>( \
+    const auto by16 = [](const void* p) { return (uintptr_t)p % 16 == 0; };
+    if (d % 8 == 0 && dv % 4 == 0 && row_width % 4 == 0 && width <= 4 * 8 * 512 && by16(proj) && by16(bias) && by16(wq) &&
+        by16(wk) && by16(q_out) && by16(k_pages)) {
+#define WN_GO(T, NT, C) whole_norm_store_vec_kernel<T, NT, C><<<n_tokens, NT, 0, stream>>>( \
             proj, row_width, bias, wq, wk, (T*)q_out, (T*)k_pages, (T*)v_pages, tok_seq, tok_pos, table, table_stride, \
             H, G, d, dv, eps, temp_coef, temp_every, values_are_keys)
 #define WN_BY_WIDTH(T) do { \
-            if (width <= 4 * WN_THREADS) WN_GO(T, 1); \
-            else if (width <= 8 * WN_THREADS) WN_GO(T, 2); \
-            else WN_GO(T, 4); \
+            if (width <= 1024) WN_GO(T, 256, 1); \
+            else if (width <= 2048) WN_GO(T, 512, 1); \
+            else if (width <= 4096) WN_GO(T, 512, 2); \
+            else if (width <= 8192) WN_GO(T, 512, 4); \
+            else WN_GO(T, 512, 8); \
         } while (0)
         if (is_bf16) WN_BY_WIDTH(bf16_t);
         else WN_BY_WIDTH(float);

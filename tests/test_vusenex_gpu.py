@@ -231,6 +231,47 @@ def test_the_norm_over_the_whole_projection_the_temperature_and_the_cache(dtype,
     assert torch.equal(q, q2)
 
 
+# widths on either side of 1,024, 2,048, 4,096, 8,192 and 16,384, where the rows are split in another way; values of their
+# own, also of another width; row strides of whole groups of four (the last: not) and what is not added or normed
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("H,G,d,dv,own,more", [
+    (4, 2, 8, 8, False, 0), (12, 4, 64, 64, False, 4), (13, 4, 64, 64, False, 0), (8, 4, 72, 20, True, 0),
+    (24, 8, 64, 64, False, 8), (25, 8, 64, 64, False, 0), (24, 4, 128, 128, True, 0), (25, 8, 128, 128, False, 4),
+    (48, 16, 128, 128, False, 0), (40, 8, 144, 100, True, 4), (57, 8, 128, 128, False, 0), (96, 16, 128, 128, True, 0),
+    (97, 16, 128, 128, True, 4), (13, 4, 64, 64, True, 2)])
+def test_the_norm_over_the_whole_projection_at_every_split_of_its_rows(dtype, tol, H, G, d, dv, own, more):
+    from gpt_fast_amd.ops import scored_attention as SA
+    torch.manual_seed(H + d)
+    lens, starts = [66, 1, 3], [0, 130, 62]
+    n_pages, tables, table, tok_seq, tok_pos, pos = _table_and_positions(lens, starts)
+    nq, nk, width = H * d, G * d, (H + G) * d + (G * dv if own else 0)
+    proj = torch.randn(sum(lens), width + more, device=DEV) * 2
+    qw, kw = 1 + 0.3 * torch.randn(nq, device=DEV), 1 + 0.3 * torch.randn(nk, device=DEV)
+    seqs = [b for b, l in enumerate(lens) for _ in range(l)]
+    for bias, eps in ((torch.randn(width, device=DEV), 1e-4), (None, 1e-4), (torch.randn(width, device=DEV), None)):
+        k_pages = torch.zeros(n_pages, G, 64, d, device=DEV, dtype=dtype)
+        v_pages = torch.zeros(n_pages, G, dv, 64, device=DEV, dtype=dtype)
+
+        def run(rows, pages):
+            return SA.whole_norm_store(proj[:rows], bias, qw if eps else None, kw if eps else None, tok_seq, tok_pos, table,
+                                       *(pages or (None, None)), H, G, d, dv, eps, 0.5, 16, not own, dtype)
+        q = run(sum(lens), (k_pages, v_pages))
+        x = proj[:, :width].double().cpu() + (0 if bias is None else bias.double().cpu())
+        want_q, want_k = x[:, :nq], x[:, nq:nq + nk]
+        want_v = (x[:, nq + nk:] if own else want_k).reshape(-1, G, dv)
+        if eps:
+            want_q, want_k = P.unit_rms(want_q, eps) * qw.double().cpu(), P.unit_rms(want_k, eps) * kw.double().cpu()
+        want_q = want_q * torch.tensor([1 + 0.5 * math.log((p + 1) // 16 + 1) for p in pos], dtype=torch.float64)[:, None]
+        want_k = want_k.reshape(-1, G, d)
+        assert rel_err(q.view(-1, nq), want_q) < tol
+        k, v = _cache_rows(k_pages, v_pages, d, dv)
+        at = torch.tensor([tables[b][p // 64] for b, p in zip(seqs, pos)]), torch.tensor(pos) % 64
+        assert rel_err(k[at[0], :, at[1]], want_k) < tol
+        assert rel_err(v[at[0], :, :, at[1]], want_v) < tol
+        # nothing stored, and fewer rows: the same queries
+        assert torch.equal(run(sum(lens), None), q) and torch.equal(run(5, None), q[:5])
+
+
 def _plain_sink_attention(q, k, v, start, scale, r1, r2, sink):
     """q [T, H, d] are the last T of the sequence's tokens; k [L, G, d], v [L, G, dv]."""
     T, H, _ = q.shape
