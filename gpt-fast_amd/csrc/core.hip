@@ -1224,7 +1224,8 @@ extern "C" int gfa_silu_mul(const void* gu, void* out, int n_rows, int I, int is
 // What bounds a layer of few rows is its chain of kernels, 5 to 10 us each whatever they do: a norm 5, the rotation
 // 5.5, the gate 5 beside products of 7 to 10 (four rows, 768 columns).  Every workgroup reads all of x
 // anyway, so each works the rows' factors out for itself, while its first weights are on the way: five kernels a
-// layer and not nine, four requests of 20 to 200 tokens and then 12 steps on 12 layers of 768 columns 12.5 -> 11.0 ms.
+// layer and not nine, four requests of 20 to 200 tokens and then 12 steps on 12 layers of 768 columns 12.5 -> 11.0 ms
+// (few_row_f32_fused: up to where).
 //
 // The same bits as rmsnorm_vec_kernel, gemm_f32_kernel and the kernels behind them: the squares are added by as
 // many lanes and in the order of that norm kernel's (256 or 1,024 threads by the width), the products as four chains of
@@ -1372,23 +1373,52 @@ __global__ __launch_bounds__(256, 2) void normed_gemm_f32_kernel(
     }
 }
 
-static size_t few_row_up(size_t n) { return (n + 255) / 256 * 256; }
-
-extern "C" long gfa_few_row_work_bytes_f32(int M, int I, int H, int hd) {
-    return (long)(2 * few_row_up((size_t)M * H * hd * 4) + few_row_up((size_t)M * I * 4));
+// Whether the products work the norms out themselves.  Every workgroup then goes through all rows again, 256 float4 at
+// a time up to 1,024 columns and 1,024 beyond; with more rows or wider ones the separate kernels are the faster way.
+// us a layer, fused and separate (30 keys): 288 columns, 12 rows 36.4, 38.9; 16 40.4, 40.4; 512, 10 42.4, 42.9; 12 45.2,
+// 43.9; 768, 4 39.5, 45.5; 10 47.3, 48.3; 12 50.4, 49.8; 1,024, 10 58.3, 60.4; 12 62.1, 62.2; 1,536, 3 80.3, 81.5; 5 86.7,
+// 84.3; 2,048, 1 79, 84; 3 87.4, 87.3; 4 91, 89; 16 141, 110; 3,072, 2 139, 141; 4 150, 147; 4,096, 1 215, 220; 2 222,
+// 219; 16 363, 306.
+static bool few_row_f32_fused(int M, int D) {
+    return D <= 1024 ? M <= 10 || M * D <= 4608 : D <= 4096 && M * D <= 6144;
 }
 
-// The layers' launches, five a layer.
+struct FewRowWorkF32 {
+    size_t q, y, h, xn, qkv, gu, bytes;
+    bool fused;
+    FewRowWorkF32(int M, int D, int I, int H, int Hkv, int hd) {
+        fused = few_row_f32_fused(M, D);
+        size_t at = 0;
+        auto take = [&](size_t n) { const size_t o = at; at += (n * 4 + 255) / 256 * 256; return o; };
+        q = take((size_t)M * H * hd);
+        y = take((size_t)M * H * hd);
+        h = take((size_t)M * I);
+        xn = take(fused ? 0 : (size_t)M * D);
+        qkv = take(fused ? 0 : (size_t)M * (H + 2 * Hkv) * hd);
+        gu = take(fused ? 0 : (size_t)M * 2 * I);
+        bytes = at;
+    }
+};
+
+extern "C" long gfa_few_row_work_bytes_f32(int M, int D, int I, int H, int Hkv, int hd) {
+    return (long)FewRowWorkF32(M, D, I, H, Hkv, hd).bytes;
+}
+
+// The layers' launches: five a layer, nine where norms, rotation and gate are kernels of their own.
 extern "C" int gfa_few_row_layers_f32(const FewRowLayer* layers, int n_layers, const FewRowStep* step, hipStream_t stream) {
     const FewRowStep& s = *step;
     const int inner = s.H * s.hd;
-    if (n_layers <= 0 || s.M <= 0 || s.M > 16 || s.D <= 0 || s.D % 4 || s.D > 4096 || s.I <= 0 || s.I % 4 || s.hd <= 0 ||
-        s.hd % 16 || s.hd > 256 || s.rot % 2 || s.rot > s.hd || (s.gate_mode != 0 && s.gate_mode != 1) ||
+    if (n_layers <= 0 || s.M <= 0 || s.M > 16 || s.D <= 0 || s.D % 4 || s.D > 4096 || s.I <= 0 || s.I % 4 ||
+        s.hd <= 0 || s.hd % 16 || s.hd > 256 || s.rot % 2 || s.rot > s.hd || (s.gate_mode != 0 && s.gate_mode != 1) ||
         (uintptr_t)s.residual % 16 || (uintptr_t)s.work % 16)
         return (int)hipErrorInvalidValue;
-    float* q = (float*)s.work;
-    float* y = (float*)((char*)q + few_row_up((size_t)s.M * inner * 4));
-    float* h = (float*)((char*)y + few_row_up((size_t)s.M * inner * 4));
+    const FewRowWorkF32 at(s.M, s.D, s.I, s.H, s.Hkv, s.hd);
+    float* q = (float*)((char*)s.work + at.q);
+    float* y = (float*)((char*)s.work + at.y);
+    float* h = (float*)((char*)s.work + at.h);
+    float* xn = (float*)((char*)s.work + at.xn);
+    float* qkv = (float*)((char*)s.work + at.qkv);
+    float* gu = (float*)((char*)s.work + at.gu);
     const int n_qkv = (s.H + 2 * s.Hkv) * s.hd;
     int rc = 0;
     for (int l = 0; l < n_layers && rc == 0; ++l) {
@@ -1396,29 +1426,48 @@ extern "C" int gfa_few_row_layers_f32(const FewRowLayer* layers, int n_layers, c
         if ((uintptr_t)L.wqkv % 16 || (uintptr_t)L.w13 % 16 || (uintptr_t)L.norm_mixer % 16 || (uintptr_t)L.norm_ffn % 16)
             return (int)hipErrorInvalidValue;
         NormedEpilogue e = {};
-        e.q = q;
-        e.k_pages = (float*)L.k_pages;
-        e.v_pages = (float*)L.v_pages;
-        e.freqs = s.freqs;
-        e.tok_seq = s.tok_seq;
-        e.tok_pos = s.tok_pos;
-        e.table = L.table;
-        e.table_stride = s.table_stride;
-        e.H = s.H; e.Hkv = s.Hkv; e.hd = s.hd; e.rot = s.rot;
-        normed_gemm_f32_kernel<2><<<n_qkv / 16, 256, 0, stream>>>(s.residual, L.norm_mixer, (const float*)L.wqkv, s.M, n_qkv,
-                                                                  s.D, s.eps_mixer, e);
+        if (at.fused) {
+            e.q = q;
+            e.k_pages = (float*)L.k_pages;
+            e.v_pages = (float*)L.v_pages;
+            e.freqs = s.freqs;
+            e.tok_seq = s.tok_seq;
+            e.tok_pos = s.tok_pos;
+            e.table = L.table;
+            e.table_stride = s.table_stride;
+            e.H = s.H; e.Hkv = s.Hkv; e.hd = s.hd; e.rot = s.rot;
+            normed_gemm_f32_kernel<2><<<n_qkv / 16, 256, 0, stream>>>(s.residual, L.norm_mixer, (const float*)L.wqkv, s.M,
+                                                                      n_qkv, s.D, s.eps_mixer, e);
+        } else {
+            rc = gfa_rmsnorm(s.residual, L.norm_mixer, nullptr, xn, 0, s.M, s.D, s.eps_mixer, stream);
+            if (rc) break;
+            rc = gfa_gemm_f32(xn, (const float*)L.wqkv, qkv, s.M, n_qkv, s.D, s.D, n_qkv, 0, stream);
+            if (rc) break;
+            rc = gfa_rope_cache_write(qkv, q, L.k_pages, L.v_pages, s.freqs, s.tok_seq, s.tok_pos, L.table, s.table_stride,
+                                      s.n_seqs, s.M, s.H, s.Hkv, s.hd, s.rot, 0, 0, stream);
+            if (rc) break;
+        }
         rc = gfa_attention_generic(q, L.k_pages, L.v_pages, s.tok_seq, s.tok_pos, L.table, s.table_stride, y, s.M, s.H,
                                    s.Hkv, s.hd, s.scale, s.window, 0, stream);
         if (rc) break;
         rc = gfa_gemm_f32(y, (const float*)L.wo, s.residual, s.M, s.D, inner, inner, s.D, 1, stream);
         if (rc) break;
-        e.out = h;
-        if (s.gate_mode == 0)
-            normed_gemm_f32_kernel<0><<<(s.I + 7) / 8, 256, 0, stream>>>(s.residual, L.norm_ffn, (const float*)L.w13, s.M,
-                                                                           s.I, s.D, s.eps_ffn, e);
-        else
-            normed_gemm_f32_kernel<1><<<(s.I + 7) / 8, 256, 0, stream>>>(s.residual, L.norm_ffn, (const float*)L.w13, s.M,
-                                                                           s.I, s.D, s.eps_ffn, e);
+        if (at.fused) {
+            e.out = h;
+            if (s.gate_mode == 0)
+                normed_gemm_f32_kernel<0><<<(s.I + 7) / 8, 256, 0, stream>>>(s.residual, L.norm_ffn, (const float*)L.w13,
+                                                                              s.M, s.I, s.D, s.eps_ffn, e);
+            else
+                normed_gemm_f32_kernel<1><<<(s.I + 7) / 8, 256, 0, stream>>>(s.residual, L.norm_ffn, (const float*)L.w13,
+                                                                              s.M, s.I, s.D, s.eps_ffn, e);
+        } else {
+            rc = gfa_rmsnorm(s.residual, L.norm_ffn, nullptr, xn, 0, s.M, s.D, s.eps_ffn, stream);
+            if (rc) break;
+            rc = gfa_gemm_f32(xn, (const float*)L.w13, gu, s.M, 2 * s.I, s.D, s.D, 2 * s.I, 0, stream);
+            if (rc) break;
+            rc = gfa_gate_mul(gu, h, s.M, s.I, s.gate_mode, 0.f, 0, stream);
+            if (rc) break;
+        }
         rc = gfa_gemm_f32(h, (const float*)L.w2, s.residual, s.M, s.D, s.I, s.I, s.D, 1, stream);
     }
     return rc;

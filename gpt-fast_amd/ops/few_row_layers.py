@@ -26,7 +26,7 @@ class _Step(ctypes.Structure):
 def takes(n_rows: int, dim: int, hidden: int, n_heads: int, n_kv_heads: int, head_dim: int, rotary_dim: int,
           dtype=torch.bfloat16) -> bool:
     """Whether the step's products and attention are the kernels that the entry of this type launches.  The float32 one
-    works the norms out inside the products: rows that the norm's own kernel keeps one float4 a thread of."""
+    may work the norms out inside the products: rows that the norm's own kernel keeps one float4 a thread of."""
     if dtype == torch.float32 and dim > 4096:
         return False
     return (0 < n_rows <= MAX_ROWS and dim % 8 == 0 and hidden % 8 == 0 and head_dim % 16 == 0 and head_dim <= 256
@@ -108,7 +108,7 @@ def run_layers(layers, x, residual, freqs, rotary_dim: int, batch, n_heads: int,
     if x is None:
         lib = library("core")
         lib.gfa_few_row_work_bytes_f32.restype = ctypes.c_long
-        size = lib.gfa_few_row_work_bytes_f32(_i(M), _i(inner), _i(H), _i(hd))
+        size = lib.gfa_few_row_work_bytes_f32(_i(M), _i(D), _i(inner), _i(H), _i(G), _i(hd))
         step.gate_mode = GATE_ACTIVATIONS[activation]
         launch = lib.gfa_few_row_layers_f32
     else:
