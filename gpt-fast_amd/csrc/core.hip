@@ -974,16 +974,17 @@ __global__ __launch_bounds__(AG_THREADS) void attention_generic_kernel(
 // kernel above walks all keys' values one after the other: four requests of the 110M shape, 20 to 200 tokens
 // and then 12 steps, 21.4 -> 12.7 ms with it.
 // A row's result depends on its position and window alone.  HD: head size rounded up to 64.
-// Head sizes up to 64 (EARLY): a wave's next page is asked for, keys and values at once, before anything waits - the
+// EARLY (head sizes up to 64): a wave's next page is asked for, keys and values at once, before anything waits - the
 // first one beside the query, not behind it: 11.01 -> 10.61 ms for the same requests (with the products of
-// normed_gemm_f32_kernel); larger heads do not hold a page in registers.
-template <int HD>
+// normed_gemm_f32_kernel); larger heads do not hold a page in registers.  It pays where reads come from memory and few
+// waves hide them, and costs the reads of waves that have no page: attention_f32_early.
+template <int HD, bool EARLY>
 __global__ __launch_bounds__(256) void attention_f32_kernel(
         const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
         const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, const int* __restrict__ table,
         int table_stride, float* __restrict__ out, int H, int Hkv, int hd, float scale, int window) {
     constexpr int PER = HD / 64;
-    constexpr bool EARLY = HD == 64;
+    static_assert(!EARLY || HD == 64, "a page of larger heads does not fit the registers");
     __shared__ __attribute__((aligned(16))) float qs[HD];
     __shared__ __attribute__((aligned(16))) float ps[4][GFA_PAGE];
     __shared__ float merged[4][HD + 2];
@@ -1104,6 +1105,19 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
     }
 }
 
+// Whether a step asks early; pages: the most that its table has for a sequence.  Not where there are many workgroups (one
+// a token and head) and they walk many pages, or share the keys of a group, which then are in the caches.  us, early and
+// not, heads of 64, prompts' keys out of the caches and single tokens' out of memory: 12 heads, a token behind 30
+// keys 5.6, 6.7; 16 behind 1,000 25.7, 26.2; prompts of 8 x 200 123, 132; 600 3.12 ms of a model's step either way; 900 124,
+// 119; 2,048 484, 459, with a window of 256 231, 257; 300 behind 2,000 151, 142.  32 heads on 4: a token behind
+// 1,000 15.6, 17.2; prompts of 100 23.7, 20.4; 4 x 150 116, 109; 2,048 1,267, 1,192, with a window 596, 635.
+// Heads of 48, whose loads are not whole lines: 900 64, 75; 2,048 237, 241.
+static bool attention_f32_early(int n_tokens, int H, int Hkv, int hd, int pages, int window) {
+    if (window > 0 && window / GFA_PAGE + 2 < pages) pages = window / GFA_PAGE + 2;
+    if ((long long)n_tokens * H < 2048 || hd == 48) return hd <= 64;
+    return hd <= 64 && pages < 10 && (window > 0 || H < 4 * Hkv);
+}
+
 extern "C" int gfa_attention_generic(const void* q, const void* k_pages, const void* v_pages,
                                      const int* tok_seq, const int* tok_pos, const int* table,
                                      int table_stride, void* out, int n_tokens, int H, int Hkv,
@@ -1114,11 +1128,12 @@ extern "C" int gfa_attention_generic(const void* q, const void* k_pages, const v
     dim3 grid(n_tokens, H);
     // 16-byte loads of the cache's operand order need it to begin at such an address
     if (!is_bf16 && hd % 16 == 0 && hd <= 256 && (uintptr_t)k_pages % 16 == 0 && (uintptr_t)v_pages % 16 == 0) {
-#define AF_GO(HD) attention_f32_kernel<HD><<<grid, 256, 0, stream>>>((const float*)q, (const float*)k_pages, \
+#define AF_GO(HD, EARLY) attention_f32_kernel<HD, EARLY><<<grid, 256, 0, stream>>>((const float*)q, (const float*)k_pages, \
         (const float*)v_pages, tok_seq, tok_pos, table, table_stride, (float*)out, H, Hkv, hd, scale, window)
-        if (hd <= 64) AF_GO(64);
-        else if (hd <= 128) AF_GO(128);
-        else AF_GO(256);
+        if (attention_f32_early(n_tokens, H, Hkv, hd, table_stride, window)) AF_GO(64, true);
+        else if (hd <= 64) AF_GO(64, false);
+        else if (hd <= 128) AF_GO(128, false);
+        else AF_GO(256, false);
 #undef AF_GO
         return GFA_LAUNCH_RESULT();
     }

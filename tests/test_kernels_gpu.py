@@ -468,6 +468,21 @@ def _attention_ref(q, k, v, pos, scale, window):
     return out
 
 
+@pytest.mark.parametrize("H,G,hd,S,window", [(12, 12, 64, 660, 0), (12, 12, 64, 660, 100), (32, 4, 32, 130, 0), (8, 4, 48, 700, 0),
+                                              (4, 4, 16, 630, 0)])
+def test_a_float32_row_is_the_same_among_few_and_among_many(H, G, hd, S, window):
+    """A prompt of many rows does not ask for its pages early, single tokens do: the same arithmetic, the same bits."""
+    k_pages, v_pages, table, ks, vs = _paged([S], G, hd, torch.float32, S + hd)
+    q = torch.randn(S, H, hd, generator=torch.Generator().manual_seed(hd)).to(DEV)
+    seq = torch.zeros(S, dtype=torch.int32, device=DEV)
+    pos = torch.arange(S, dtype=torch.int32, device=DEV)
+    out = K().attention_generic(q, k_pages, v_pages, seq, pos, table, hd ** -0.5, window)
+    for p in (0, 63, 64, 129, S // 2, S - 1):
+        one = K().attention_generic(q[p:p + 1], k_pages, v_pages, seq[:1], pos[p:p + 1], table, hd ** -0.5, window)
+        assert torch.equal(one[0], out[p]), p
+        close(out[p], _attention_ref(q[p].cpu(), ks[0], vs[0], p, hd ** -0.5, window), 1e-5)
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 1.5e-2)])
 @pytest.mark.parametrize("H,G,hd,window", [
     (4, 4, 16, 0), (6, 2, 48, 0), (8, 1, 128, 0), (3, 3, 80, 0), (4, 2, 64, 37), (2, 1, 256, 100),
