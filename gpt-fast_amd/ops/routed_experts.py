@@ -3,6 +3,7 @@ the chosen experts.  Shape checks on the host, then the launch."""
 import ctypes
 import functools
 import math
+from statistics import NormalDist
 from typing import Optional
 
 import torch
@@ -299,83 +300,79 @@ def expert_tiles(offsets: torch.Tensor, n_experts: int, pairs: int) -> torch.Ten
     return tiles
 
 
+@functools.lru_cache(maxsize=256)
+def _shares(n: int):
+    """The shares of n experts over their mean, spread as exp(0.4 normal): its quantiles."""
+    spread = [math.exp(0.4 * NormalDist().inv_cdf((i + 0.5) / n)) for i in range(n)]
+    return [v * n / sum(spread) for v in spread]
+
+
 def _tiles(pairs: int, n_experts: int, rows: int, F: int, columns: int) -> float:
-    """Tiles of ``rows`` x ``columns`` that the experts' products have on average, their shares of the pairs spread
-    evenly from half to one and a half of the mean."""
+    """Tiles of up to ``rows`` x ``columns`` that the experts' products have if the experts' shares are :func:`_shares`
+    (of 128 at most, each then of several experts)."""
+    n = min(n_experts, 128)
     mean = pairs / n_experts
-    of_one = sum(min(1.0, 1.5 - rows * k / mean) for k in range(math.ceil(1.5 * mean / rows)))
+    of_one = sum(math.ceil(mean * share / rows) for share in _shares(n)) / n
     return of_one * min(n_experts, pairs) * ((F + columns - 1) // columns)
 
 
 @functools.lru_cache(maxsize=4096)
 def tall_tiles_win(n_experts: int, pairs: int, F: int, K: int, mode: int, units: int) -> bool:
     """Whether 256 x 256 tiles, which read each operand half as often and are only as high as their rows (steps of 64),
-    make the products of :func:`rows_tile`'s arguments fastest.  Microseconds, shares spread as exp(0.4 normal), tiles of
-    128 x 128 and these: 32 experts, 4,096 -> 3,584, x 40 rows 192, 192; x 64 202, 211; x 100 256, 222; x 140 302, 247;
-    x 222 385, 338; x 450 616, 504; 64 of them, 4,096 -> 2 x 2,048, x 64 506, 434; x 180 779, 601; 128, 2,048 ->
-    4,096, x 64 461, 467; x 140 639, 571.  Not where 128 x 128 tiles need no second round (8, 4,096 -> 3,584, x 222 94,
-    119), nor where these need one for little (16, 4,096 -> 3,584, x 222 179, 210, 1.18 rounds; x 300 250, 228, 1.44;
-    16, 2,048 -> 4,096, x 180 96, 101, 1.08; x 222 125, 109, 1.35).  Up to K = 1,024 it is either by some percent."""
-    if K <= 1024 or pairs < 64 * n_experts:
+    make the products of :func:`rows_tile`'s arguments fastest.
+
+    What decides is the rounds of the chip that either needs.  Fitted to the times: one of these tiles to a unit takes
+    1.15 times as long as two of 128 x 128 that share it, nearly whatever its height, and a last round of one small
+    tile to a unit 0.65 of one of two.  Microseconds, 128 x 128 and these (means of two draws of shares spread as
+    :func:`_shares`): 16 experts, 3,584 -> 4,096, x 120 rows 159, 123; x 140, a second round of these, 162, 172; x 222 215,
+    187; 32, 4,096 -> 3,584, x 64 201, 210; x 100 267, 227; x 222 390, 346; 8, 3,584 -> 4,096, x 180 82, 98; x 222, a
+    second round of the small ones, 132, 101; 32, 2,816 -> 2,048, x 140 137, 153.  Shares that are not the assumed ones
+    can end a round elsewhere: 16, 5,120 -> 2 x 1,536, x 120, counted as a little more than a round of small ones, needed
+    one: 130, 154.  Over 935 such points from 36 rows an expert on what the two rules choose is 0.9 % off the fastest
+    kernel on average and more than 5 % at 62.  Up to K = 1,024 :func:`rows_tile` says, but for sums of K = 1,024 from
+    400 rows an expert on: 1,024 -> 2,048, x 600 older kernel, 128 x 128, these: 16 experts 78, 65, 68; 32 144, 141,
+    119; 128 537, 543, 481."""
+    if pairs < 36 * n_experts or K < 1024 or K == 1024 and (mode != 0 or pairs < 400 * n_experts):
         return False
     gated = mode == 2
-    if _tiles(pairs, n_experts, 128, F, 64 if gated else 128) <= 2 * units:
-        return False
-    return not 1.0 < _tiles(pairs, n_experts, 256, F, 128 if gated else 256) / units < 1.3
+    small = _tiles(pairs, n_experts, 128, F, 64 if gated else 128) / (2 * units)
+    tall = _tiles(pairs, n_experts, 256, F, 128 if gated else 256) / units
+    last = small % 1.0
+    rounds = small // 1.0 + (0.0 if last == 0.0 else max(0.65, 0.3 + 0.7 * last))
+    return 1.15 * math.ceil(tall) < rounds
 
 
 @functools.lru_cache(maxsize=4096)
 def rows_tile(n_experts: int, pairs: int, F: int, K: int, mode: int, units: int) -> int:
     """Which kernel makes the experts' products of ``pairs`` rows of K into rows of F on ``units`` compute units
-    (``mode`` 0: the sums, 1: an activation of them, 2: a gated one): 1, 2 or 4 for the tile kernel
-    (csrc/prompt_tile.h) with tiles of 64 x 256, 128 x 128 or 256 x 256 rows of x and of W, 0 for the older one
+    (``mode`` 0: the sums, 1: an activation of them, 2: a gated one) where :func:`tall_tiles_win` does not say so: 1 or 2
+    for the tile kernel (csrc/prompt_tile.h) with tiles of 64 x 256 or 128 x 128 rows of x and of W, 0 for the older one
     (``expert_tile_kernel``, which needs :func:`expert_tiles`).
 
-    Asked where :func:`tall_tiles_win` does not say so; its measurements of tile 4 are of tiles that are 256 high
-    whatever their rows.
-
-    The rows of an expert are known on the device alone; on the host there is their mean.  A round of the chip is one
-    tile 4 to a unit, two of tile 1 or 2, three of the older kernel's.  Microseconds, n x m being n experts of m rows
+    The rows of an expert are known on the device alone; on the host there is their mean.  A round of the chip is
+    two of tile 1 or 2 to a unit, three of the older kernel's.  Microseconds, n x m being n experts of m rows
     on average:
 
     * From 36 rows on shares above 64 become frequent, whose matrices the 64 x 256 tile reads twice: 64 x 34,
       1,280 -> 2,048 tile 1 68, tile 2 76; 32 x 39, 3,584 -> 4,096 219, 179.  Below, where its workgroups
       are fewer than the units, tile 2 has twice as many: 8 x 10, 4,096 -> 2 x 2,048 74, 68.
-    * Where tile 2 does not need a second round it is the best: 8 x 400, 1,024 -> 2 x 512 older 23, tile 2 19, tile 4
-      38; 8 x 170, 4,096 -> 2 x 2,048 101, 90, 109, but x 222, beyond the round, 131, 143, 114.
+    * Where tile 2 does not need a second round it is the best: 8 x 400, 1,024 -> 2 x 512 older 23, tile 2 19; 8 x 170,
+      4,096 -> 2 x 2,048 101, 90.
     * Up to K = 1,024 a tile is over so soon that its first loads and its last stores show; over some rounds the older
       kernel, three to a unit, hides them best: 64 x 62, 1,024 -> 2 x 1,024 69, tile 2 77; 128 x 62, 768 -> 2,048 100,
       110; 256 x 140, 512 -> 2 x 1,024 207, 253.  Over fewer it is not worth the list (3 to 8 us): 64 x 62, 768 ->
-      2,048 64, 58; 128 x 127, 512 -> 2 x 256 37, 31.  Sums alone of K = 1,024: 128 x 222, 1,024 -> 4,096 older 473,
-      tile 4 475; x 400 724, 686.
-    * 256 x 256 tiles read each operand half as often, but a router that prefers some experts leaves many of them
-      nearly empty.  Both products of 32 experts, 4,096 -> 2 x 2,048 -> 4,096, as the routers of random weights of two
-      designs choose, older, tile 2, tile 4: x 112 451, 473, 521 and 460, 447, 524; x 128 474, 490, 528 and 507, 510,
-      546; x 162 525, 539, 536 and 572, 553, 544; x 181 552, 586, 541 and 591, 579, 551; x 256 682, 671, 670 and 758,
-      744, 677.  4,096 -> 3,584 -> 4,096, each: x 128 286, 284, 310; x 181 343, 337, 349; x 225 388, 377, 384.  With
-      even shares they win sooner (the first: x 128 616, 550, 510; x 160 685, 640, 524).  A second or third round that
-      they hardly need costs more than that: 16 x 190, 4,096 -> 4,096 tile 2 183, tile 4 222; x 222 233, 224; x 300
-      259, 228; 64 x 222, 2,048 -> 1,024 137, 155."""
+      2,048 64, 58; 128 x 127, 512 -> 2 x 256 37, 31."""
     gated = mode == 2
     if pairs < 36 * n_experts:
         columns = 128 if gated else 256
         return 1 if min(n_experts, pairs) * ((F + columns - 1) // columns) >= units else 2
     small = _tiles(pairs, n_experts, 128, F, 64 if gated else 128)
-    if small <= 2 * units:
-        return 2
-    if K <= 1024:
-        if mode == 0 and K == 1024 and pairs >= 400 * n_experts:
-            return 4
-        return 0 if small >= min(8, 4096 / K) * units else 2
-    rounds = _tiles(pairs, n_experts, 256, F, 128 if gated else 256) / units
-    if 1.0 < rounds < 3.1 and 0.0 < rounds % 1.0 < (0.35 if K <= 2048 else 0.3):
-        return 2
-    return 4 if pairs >= 160 * n_experts else 2
+    return 0 if K <= 1024 and small > 2 * units and small >= min(8, 4096 / K) * units else 2
 
 
 def _tile_of(w: torch.Tensor, mode: int, pairs: int) -> int:
-    """:func:`tall_tiles_win`, then :func:`rows_tile`, where the tile kernel takes these experts (inner sizes of whole pieces of 64, results of
-    whole 16 bytes, matrices below 4 GiB), else 0."""
+    """4, tiles of 256 x 256, where :func:`tall_tiles_win`, else what :func:`rows_tile` says, where the tile kernel takes these
+    experts (inner sizes of whole pieces of 64, results of whole 16 bytes, matrices below 4 GiB), else 0."""
     E, N, K = w.shape
     F = N // 2 if mode == 2 else N
     if K % 64 != 0 or F % 8 != 0 or not 0 < N * K * 2 < 1 << 32:

@@ -1,18 +1,30 @@
 """Which form the experts' products take, by their sizes and the chip."""
+import pytest
 
 
-def test_tall_tiles_by_rows_rounds_and_inner_size():
-    from gpt_fast_amd.ops.routed_experts import tall_tiles_win
+def _tile(E, m, K, F, mode, units=256):
+    from gpt_fast_amd.ops.routed_experts import rows_tile, tall_tiles_win
+    sizes = (E, int(m * E), F, K, mode, units)
+    return 4 if tall_tiles_win(*sizes) else rows_tile(*sizes)
 
-    def wins(E, F, K, mode, means, units=256):
-        return [tall_tiles_win(E, int(m * E), F, K, mode, units) for m in means]
-    assert wins(32, 3584, 4096, 1, (1, 63, 64, 100, 800)) == [False, False, True, True, True]
-    # a round of 128 x 128 tiles; a round of these; a little more than one; clearly more
-    assert wins(8, 3584, 4096, 1, (180, 300)) == [False, True]
-    assert wins(16, 3584, 4096, 1, (180, 222, 300)) == [True, False, True]
-    assert wins(128, 4096, 1024, 0, (100, 400)) == [False, False]
-    # a gated product's tiles make half the columns
-    assert wins(16, 2048, 4096, 2, (100,)) == wins(16, 4096, 4096, 0, (100,)) == [True]
+
+# measured, a tile of 128 x 128 against one of 256 x 256: products where the one chosen is at least 3 % faster
+@pytest.mark.parametrize("E,m,K,F,mode,tile", [
+    (16, 120, 3584, 4096, 0, 4), (16, 140, 3584, 4096, 0, 2), (16, 222, 3584, 4096, 0, 4), (32, 64, 4096, 3584, 1, 2),
+    (32, 100, 4096, 3584, 1, 4), (32, 222, 4096, 3584, 1, 4), (8, 180, 3584, 4096, 0, 2), (8, 222, 3584, 4096, 0, 4),
+    (32, 140, 2816, 2048, 1, 2), (16, 222, 4096, 3584, 1, 2), (16, 80, 2048, 7168, 0, 2), (16, 140, 4096, 2048, 2, 2),
+    (16, 80, 2048, 4096, 0, 4), (16, 222, 5120, 1536, 2, 4), (64, 180, 4096, 2048, 2, 4), (128, 140, 2048, 4096, 0, 4)])
+def test_the_tile_that_was_measured_faster(E, m, K, F, mode, tile):
+    assert _tile(E, m, K, F, mode) == tile
+
+
+def test_tiles_by_rows_and_inner_size():
+    assert [_tile(32, m, 4096, 3584, 1) for m in (0.5, 1, 35, 36)] == [2, 1, 1, 2]
+    assert [_tile(128, m, 1024, 4096, 0) for m in (100, 399, 400)] == [0, 0, 4]
+    assert [_tile(128, m, 1024, 4096, 1) for m in (100, 400)] == [0, 0]
+    # a gated product's tiles make half the columns, and a chip of half the units is full with half the columns
+    assert all(_tile(16, m, 4096, 2048, 2) == _tile(16, m, 4096, 4096, 0) == _tile(16, m, 4096, 2048, 0, 128)
+               for m in (40, 80, 100, 140, 200, 300))
 
 
 def test_two_pieces_ahead_where_every_workgroup_that_can_have_work_is_on_the_chip():
