@@ -201,7 +201,8 @@ class RoutedExperts(Part):
         """The feed-forward's output alone, float32 [N, D]."""
         s = self.spec
         z = L.linear(x, self.w_router, out_dtype=torch.float32)
-        ordered = self._grouped(x, batch) and RE.orders_with_route(x.shape[0], self.n_choices, s.n_groups)
+        ordered = self._grouped(x, batch) and \
+            RE.orders_sooner_with_route(x.shape[0], self.n_choices, s.n_groups, s.keep_groups)
         chosen, weights, *lists = RE.route(z, self.n_choices, s.top, s.n_groups, s.keep_groups, s.weight_eps,
                                            scoring=s.scoring, correction=self.correction, group_top=s.group_top,
                                            ordered=ordered)

@@ -32,3 +32,10 @@ def test_two_pieces_ahead_where_every_workgroup_that_can_have_work_is_on_the_chi
     # 32 tiles of 16 rows: 24 experts on 256 units, whether the experts or the pairs are fewer
     assert [_pieces_ahead(E, P, 512, 256) for E, P in ((24, 99), (25, 99), (64, 24), (64, 25))] == [2, 1, 2, 1]
     assert [_pieces_ahead(1, 1, rows, 1) for rows in (1, 48, 49)] == [2, 2, 1]
+
+
+def test_the_routers_launch_orders_where_its_tokens_do_not_crowd_one_compute_unit():
+    from gpt_fast_amd.ops.routed_experts import orders_sooner_with_route as sooner
+    assert [sooner(n, 32, 4, 2) for n in (1, 8, 9, 16)] == [True, True, False, False]
+    assert [sooner(n, 256, 8, 4) for n in (4, 5)] == [True, False]
+    assert [sooner(n, 32, 4, 4) for n in (9, 16, 17)] == [True, True, False]
