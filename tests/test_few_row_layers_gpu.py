@@ -13,7 +13,7 @@ SHAPES = {"16": (64, 4, 4, 16, 176, 3), "48": (200, 10, 5, 48, 328, 2), "128": (
           "1032": (1032, 4, 4, 64, 1104, 2), "4096": (4096, 4, 1, 64, 40, 2)}
 
 
-def _engine(tmp_path, shape, dtype="bfloat16"):
+def _config(shape):
     import gpt_fast_amd as gfa
     hidden, heads, kv_heads, head_dim, inner, layers = SHAPES[shape]
     config = {"architectures": ["LlamaForCausalLM"], "model_type": "llama", "hidden_size": hidden,
@@ -22,7 +22,13 @@ def _engine(tmp_path, shape, dtype="bfloat16"):
               "max_position_embeddings": 4096, "rope_theta": 10000.0, "rms_norm_eps": 1e-5,
               "rope_scaling": None, "tie_word_embeddings": False}
     arch = gfa.config.registry.architecture_of(config)
-    gfa.write_random_model(str(tmp_path), arch, arch.read_config(config), seed=5, dtype=dtype, std=0.05)
+    return arch, arch.read_config(config)
+
+
+def _engine(tmp_path, shape, dtype="bfloat16"):
+    import gpt_fast_amd as gfa
+    arch, config = _config(shape)
+    gfa.write_random_model(str(tmp_path), arch, config, seed=5, dtype=dtype, std=0.05)
     return gfa.Engine.from_folder(str(tmp_path), dtype=dtype, device="cuda:0", max_tokens=16384)
 
 
@@ -30,15 +36,38 @@ def _engine(tmp_path, shape, dtype="bfloat16"):
 @pytest.mark.parametrize("shape", SHAPES, ids=str)
 def test_one_call_launches_what_the_layers_launch(tmp_path, shape, dtype, monkeypatch):
     """float32: the norms, the rotation and the gate are worked out inside the products, to the same bits."""
+    _same_bits(_engine(tmp_path, shape, dtype), SHAPES[shape][5], monkeypatch)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("shape,window,rotary,activation", [("16", 3, 8, "gelu_tanh"), ("128", 70, 64, "silu"), ("48", None, 2, "gelu_tanh"),
+                                                            ("1032", 1, 30, "gelu_tanh"), ("4096", 100, 64, "gelu_tanh")])
+def test_with_a_window_a_part_of_the_rotation_and_the_other_gate(shape, window, rotary, activation, dtype, monkeypatch):
+    import dataclasses
+    import gpt_fast_amd as gfa
+    from gpt_fast_amd.weights.random_init import random_parameters
+    arch, config = _config(shape)
+    plan = arch.plan(config)
+
+    def changed(layer):
+        position = dataclasses.replace(layer.mixer.position, rotary_dim=rotary)
+        return dataclasses.replace(layer, mixer=dataclasses.replace(layer.mixer, window=window, position=position),
+                                   feed_forward=dataclasses.replace(layer.feed_forward, activation=activation))
+    plan = dataclasses.replace(plan, layers=[changed(layer) for layer in plan.layers])
+    params = random_parameters(arch.bindings(config), 5, dtype, "cuda:0", std=0.05, norm_std=0.1, tie=False)
+    _same_bits(gfa.Engine.from_plan(plan, params, dtype, "cuda:0", max_tokens=16384), SHAPES[shape][5], monkeypatch)
+
+
+def _same_bits(engine, n_layers, monkeypatch):
     import gpt_fast_amd as gfa
     from gpt_fast_amd.ops import few_row_layers as F
     calls, run = [], F.run_layers
     monkeypatch.setattr(F, "run_layers", lambda layers, *a, **k: (calls.append(len(layers)), run(layers, *a, **k))[1])
-    engine = _engine(tmp_path, shape, dtype)
     ends = list(engine.model.few_rows.ends)
-    assert ends == [SHAPES[shape][5]] * SHAPES[shape][5]
+    assert ends == [n_layers] * n_layers
     # held tokens, then the tokens of the step: one each (a context that is split among them), a short prompt, both
-    # together, a prompt whose attention is the tiled kernel's
+    # together, a prompt whose attention is the tiled kernel's; in float32 the products make the norms themselves for some
+    # of these and not for others
     steps = [([2100], [1]), ([31, 64, 5], [1, 1, 1]), ([3] * 16, [1] * 16), ([0], [5]), ([40, 0], [1, 9]), ([0], [16])]
     for held, new in steps:
         got = []
@@ -51,7 +80,7 @@ def test_one_call_launches_what_the_layers_launch(tmp_path, shape, dtype, monkey
             del calls[:]
             got.append(engine.step([gfa.Entry(s, util.random_tokens(320, n, 50 + i), want=list(range(n)))
                                     for i, (s, n) in enumerate(zip(slots, new))]))
-            assert calls == ([] if apart else [SHAPES[shape][5]])
+            assert calls == ([] if apart else [n_layers])
             for s in slots:
                 engine.end_sequence(s)
         assert torch.isfinite(got[0]).all()
