@@ -19,9 +19,19 @@ def _plain_layer(block) -> bool:
         return False
     f, p = block.feed_forward.spec, block.mixer.position
     norms = (RMSNorm, ScalarRMSNorm)                     # both hold a float32 weight per column
-    return (type(block.mixer_norm) in norms and type(block.feed_forward_norm) in norms
+    return (type(block.mixer_norm) in norms and type(block.feed_forward_norm) in norms and not _own_forward(block)
             and type(p) is RotaryPosition and p.spec.layout == "interleaved"
             and f.activation in F.GATE_MODES and f.limit is None)
+
+
+def _own_forward(block) -> bool:
+    """A ``forward`` put on the object itself, over its class's."""
+    return ("forward" in block.__dict__ or "forward" in block.mixer.__dict__ or "forward" in block.feed_forward.__dict__
+            or "forward" in block.mixer_norm.__dict__ or "forward" in block.feed_forward_norm.__dict__)
+
+
+def _parts(block):
+    return (block, block.mixer, block.mixer.position, block.feed_forward, block.mixer_norm, block.feed_forward_norm)
 
 
 def _alike(a, b) -> bool:
@@ -37,31 +47,48 @@ class FewRowRuns:
     run of layers costs a recorded step what the call saves an eager one."""
 
     def __init__(self, plan, blocks, runtime):
-        order = plan.order
+        self.plan, self.dtype = plan, runtime.dtype
+        self._find(blocks)
+
+    def _find(self, blocks):
+        order, is_float32 = self.plan.order, self.dtype == torch.float32
         self.blocks = [blocks[run.layer] for run in order]
         self.ends = [0] * len(order)
-        self.dtype = runtime.dtype
-        if plan.streams is not None:
+        self.parts = [None] * len(order)
+        if self.plan.streams is not None:
             return
         for n in reversed(range(len(order))):
             if not _plain_layer(self.blocks[n]) or order[n].cache_from is not None:
                 continue
+            self.parts[n] = _parts(self.blocks[n])
             behind = n + 1
             if behind == len(order) or getattr(order[behind], "enter", None) is not None \
-                    or runtime.is_float32 and not self._joins(n, behind) or not getattr(self.blocks[behind], "takes_prepared", False):
+                    or is_float32 and not self._joins(n, behind) or not getattr(self.blocks[behind], "takes_prepared", False):
                 self.ends[n] = behind
                 continue
             if self._joins(n, behind):
                 self.ends[n] = self.ends[behind]
 
+    def _as_found(self, n: int, blocks) -> bool:
+        """Whether run n's layer still has the parts that were looked at: a program may put one of its own, or a
+        ``forward`` of its own, in a part's place at any time."""
+        block = blocks[self.plan.order[n].layer]
+        was, mixer, position, feed_forward, mixer_norm, ff_norm = self.parts[n]
+        return (block is was and block.mixer is mixer and mixer.position is position and block.feed_forward is feed_forward
+                and block.mixer_norm is mixer_norm and block.feed_forward_norm is ff_norm and not _own_forward(block))
+
     def _joins(self, n: int, behind: int) -> bool:
         return bool(self.ends[behind]) and _alike(self.blocks[n], self.blocks[behind])
 
-    def take(self, n: int, stream, batch, cache) -> int:
+    def take(self, n: int, stream, batch, cache, blocks) -> int:
         """Run the plain layers from run ``n`` on over the stream, if this step's rows are few enough;
-        the number of runs taken (0: none)."""
+        the number of runs taken (0: none).  ``blocks``: the model's, by layer."""
+        if not 0 < batch.n_tokens <= F.MAX_ROWS or not self.ends[n]:
+            return 0
+        if not all(self._as_found(i, blocks) for i in range(n, self.ends[n])):
+            self._find(blocks)
         end = self.ends[n]
-        if not end or not 0 < batch.n_tokens <= F.MAX_ROWS:
+        if not end:
             return 0
         first = self.blocks[n]
         m, f = first.mixer.spec, first.feed_forward.spec

@@ -222,7 +222,7 @@ class DecoderModel:
                 stream = ResidualStream(self.enter_steps[run.enter].forward(
                     stream.tensor, embedded, batch))
             if self.tap is None:
-                taken = n + self.few_rows.take(n, stream, batch, cache)
+                taken = n + self.few_rows.take(n, stream, batch, cache, self.blocks)
                 if taken > n:
                     continue
             block = self.blocks[run.layer]

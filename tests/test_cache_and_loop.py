@@ -632,6 +632,60 @@ def test_a_registered_norm_derived_from_the_librarys_is_not_replaced_in_few_row_
             assert ends(dtype, **{name: own}) == ([1, 0] if dtype == torch.float32 else [0, 0])
 
 
+def test_a_part_put_in_a_built_models_place_is_not_passed_by_in_few_row_steps(monkeypatch):
+    """What the native call takes over is looked at again at every step: a norm, a feed-forward, a whole block or a
+    ``forward`` of its own that a program puts into a built model runs, as it does in longer steps."""
+    import types
+    from gpt_fast_amd.architectures.llama import llama_plan
+    from gpt_fast_amd.config.llama import LlamaConfig
+    from gpt_fast_amd.parts import Runtime, few_rows
+    from gpt_fast_amd.parts.feed_forward import GatedFeedForward
+    from gpt_fast_amd.parts.model import DecoderModel
+    from gpt_fast_amd.parts.norm import RMSNorm
+
+    class Doubled(RMSNorm):
+        pass
+
+    class Other(GatedFeedForward):
+        pass
+
+    taken = []
+    monkeypatch.setattr(few_rows.F, "run_layers", lambda layers, *a: taken.append(len(layers)))
+    batch = types.SimpleNamespace(n_tokens=1, table=lambda group: torch.zeros(1, 2))
+    entry = types.SimpleNamespace(writes=True, group_id=0, k_pages=None, v_pages=None)
+    cache = types.SimpleNamespace(entries=[entry, entry])
+    stream = types.SimpleNamespace(tensor=None)
+
+    def step(change):
+        rt = Runtime(torch.float32, "cpu")
+        model = DecoderModel(llama_plan(LlamaConfig.from_dict(util.TINY_A)), rt)
+        g = torch.Generator().manual_seed(0)
+        for block in model.blocks:
+            block.bind({k: torch.randn(p.shape, generator=g) for k, p in block.parameters().items()})
+        change(model, model.blocks[1], rt)
+        del taken[:]
+        return model.few_rows.take(0, stream, batch, cache, model.blocks), taken[:]
+
+    assert step(lambda model, b, rt: None) == (2, [2])
+
+    def norm(model, b, rt):
+        b.feed_forward_norm = Doubled(b.feed_forward_norm.spec, rt)
+
+    def feed_forward(model, b, rt):
+        b.feed_forward = Other(b.feed_forward.spec, rt)
+
+    def block(model, b, rt):
+        model.blocks[1] = types.SimpleNamespace()
+
+    def blocks(model, b, rt):
+        model.blocks = [model.blocks[0], types.SimpleNamespace()]
+
+    def forward(model, b, rt):
+        b.mixer.forward = lambda *a: None
+    for change in (norm, feed_forward, block, blocks, forward):
+        assert step(change) == (1, [1]), change
+
+
 def test_residual_stream_runs_what_was_put_off_before_any_read():
     """The stream holds at most one part's last kernels back; every read - the rows of a norm
     or the tensor itself - runs them first, telling them the norm that reads (only if all
