@@ -53,8 +53,8 @@ def test_gate_inside_the_grouped_product(n, E, top, F, K, activation, limit):
     want = kernels.gate_mul_sums(sums, activation, limit)
     got = RE.grouped_rows(x, order, top, w, offsets, activation, n, True, limit)
     assert got.shape == want.shape and got.dtype == torch.bfloat16
-    # the same sums but for where a tile's rows of W begin to be walked: float32 sums in another order (1e-6 of their
-    # size), which now and then round to the neighbouring bfloat16 (2^-8)
+    # the same sums at these sizes, and the gate's own arithmetic in either kernel, one rounding apart: now and then the
+    # neighbouring bfloat16 (2^-8)
     assert rel_err(got, want) <= 2.0 ** -8
 
 
