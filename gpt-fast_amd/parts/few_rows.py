@@ -1,7 +1,9 @@
-"""Runs of plain decoder layers whose few-row steps are launched by one native call."""
+"""Runs of plain decoder layers whose few-row steps are launched by one native call, or are one launch."""
 import torch
 
+from ..ops import attention_bf16 as A
 from ..ops import few_row_layers as F
+from ..ops import resident_layers as R
 from ..ops.linear import HalfNormed
 from .attention import Attention
 from .block import PreNormBlock
@@ -101,6 +103,15 @@ class FewRowRuns:
         layers = [F.Layer(b.mixer.wqkv, b.mixer.wo, b.feed_forward.w13, b.feed_forward.w2, b.mixer_norm.weight,
                           b.feed_forward_norm.weight, e.k_pages, e.v_pages, batch.table(e.group_id))
                   for b, e in zip(self.blocks[n:end], entries)]
+        p, sizes = m.position, (m.dim, f.hidden, m.n_heads, m.n_kv_heads, m.head_dim)
+        if self.dtype == torch.bfloat16 and R.takes(batch.n_tokens, *sizes, p.rotary_dim) \
+                and R.pays(end - n, batch.n_tokens, batch.n_seqs, layers[0].table.shape[1], *sizes,
+                           A.compute_units(layers[0].w2.device)) \
+                and R.aligned(layers, stream.tensor):
+            R.run(layers, stream.tensor, first.mixer.position.freqs, p.rotary_dim, batch, m.n_heads, m.n_kv_heads, m.head_dim,
+                  first.mixer.window, first.mixer_norm.spec.eps, first.feed_forward_norm.spec.eps, first.mixer.scale,
+                  f.activation)
+            return end - n
         x = None                                         # in float32 the first product makes its norm itself
         if self.dtype == torch.bfloat16:
             x = stream.normed(first.mixer_norm, reader=first.mixer)
