@@ -273,7 +273,7 @@ struct SkinnyExtra {
 // Rows per record of the sums-of-squares shares for M rows of x.
 extern "C" int gfa_share_rows(int M) { return M <= 4 ? 4 : M <= 8 ? 8 : M <= 16 ? 16 : M <= 32 ? 32 : 64; }
 
-// TILES = 2 (nine to 48 rows of x, wide matrices, not the gate): a workgroup takes two
+// TILES = 2 (tiles_per_workgroup, not the gate): a workgroup takes two
 // tiles of W's rows, one below the other, against the same fragments of x.  With sixteen
 // rows every workgroup reads as many bytes of x as of W; two tiles halve that, at half as
 // many workgroups, which pays where those still fill the chip.
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(512) void skinny_mfma_kernel(
     constexpr int NT = (IS_GATE(MODE)) ? 1 : TILES;          // tiles of output columns per workgroup
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, NW = blockDim.x >> 6;
-    // th (12..16) rows of W per tile: the host picks it so that the tiles divide evenly
+    // th (8..16) rows of W per tile: the host picks it so that the tiles divide evenly
     // over the compute units; operand rows th..15 repeat row th - 1 and are never stored
     const int n0 = blockIdx.x * th * NT;
     char* stage = smem + (size_t)wave * (RT * SM_TILE);
@@ -688,21 +688,23 @@ static int compute_units() {
     return cus;
 }
 
-// Rows of W per workgroup (12..16, in steps of `step`) for a product with N output columns:
-// the height at which the compute unit with the most tiles streams the fewest rows - with
-// 16 rows, 6144 columns are 384 tiles on 256 compute units, half of which stream twice as
-// much as the others; with 12 rows they are 512, two each.  The taller tile on a tie.  Not
+// Rows of W per tile (in steps of `step`) for a product with N output columns: the height at which the compute unit
+// with the most tiles streams the fewest rows - with 16 rows, 6144 columns are 384 tiles on 256 compute units, half of
+// which stream twice as much as the others; with 12 rows they are 512, two each.  The taller tile on a tie.  Not
 // below 12: every tile reads all of x, so lower tiles cost in x what they save in W (10240
-// columns at 8 rows, 1280 tiles for 640, measured 54 against 41 us at 16 rows of x).
-static int pick_tile_rows(int N, int step, int nt = 1) {
+// columns at 8 rows, 1280 tiles for 640, measured 54 against 41 us at 16 rows of x).  Pairs of tiles (nt 2) read x
+// once for both, `x_rows` of it, which is then counted: down to 8.
+static int pick_tile_rows(int N, int step, int nt, int x_rows) {
     const int cus = compute_units();
-    const long tiles16 = (N + 16 * nt - 1) / (16 * nt);
-    const long cost16 = ((tiles16 + cus - 1) / cus) * 16;
+    auto cost_of = [&](int th) {
+        const long tiles = (N + th * nt - 1) / (th * nt);
+        return ((tiles + cus - 1) / cus) * (nt == 2 ? 2 * th + x_rows : th);
+    };
+    const long cost16 = cost_of(16);
     int best = 16;
     long best_cost = cost16;
-    for (int th = 16 - step; th >= 12; th -= step) {
-        const long tiles = (N + th * nt - 1) / (th * nt);
-        const long cost = ((tiles + cus - 1) / cus) * th;
+    for (int th = 16 - step; th >= (nt == 2 ? 8 : 12); th -= step) {
+        const long cost = cost_of(th);
         if (cost < best_cost) {
             best = th;
             best_cost = cost;
@@ -719,15 +721,24 @@ static int pick_tile_rows(int N, int step, int nt = 1) {
 // of W, 128 workgroups, a loss of a fifth).  Not the gate, which multiplies two sets of rows
 // against the same x already: with two tiles of each, 242 registers, the step at sixteen rows
 // lost 5 % (8B and 70B shapes) although the kernel alone gained 3 %.
+//
+// Up to 16 rows of x also where single tiles of 16 would go on the chip a second time and pairs of lower ones do not.  Single
+// and pairs, us: 4608 x 4096 4 rows of x 10.8, 9.5; 8 10.9, 9.6; 16 14.4, 11.2; 5120 x 4096 11.1, 9.9; 11.0, 10.1; 14.4,
+// 11.7; 5632 x 4096 11.0, 11.2; 11.2, 10.7; 14.6, 12.2; 6176 x 4096 11.5, 11.7; 11.7, 11.2; 14.7, 12.7; 5120 x 7168 16.9,
+// 14.4; 17.3, 15.1; 22.5, 17.5.  Twice: 9216 x 4096, 16 rows 20.0, 18.1; 8 rows 15.5, 15.3.  With 4096 columns, one round
+// either way, 7.9, 9.1; 8.2, 9.2; 9.5, 10.7.
 static int tiles_per_workgroup(int mode, int M, int N) {
+    const int cus = compute_units();
+    if (IS_GATE(mode)) return 1;
+    if (M <= 16) return N > 16 * cus && (M > 8 || N < (M > 4 ? 24 : 22) * cus) ? 2 : 1;
     // 33..48 rows: only where the registers hold it (the plain epilogues)
     const int most = (mode == 2 || mode == 4) ? 32 : 48;
-    return (!IS_GATE(mode) && M > 8 && M <= most && N >= 24 * compute_units()) ? 2 : 1;
+    return M <= most && N >= 24 * cus ? 2 : 1;
 }
 
 // Tile height the launcher below uses for this mode, these rows of x and this width.
 static int tile_rows(int mode, int M, int N) {
-    return pick_tile_rows(N, (mode == 2 || mode == 4) ? 4 : 1, tiles_per_workgroup(mode, M, N));
+    return pick_tile_rows(N, (mode == 2 || mode == 4) ? 4 : 1, tiles_per_workgroup(mode, M, N), M > 8 ? 16 : M > 4 ? 8 : 4);
 }
 
 // Workgroups the launcher below starts for this mode, M <= 16 rows of x and N columns (the
@@ -743,7 +754,7 @@ static int launch_skinny_mfma(const bf16_t* x, const bf16_t* w, void* out, int M
                               int ldo, int gate_rows, const SkinnyExtra& ex, hipStream_t stream) {
     const int ct = (M + 15) / 16;
     // the epilogues that add into the residual stream or rotate pairs work on groups of
-    // four columns: their tiles are 12 or 16 rows high
+    // four columns: their tiles are 8, 12 or 16 rows high
     const int nt = tiles_per_workgroup(MODE, M, N);
     const int th = ct == 1 ? tile_rows(MODE, M, N) : 16;
     const int tiles = (N + th * nt - 1) / (th * nt);     // workgroups
@@ -786,7 +797,9 @@ static int launch_skinny_mfma(const bf16_t* x, const bf16_t* w, void* out, int M
 #define GFA_LAUNCH_MFMA(CTV, XPV, XFV, NTV) GFA_LAUNCH_MFMA_L(CTV, XPV, XFV, NTV, 1)
     switch (ct) {
         case 1:                                          // columns of the x operand that stand
-            if (M <= 4) GFA_LAUNCH_MFMA(1, 4, false, 1);   // for no row carry later steps of k
+            if (M <= 4 && nt == 2) GFA_LAUNCH_MFMA(1, 4, false, (IS_GATE(MODE) ? 1 : 2));   // for no row carry later steps of k
+            else if (M <= 4) GFA_LAUNCH_MFMA(1, 4, false, 1);
+            else if (M <= 8 && nt == 2) GFA_LAUNCH_MFMA(1, 2, false, (IS_GATE(MODE) ? 1 : 2));
             else if (M <= 8) GFA_LAUNCH_MFMA(1, 2, false, 1);
             else if (nt == 2) GFA_LAUNCH_MFMA(1, 1, true, (IS_GATE(MODE) ? 1 : 2));
             else GFA_LAUNCH_MFMA(1, 1, true, 1);

@@ -139,7 +139,7 @@ def can_chain_norm(n_rows: int, n_out: int, inner: int) -> bool:
 def skinny_into_chain(x, w: torch.Tensor, residual: torch.Tensor, next_g: torch.Tensor):
     """residual += x w^T, and the first half of the RMS norm that follows: returns
     ``xg`` = bfloat16(new residual * next_g) as :class:`ChunkedRows` and ``ssq`` float32
-    [workgroups, R]: per workgroup (one or two tiles of 12 to 16 columns) its share of each row's sum of
+    [workgroups, R]: per workgroup (one tile of 12 to 16 columns or two of 8 to 16) its share of each row's sum of
     squares, R = 4, 8, 16, 32 or 64 rows per record (the least that holds M).  Up to 64 rows; x a
     tensor [M, K] or :class:`ChunkedRows` (the gate's result, left so on request)."""
     chunked = isinstance(x, ChunkedRows)
