@@ -14,7 +14,7 @@
 // (16 KB) under way in registers, across the ends of tiles; behind its last tile it asks for the next product's first
 // blocks, RL_PACE at a time: a chip's worth of loads in flight makes every store, counter and poll of the phases' meeting
 // wait behind it, and asking for all of them at once, or more into the second-level cache, measured slower (8B, 1 row:
-// 2741 us a step; two at a time 2830, all at once 2840, three more blocks into the cache 3000).  The other four waves: one
+// 2741 us a step; two at a time 2820, all at once 2830, three more blocks into the cache 3000).  The other four waves: one
 // waits for the phase before and finishes the products (sum over the streamers, norm, rotation, gate, residual,
 // stores), three bring x into shared memory and work on attention.
 //
