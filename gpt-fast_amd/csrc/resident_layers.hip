@@ -13,23 +13,26 @@
 // nothing but read weights and multiply.  While a product's x is there each has RL_RING blocks of 16 rows x 128 columns
 // (16 KB) under way in registers, across the ends of tiles; behind its last tile it asks for the next product's first
 // blocks, RL_PACE at a time: a chip's worth of loads in flight makes every store, counter and poll of the phases' meeting
-// wait behind it, and asking for all of them at once, or more into the second-level cache, measured slower (8B, 1 row:
-// 2741 us a step; two at a time 2820, all at once 2830, three more blocks into the cache 3000).  The other four waves: one
+// wait behind it, and asking for all of them at once, or more into the second-level cache, measured slower (8B, 1 row,
+// 16 counters: 2741 us a step; two at a time 2820, all at once 2830, three more blocks into the cache 3000).  The other four waves: one
 // waits for the phase before and finishes the products (sum over the streamers, norm, rotation, gate, residual,
 // stores), three bring x into shared memory and work on attention.
 //
 // Loads of 4 rows x 256 bytes, past the caches, stream at 7.0 TB/s, 16 rows x 64 bytes (the
 // order of the matrix cores' operands) at 6.0: so the blocks pass through a piece of shared memory of the wave's own.
 //
-// Measured, us a decode step, five launches a layer -> this: 110M shape (12 layers, 768 wide) 1 row 333 -> 306,
-// 8 rows of 200 keys 375 -> 349; 8B shape 1 row of 200 keys 2990 -> 2740 (its weights take 2150 at 7.0 TB/s),
-// 8 rows 3090 -> 2990, 1 row of 6000 keys 3240 -> 3149; 8 new tokens of one sequence behind 6000 keys 10300 -> 3710 (the
-// attention of prompts has too few workgroups there).  What is left over the stream, of an 8B layer's 78 us 16:
-// four meetings under load, 1.3 to 4.7 each, and attention, 5 and its own meeting.
+// Measured, us a decode step, five launches a layer -> this: 110M shape (12 layers, 768 wide) 1 row 333 -> 286,
+// 8 rows of 200 keys 375 -> 321; 8B shape 1 row of 200 keys 2990 -> 2676 (its weights take 2150 at 7.0 TB/s, the head's with
+// them), 8 rows 3090 -> 2917, 1 row of 2000 keys 3110 -> 2853; 8 new tokens of one sequence behind 6000 keys 10300 -> 3710 (the
+// attention of prompts has too few workgroups there).  What is left over the stream is the meetings, 1 to 4 us each under
+// load, and attention, 5 and its own meeting.
 //
 // Between phases: results are stored through to memory (agent scope), and once they are there the workgroup adds
-// one to one of sixteen counters in lines of their own; the next phase polls all sixteen.  256 workgroups meet in
-// 1.3 us so (one counter 3.9 us, one flag a workgroup 2.2 to 3.2).  What a phase leaves lies in memory that this launch
+// one to one of 64 counters in lines of their own; the next phase polls all of them, one a lane.  Additions to a line wait for one
+// another, longer the more loads are under way: with 8, 16, 32, 64 counters a step of the 110M shape takes 323, 306, 293, 286 us
+// at 1 row and 376, 352, 336, 321 at 8 rows, of the 8B shape 2800, 2746, 2700, 2676 and 3084, 2998, 2952, 2917; lines of 128 and 512
+// bytes take as long as these of 256.  (256 workgroups that do nothing else meet in 1.3 us with 16, 3.9 with one, 2.2 to 3.2
+// with a flag each.)  What a phase leaves lies in memory that this launch
 // has not touched before, so that no cache can hold an older copy: every layer has its own buffers.  The counters only grow:
 // nothing arrives for a phase before the one in front of it is complete.
 //
@@ -55,7 +58,7 @@
 #define RL_SHARE 8                    // blocks of 32 keys that a share of a context has at least, and
 #define RL_SHARE_COST 6               // blocks that a share costs beside its own
 #define RL_SUMS (RL_STREAMERS * 2 * 64)   // floatx4 of a tile's partial sums
-#define RL_COUNTERS 16
+#define RL_COUNTERS 64
 #define RL_LINE 64                    // ints from one counter to the next
 #define RL_NOWHERE 0xfffff000u        // an offset behind every matrix: reads as zero
 #define RL_MOST_BYTES 0xffff0000l
@@ -641,7 +644,7 @@ __device__ __forceinline__ bool rl_join_heads(const Args& a, char* work, const R
     return complete;
 }
 
-// What is waited for: cumulative counts of the sixteen counters, lane c < 16 holding counter c's.
+// What is waited for: cumulative counts of the counters, lane c holding counter c's.
 struct RlWait {
     int* counters;
     int need, lane;
