@@ -22,15 +22,15 @@
 // order of the matrix cores' operands) at 6.0: so the blocks pass through a piece of shared memory of the wave's own.
 //
 // Measured, us a decode step, five launches a layer -> this: 110M shape (12 layers, 768 wide) 1 row 333 -> 286,
-// 8 rows of 200 keys 375 -> 321; 8B shape 1 row of 200 keys 2990 -> 2676 (its weights take 2150 at 7.0 TB/s, the head's with
-// them), 8 rows 3090 -> 2917, 1 row of 2000 keys 3110 -> 2853; 8 new tokens of one sequence behind 6000 keys 10300 -> 3710 (the
+// 8 rows of 200 keys 375 -> 317; 8B shape 1 row of 200 keys 2990 -> 2660 (its weights take 2150 at 7.0 TB/s, the head's with
+// them), 8 rows 3090 -> 2896; 8 new tokens of one sequence behind 6000 keys 10300 -> 3710 (the
 // attention of prompts has too few workgroups there).  What is left over the stream is the meetings, 1 to 4 us each under
 // load, and attention, 5 and its own meeting.
 //
 // Between phases: results are stored through to memory (agent scope), and once they are there the workgroup adds
-// one to one of 64 counters in lines of their own; the next phase polls all of them, one a lane.  Additions to a line wait for one
-// another, longer the more loads are under way: with 8, 16, 32, 64 counters a step of the 110M shape takes 323, 306, 293, 286 us
-// at 1 row and 376, 352, 336, 321 at 8 rows, of the 8B shape 2800, 2746, 2700, 2676 and 3084, 2998, 2952, 2917; lines of 128 and 512
+// one to one of 128 counters in lines of their own; the next phase polls all of them, two a lane.  Additions to a line wait for one
+// another, longer the more loads are under way: with 8, 16, 32, 64, 128 counters a step of the 110M shape takes 323, 306, 293, 286,
+// 286 us at 1 row and 376, 352, 336, 321, 317 at 8 rows, of the 8B shape 2800, 2746, 2700, 2676, 2660 and 3084, 2998, 2952, 2917, 2896; lines of 128 and 512
 // bytes take as long as these of 256.  (256 workgroups that do nothing else meet in 1.3 us with 16, 3.9 with one, 2.2 to 3.2
 // with a flag each.)  What a phase leaves lies in memory that this launch
 // has not touched before, so that no cache can hold an older copy: every layer has its own buffers.  The counters only grow:
@@ -58,7 +58,7 @@
 #define RL_SHARE 8                    // blocks of 32 keys that a share of a context has at least, and
 #define RL_SHARE_COST 6               // blocks that a share costs beside its own
 #define RL_SUMS (RL_STREAMERS * 2 * 64)   // floatx4 of a tile's partial sums
-#define RL_COUNTERS 64
+#define RL_COUNTERS 128
 #define RL_LINE 64                    // ints from one counter to the next
 #define RL_NOWHERE 0xfffff000u        // an offset behind every matrix: reads as zero
 #define RL_MOST_BYTES 0xffff0000l
@@ -644,21 +644,22 @@ __device__ __forceinline__ bool rl_join_heads(const Args& a, char* work, const R
     return complete;
 }
 
-// What is waited for: cumulative counts of the counters, lane c holding counter c's.
+// What is waited for: cumulative counts of the counters, lane c holding those of counters c and 64 + c.
 struct RlWait {
     int* counters;
     int need, lane;
     bool lost;
+    int need1 = 0;                        // of the second counter
     __device__ __forceinline__ void expect(int arrivals) {
-        if (lane < RL_COUNTERS) need += (unsigned)(arrivals + RL_COUNTERS - 1 - lane) / RL_COUNTERS;
+        need += (unsigned)(arrivals + RL_COUNTERS - 1 - lane) / RL_COUNTERS;
+        need1 += (unsigned)(arrivals + RL_COUNTERS - 1 - 64 - lane) / RL_COUNTERS;
     }
     __device__ __forceinline__ void all() {
         if (lost) return;
         int polls = 0;
         for (;;) {
-            int seen = need;
-            if (lane < RL_COUNTERS) seen = rl_get(counters + lane * RL_LINE);
-            if (__all(seen >= need)) break;
+            const int seen = rl_get(counters + lane * RL_LINE), seen1 = rl_get(counters + (64 + lane) * RL_LINE);
+            if (__all(seen >= need && seen1 >= need1)) break;
             if (++polls == RL_MAX_POLLS) {
                 lost = true;
                 break;

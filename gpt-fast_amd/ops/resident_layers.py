@@ -27,7 +27,7 @@ def takes(n_rows: int, dim: int, hidden: int, n_heads: int, n_kv_heads: int, hea
 def pays(n_layers: int, n_rows: int, n_seqs: int, table_pages: int, dim: int, hidden: int, n_heads: int, n_kv_heads: int,
          head_dim: int, units: int) -> bool:
     """Whether one launch that stays on its ``units`` compute units takes less time than five launches a layer
-    (ops.few_row_layers), both measured on 256 units, in us a step (this side when its phases met through 16 counters, not 64:
+    (ops.few_row_layers), both measured on 256 units, in us a step (this side when its phases met through 16 counters, not 128:
     2 to 9 % longer than now):
 
     - From 8 layers on: meeting at the start costs what some layers give.  768 wide, 1 row: 3 layers 118 -> 130, 6 layers
