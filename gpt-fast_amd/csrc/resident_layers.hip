@@ -572,7 +572,7 @@ __device__ __forceinline__ bool rl_join_heads(const Args& a, char* work, const R
 #pragma unroll
     for (int q = 0; q < DQ; ++q) o[q] = floatx4_t{0.f, 0.f, 0.f, 0.f};
     auto merge = [&](float mw, float lw, const floatx4_t (&other)[DQ]) {
-        if (mw == -INFINITY) return;
+        if (mw == -INFINITY && lw == 0.f) return;          // saw no key; scores that are no numbers leave lw NaN, and that stays
         const float m_new = fmaxf(m, mw);
         const float keep = __builtin_amdgcn_exp2f(m - m_new), add = __builtin_amdgcn_exp2f(mw - m_new);
         l = l * keep + lw * add;

@@ -1,0 +1,80 @@
+"""One plain layer over a few rows (csrc/resident_layers.hip, and beside it the launches of one kernel at a time,
+csrc/gemm_bf16.hip: gfa_few_row_layers_bf16), row by row, with the keys and values that it writes."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+import util
+
+pytestmark = pytest.mark.gpu
+DEV, PAGE, EPS = "cuda:0", 64, 1e-5
+
+
+def _problem(D, H, G, hd, inner, held, new, window=0, rot=None, seed=0, extra_pages=0):
+    """A layer, its inputs and a cache that holds ``held`` tokens of each sequence; slots that hold none are NaN."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+
+    def randn(*shape, std=1.0):
+        return torch.randn(*shape, generator=g, device=DEV) * std
+    rot = hd if rot is None else rot
+    M, longest = sum(new), max(h + n for h, n in zip(held, new))
+    width = -(-longest // PAGE) + extra_pages
+    n_pages = width * len(held) + 2
+    table = torch.randperm(n_pages, generator=g, device=DEV)[:width * len(held)].view(len(held), width).int()
+    keys = torch.full((n_pages, G, PAGE, hd), float("nan"), device=DEV, dtype=torch.bfloat16)
+    values = torch.full((n_pages, G, hd, PAGE), float("nan"), device=DEV, dtype=torch.bfloat16)
+    for i, h in enumerate(held):
+        for at in range(0, h, PAGE):
+            n, page = min(PAGE, h - at), int(table[i, at // PAGE])
+            keys[page, :, :n] = randn(G, n, hd).bfloat16()
+            values[page, :, :, :n] = randn(G, hd, n).bfloat16()
+    p = SimpleNamespace(
+        D=D, H=H, G=G, hd=hd, inner=inner, rot=rot, window=window, scale=hd ** -0.5, held=held, new=new, keys=keys, values=values,
+        wqkv=randn((H + 2 * G) * hd, D, std=D ** -0.5).bfloat16(), wo=randn(D, H * hd, std=(H * hd) ** -0.5).bfloat16(),
+        w13=randn(2 * inner, D, std=D ** -0.5).bfloat16(), w2=randn(D, inner, std=inner ** -0.5).bfloat16(),
+        norm_mixer=1 + 0.1 * randn(D), norm_ffn=1 + 0.1 * randn(D), table=table, residual=randn(M, D),
+        freqs=10000.0 ** (-torch.arange(0, rot, 2, device=DEV).float() / rot))
+    ints = dict(dtype=torch.int32, device=DEV)
+    starts = [sum(new[:i]) for i in range(len(new) + 1)]
+    p.batch = SimpleNamespace(
+        tok_seq=torch.tensor([i for i, n in enumerate(new) for _ in range(n)], **ints),
+        tok_pos=torch.tensor([h + t for h, n in zip(held, new) for t in range(n)], **ints),
+        start_pos=torch.tensor(held, **ints), q_start=torch.tensor(starts, **ints), n_seqs=len(new), n_tokens=M, max_q_len=max(new))
+    return p
+
+
+def _run(p, way, **options):
+    """(the stream behind the layer, its keys and values as [page, G, slot, d] and [page, G, d, slot])."""
+    from gpt_fast_amd.ops import few_row_layers as F
+    from gpt_fast_amd.ops import resident_layers as R
+    k_pages, v_pages = util.to_cache_order(p.keys, p.values)
+    layer = F.Layer(p.wqkv, p.wo, p.w13, p.w2, p.norm_mixer, p.norm_ffn, k_pages, v_pages, p.table)
+    stream = p.residual.clone()
+    if way == "resident":
+        R.run([layer], stream, p.freqs, p.rot, p.batch, p.H, p.G, p.hd, p.window, EPS, EPS, p.scale, "silu", **options)
+    else:
+        x = stream * (stream.square().mean(1, keepdim=True) + EPS).rsqrt() * p.norm_mixer
+        F.run_layers([layer], x.bfloat16(), stream, p.freqs, p.rot, p.batch, p.H, p.G, p.hd, p.window, EPS, EPS, p.scale, "silu")
+    return (stream,) + util.from_cache_order(k_pages, v_pages)
+
+
+# head size, heads, key/value heads, window, the newest token's position; the keys that are no numbers: all that a wave sees, the
+# first time the only one of its block of 32 that the window shows, the last time all of a share of a long context
+NO_NUMBERS = [(64, 4, 4, 65, 95, 31, 32), (128, 8, 2, 0, 70, 32, 64), (48, 6, 3, 0, 40, 0, 32), (16, 2, 2, 0, 96, 64, 96),
+              (64, 2, 1, 0, 2100, 0, 256)]
+
+
+@pytest.mark.parametrize("way", ["resident"])
+@pytest.mark.parametrize("hd,H,G,window,pos,first,end", NO_NUMBERS)
+def test_a_part_of_a_context_that_is_no_number_makes_the_row_no_number(hd, H, G, window, pos, first, end, way):
+    """Every column of the layer's result reads every head, so the row is NaN from end to end; the other sequence's row keeps
+    its bits."""
+    p = _problem(128, H, G, hd, 136, [pos, pos], [1, 1], window=window)
+    want = _run(p, way)[0]
+    assert bool(torch.isfinite(want).all())
+    for key in range(first, end):
+        p.keys[int(p.table[0, key // PAGE]), :, key % PAGE] = float("nan")
+    got = _run(p, way)[0]
+    assert bool(torch.isnan(got[0]).all())
+    assert torch.equal(got[1], want[1])
