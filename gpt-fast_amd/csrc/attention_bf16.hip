@@ -407,8 +407,8 @@ __global__ __launch_bounds__(RT == 1 ? 512 : 256) void attention_mfma_kernel(
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 const float mw = sm_ml[(((w - 1) * RT + rt) * 16 + li) * 2];
-                if (mw == -INFINITY) continue;
                 const float lw = sm_ml[(((w - 1) * RT + rt) * 16 + li) * 2 + 1];
+                if (mw == -INFINITY && lw == 0.f) continue;    // saw no key; scores that are no numbers leave lw NaN
                 const float m_new = fmaxf(m[rt], mw);
                 const float a = __builtin_amdgcn_exp2f(m[rt] - m_new);     // 0 if this wave saw no key
                 const float b = __builtin_amdgcn_exp2f(mw - m_new);

@@ -65,7 +65,7 @@ NO_NUMBERS = [(64, 4, 4, 65, 95, 31, 32), (128, 8, 2, 0, 70, 32, 64), (48, 6, 3,
               (64, 2, 1, 0, 2100, 0, 256)]
 
 
-@pytest.mark.parametrize("way", ["resident"])
+@pytest.mark.parametrize("way", ["resident", "one by one"])
 @pytest.mark.parametrize("hd,H,G,window,pos,first,end", NO_NUMBERS)
 def test_a_part_of_a_context_that_is_no_number_makes_the_row_no_number(hd, H, G, window, pos, first, end, way):
     """Every column of the layer's result reads every head, so the row is NaN from end to end; the other sequence's row keeps
