@@ -37,9 +37,11 @@
 // nothing arrives for a phase before the one in front of it is complete.
 //
 // Waiting cannot lock up, whatever part of the grid the chip has room for: nothing is waited for but workgroups that
-// run.  They are counted at the start.  If all are there, workgroup b is worker b of all.  If some are not
-// there after a while (another launch holds their place), those that run close the list and share the work
-// among themselves; what starts later finds the list closed and ends.
+// run.  A phase's work is cut into as many parts as the grid has workgroups.  They are counted at the start: if all are there,
+// workgroup b takes part b of every phase.  If some are not there after a while (another launch holds their place), those that
+// run close the list and share all parts among themselves, worker v of V taking parts v, v + V, ...; what starts later
+// waits for the next layer, in front of which the list is made anew, until all are there.  So a launch that begins on a busy chip has the
+// rest of it as soon as it is free, and every result has the same bits whoever worked it out.
 #include "few_row_layers.h"
 #include <cstring>
 
@@ -99,17 +101,22 @@ struct ResidentArgs {
     size_t work_stride;
     unsigned off_q, off_po, off_pml;
     int n_layers, M, D, I, H, Hkv, hd, rot, table_stride, window, pad, gate_mode;
-    int start_polls, seal_polls;          // polls before the list of workers is closed, and then sealed
+    int start_polls, seal_polls;          // polls before the list of workers is closed, and then the first layer's
     float scale_log2;
 };
 
-// The words of a launch, in ints: [0] groups of workgroups that are there and the closed bit, [RL_LINE] workers after closing
-// and the sealed bit, then the groups' and the phases' counters, then one word per (token, kv head) for its shares.
+// The words of a launch, in ints: [0] groups of workgroups that are there and the closed bit, then the groups' and the phases'
+// counters, per layer its list of workers (how many, how many of them worked on the layer before, the closed bit), then one word
+// per (token, kv head) for its shares.
 #define RL_CLOSED (1 << 30)
+#define RL_BEFORE (1 << 15)
+#define RL_COUNT (RL_BEFORE - 1)
 #define RL_GROUPS 16
-#define RL_AT_GROUPS (2 * RL_LINE)
+#define RL_LIST 16                    // ints from one list to the next
+#define RL_AT_GROUPS RL_LINE
 #define RL_AT_COUNTERS (RL_AT_GROUPS + RL_GROUPS * RL_LINE)
-#define RL_AT_SPLITS (RL_AT_COUNTERS + RL_COUNTERS * RL_LINE)
+#define RL_AT_LISTS (RL_AT_COUNTERS + RL_COUNTERS * RL_LINE)
+#define RL_AT_SPLITS (RL_AT_LISTS + RL_MAX_LAYERS * RL_LIST)
 #define RL_MAX_POLLS (1 << 22)        // seconds: a wait that runs out leaves NaN
 
 typedef const __attribute__((address_space(4))) ResidentArgs RlArgs;
@@ -133,36 +140,33 @@ __device__ __forceinline__ unsigned rl_two(float a, float b) {
     return (unsigned)float_to_bf16(a) | (unsigned)float_to_bf16(b) << 16;
 }
 
-// One product of a layer, as this worker sees it.
+// One part of a product of a layer.
 struct RlProduct {
     const bf16_t* w;
     unsigned bytes;
     int K, gate;                          // gate: rows between a column's two rows of W, or 0
-    int base, rows;                       // this worker's rows of W, in tiles of sixteen; both multiples of four
+    int base, rows;                       // the part's rows of W, in tiles of sixteen; both multiples of four
     int pieces;                           // of 128 columns: those of the streamer that has the most
     int chunk, chunks;                    // pieces of x that lie in shared memory at a time; 1 chunk: all of x, as it is
 };
 
 // What is the same in every layer, worked out once and kept in shared memory.
 struct RlPlan {
-    int base, rows, K, gate;
-    int pieces, chunk, chunks, arrivals;  // arrivals: workers that have rows
+    int N, share, K, gate;                // share: rows of a part
+    int pieces, chunk, chunks, arrivals;  // arrivals: parts that have rows
     unsigned bytes, off_in, off_out, off_share;
     unsigned off_sums, unused[3];
 };
 
-// Rows per worker of N rows.
-__device__ __forceinline__ int rl_share(int N, int V) { return ((N >> 2) + V - 1) / V * 4; }
-
 template <typename Args>
-__device__ __forceinline__ void rl_make_plan(const Args& a, RlPlan* plan, int phase, int v, int V) {
+__device__ __forceinline__ void rl_make_plan(const Args& a, RlPlan* plan, int phase, int parts) {
     RlPlan t = {};
-    const int N = a.N[phase], share = rl_share(N, V);
+    const int N = a.N[phase], share = ((N >> 2) + parts - 1) / parts * 4;
+    t.N = N;
+    t.share = share;
     t.K = a.K[phase];
     t.gate = a.gate[phase];
     t.bytes = (unsigned)(N + t.gate) * (unsigned)t.K * 2u;
-    t.base = v * share;
-    t.rows = t.base >= N ? 0 : N - t.base < share ? N - t.base : share;
     t.arrivals = share > 0 ? (N + share - 1) / share : 0;
     const int T = (t.K + RL_PIECE - 1) / RL_PIECE;
     t.pieces = (T + RL_STREAMERS - 1) / RL_STREAMERS;
@@ -184,7 +188,7 @@ __device__ __forceinline__ void rl_make_plan(const Args& a, RlPlan* plan, int ph
 __device__ __forceinline__ int rl_same(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 template <typename Args>
-__device__ __forceinline__ RlProduct rl_product(const Args& a, const RlPlan* plan, int layer, int phase) {
+__device__ __forceinline__ RlProduct rl_product(const Args& a, const RlPlan* plan, int layer, int phase, int part) {
     RlProduct p;
     const bool is = layer < a.n_layers;                    // behind the last layer: a product without rows
     p.w = a.layer[is ? layer : 0].w[phase];
@@ -192,8 +196,9 @@ __device__ __forceinline__ RlProduct rl_product(const Args& a, const RlPlan* pla
     p.bytes = rl_same(t.bytes);
     p.K = rl_same(t.K);
     p.gate = rl_same(t.gate);
-    p.base = rl_same(t.base);
-    p.rows = is ? rl_same(t.rows) : 0;
+    const int share = rl_same(t.share), left = rl_same(t.N) - part * share;
+    p.base = part * share;
+    p.rows = !is || left <= 0 ? 0 : left < share ? left : share;
     p.pieces = rl_same(t.pieces);
     p.chunk = rl_same(t.chunk);
     p.chunks = rl_same(t.chunks);
@@ -675,10 +680,33 @@ struct RlWait {
     }
 };
 
-// Who works: (worker, workers) of this workgroup, or worker < 0.  By one lane.
-__device__ __forceinline__ int2 rl_join(int* words, int start_polls, int seal_polls) {
+// The place of a workgroup: worker v of V, from a layer on; v < 0: nothing to do.
+struct RlPlace {
+    int v, V, layer;
+};
+
+// Into the list of the first layer from `layer` on that is not closed yet, and waits until it is.  By one lane.
+__device__ __forceinline__ RlPlace rl_enlist(int* lists, int layer, int n_layers) {
+    for (; layer < n_layers; ++layer) {
+        int* list = lists + layer * RL_LIST;
+        int seen = rl_get(list);
+        while (!(seen & RL_CLOSED))
+            if (__hip_atomic_compare_exchange_strong(list, &seen, seen + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED, AGENT)) {
+                const int v = seen & RL_COUNT;
+                while (!((seen = rl_get(list)) & RL_CLOSED)) __builtin_amdgcn_s_sleep(2);
+                return {v, seen & RL_COUNT, layer};
+            }
+    }
+    return {-1, 0, 0};
+}
+
+// Who works at the start.  By one lane.  Those that are here wait for the others about as long as a layer would take them, a tenth
+// of start_polls for all of the grid (8B: 76 us, 100 polls): a long wait is lost if nobody comes, a layer by few workers if they
+// come soon.
+__device__ __forceinline__ RlPlace rl_join(int* words, int n_layers, int start_polls, int seal_polls) {
     const int b = blockIdx.x, n = gridDim.x, group = b % RL_GROUPS;
     const int groups = n < RL_GROUPS ? n : RL_GROUPS, of_group = (n - group + RL_GROUPS - 1) / RL_GROUPS;
+    int* lists = words + RL_AT_LISTS;
     int state = 0;
     if (__hip_atomic_fetch_add(words + RL_AT_GROUPS + group * RL_LINE, 1, __ATOMIC_RELAXED, AGENT) == of_group - 1) {
         state = rl_get(words);                             // the last of its group: the group is there
@@ -686,31 +714,33 @@ __device__ __forceinline__ int2 rl_join(int* words, int start_polls, int seal_po
                !__hip_atomic_compare_exchange_strong(words, &state, state + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED, AGENT)) {}
     }
     int polls = 0;
-    bool closed_here = false;
     for (;;) {
         state = rl_get(words);
-        if (state == groups) return make_int2(b, n);       // all are there
-        if (state & RL_CLOSED) break;
+        if (state == groups) return {b, n, 0};             // all are there
+        if (state & RL_CLOSED) return rl_enlist(lists, 0, n_layers);
         if (++polls >= start_polls) {
-            closed_here = __hip_atomic_compare_exchange_strong(words, &state, state | RL_CLOSED, __ATOMIC_RELAXED, __ATOMIC_RELAXED, AGENT);
-            continue;
+            int here = 0;
+            for (int i = 0; i < groups; ++i) here += rl_get(words + RL_AT_GROUPS + i * RL_LINE);
+            if (10 * here * polls >= start_polls * n &&
+                __hip_atomic_compare_exchange_strong(words, &state, state | RL_CLOSED, __ATOMIC_RELAXED, __ATOMIC_RELAXED, AGENT))
+                break;
         }
         __builtin_amdgcn_s_sleep(2);
     }
-    // some are not: those that come here before the list is sealed share the work
-    int* list = words + RL_LINE;
-    int mine = rl_get(list);
-    for (;;) {
-        if (mine & RL_CLOSED) return make_int2(-1, 0);
-        if (__hip_atomic_compare_exchange_strong(list, &mine, mine + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED, AGENT)) break;
-    }
-    if (closed_here) {
-        for (int i = 0; i < seal_polls; ++i) __builtin_amdgcn_s_sleep(2);
-        __hip_atomic_fetch_or(list, RL_CLOSED, __ATOMIC_RELAXED, AGENT);
-    }
-    int sealed;
-    while (!((sealed = rl_get(list)) & RL_CLOSED)) __builtin_amdgcn_s_sleep(2);
-    return make_int2(mine, sealed & ~RL_CLOSED);
+    // some are not: those that come here before the first layer's list is closed share the work
+    const int v = __hip_atomic_fetch_add(lists, 1, __ATOMIC_RELAXED, AGENT);
+    for (int i = 0; i < seal_polls; ++i) __builtin_amdgcn_s_sleep(2);
+    return {v, __hip_atomic_fetch_or(lists, RL_CLOSED, __ATOMIC_RELAXED, AGENT), 0};
+}
+
+// Who works on the next layer: the V that worked on the one before, the last of which closes the list, and those that came
+// before that.  By one lane.
+__device__ __forceinline__ int2 rl_join_again(int* list, int V) {
+    int seen = __hip_atomic_fetch_add(list, RL_BEFORE + 1, __ATOMIC_RELAXED, AGENT);
+    const int v = seen & RL_COUNT;
+    if (seen / RL_BEFORE + 1 == V) return make_int2(v, __hip_atomic_fetch_or(list, RL_CLOSED, __ATOMIC_RELAXED, AGENT) & RL_COUNT);
+    while (!((seen = rl_get(list)) & RL_CLOSED)) __builtin_amdgcn_s_sleep(2);
+    return make_int2(v, seen & RL_COUNT);
 }
 
 __device__ __forceinline__ float rl_gate(int mode, float a) {
@@ -721,48 +751,61 @@ __device__ __forceinline__ float rl_gate(int mode, float a) {
 // Lane i of every sixteen gets the value of lane (i + n) % 16.
 #define RL_TURNED(x, n) __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x120 + 16 - (n), 0xf, 0xf, false))
 
-template <int DS, bool FULL>
-__global__ __launch_bounds__(RL_THREADS) void resident_layers_kernel(const ResidentArgs) {
-    RlArgs& a = *(RlArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-    extern __shared__ __attribute__((aligned(128))) char smem[];
+// A worker's way through the layers.  WHOLE: all workgroups are there, and every part of a phase has one worker from the first
+// layer to the last.  In a body of its own: in one body for both forms more is alive than there are registers for, and a step of the 8B
+// shape takes 2,880 us instead of 2,667 at 1 row, 3,108 instead of 2,892 at 8.
+template <int DS, bool FULL, bool WHOLE, typename Args>
+__device__ __forceinline__ void rl_work(const Args& a, char* smem, int v, int V, int first_layer) {
     char* x_lds = smem;
     char* stages = smem + RL_X_BYTES;
     floatx4_t* sums = (floatx4_t*)(stages + RL_STREAMERS * RL_STAGE);
     int* place = (int*)(sums + 2 * RL_SUMS);
-    int* first = place + 16;
-    RlPlan* plan = (RlPlan*)(first + 32);
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (threadIdx.x == 0) {
-        const int2 w = rl_join(a.words, a.start_polls, a.seal_polls);
-        place[0] = w.x;
-        place[1] = w.y;
-    }
-    lds_barrier();
-    const int v = __builtin_amdgcn_readfirstlane(place[0]), V = __builtin_amdgcn_readfirstlane(place[1]);
-    if (v < 0) return;
-    if (threadIdx.x < 5) rl_make_plan(a, plan, threadIdx.x, v, V);
-    if (wave == 1) rl_make_shares(a, first, lane);
-    lds_barrier();
+    const int* first = place + 16;
+    const RlPlan* plan = (RlPlan*)(first + 32);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), parts = gridDim.x;
+    if (WHOLE) first_layer = 0;
+    // where some are missing all waves meet twice between layers: the new list is there; all have read it
+    auto new_list = [&] {
+        lds_barrier();
+        v = rl_same(place[0]);
+        V = rl_same(place[1]);
+        lds_barrier();
+    };
     const int pad = a.pad, pairs = a.M * a.Hkv;
     const int items = rl_same(first[a.M]) * a.Hkv;
     const bool shared = items > pairs;
     if (wave < RL_STREAMERS) {
         rl_u4 ring[RL_RING][4];
         RlCursor c;
-        RlProduct p = rl_product(a, plan, 0, 0);
+        char* stage = stages + wave * RL_STAGE;
+        int layer = first_layer, phase = 0, part = v;
+        RlProduct p = rl_product(a, plan, layer, 0, v);
         rl_seek(c, p, wave);
 #pragma unroll
         for (int i = 0; i < RL_RING; ++i) rl_ask(c, ring[i], lane);
-        char* stage = stages + wave * RL_STAGE;
-        int layer = 0, phase = 0;
 #pragma unroll 1
         while (layer < a.n_layers) {
-            const int next_phase = phase == 0 ? 2 : phase == 4 ? 0 : phase + 1, next_layer = layer + (phase == 4);
-            const RlProduct next = rl_product(a, plan, next_layer, next_phase);
+            bool part_left = false;
+            if (!WHOLE) {
+                part_left = part + V < parts;
+                part = part_left ? part + V : v;
+            }
+            const int next_phase = part_left ? phase : phase == 0 ? 2 : phase == 4 ? 0 : phase + 1;
+            const int next_layer = layer + (phase == 4 && !part_left);
+            const bool other_list = !WHOLE && next_layer != layer && V < parts;   // the next part is not known yet
+            RlProduct next = rl_product(a, plan, other_list ? a.n_layers : next_layer, next_phase, part);
             rl_stream(p, next, c, ring, wave, lane, pad, x_lds, stage, sums);
-            if (phase == 0)                                // attention: the other waves'
+            if (phase == 0 && !part_left)                  // attention: the other waves'
                 for (int item = v; item < items; item += V)
                     for (int i = 0; i < RL_ITEM_MEETINGS(shared); ++i) lds_barrier();
+            if (other_list && next_layer < a.n_layers) {
+                new_list();
+                part = v;
+                next = rl_product(a, plan, next_layer, 0, v);
+                rl_seek(c, next, wave);
+#pragma unroll
+                for (int i = 0; i < RL_RING; ++i) rl_ask(c, ring[i], lane);
+            }
             p = next;
             phase = next_phase;
             layer = next_layer;
@@ -774,7 +817,7 @@ __global__ __launch_bounds__(RL_THREADS) void resident_layers_kernel(const Resid
         const int aux = wave - RL_STREAMERS;
         __builtin_amdgcn_s_setprio(2);
 #pragma unroll 1
-        for (int at = 0; at < 5 * a.n_layers; ++at) {
+        for (int at = 5 * first_layer; at < 5 * a.n_layers; ++at) {
             const int layer = at / 5, phase = at - 5 * layer;
             char* work = a.work + (size_t)layer * a.work_stride;
             if (phase == 1) {
@@ -782,29 +825,33 @@ __global__ __launch_bounds__(RL_THREADS) void resident_layers_kernel(const Resid
                     const RlItem it(a, first, item);
                     rl_attend<DS, FULL>(a, a.layer[layer], work, it, x_lds, aux, [] { lds_barrier(); });
                     lds_barrier();
-                    rl_join_heads<DS, FULL>(a, work, it, layer, x_lds, aux, shared, place + 2);
+                    rl_join_heads<DS, FULL>(a, work, it, layer, x_lds, aux, shared, place + 3);
                 }
                 continue;
             }
-            const RlProduct p = rl_product(a, plan, layer, phase);
-            if (p.rows == 0) continue;
-            const char* x = work + (unsigned)rl_same(plan[phase].off_in);
-            lds_barrier();
-            int chunk_begin = 0;
-            for (int n = 0, of = ((p.rows + 15) >> 4) * p.chunks; n <= of; ++n) {
-                if (n == 0 || (p.chunks > 1 && n < of))
-                    rl_bring(p, x, pad, chunk_begin, x_lds + (n & 1) * RL_X_HALF, aux - 1, lane);
-                chunk_begin += p.chunk;
-                if (chunk_begin >= p.pieces) chunk_begin = 0;
+            int part = v;
+            do {
+                const RlProduct p = rl_product(a, plan, layer, phase, part);
+                if (p.rows == 0) break;
+                const char* x = work + (unsigned)rl_same(plan[phase].off_in);
                 lds_barrier();
-            }
+                int chunk_begin = 0;
+                for (int n = 0, of = ((p.rows + 15) >> 4) * p.chunks; n <= of; ++n) {
+                    if (n == 0 || (p.chunks > 1 && n < of))
+                        rl_bring(p, x, pad, chunk_begin, x_lds + (n & 1) * RL_X_HALF, aux - 1, lane);
+                    chunk_begin += p.chunk;
+                    if (chunk_begin >= p.pieces) chunk_begin = 0;
+                    lds_barrier();
+                }
+            } while (!WHOLE && (part += V) < parts);
+            if (!WHOLE && phase == 4 && V < parts && layer + 1 < a.n_layers) new_list();
         }
         return;
     }
 
     // the one that waits for the phase before and finishes products and attention
     const int fi = lane & 15, fg = lane >> 4;
-    const int base_d = rl_same(plan[2].base), rows_d = rl_same(plan[2].rows), with_d = rl_same(plan[2].arrivals);
+    const int with_d = rl_same(plan[2].arrivals);
     RlWait wait = {a.words + RL_AT_COUNTERS, 0, lane, false};
 
     // four columns n.. of the stream: their normed half; returns the sum of their squares
@@ -812,11 +859,18 @@ __global__ __launch_bounds__(RL_THREADS) void resident_layers_kernel(const Resid
         rl_put8((bf16_t*)x + chunked_elem(fi, n, pad), rl_two(r.x * g.x, r.y * g.y), rl_two(r.z * g.z, r.w * g.w));
         return fmaf(r.x, r.x, fmaf(r.y, r.y, fmaf(r.z, r.z, r.w * r.w)));
     };
-    // this worker's share of the rows' sums of squares
-    auto leave_share = [&](float part, char* s) {
-        part += __shfl_xor(part, 16, GFA_WAVE);
-        part += __shfl_xor(part, 32, GFA_WAVE);
-        if (fg == 0 && fi < pad) rl_put((float*)s + (size_t)v * pad + fi, part);
+    // a part's share of the rows' sums of squares
+    auto leave_share = [&](float sum, char* s, int part) {
+        sum += __shfl_xor(sum, 16, GFA_WAVE);
+        sum += __shfl_xor(sum, 32, GFA_WAVE);
+        if (fg == 0 && fi < pad) rl_put((float*)s + (size_t)part * pad + fi, sum);
+    };
+    // four columns of the stream: one worker's from the first layer to the last, or another one's in every layer
+    auto stream_at = [&](int n) {
+        const float* at = a.residual + (size_t)fi * a.D + n;
+        if (WHOLE) return *(const float4*)at;
+        const float2 lo = rl_get8(at), hi = rl_get8(at + 2);
+        return make_float4(lo.x, lo.y, hi.x, hi.y);
     };
     // What finishing the first tile of a product needs beside the sums stays here: the stream's columns, and of the rotation
     // what is the same in every layer.
@@ -834,24 +888,30 @@ __global__ __launch_bounds__(RL_THREADS) void resident_layers_kernel(const Resid
     };
     {
         __builtin_amdgcn_s_setprio(3);                     // others wait for what this wave does
-        if (v < with_d) {                                  // the norm before the first layer
-            float part = 0.f;
-            for (int n = base_d + fg * 4; n < base_d + rows_d; n += 16)
+        for (int part = v; part < with_d && first_layer == 0; part += WHOLE ? with_d : V) {   // the norm before the first layer
+            const RlProduct d = rl_product(a, plan, 0, 2, part);
+            float sum = 0.f;
+            for (int n = d.base + fg * 4; n < d.base + d.rows; n += 16)
                 if (fi < a.M) {
                     const float4 r = *(const float4*)(a.residual + (size_t)fi * a.D + n);
-                    part += leave_normed(n, r, *(const float4*)(a.norm_first + n), a.work + a.off_in[0]);
-                    if (n < base_d + 16) stream0 = r;
+                    sum += leave_normed(n, r, *(const float4*)(a.norm_first + n), a.work + a.off_in[0]);
+                    if (n < d.base + 16) stream0 = r;
                 }
-            leave_share(part, a.work + a.off_sums[0]);
-            wait.arrive(v);
+            leave_share(sum, a.work + a.off_sums[0], part);
+            wait.arrive(part);
         }
         wait.expect(with_d);
+        for (int n = 0; n < first_layer; ++n) {            // what others have done
+            wait.expect(rl_same(plan[0].arrivals));
+            wait.expect(pairs);
+            for (int phase = 2; phase < 5; ++phase) wait.expect(rl_same(plan[phase].arrivals));
+        }
         if (fi < a.M) pos = a.tok_pos[fi];
-        const int n = rl_same(plan[0].base) + fg * 4;
+        const int n = v * rl_same(plan[0].share) + fg * 4;
         if (fi < a.M && n < a.N[0]) angles(n, cs0, sn0);
     }
 
-    for (int layer = 0; layer < a.n_layers; ++layer) {
+    for (int layer = first_layer; layer < a.n_layers; ++layer) {
         const auto& L = a.layer[layer];
         char* work = a.work + (size_t)layer * a.work_stride;
 #pragma unroll 1
@@ -862,13 +922,15 @@ __global__ __launch_bounds__(RL_THREADS) void resident_layers_kernel(const Resid
                     if (item == v) wait.all();
                     lds_barrier();
                     lds_barrier();
-                    if (rl_join_heads<DS, FULL>(a, work, it, layer, x_lds, 0, shared, place + 2)) wait.arrive(it.pair);
+                    if (rl_join_heads<DS, FULL>(a, work, it, layer, x_lds, 0, shared, place + 3)) wait.arrive(it.pair);
                 }
                 wait.expect(pairs);
                 continue;
             }
-            const RlProduct p = rl_product(a, plan, layer, phase);
-            if (p.rows > 0) {
+            int part = v;
+            do {
+                const RlProduct p = rl_product(a, plan, layer, phase, part);
+                if (p.rows == 0) break;
                 const int tiles = (p.rows + 15) >> 4;
                 {
                     const float* norm = L.norm[phase];
@@ -883,15 +945,16 @@ __global__ __launch_bounds__(RL_THREADS) void resident_layers_kernel(const Resid
                         if (mine) {
                             if (phase == 0) {
                                 if (n >= a.H * a.hd) page = L.table[(size_t)a.tok_seq[fi] * a.table_stride + pos / GFA_PAGE];
-                                if (j > 0) angles(n, cs, sn);
+                                if (j > 0 || !WHOLE) angles(n, cs, sn);
                             } else if (phase != 3) {
-                                if (j > 0) res = *(const float4*)(a.residual + (size_t)fi * a.D + n);
+                                if (j > 0) res = stream_at(n);
                                 if (norm) g = *(const float4*)(norm + n);
                             }
                         }
                     };
                     ask_operands(0);
                     wait.all();
+                    if (!WHOLE && mine && (phase == 2 || phase == 4)) res = stream_at(n);
                     lds_barrier();
                     // the norm's other half: all workers' shares, sixteen bytes a lane, all of them under way at once;
                     // lane l's numbers are of rows 4 l + e: of every fourth row, or of two or all rows in turn
@@ -937,7 +1000,7 @@ __global__ __launch_bounds__(RL_THREADS) void resident_layers_kernel(const Resid
                     }
                     if (wait.lost) rs = __builtin_nanf("");
                     const unsigned out = rl_same(plan[phase].off_out);
-                    float part = 0.f;
+                    float squares = 0.f;
                     for (int j = 0; j < tiles; ++j) {
                         const bool last = j + 1 == tiles;
                         for (int c = 0; c < p.chunks; ++c) lds_barrier();
@@ -983,25 +1046,61 @@ __global__ __launch_bounds__(RL_THREADS) void resident_layers_kernel(const Resid
                                 rl_put8((bf16_t*)(work + a.off_in[4]) + chunked_elem(fi, n, pad), rl_two(h[0], h[1]), rl_two(h[2], h[3]));
                             } else {
                                 res.x += v0[0]; res.y += v0[1]; res.z += v0[2]; res.w += v0[3];
-                                if (norm) part += leave_normed(n, res, g, work + out);
+                                if (norm) squares += leave_normed(n, res, g, work + out);
                             }
                         }
+                        float* out_stream = a.residual + (size_t)fi * a.D + n;
+                        if (!WHOLE && mine && (phase == 2 || phase == 4)) {
+                            rl_put8(out_stream, __float_as_uint(res.x), __float_as_uint(res.y));
+                            rl_put8(out_stream + 2, __float_as_uint(res.z), __float_as_uint(res.w));
+                        }
                         if (last) {
-                            if (norm) leave_share(part, work + (unsigned)rl_same(plan[phase].off_share));
-                            wait.arrive(v);
+                            if (norm) leave_share(squares, work + (unsigned)rl_same(plan[phase].off_share), part);
+                            wait.arrive(part);
                         }
                         // the stream itself is this wave's alone, and of the first tile it stays in registers
-                        if (phase == 2 || phase == 4) {
+                        if (WHOLE && (phase == 2 || phase == 4)) {
                             if (j == 0) stream0 = res;
-                            if (mine && (j > 0 || layer + 1 == a.n_layers)) *(float4*)(a.residual + (size_t)fi * a.D + n) = res;
+                            if (mine && (j > 0 || layer + 1 == a.n_layers)) *(float4*)out_stream = res;
                         }
                         if (!last) ask_operands(j + 1);
                     }
                 }
-            }
+            } while (!WHOLE && (part += V) < parts);
             wait.expect(rl_same(plan[phase].arrivals));
         }
+        if (!WHOLE && V < parts && layer + 1 < a.n_layers) {
+            if (lane == 0) {
+                const int2 w = rl_join_again(a.words + RL_AT_LISTS + (layer + 1) * RL_LIST, V);
+                place[0] = w.x;
+                place[1] = w.y;
+            }
+            new_list();
+        }
     }
+}
+
+template <int DS, bool FULL>
+__global__ __launch_bounds__(RL_THREADS) void resident_layers_kernel(const ResidentArgs) {
+    RlArgs& a = *(RlArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    extern __shared__ __attribute__((aligned(128))) char smem[];
+    int* place = (int*)(smem + RL_X_BYTES + RL_STREAMERS * RL_STAGE + 2 * RL_SUMS * 16);
+    int* first = place + 16;
+    RlPlan* plan = (RlPlan*)(first + 32);
+    if (threadIdx.x == 0) {
+        const RlPlace w = rl_join(a.words, a.n_layers, a.start_polls, a.seal_polls);
+        place[0] = w.v;
+        place[1] = w.V;
+        place[2] = w.layer;
+    }
+    lds_barrier();
+    const int v = rl_same(place[0]), V = rl_same(place[1]), first_layer = rl_same(place[2]);
+    if (v < 0) return;
+    if (threadIdx.x < 5) rl_make_plan(a, plan, threadIdx.x, gridDim.x);
+    if (rl_same(threadIdx.x >> 6) == 1) rl_make_shares(a, first, threadIdx.x & 63);
+    lds_barrier();
+    if (V == (int)gridDim.x && first_layer == 0) rl_work<DS, FULL, true>(a, smem, v, V, 0);
+    else rl_work<DS, FULL, false>(a, smem, v, V, first_layer);
 }
 
 __global__ __launch_bounds__(256) void resident_zero_kernel(int* words, int n) {
@@ -1103,8 +1202,8 @@ extern "C" int gfa_resident_layers_bf16(const FewRowLayer* layers, int n_layers,
     a.pad = rl_rows_kept(s.M);
     a.gate_mode = s.gate_mode;
     a.scale_log2 = s.scale * 1.4426950408889634f;
-    a.start_polls = start_polls > 0 ? start_polls : 1000;
-    a.seal_polls = 200;
+    a.start_polls = start_polls > 0 && start_polls < 1000 ? start_polls : 1000;
+    a.seal_polls = a.start_polls < 100 ? 2 * a.start_polls : 200;
     a.words = (int*)s.work;
     a.work = (char*)s.work + rl_word_bytes(s.M, s.Hkv);
     rl_lay_out(a, units);

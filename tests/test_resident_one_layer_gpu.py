@@ -44,19 +44,27 @@ def _problem(D, H, G, hd, inner, held, new, window=0, rot=None, seed=0, extra_pa
     return p
 
 
+def _layer(p):
+    """The layer with a cache of its own in the kernels' order."""
+    from gpt_fast_amd.ops import few_row_layers as F
+    return F.Layer(p.wqkv, p.wo, p.w13, p.w2, p.norm_mixer, p.norm_ffn, *util.to_cache_order(p.keys, p.values), p.table)
+
+
+def _resident(p, layers, stream, **options):
+    from gpt_fast_amd.ops import resident_layers as R
+    R.run(layers, stream, p.freqs, p.rot, p.batch, p.H, p.G, p.hd, p.window, EPS, EPS, p.scale, "silu", **options)
+
+
 def _run(p, way, **options):
     """(the stream behind the layer, its keys and values as [page, G, slot, d] and [page, G, d, slot])."""
     from gpt_fast_amd.ops import few_row_layers as F
-    from gpt_fast_amd.ops import resident_layers as R
-    k_pages, v_pages = util.to_cache_order(p.keys, p.values)
-    layer = F.Layer(p.wqkv, p.wo, p.w13, p.w2, p.norm_mixer, p.norm_ffn, k_pages, v_pages, p.table)
-    stream = p.residual.clone()
+    layer, stream = _layer(p), p.residual.clone()
     if way == "resident":
-        R.run([layer], stream, p.freqs, p.rot, p.batch, p.H, p.G, p.hd, p.window, EPS, EPS, p.scale, "silu", **options)
+        _resident(p, [layer], stream, **options)
     else:
         x = stream * (stream.square().mean(1, keepdim=True) + EPS).rsqrt() * p.norm_mixer
         F.run_layers([layer], x.bfloat16(), stream, p.freqs, p.rot, p.batch, p.H, p.G, p.hd, p.window, EPS, EPS, p.scale, "silu")
-    return (stream,) + util.from_cache_order(k_pages, v_pages)
+    return (stream,) + util.from_cache_order(layer.k_pages, layer.v_pages)
 
 
 # head size, heads, key/value heads, window, the newest token's position; the keys that are no numbers: all that a wave sees, the
@@ -78,3 +86,36 @@ def test_a_part_of_a_context_that_is_no_number_makes_the_row_no_number(hd, H, G,
     got = _run(p, way)[0]
     assert bool(torch.isnan(got[0]).all())
     assert torch.equal(got[1], want[1])
+
+
+def test_a_launch_that_begins_on_a_busy_chip_has_the_rest_of_it_once_it_is_free():
+    """32 layers of 4,096 beside two, then four, launches of as many that leave them eight compute units: they
+    stay with the eight for a layer, not to their end, which would take 32 times as long as on the whole chip; and what they
+    compute has the same bits."""
+    p = _problem(4096, 32, 8, 128, 14336, [200, 31], [1, 1])
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    mine_layers, other_layers = ([_layer(p) for _ in range(32)] for _ in range(2))      # one set of weights, a cache each
+    mine, others = torch.cuda.Stream(), torch.cuda.Stream()
+    other_rows = p.residual.clone()
+
+    def timed(**options):
+        stream = p.residual.clone()
+        torch.cuda.synchronize()
+        begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        for _ in range(options.pop("beside", 0)):
+            with torch.cuda.stream(others):
+                _resident(p, other_layers, other_rows, workgroups=units - 8)
+        with torch.cuda.stream(mine):
+            begin.record()
+            _resident(p, mine_layers, stream, **options)
+            end.record()
+        torch.cuda.synchronize()
+        return stream, begin.elapsed_time(end)
+    timed()
+    want, alone = timed()
+    assert bool(torch.isfinite(want).all())
+    for beside in (2, 4):
+        got, took = timed(beside=beside, start_polls=1)
+        print(f"alone {alone:.2f} ms, beside {beside} launches {took:.2f} ms", flush=True)
+        assert torch.equal(got, want)
+        assert took < 8 * alone
