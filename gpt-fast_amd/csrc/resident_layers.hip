@@ -99,7 +99,9 @@ struct ResidentArgs {
     int* words;                           // zero at the start: RlWords below
     char* work;                           // per layer work_stride bytes: the buffers below
     size_t work_stride;
-    unsigned off_q, off_po, off_pml;
+    unsigned off_q;
+    size_t off_po, off_pml;               // sums of the contexts' shares, behind the layers' buffers: one place for all layers,
+                                          // read past the caches, written again only when the layer that read them is complete
     int n_layers, M, D, I, H, Hkv, hd, rot, table_stride, window, pad, gate_mode;
     int start_polls, seal_polls;          // polls before the list of workers is closed, and then the first layer's
     float scale_log2;
@@ -596,8 +598,8 @@ __device__ __forceinline__ bool rl_join_heads(const Args& a, char* work, const R
     if (shared) {
         // [item][R][hd] and [item][R][2], this lane's dims of its head
         const int row = li < R ? li : 0;
-        float* po = (float*)(work + a.off_po);
-        float* pml = (float*)(work + a.off_pml);
+        float* po = (float*)(a.work + a.off_po);
+        float* pml = (float*)(a.work + a.off_pml);
         if (it.splits > 1 && li < R) {
 #pragma unroll
             for (int q = 0; q < DQ; ++q)
@@ -1118,11 +1120,12 @@ static int rl_units() {
     return units;
 }
 
-// The buffers of a launch: sizes and places.  Returns the bytes of all of them.
+// The buffers of a launch: sizes and places.  Returns the bytes of all of them: 32 layers of the 8B shape 3 MB at 1 row, 19 at 8 (36 and
+// 52 with partial sums in every layer).
 static size_t rl_lay_out(ResidentArgs& a, int units) {
     const size_t pad = a.pad, D = a.D, heads = (size_t)a.H * a.hd;
     size_t off = 0;
-    auto take = [&](size_t bytes) { const size_t at = off; off = (off + bytes + 255) / 256 * 256; return (unsigned)at; };
+    auto take = [&](size_t bytes) { const size_t at = off; off = (off + bytes + 255) / 256 * 256; return at; };
     a.off_in[0] = take(pad * D * 2);
     a.off_sums[0] = take((D + 3) / 4 * pad * 4);
     a.off_q = take((size_t)a.M * heads * 2);
@@ -1130,17 +1133,18 @@ static size_t rl_lay_out(ResidentArgs& a, int units) {
     a.off_in[3] = take(pad * D * 2);
     a.off_sums[3] = take((D + 3) / 4 * pad * 4);
     a.off_in[4] = take(pad * (size_t)a.I * 2);
-    const long pairs = (long)a.M * a.Hkv, of_token = (a.table_stride * 2 + RL_SHARE - 1) / RL_SHARE;
-    const long most = 2l * (units > pairs ? units : pairs);
-    const size_t partials = of_token > 1 ? (most < pairs * of_token ? most : pairs * of_token) * (a.H / a.Hkv) : 0;
-    a.off_po = take(partials * a.hd * 4);
-    a.off_pml = take(partials * 2 * 4);
     a.work_stride = off;
     a.off_out[2] = a.off_in[3];
     a.off_share[2] = a.off_sums[3];
     a.off_out[4] = (unsigned)off + a.off_in[0];
     a.off_share[4] = (unsigned)off + a.off_sums[0];
-    return off * a.n_layers;
+    off *= a.n_layers;
+    const long pairs = (long)a.M * a.Hkv, of_token = (a.table_stride * 2 + RL_SHARE - 1) / RL_SHARE;
+    const long most = 2l * (units > pairs ? units : pairs);
+    const size_t partials = of_token > 1 ? (most < pairs * of_token ? most : pairs * of_token) * (a.H / a.Hkv) : 0;
+    a.off_po = take(partials * a.hd * 4);
+    a.off_pml = take(partials * 2 * 4);
+    return off;
 }
 
 static size_t rl_word_bytes(int M, int Hkv) { return ((size_t)(RL_AT_SPLITS + M * Hkv) * 4 + 255) / 256 * 256; }

@@ -119,3 +119,17 @@ def test_a_launch_that_begins_on_a_busy_chip_has_the_rest_of_it_once_it_is_free(
         print(f"alone {alone:.2f} ms, beside {beside} launches {took:.2f} ms", flush=True)
         assert torch.equal(got, want)
         assert took < 8 * alone
+
+
+def test_the_work_memory_holds_the_partial_sums_of_one_layer():
+    """8B shape, 8 rows: 32 layers' rows and one set of partial sums, which 64 pages of table allow two a compute unit of."""
+    import ctypes
+    from gpt_fast_amd.ops.library import library
+    size = library("resident_layers").gfa_resident_work_bytes
+    size.restype = ctypes.c_long
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    sizes = [size(n, 8, 4096, 14336, 32, 8, 128, 64) for n in (1, 2, 32)]
+    assert sizes[2] - sizes[1] == 30 * (sizes[1] - sizes[0])
+    partials = 2 * max(units, 64) * 4 * (128 + 2) * 4
+    rows = 8 * (2 * (3 * 4096 + 2 * 4096 + 14336) + 2 * 4096)         # x of four products, q, shares of the squares at one for four
+    assert sizes[1] - sizes[0] < 1.1 * rows and sizes[0] < 1.1 * (rows + partials) + 65536
