@@ -64,6 +64,7 @@
 #define RL_LINE 64                    // ints from one counter to the next
 #define RL_NOWHERE 0xfffff000u        // an offset behind every matrix: reads as zero
 #define RL_MOST_BYTES 0xffff0000l
+#define RL_MOST_COLUMNS (1 << 23)     // of a row of x: sixteen of them, and all buffers of a layer, have 32-bit offsets
 
 typedef unsigned int rl_u4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_t;
@@ -1176,7 +1177,7 @@ extern "C" int gfa_resident_layers_bf16(const FewRowLayer* layers, int n_layers,
     if (n_layers <= 0 || n_layers > RL_MAX_LAYERS || s.M <= 0 || s.M > RL_MAX_ROWS || s.D <= 0 || s.D % 8 || s.I <= 0 || s.I % 8 ||
         s.H <= 0 || s.Hkv <= 0 || s.H % s.Hkv || s.H / s.Hkv > 16 || s.hd <= 0 || s.hd % 16 || s.hd > 128 || s.rot < 0 || s.rot % 2 ||
         s.rot > s.hd || s.table_stride <= 0 || (s.gate_mode != 3 && s.gate_mode != 6) || units <= 0 ||
-        (long)s.D * s.I * 4 >= RL_MOST_BYTES || (long)s.D * (s.H + 2 * s.Hkv) * s.hd * 2 >= RL_MOST_BYTES)
+        s.D >= RL_MOST_COLUMNS || s.I >= RL_MOST_COLUMNS || (long)s.H * s.hd >= RL_MOST_COLUMNS || (long)s.D * s.I * 4 >= RL_MOST_BYTES || (long)s.D * (s.H + 2 * s.Hkv) * s.hd * 2 >= RL_MOST_BYTES)
         return (int)hipErrorInvalidValue;
     ResidentArgs a = {};
     for (int i = 0; i < n_layers; ++i) {

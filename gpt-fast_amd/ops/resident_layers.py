@@ -12,6 +12,7 @@ from .library import KernelError, check, library, require_contiguous, require_de
 MAX_ROWS = 16
 X_BYTES = 88 * 1024          # of shared memory for the rows that a product multiplies (RL_X_BYTES)
 MOST_BYTES = 0xffff0000      # of one matrix: offsets into it are 32-bit
+MOST_COLUMNS = 1 << 23       # of a row of x: so are those into a layer's rows
 
 _p, _i = ctypes.c_void_p, ctypes.c_int
 
@@ -20,7 +21,7 @@ def takes(n_rows: int, dim: int, hidden: int, n_heads: int, n_kv_heads: int, hea
     """Whether the kernel computes such layers at all."""
     return (0 < n_rows <= MAX_ROWS and dim % 8 == 0 and hidden % 8 == 0 and head_dim % 16 == 0 and head_dim <= 128
             and n_heads % n_kv_heads == 0 and n_heads // n_kv_heads <= 16 and rotary_dim % 2 == 0
-            and 0 < rotary_dim <= head_dim and 4 * dim * hidden < MOST_BYTES
+            and 0 < rotary_dim <= head_dim and max(dim, hidden, n_heads * head_dim) < MOST_COLUMNS and 4 * dim * hidden < MOST_BYTES
             and 2 * dim * (n_heads + 2 * n_kv_heads) * head_dim < MOST_BYTES)
 
 

@@ -176,3 +176,11 @@ def test_what_the_kernel_takes_and_what_begins_where_it_reads():
     assert R.aligned([SimpleNamespace(**whole)] * 2, residual) and not R.aligned([SimpleNamespace(**whole)], residual[1:])
     for n in names:
         assert not R.aligned([SimpleNamespace(**whole), SimpleNamespace(**{**whole, n: whole[n][1:]})], residual), n
+
+
+def test_rows_whose_offsets_do_not_fit_into_32_bits_are_not_taken():
+    """Sixteen rows of 2^27 - 8 columns are 2^32 - 256 bytes: what lies behind them in a layer's buffers is out of reach."""
+    from gpt_fast_amd.ops import resident_layers as R
+    assert R.takes(16, 8, (1 << 23) - 8, 8, 1, 16, 2)
+    assert not R.takes(16, 8, 1 << 23, 8, 1, 16, 2) and not R.takes(16, 8, (1 << 27) - 8, 8, 1, 16, 2)
+    assert not R.takes(16, 8, 8, 1 << 19, 1 << 19, 16, 2)
