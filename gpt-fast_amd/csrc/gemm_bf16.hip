@@ -253,7 +253,7 @@ struct SkinnyExtra {
     int table_stride, H, Hkv, hd, rot;
     // A norm spread over two kernels (one tile of rows).  The kernel that completes the
     // residual stream (MODE 2) also writes xg_out = bfloat16(new residual * next_g) (chunked) and
-    // ssq_out [gfa_skinny_workgroups(2, M, N), share_rows]: each workgroup's share of its rows' sums of squares (float,
+    // ssq_out [gfa_skinny_workgroups(2, M, N, K), share_rows]: each workgroup's share of its rows' sums of squares (float,
     // from the float residual).  The next product takes xg as its x, adds the shares in a fixed
     // order (ssq_in [t_in, share_rows]) and scales its result by rsqrt(sum / K + eps): a factor per row
     // commutes with the product, so this is the RMS norm of model.py:236-241.
@@ -722,30 +722,41 @@ static int pick_tile_rows(int N, int step, int nt, int x_rows) {
 // against the same x already: with two tiles of each, 242 registers, the step at sixteen rows
 // lost 5 % (8B and 70B shapes) although the kernel alone gained 3 %.
 //
-// Up to 16 rows of x also where single tiles of 16 would go on the chip a second time and pairs of lower ones do not.  Single
-// and pairs, us: 4608 x 4096 4 rows of x 10.8, 9.5; 8 10.9, 9.6; 16 14.4, 11.2; 5120 x 4096 11.1, 9.9; 11.0, 10.1; 14.4,
-// 11.7; 5632 x 4096 11.0, 11.2; 11.2, 10.7; 14.6, 12.2; 6176 x 4096 11.5, 11.7; 11.7, 11.2; 14.7, 12.7; 5120 x 7168 16.9,
-// 14.4; 17.3, 15.1; 22.5, 17.5.  Twice: 9216 x 4096, 16 rows 20.0, 18.1; 8 rows 15.5, 15.3.  With 4096 columns, one round
-// either way, 7.9, 9.1; 8.2, 9.2; 9.5, 10.7.
-static int tiles_per_workgroup(int mode, int M, int N) {
+// Up to 16 rows of x also where single tiles of 16 would go on the chip a second time and pairs of lower ones do not, as far as
+// the columns of W are long enough for what a pair takes longer to begin and to end.  Single tiles and pairs, us:
+//   4608 rows x 4096, 4 rows of x 10.1, 9.6; 8 10.9, 9.6; 9 11.7, 10.3; 16 14.3, 11.3; 5120 x 8192 17.1, 16.0; 19.0, 16.8; 16 24.5, 19.1
+//   13..16 rows: 4608 x 512 4.7, 4.6; x 1024 6.1, 5.7; x 2048 9.0, 8.0
+//   9..12, 9 and 12: x 1536 6.5, 6.5; 6.8, 6.7, 5632 x 1536 6.6, 6.9; 6.9, 7.1; 4608 x 3072 9.8, 8.7; 10.7, 9.2
+//   5..8, 6 and 8: x 1536 5.9, 6.2; 6.2, 6.2; 5120 x 1536 5.9, 6.3; 6.1, 6.4; x 3072 9.0, 8.4; 9.3, 8.7
+//   2..4, 2 and 4: x 1536 5.8, 6.2; 5.7, 6.1; 5120 x 3072 8.7, 9.0; 8.5, 8.5; x 4096 10.6, 10.6; 10.4, 10.0; 5376 x 4096 10.6, 10.9;
+//   10.4, 10.3
+// With the rotation behind them pairs take longer to end: 5120 x 4096 4 rows 11.1, 11.6; 8 12.0, 12.1; 9 12.9, 13.1; 10 13.4, 13.1; 16 15.0, 14.0;
+// x 2048 8 rows 8.2, 8.9; 14 9.3, 9.6; 4608 x 8192 4 rows 16.8, 17.6; 16 24.1, 20.9.
+// From 24 rows of W per compute unit on, two rounds either way, up to 8 rows: 6144 x 4096 8 rows 11.2, 11.3; 7168 11.9, 12.3; 8192 12.7, 14.7; into
+// the stream 13.2, 15.4.  With 4096 rows of W, one round either way, 7.9, 9.1; 8.2, 9.2; 16 rows 9.5, 10.7.
+static int tiles_per_workgroup(int mode, int M, int N, int K) {
     const int cus = compute_units();
     if (IS_GATE(mode)) return 1;
-    if (M <= 16) return N > 16 * cus && (M > 8 || N < (M > 4 ? 24 : 22) * cus) ? 2 : 1;
+    if (M <= 16 && N < 24 * cus) {
+        if (N <= 16 * cus) return 1;
+        if (mode == 4) return M > 9 && K >= 4096 ? 2 : 1;
+        return K >= (M > 12 ? 0 : M > 8 ? 2048 : M > 4 ? 3072 : 4096) && (M > 4 || N <= 20 * cus) ? 2 : 1;
+    }
     // 33..48 rows: only where the registers hold it (the plain epilogues)
     const int most = (mode == 2 || mode == 4) ? 32 : 48;
-    return M <= most && N >= 24 * cus ? 2 : 1;
+    return M > 8 && M <= most && N >= 24 * cus ? 2 : 1;
 }
 
 // Tile height the launcher below uses for this mode, these rows of x and this width.
-static int tile_rows(int mode, int M, int N) {
-    return pick_tile_rows(N, (mode == 2 || mode == 4) ? 4 : 1, tiles_per_workgroup(mode, M, N), M > 8 ? 16 : M > 4 ? 8 : 4);
+static int tile_rows(int mode, int M, int N, int K) {
+    return pick_tile_rows(N, (mode == 2 || mode == 4) ? 4 : 1, tiles_per_workgroup(mode, M, N, K), M > 8 ? 16 : M > 4 ? 8 : 4);
 }
 
-// Workgroups the launcher below starts for this mode, M <= 16 rows of x and N columns (the
+// Workgroups the launcher below starts for this mode, M <= 16 rows of x and a matrix of [N, K] (the
 // two-kernel norm's shares are one record per workgroup of mode 2, so its callers size
 // their buffers by it).
-extern "C" int gfa_skinny_workgroups(int mode, int M, int N) {
-    const int per = (M <= 16 ? tile_rows(mode, M, N) : 16) * tiles_per_workgroup(mode, M, N);
+extern "C" int gfa_skinny_workgroups(int mode, int M, int N, int K) {
+    const int per = (M <= 16 ? tile_rows(mode, M, N, K) : 16) * tiles_per_workgroup(mode, M, N, K);
     return (N + per - 1) / per;
 }
 
@@ -755,8 +766,8 @@ static int launch_skinny_mfma(const bf16_t* x, const bf16_t* w, void* out, int M
     const int ct = (M + 15) / 16;
     // the epilogues that add into the residual stream or rotate pairs work on groups of
     // four columns: their tiles are 8, 12 or 16 rows high
-    const int nt = tiles_per_workgroup(MODE, M, N);
-    const int th = ct == 1 ? tile_rows(MODE, M, N) : 16;
+    const int nt = tiles_per_workgroup(MODE, M, N, K);
+    const int th = ct == 1 ? tile_rows(MODE, M, N, K) : 16;
     const int tiles = (N + th * nt - 1) / (th * nt);     // workgroups
     const int RT = (IS_GATE(MODE)) ? 2 : nt;                 // tiles of W staged per wave
     const int pieces = (K + SM_SUBK - 1) / SM_SUBK;
@@ -884,7 +895,7 @@ extern "C" int gfa_qkv_rope_store_bf16(const void* x, const float* ssq_in, int t
 // residual [M, N] += x w^T for up to 64 rows, and the first half of the norm that follows:
 // xg_out = bfloat16(new residual * next_g), kept chunked ([N / 8][share_rows][8], see
 // chunked_elem), ssq_out [tiles, share_rows] = the workgroups' shares of the rows' sums of
-// squares, tiles = gfa_skinny_workgroups(2, M, N); share_rows = gfa_share_rows(M).
+// squares, tiles = gfa_skinny_workgroups(2, M, N, K); share_rows = gfa_share_rows(M).
 // N a multiple of 8.  x_chunked: x is kept chunked too (pad gfa_share_rows(M)), as the gate
 // of gfa_skinny_after_chain_bf16 leaves its result on request.
 extern "C" int gfa_skinny_into_chain_bf16(const void* x, int x_chunked, const void* w,
@@ -957,17 +968,20 @@ extern "C" int gfa_skinny_bf16(const void* x, const void* w, void* out, int M, i
 
 struct FewRowWork {
     size_t q, y, xa, sa, h, xb, sb, po, pml, bytes;
+    int records_a, records_b;             // of sa, behind the output projection, and of sb, behind the feed-forward
     FewRowWork(int M, int D, int I, int H, int hd, int splits) {
-        const size_t pad = gfa_share_rows(M), heads = (size_t)H * hd, records = gfa_skinny_workgroups(2, M, D);
+        const size_t pad = gfa_share_rows(M), heads = (size_t)H * hd;
+        records_a = gfa_skinny_workgroups(2, M, D, H * hd);
+        records_b = gfa_skinny_workgroups(2, M, D, I);
         size_t at = 0;
         auto take = [&](size_t n) { const size_t o = at; at += (n + 255) / 256 * 256; return o; };
         q = take((size_t)M * heads * 2);
         y = take(pad * heads * 2);
         xa = take(pad * D * 2);
-        sa = take(records * pad * 4);
+        sa = take(records_a * pad * 4);
         h = take(pad * (size_t)I * 2);
         xb = take(pad * D * 2);
-        sb = take(records * pad * 4);
+        sb = take(records_b * pad * 4);
         po = take(splits > 1 ? (size_t)splits * M * heads * 4 : 0);
         pml = take(splits > 1 ? (size_t)splits * M * H * 2 * 4 : 0);
         bytes = at;
@@ -986,7 +1000,7 @@ extern "C" int gfa_few_row_layers_bf16(const FewRowLayer* layers, int n_layers, 
         return (int)hipErrorInvalidValue;
     const FewRowWork at(s.M, s.D, s.I, s.H, s.hd, s.n_splits);
     char* w = (char*)s.work;
-    const int records = gfa_skinny_workgroups(2, s.M, s.D), inner = s.H * s.hd;
+    const int inner = s.H * s.hd;
     // one token for each sequence and a group that fits one tile: the heads' results stay chunked
     const int chunked = !s.rows_tiled && s.one_token_each && s.max_tiles == 1;
     const void* x = s.x0;
@@ -1009,7 +1023,7 @@ extern "C" int gfa_few_row_layers_bf16(const FewRowLayer* layers, int n_layers, 
                                         (float*)(w + at.sa), stream);
         if (rc) break;
         const bool last = l + 1 == n_layers;               // nothing takes halves: plain rows, as for any product
-        rc = gfa_skinny_after_chain_bf16(w + at.xa, (const float*)(w + at.sa), records, s.eps_ffn, L.w13, w + at.h, s.M, s.I,
+        rc = gfa_skinny_after_chain_bf16(w + at.xa, (const float*)(w + at.sa), at.records_a, s.eps_ffn, L.w13, w + at.h, s.M, s.I,
                                          s.D, s.I, s.gate_mode, s.I, !last, stream);
         if (rc) break;
         if (!last) {
@@ -1022,7 +1036,7 @@ extern "C" int gfa_few_row_layers_bf16(const FewRowLayer* layers, int n_layers, 
         }
         x = w + at.xb;
         ssq = (const float*)(w + at.sb);
-        shares = records;
+        shares = at.records_b;
     }
     return rc;
 }

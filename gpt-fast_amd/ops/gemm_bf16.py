@@ -154,7 +154,7 @@ def skinny_into_chain(x, w: torch.Tensor, residual: torch.Tensor, next_g: torch.
     if N % 8 or K % 8:                                   # up to MAX_ROWS rows: checked above
         raise KernelError(f"skinny_into_chain: [{M}, {K}] x [{N}, {K}] is outside this kernel")
     xg = ChunkedRows(M, N, w.device)
-    records = library("gemm_bf16").gfa_skinny_workgroups(_i(2), _i(M), _i(N))   # one per workgroup
+    records = library("gemm_bf16").gfa_skinny_workgroups(_i(2), _i(M), _i(N), _i(K))   # one per workgroup
     ssq = torch.empty((records, share_rows(M)), dtype=torch.float32, device=w.device)
     check(library("gemm_bf16").gfa_skinny_into_chain_bf16(
         ptr(x.data if chunked else x), _i(int(chunked)), ptr(w), ptr(residual), _i(M), _i(N), _i(K),

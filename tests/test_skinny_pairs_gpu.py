@@ -85,3 +85,60 @@ def test_rotation_and_cache_write(heads, kv_heads, M):
         page = int(table[0, p // 64])
         _close(keys[page, :, p % 64], want[m, heads:heads + kv_heads], K, True)
         _close(values[page, :, :, p % 64], want[m, heads + kv_heads:], K, True)
+
+
+# pairs are a matter of long columns where the rows of x are few: (rows of x, columns of W) on both sides of each line
+LINES = [(2, 4096), (4, 4096), (4, 4088), (5, 3072), (8, 3064), (9, 2048), (12, 2040), (13, 64), (9, 4096), (10, 4088), (10, 4096)]
+
+
+def _within(got, want, x, w, rounded):
+    """Sums of K products in float32, in any order: within K 2^-24 of the sum of their magnitudes."""
+    bound = x.shape[1] * 2 ** -24 * (x.float().abs() @ w.float().abs().t()) + (2 ** -8 * want.abs() if rounded else 0)
+    assert bool(((got.double() - want.double()).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("per_unit", [17, 19.5, 20, 21.5, 23.5])
+@pytest.mark.parametrize("M,K", LINES)
+def test_both_sides_of_every_line(M, K, per_unit):
+    from gpt_fast_amd.ops import gemm_bf16 as G
+    N = _width(per_unit, 64)
+    g = torch.Generator(device=DEV).manual_seed(N + M)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = torch.randn(N, K, generator=g, device=DEV).bfloat16()
+    want = x.float() @ w.float().t()
+    _within(G.skinny(x, w, out_dtype=torch.float32), want, x, w, False)
+    residual, weight = torch.randn(M, N, generator=g, device=DEV), 1 + 0.1 * torch.randn(N, generator=g, device=DEV)
+    stream = residual + want
+    xg, ssq = G.skinny_into_chain(x, w, residual, weight)
+    _within(residual, stream, x, w, True)
+    assert util.rel_err(ssq.sum(0)[:M], stream.square().sum(1)) < 2 ** -10
+    hd, kv_heads = 64, 4
+    heads = N // hd - 2 * kv_heads
+    pos = (torch.arange(M, device=DEV) * 5 + 3).int()
+    seq = torch.zeros(M, dtype=torch.int32, device=DEV)
+    table = torch.tensor([[2, 0]], dtype=torch.int32, device=DEV)
+    k_pages = torch.zeros(3, kv_heads, 64, hd, dtype=torch.bfloat16, device=DEV)
+    v_pages = torch.zeros(3, kv_heads, hd, 64, dtype=torch.bfloat16, device=DEV)
+    freqs = torch.zeros(hd // 2, device=DEV)                          # no turn: the projection itself
+    q = G.qkv_rope_store(x, w, freqs, seq, pos, table, k_pages, v_pages, heads, kv_heads, hd, hd)
+    _within(q.view(M, -1), want[:, :heads * hd], x, w[:heads * hd], True)
+    keys, values = util.from_cache_order(k_pages, v_pages)
+    at = (table[0, pos.long() // 64].long(), pos.long() % 64)
+    got = torch.cat([keys[at[0], :, at[1]].reshape(M, -1), values[at[0], :, :, at[1]].reshape(M, -1)], 1)
+    _within(got, want[:, heads * hd:], x, w[heads * hd:], True)
+
+
+def test_where_pairs_begin():
+    """One workgroup a tile of at least twelve rows of W, or a pair: fewer than a round of the chip."""
+    import ctypes
+    from gpt_fast_amd.ops.library import library
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    workgroups, i = library("gemm_bf16").gfa_skinny_workgroups, ctypes.c_int
+
+    def pairs(mode, M, K, per_unit):
+        return workgroups(i(mode), i(M), i(_width(per_unit)), i(K)) <= units
+    for M, K in ((4, 4096), (8, 3072), (12, 2048), (16, 8)):
+        assert pairs(0, M, K, 18) and pairs(2, M, K, 18) and (M > 8 or not pairs(0, M, K, 24.1))
+        assert K == 8 or not pairs(0, M, K - 8, 18)
+    assert not pairs(0, 4, 4096, 20.5) and pairs(0, 5, 4096, 20.5)
+    assert pairs(4, 10, 4096, 18) and not pairs(4, 9, 4096, 18) and not pairs(4, 16, 4088, 18)
