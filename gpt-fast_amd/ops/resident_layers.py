@@ -26,26 +26,45 @@ def takes(n_rows: int, dim: int, hidden: int, n_heads: int, n_kv_heads: int, hea
 
 
 def pays(n_layers: int, n_rows: int, n_seqs: int, table_pages: int, dim: int, hidden: int, n_heads: int, n_kv_heads: int,
-         head_dim: int, units: int) -> bool:
+         head_dim: int, units: int, window: int = 0) -> bool:
     """Whether one launch that stays on its ``units`` compute units takes less time than five launches a layer
-    (ops.few_row_layers), both measured on 256 units, in us a step (this side when its phases met through 16 counters, not 128:
-    2 to 9 % longer than now):
+    (ops.few_row_layers), both measured on 256 units, in us for the layers alone, 200 keys a row where nothing else is said
+    (some 1,800 steps of 31 shapes):
 
-    - From 8 layers on: meeting at the start costs what some layers give.  768 wide, 1 row: 3 layers 118 -> 130, 6 layers
-      190 -> 190, 12 layers 333 -> 306; 288 wide, 8 layers 215 -> 204; 4096 wide (8B) 2 layers 373 -> 380, 4 layers 554 -> 542,
-      8 layers 895 -> 851, 32 layers 2990 -> 2740.
+    - From 8 layers on: meeting at the start costs what some layers give.  1 row and 8 rows: 288 wide, 2 layers 51 -> 66, 54 -> 65;
+      5 layers 118 -> 119, 122 -> 118; 8 layers 184 -> 169, 192 -> 172; 768 wide 4 layers 106 -> 108, 112 -> 112; 8 layers 205 -> 185,
+      225 -> 194; 8B 3 layers 266 -> 258, 276 -> 282; 8 layers 701 -> 642, 718 -> 699; 70B 10 layers 3051 -> 2772, 3044 -> 2960.
+      Five to seven layers of most shapes would gain 1 to 8 % too.
     - More than 8 rows only where those of the widest product fit the two halves of their shared memory one after
-      the other.  12 rows: 768 wide 400 -> 370, 2048 wide (5632 inner) 577 -> 558, 3072 (8192) 828 -> 873, 8B 3365 -> 3646.
-    - As many pairs of a row and a key/value head as units at most: 6656 wide, 52 heads, 12 layers: 4 rows 2366 -> 2329, 8 rows
-      2506 -> 2696.
-    - One or two sequences with one new token each, up to 12288 keys: attention that has the chip to itself then
-      reads the cache at 5.1 TB/s, beside waves that hold weights at 3.6.  8B, 1 row: 6000 keys 3240 -> 3149, 12000 keys
-      3359 -> 3347, 30000 keys 3755 -> 3827.  Several new tokens of a sequence pay at any length: 8 behind 6000 keys
-      10300 -> 3710; so do more sequences: 4 of 15000 keys 4470 -> 4343, 8 of which one has 16000 4310 -> 3740."""
+      the other.  12 layers of 12 rows: 768 wide 358 -> 290, 2048 wide (5632 inner) 514 -> 466, 3072 (8192) 754 -> 778,
+      8B 1199 -> 1288, 5120 (13824) 1836 -> 2210.
+    - As many pairs of a row and a key/value head as units at most.  12 layers 5120 wide, 40 such heads: 6 rows 1638 -> 1594, 8 rows
+      1692 -> 1674; 10 layers 6656 wide, 52 heads: 4 rows 1963 -> 1858, 5 rows 2063 -> 2195.
+    - One or two sequences with one new token each, up to 12288 keys.  12 layers of 8B, 1 row: 12000 keys 1210 -> 1169, 30000
+      keys 1381 -> 1367, 1 %, which is less than two machines differ by.
+    - One new token for each sequence: up to 4608 keys, and of all rows' and heads' blocks of 32 keys no more than 24 a unit.  Attention by three
+      waves of a workgroup has fewer keys under way than a launch of its own, and from some length on that costs more
+      than the meetings save.  12 layers, 4000, 6000 and 12000 keys: 1024 wide, 4 kv heads of 128, 1 row 387 -> 354, 396 -> 380, 437 -> 459; heads of 32,
+      1 row, 3500 and 5000 keys 346 -> 322, 341 -> 354.  768 wide, heads of 64 (12 blocks a unit with 8 rows of 1000 keys): 8 rows of 1000, 2000, 6000 keys
+      420 -> 357, 504 -> 447, 724 -> 749; 16 rows of 500, 1500 and 5000 keys 388 -> 352, 494 -> 523, 831 -> 1180; 512 wide, heads of 32, 16 rows
+      of 1500 keys 411 -> 485.  All contexts are taken to be as long as the table: which are shorter is known on the device
+      only, and may change from replay to replay.  (One long context among short ones gains: 768 wide, 8 rows, one of 6000 keys 450 -> 376.)
+      With a window the keys are the window's: 768 wide, 8 rows of 10000 keys, window 1024 420 -> 357, 4096 619 -> 623.
+    - But for heads of 128, eight or more of keys and values: at any length: 8B, 8 rows of 20000 keys 2438 -> 2329; a 7B shape, 8 rows of 16000
+      5403 -> 5160, 4 rows of 30000 4988 -> 4825.  Blocks of such heads are large enough.  Four of them: 1 row of 30000 keys
+      10 to 16 % slower.
+    - Several new tokens of a sequence pay at any length, since the attention of prompts has too few workgroups there: 2048 wide, 8 behind 6000
+      keys 1211 -> 511; 768 wide, 15 rows of 5000 keys and one more for one of them 2249 -> 1164."""
     widest = max(dim, hidden, n_heads * head_dim)
+    keys = table_pages * PAGE
+    if window > 0:
+        keys = min(keys, window)
+    one_each = n_rows <= n_seqs
+    few_keys = keys <= 4608 and n_rows * n_kv_heads * -(-keys // 32) <= 24 * units
+    large_blocks = head_dim == 128 and n_kv_heads >= 8 and (n_rows > 2 or keys <= 12288)
     return (n_layers >= 8 and n_rows * n_kv_heads <= units
             and (n_rows <= 8 or 2 * MAX_ROWS * widest <= 2 * X_BYTES)
-            and (n_rows > 2 or n_rows > n_seqs or table_pages * PAGE <= 12288))
+            and (not one_each or few_keys or large_blocks))
 
 
 def aligned(layers, residual) -> bool:

@@ -106,7 +106,7 @@ class FewRowRuns:
         p, sizes = m.position, (m.dim, f.hidden, m.n_heads, m.n_kv_heads, m.head_dim)
         if self.dtype == torch.bfloat16 and R.takes(batch.n_tokens, *sizes, p.rotary_dim) \
                 and R.pays(end - n, batch.n_tokens, batch.n_seqs, layers[0].table.shape[1], *sizes,
-                           A.compute_units(layers[0].w2.device)) \
+                           A.compute_units(layers[0].w2.device), first.mixer.window) \
                 and R.aligned(layers, stream.tensor):
             R.run(layers, stream.tensor, first.mixer.position.freqs, p.rotary_dim, batch, m.n_heads, m.n_kv_heads, m.head_dim,
                   first.mixer.window, first.mixer_norm.spec.eps, first.feed_forward_norm.spec.eps, first.mixer.scale,

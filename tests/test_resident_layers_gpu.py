@@ -184,3 +184,20 @@ def test_rows_whose_offsets_do_not_fit_into_32_bits_are_not_taken():
     assert R.takes(16, 8, (1 << 23) - 8, 8, 1, 16, 2)
     assert not R.takes(16, 8, 1 << 23, 8, 1, 16, 2) and not R.takes(16, 8, (1 << 27) - 8, 8, 1, 16, 2)
     assert not R.takes(16, 8, 8, 1 << 19, 1 << 19, 16, 2)
+
+
+def test_the_rule_on_long_contexts():
+    """Steps that took longer in one launch than in five a layer, and beside each one that did not."""
+    from gpt_fast_amd.ops import resident_layers as R
+
+    def pays(rows, keys, sizes, window=0, seqs=None):
+        return R.pays(12, rows, seqs or rows, -(-keys // 64), *sizes, 256, window)
+    small, heads_of_32 = (768, 2048, 12, 12, 64), (512, 1376, 16, 16, 32)
+    assert pays(8, 2000, small) and not pays(8, 4000, small)
+    assert pays(16, 900, small) and not pays(16, 1500, small) and not pays(16, 5000, small)
+    assert pays(8, 1500, heads_of_32) and not pays(16, 1500, heads_of_32) and not pays(1, 5000, heads_of_32)
+    assert not pays(3, 30000, (2048, 5632, 32, 4, 64)) and not pays(3, 30000, (2048, 5632, 16, 2, 128))
+    assert not pays(8, 3000, (2560, 6912, 32, 32, 80))
+    for rows in (3, 4, 8):
+        assert pays(rows, 30000, (4096, 14336, 32, 8, 128)) and pays(rows, 16000, (4096, 11008, 32, 32, 128))
+    assert pays(8, 30000, small, window=1024) and pays(8, 30000, small, seqs=7)
