@@ -32,9 +32,14 @@
 // another, longer the more loads are under way: with 8, 16, 32, 64, 128 counters a step of the 110M shape takes 323, 306, 293, 286,
 // 286 us at 1 row and 376, 352, 336, 321, 317 at 8 rows, of the 8B shape 2800, 2746, 2700, 2676, 2660 and 3084, 2998, 2952, 2917, 2896; lines of 128 and 512
 // bytes take as long as these of 256.  (256 workgroups that do nothing else meet in 1.3 us with 16, 3.9 with one, 2.2 to 3.2
-// with a flag each.)  What a phase leaves lies in memory that this launch
-// has not touched before, so that no cache can hold an older copy: every layer has its own buffers.  The counters only grow:
-// nothing arrives for a phase before the one in front of it is complete.
+// with a flag each.)  What a phase leaves is read at agent scope
+// like the counters, and lies in memory that this launch has not read before: every layer has its own buffers.  Workgroups of several dies
+// write parts of one line (of a norm's shares, four bytes each), and a cache that holds such a line after its own part was stored through may
+// not be believed about the others.  That order between workgroups is the hardware's (stores at agent scope, vmcnt(0), an addition;
+// a poll that sees it, then loads at agent scope), not the language's, whose fences write back and drop second-level caches that
+// hold nothing of this: us a step, 110M shape 1 row, 8B shape 1 and 8 rows: 256, 2492, 2723 without; with the acquiring
+// fences 315, 2631, 2840, with both 527, 4120, 4346; reading at agent scope instead of through the caches costs nothing, 257, 2482, 2706.
+// The counters only grow: nothing arrives for a phase before the one in front of it is complete.
 //
 // Waiting cannot lock up, whatever part of the grid the chip has room for: nothing is waited for but workgroups that
 // run.  A phase's work is cut into as many parts as the grid has workgroups.  They are counted at the start: if all are there,
@@ -62,6 +67,7 @@
 #define RL_SUMS (RL_STREAMERS * 2 * 64)   // floatx4 of a tile's partial sums
 #define RL_COUNTERS 128
 #define RL_LINE 64                    // ints from one counter to the next
+#define RL_AT_AGENT 16                // cache policy of a load (sc1): as an atomic load at agent scope
 #define RL_NOWHERE 0xfffff000u        // an offset behind every matrix: reads as zero
 #define RL_MOST_BYTES 0xffff0000l
 #define RL_MOST_COLUMNS (1 << 23)     // of a row of x: sixteen of them, and all buffers of a layer, have 32-bit offsets
@@ -133,6 +139,10 @@ template <typename T> __device__ __forceinline__ T rl_get(const T* p) { return _
 __device__ __forceinline__ float2 rl_get8(const float* p) {
     const unsigned long long v = __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, AGENT);
     return make_float2(__uint_as_float((unsigned)v), __uint_as_float((unsigned)(v >> 32)));
+}
+__device__ __forceinline__ rl_u4 rl_get16(const void* p) {
+    const float2 lo = rl_get8((const float*)p), hi = rl_get8((const float*)p + 2);
+    return rl_u4{__float_as_uint(lo.x), __float_as_uint(lo.y), __float_as_uint(hi.x), __float_as_uint(hi.y)};
 }
 __device__ __forceinline__ void rl_all_landed() {
     asm volatile("" ::: "memory");
@@ -361,7 +371,7 @@ __device__ __forceinline__ void rl_bring(const RlProduct& p, const char* x, int 
             const int s = n / part;
             from = (rl_first_piece(p.K, s) + chunk_begin) * piece_bytes + ((n - s * part) << 10);
         }
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(to + (n << 10)), 16, from + lane * 16, 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(to + (n << 10)), 16, from + lane * 16, 0, 0, RL_AT_AGENT);
     }
     rl_all_landed();
 }
@@ -464,14 +474,14 @@ __device__ __forceinline__ void rl_attend(const Args& a, const LayerT& L, const 
 #pragma unroll
             for (int ds = 0; ds < DS; ++ds)
                 kf[kt][ds].u = __builtin_amdgcn_raw_buffer_load_b128(
-                    rs, FULL || ds * 32 + lg * 8 < hd ? key_lane + ds * 2048 + kt * 256 : (int)RL_NOWHERE, at, 0);
+                    rs, FULL || ds * 32 + lg * 8 < hd ? key_lane + ds * 2048 + kt * 256 : (int)RL_NOWHERE, at, RL_AT_AGENT);
     };
     auto ask_values = [&](int page, int kb) {
         const auto rs = region(L.v_pages, page);
         const int at = (kb & 1) * 1024;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
-            vf[dt].u = __builtin_amdgcn_raw_buffer_load_b128(rs, FULL || dt * 16 < hd ? value_lane + dt * 2048 : (int)RL_NOWHERE, at, 0);
+            vf[dt].u = __builtin_amdgcn_raw_buffer_load_b128(rs, FULL || dt * 16 < hd ? value_lane + dt * 2048 : (int)RL_NOWHERE, at, RL_AT_AGENT);
     };
     int kb = kb_begin + wave - 1;
     int page = kb < kb_end ? pages[kb >> 1] : 0, page_behind = kb + 3 < kb_end ? pages[(kb + 3) >> 1] : 0;
@@ -487,7 +497,7 @@ __device__ __forceinline__ void rl_attend(const Args& a, const LayerT& L, const 
 #pragma unroll
         for (int ds = 0; ds < DS; ++ds) {
             const int d = ds * 32 + lg * 8;
-            qf[ds].u = (valid && (FULL || d < hd)) ? *(const rl_u4*)(q + d) : rl_u4{0, 0, 0, 0};
+            qf[ds].u = (valid && (FULL || d < hd)) ? rl_get16(q + d) : rl_u4{0, 0, 0, 0};
         }
     }
     if (kb < kb_end && !early) {
@@ -971,7 +981,7 @@ __device__ __forceinline__ void rl_work(const Args& a, char* smem, int v, int V,
                         for (int at = 0; at < all; at += 8192) {
                             rl_u4 shares[8];
 #pragma unroll
-                            for (int i = 0; i < 8; ++i) shares[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, at + (i * 64 + lane) * 16, 0, 0);
+                            for (int i = 0; i < 8; ++i) shares[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, at + (i * 64 + lane) * 16, 0, RL_AT_AGENT);
 #pragma unroll
                             for (int i = 0; i < 8; ++i)
 #pragma unroll

@@ -88,6 +88,20 @@ def test_a_part_of_a_context_that_is_no_number_makes_the_row_no_number(hd, H, G,
     assert torch.equal(got[1], want[1])
 
 
+def test_repeats_have_the_same_bits():
+    """Every launch reads what its own workgroups left, also where several of them wrote parts of one line."""
+    for sizes in ((768, 12, 12, 64, 2048, [40], [1]), (264, 4, 2, 64, 1096, [9, 300, 70], [1, 1, 1])):
+        p = _problem(*sizes)
+        layers = [_layer(p) for _ in range(32)]
+        results = []
+        for _ in range(40):
+            stream = p.residual.clone()
+            _resident(p, layers, stream)
+            results.append(stream)
+        assert bool(torch.isfinite(results[0]).all())
+        assert all(torch.equal(r, results[0]) for r in results)
+
+
 def test_a_launch_that_begins_on_a_busy_chip_has_the_rest_of_it_once_it_is_free():
     """32 layers of 4,096 beside two, then four, launches of as many that leave them eight compute units: they
     stay with the eight for a layer, not to their end, which would take 32 times as long as on the whole chip; and what they
