@@ -88,6 +88,74 @@ def test_a_part_of_a_context_that_is_no_number_makes_the_row_no_number(hd, H, G,
     assert torch.equal(got[1], want[1])
 
 
+# width, heads, key/value heads, head size, inner; held tokens, new ones; window, dims turned.  Rows kept: 1, 2, 4, 8, 16.  x of a
+# product whole, and in halves: of the columns of a streamer 20 128-wide pieces of 49 at a time (one row of 49,160), 10 of 28 (two
+# rows of 28,672), 5 of 14 (four of 14,336), 2 of 11 (eight of 11,008), 2 of 8 (eight of 64 heads of 128), 1 of 3 (twelve of 3,072)
+ROW_BY_ROW = [(768, 12, 12, 64, 2048, [700, 40], [1, 1], 0, 64), (768, 12, 4, 64, 2048, [0], [4], 0, 64),
+              (128, 2, 1, 64, 49160, [33], [1], 0, 64), (256, 4, 2, 64, 28672, [90, 3], [1, 1], 0, 64),
+              (256, 4, 2, 64, 14336, [5, 6, 700], [1, 1, 1], 0, 64), (256, 4, 2, 64, 14336, [20], [4], 0, 64),
+              (264, 4, 4, 64, 11008, [9] * 5 + [2100], [1] * 5 + [3], 0, 64), (256, 64, 8, 128, 520, [70] * 8, [1] * 8, 0, 128),
+              (3072, 4, 1, 128, 136, [3] * 12, [1] * 12, 0, 128), (1032, 16, 2, 48, 1104, [2100] + [31] * 15, [1] * 16, 0, 48),
+              (200, 10, 5, 80, 328, [700, 31, 64], [1, 2, 3], 70, 30), (128, 16, 1, 128, 264, [0], [16], 0, 2)]
+
+
+def _exact(p):
+    """The layer in 64 bits: (the stream behind it, the new tokens' keys and values [M, G, hd])."""
+    f, hd, G = torch.float64, p.hd, p.G
+
+    def normed(x, weight):
+        return x * (x.square().mean(1, keepdim=True) + EPS).rsqrt() * weight.to(f)
+    stream, pos, seq = p.residual.to(f), p.batch.tok_pos.long(), p.batch.tok_seq.long()
+    M = len(pos)
+    q, k, v = (normed(stream, p.norm_mixer) @ p.wqkv.to(f).t()).view(M, -1, hd).split([p.H, G, G], 1)
+    angle = (pos[:, None].float() * p.freqs).to(f)[:, None]
+
+    def turned(x):
+        a, b = x[..., :p.rot].unflatten(-1, (-1, 2)).unbind(-1)
+        pair = torch.stack([a * angle.cos() - b * angle.sin(), b * angle.cos() + a * angle.sin()], -1)
+        return torch.cat([pair.flatten(-2), x[..., p.rot:]], -1)
+    q, k = turned(q), turned(k)
+    mixed = torch.empty_like(q)
+    for t in range(M):
+        at = torch.arange(max(0, int(pos[t]) + 1 - p.window) if p.window else 0, int(pos[t]) + 1, device=DEV)
+        page, slot = p.table[seq[t]].long()[at // PAGE], at % PAGE
+        keys, values = p.keys[page, :, slot].to(f), p.values[page, :, :, slot].to(f)          # [keys, G, hd]
+        for i in range(M):                                                # those of this step, as they were written
+            if seq[i] == seq[t] and at[0] <= pos[i] <= pos[t]:
+                keys[pos[i] - at[0]], values[pos[i] - at[0]] = k[i], v[i]
+        rows = q[t].view(G, -1, hd)
+        for g in range(G):
+            mixed[t].view(G, -1, hd)[g] = (rows[g] @ keys[:, g].t() * p.scale).softmax(-1) @ values[:, g]
+    stream = stream + mixed.reshape(M, -1) @ p.wo.to(f).t()
+    a, b = (normed(stream, p.norm_ffn) @ p.w13.to(f).t()).chunk(2, 1)
+    return stream + (torch.nn.functional.silu(a) * b) @ p.w2.to(f).t(), k, v
+
+
+@pytest.mark.parametrize("workgroups", [0, 7])
+@pytest.mark.parametrize("sizes", ROW_BY_ROW, ids=str)
+def test_every_row_and_what_it_leaves_in_the_cache(sizes, workgroups):
+    """Against 64 bits, each row by itself.  bfloat16 rounds by at most 2^-9 of a value: a key or a value through the norm's rows and
+    its own rounding, 2^-8 of the row at most beside sums in float32; what the layer adds to the stream through seven such roundings one
+    behind the other (rows, queries, probabilities, heads, rows, gate; keys and values beside them), independent of
+    one another, sqrt(7) 2^-9 < 2^-7.  A 128-wide piece left out of 14,336 columns changes a row by a tenth."""
+    D, H, G, hd, inner, held, new, window, rot = sizes
+    p = _problem(D, H, G, hd, inner, held, new, window=window, rot=rot, seed=3)
+    want, k, v = _exact(p)
+    stream, keys, values = _run(p, "resident", workgroups=workgroups)
+    at = p.batch.tok_pos.long()
+    page, slot = p.table[p.batch.tok_seq.long(), at // PAGE].long(), at % PAGE
+    for name, got, right, bound in (("stream", stream - p.residual, want - p.residual, 2 ** -7),
+                                    ("keys", keys[page, :, slot], k, 2 ** -8), ("values", values[page, :, :, slot], v, 2 ** -8)):
+        error = (got.double() - right).flatten(1).norm(dim=1) / right.flatten(1).norm(dim=1)
+        print(f"{name}: largest {float(error.max()):.5f} of {bound:.5f}", flush=True)
+        assert bool((error <= bound).all()), (name, error)           # false for NaN
+    held_still = torch.ones(keys.shape[0], PAGE, dtype=torch.bool, device=DEV)
+    held_still[page, slot] = False                                    # nothing else of the cache is written
+    for now, was in ((keys, p.keys), (values.transpose(2, 3), p.values.transpose(2, 3))):
+        now, was = now.transpose(1, 2)[held_still], was.transpose(1, 2)[held_still]
+        assert torch.equal(now.view(torch.int16), was.view(torch.int16))
+
+
 def test_repeats_have_the_same_bits():
     """Every launch reads what its own workgroups left, also where several of them wrote parts of one line."""
     for sizes in ((768, 12, 12, 64, 2048, [40], [1]), (264, 4, 2, 64, 1096, [9, 300, 70], [1, 1, 1])):
