@@ -5,19 +5,25 @@
 // (32 TM x 32 TN) with v_mfma_f32_32x32x16_bf16, formed transposed (A = W, B = x) so that a lane ends with
 // four consecutive columns of one row.  (The 32 x 32 form reads half as many operand registers per flop as
 // 16 x 16 x 32; under the chip's power limit a bare loop of it reaches 1.86 PFLOP/s on random operands
-// against 1.65.)  K is walked in pieces of 64, one 128-byte line per row, which are copied straight into
-// shared memory (global_load_lds, 16 bytes a lane) two buffers deep, their 16-byte chunks swizzled by the
-// row so that operand reads have no bank conflicts.
+// against 1.65.)  K is walked in stages of 64, one 128-byte line per row, which are copied straight into
+// shared memory (global_load_lds, 16 bytes a lane; a copy of sixteen half lines moves 67 KB a microsecond
+// into a compute unit, one of eight lines 130), their 16-byte chunks swizzled by the row so that operand
+// reads have no bank conflicts.
 //
-// What bounds it is the path into a compute unit, not the arithmetic: at 256 x 256 a piece takes 2,048
-// cycles of the matrix units and 64 KB of copies.  Hence:
+// What bounds it is how many bytes a workgroup has under way, not the way into a compute unit (130 KB a microsecond
+// out of the XCD's cache, of which the tile of 256 x 256 takes 35) and, while W comes from memory, not the arithmetic:
+// two buffers of 64 KB had some 35 KB under way at a time, 1 us of latency long.  Hence:
+//  * x and W have rings of buffers of their own in the 160 KB: two of x, whose rows other workgroups of the XCD
+//    read too, and three of W, which comes from memory and so is asked for two stages ahead (low tiles: three and
+//    three, four and four).  One round of the chip, 16 experts of 256, 192, 128, 64 rows, 4,096 x 4,096: 127, 112,
+//    104, 96 us; with two buffers of both, and lines of W asked for ahead, 146, 133, 119, 107;
 //  * operands of the next 16 k are read between the products of this one, one read per two products, and
-//    the one barrier of a piece stands before its last 16 k, so that nothing waits behind it;
-//  * copies are spread over three of a piece's four steps instead of issued in a burst (a burst fills the
-//    address unit and holds the products up);
-//  * in the tile that fills a compute unit by itself, the lines of W are asked for two pieces before they are
-//    copied (one dword of 64 lines per instruction, into shared memory that nobody reads), so that the copies find
-//    them in the XCD's cache.
+//    the one barrier of a stage stands before its last 16 k, so that nothing waits behind it;
+//  * copies are spread over a stage's four steps instead of issued in a burst (a burst fills the
+//    address unit and holds the products up), x's first, since copies land in order and x's are due sooner;
+//  * groups of neighbouring columns begin at stages of their own (below).
+// 7,108 rows of 32 experts, a prompt's shares, 4,096 -> 3,584: 322 -> 262 us, 3,584 -> 4,096: 313 -> 252; 8,024 rows,
+// 4,096 -> 2 x 2,048 362 -> 305, 2,048 -> 4,096 197 -> 166; 8,192 rows of one 4,096 x 4,096: 215 -> 205 (1,340 TFLOP/s).
 // The copies are written in asm because the compiler takes any operand read to depend on every copy in
 // flight and waits for all of them; they have no output registers, and the waits below count them.
 #pragma once
@@ -152,13 +158,27 @@ __device__ __forceinline__ void pt_find_tile(const int* __restrict__ offsets, in
 #define PT_RUN 4               // tiles of one row tile that an XCD takes together (1, 2, 4: alike; 7, 14: slower)
 #define PT_AS3(p) ((__attribute__((address_space(3))) void*)(p))
 
-// One tile of up to 64 TM rows: rows m0 .. m1 - 1, all of expert e, columns from n0 on.  ASK: the lines of W are
-// asked for ahead.
-template <int TM, int TN, int MODE, bool ASK>
+// Buffers that a workgroup keeps for stages of x and of W, in `rows` lines of 128 bytes: of W, which comes from memory, one
+// more than of x, which comes out of the XCD's cache, where there is room for it.  (Still more of W gain nothing:
+// copies land in order, so those of x that the next stage needs wait for all of W asked for before them.)
+struct PtRings {
+    int x, w;
+};
+constexpr PtRings pt_rings(int rows, int bm, int bn) {
+    PtRings best{0, 0};
+    for (int n = 2; n <= 5 && n * (bm + bn) <= rows; ++n) best = {n, n * (bm + bn) + bn <= rows ? n + 1 : n};
+    return best;
+}
+
+// One tile of up to 64 TM rows: rows m0 .. m1 - 1, all of expert e, columns from n0 on, within LDS bytes of shared
+// memory.
+template <int TM, int TN, int MODE, int LDS>
 __device__ __forceinline__ void pt_tile(const PtArgs& g, char* lds, int e, int m0, int m1, int n0) {
     constexpr int BM = 64 * TM, BN = 64 * TN;
-    constexpr int UX = BM / 32, UW = BN / 32, U = UX + UW;       // 1 KB copies (8 rows) of a wave and piece
-    constexpr int XB = BM * 128, BUF = (BM + BN) * 128;
+    constexpr int UX = BM / 32, UW = BN / 32, U = UX + UW;       // 1 KB copies (8 rows) of a wave and stage
+    constexpr PtRings RING = pt_rings(LDS / 128, BM, BN);
+    constexpr int NX = RING.x, NW = RING.w, XS = BM * 128, WS = BN * 128, W0 = NX * XS;
+    static_assert(NX >= 2 && (NX - 1) * U + UW < 64, "stages under way, counted by the wait");
     const int F = g.F, N = MODE == PT_GATE ? 2 * F : F;          // columns of out, rows of an expert's W
     const int K = g.K;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -175,10 +195,12 @@ __device__ __forceinline__ void pt_tile(const PtArgs& g, char* lds, int e, int m
         return (n < F ? n : F - 1) + ((r >> 5) & 1) * F;
     };
 #define PT_SWIZZLE(r) (((r) >> 1) & 7)
-    const int T = K / 64;                                        // pieces
-    // experts begin at different pieces: their matrices are often a power of two apart, and walked in step from
-    // the first piece they meet in the same memory channels (32 experts of 4,096 x 4,096, 40 tokens: 266 -> 190 us)
-    const int turn = (e * 8) % T;
+    const int T = K / 64;                                        // stages of the whole product
+    // experts begin at different stages: their matrices are often a power of two apart, and walked in step from
+    // the first one they meet in the same memory channels (32 experts of 4,096 x 4,096, 40 tokens: 266 -> 190 us).  So do
+    // groups of an expert's column tiles, as many as an XCD takes together (gated: twice as many; a prompt's shares: 300
+    // -> 288, 190 -> 181; every column tile for itself 333, 209: its neighbours no longer read x at the same time)
+    const int turn = (e + n0 / BN / PT_RUN) * 8 % T;
     const char* xp[UX];
     uint32_t wo[UW];
 #pragma unroll
@@ -193,20 +215,14 @@ __device__ __forceinline__ void pt_tile(const PtArgs& g, char* lds, int e, int m
         wo[i] = (uint32_t)(w_row(r) - wfirst) * (uint32_t)(K * 2) + c * 16;
     }
     const char* wbase = (const char*)(we + (size_t)wfirst * K);
-
-    // the line (of the pieces to come) that this lane asks for: one of the tile's rows of W
-    const char* line = nullptr;
-    if (ASK) {
-        static_assert(BN / PT_WAVES <= 64, "a lane asks for one line");
-        line = (const char*)(we + (size_t)w_row(wave * (BN / PT_WAVES) + lane % (BN / PT_WAVES)) * K);
-    }
     const uint32_t lds_at = (uint32_t)(uintptr_t)PT_AS3(lds);
-    // copy i of the wave (x first) of piece t into buffer b
-#define PT_COPY(i, t, b) do { \
+    // copy i of the wave (x first) into x's buffer bx or W's bw, of the stage NX or NW behind stage t; not beyond the last
+#define PT_COPY(i, t, bx, bw) do { \
         constexpr bool X = (i) < UX; \
-        const uint32_t to = __builtin_amdgcn_readfirstlane(lds_at + (b) * BUF + (X ? 0 : XB) + \
+        const uint32_t to = __builtin_amdgcn_readfirstlane(lds_at + (X ? (bx) * XS : W0 + (bw) * WS) + \
                             (wave + PT_WAVES * (X ? (i) : (i) - UX)) * 1024); \
-        const size_t at = (size_t)(uint32_t)__builtin_amdgcn_readfirstlane((t) + turn < T ? (t) + turn : (t) + turn - T) * 128; \
+        const int stage = (t) + (X ? NX : NW) < T ? (t) + (X ? NX : NW) : T - 1; \
+        const size_t at = (size_t)(uint32_t)__builtin_amdgcn_readfirstlane(stage + turn < T ? stage + turn : stage + turn - T) * 128; \
         if (X) \
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" \
                          :: "s"(to), "v"(xp[X ? (i) : 0] + at) : "memory", "m0"); \
@@ -214,15 +230,9 @@ __device__ __forceinline__ void pt_tile(const PtArgs& g, char* lds, int e, int m
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" \
                          :: "s"(to), "v"(wo[X ? 0 : (i) - UX]), "s"(wbase + at) : "memory", "m0"); \
     } while (0)
-#define PT_ASK(t) do { if (ASK) { \
-        const int piece = ((t) < T ? (t) : T - 1) + turn; \
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" \
-                     :: "s"(__builtin_amdgcn_readfirstlane(lds_at + 2 * BUF + wave * 256)), \
-                        "v"(line + (size_t)(piece < T ? piece : piece - T) * 128) : "memory", "m0"); \
-    } } while (0)
 
     const int hi = lane >> 5, swizzle = PT_SWIZZLE(lane & 31);
-    const int x_at = (wr * TM * 32 + (lane & 31)) * 128, w_at = XB + (wc * TN * 32 + (lane & 31)) * 128;
+    const int x_at = (wr * TM * 32 + (lane & 31)) * 128, w_at = W0 + (wc * TN * 32 + (lane & 31)) * 128;
     int chunk[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) chunk[s] = ((2 * s + hi) ^ swizzle) * 16;
@@ -234,47 +244,77 @@ __device__ __forceinline__ void pt_tile(const PtArgs& g, char* lds, int e, int m
 #pragma unroll
             for (int q = 0; q < 16; ++q) acc[i][j][q] = 0.f;
     PtFrag a0[TN], b0[TM], a1[TN], b1[TM];
-#define PT_READ(b, s, A, B, q) do { \
-        if ((q) < TN) A[(q) < TN ? (q) : 0].u = *(const uint4*)(lds + (b) * BUF + w_at + chunk[s] + (q) * 4096); \
-        else B[(q) < TN ? 0 : (q) - TN].u = *(const uint4*)(lds + (b) * BUF + x_at + chunk[s] + ((q) - TN) * 4096); \
+#define PT_READ(bx, bw, s, A, B, q) do { \
+        if ((q) < TN) A[(q) < TN ? (q) : 0].u = *(const uint4*)(lds + (bw) * WS + w_at + chunk[s] + (q) * 4096); \
+        else B[(q) < TN ? 0 : (q) - TN].u = *(const uint4*)(lds + (bx) * XS + x_at + chunk[s] + ((q) - TN) * 4096); \
     } while (0)
-    // the products of operands A, B; between them the reads of the next 16 k (step s of buffer b) into NA, NB
-    // and copies C0 .. C1 - 1 of piece t into buffer to
-#define PT_STEP(A, B, b, s, NA, NB, C0, C1, t, to) do { \
+    // the products of operands A, B; between them the reads of the next 16 k (step s of buffers bx, bw) into NA, NB, and
+    // copies C0 .. C1 - 1 of the stages behind t into buffers tx, tw
+#define PT_STEP(A, B, READ, bx, bw, s, NA, NB, C0, C1, t, tx, tw) do { \
         _Pragma("unroll") for (int q = 0; q < TN * TM; ++q) { \
             acc[q / TM][q % TM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A[q / TM].v, B[q % TM].v, acc[q / TM][q % TM], 0, 0, 0); \
-            _Pragma("unroll") for (int r = 0; r < TN + TM; ++r) \
-                if (r * (TN * TM) / (TN + TM) == q) PT_READ(b, s, NA, NB, r); \
+            if (READ) { _Pragma("unroll") for (int r = 0; r < TN + TM; ++r) \
+                if (r * (TN * TM) / (TN + TM) == q) PT_READ(bx, bw, s, NA, NB, r); } \
             pt_copies<C0, C1>([&](auto i) { \
-                if ((i.value - (C0)) * (TN * TM) / ((C1) - (C0)) == q) PT_COPY(i.value, t, to); }); \
+                if ((i.value - (C0)) * (TN * TM) / ((C1) - (C0)) == q) PT_COPY(i.value, t, tx, tw); }); \
             __builtin_amdgcn_sched_barrier(0); \
         } \
     } while (0)
-    // everything but the newest request (the line asked for ahead) has landed, in every wave
+    // all but the newest n copies of every wave have landed, and every wave has read its operands
 #define PT_SYNC(n) do { \
-        asm volatile("s_waitcnt vmcnt(" #n ") lgkmcnt(0)" ::: "memory"); \
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(n) : "memory"); \
         __builtin_amdgcn_s_barrier(); \
         asm volatile("" ::: "memory"); \
     } while (0)
-    constexpr int C0 = (U * 5 + 15) / 16, C1 = (U * 10 + 15) / 16;      // copies of the first, first two steps
-    pt_copies<0, U>([&](auto i) { PT_COPY(i.value, 0, 0); });
-    PT_ASK(1);
-    if (ASK) PT_SYNC(1); else PT_SYNC(0);
-    int t1 = T > 1 ? 1 : 0;                                       // the piece whose copies are under way
-    pt_copies<0, C0>([&](auto i) { PT_COPY(i.value, t1, 1); });
+    // The copies between two waits, x's first: those before CA in the last step of the stage whose buffers they take,
+    // those before CB, CC, U in the first steps of the next.
+    constexpr int CA = UX, CB = UX + UW / 3;
+    // How many copies a wave may still have under way when it goes on to the next stage, R stages being left behind
+    // this one: those behind the next stage's.  Between two waits x's copies of one stage come first, then W's of one
+    // NW - NX stages later.
+    auto left = [](int R) constexpr {
+        int n = 0;
+        for (int j = 0; j <= NX - 2; ++j) {
+            if (j < NX - 2 && NX - 1 - j <= R) n += UX;
+            if ((j < NX - 2 || NX < NW) && NW - 1 - j <= R) n += UW;
+        }
+        return n;
+    };
+    pt_copies<0, NW - 1>([&](auto s) {                           // as if the waits before the first stage had been
+        constexpr int t = s.value - (NW - 1);
+        if constexpr (t + NX - 1 >= 0) pt_copies<0, UX>([&](auto i) { PT_COPY(i.value, t - 1, t + NX - 1, 0); });
+        pt_copies<UX, U>([&](auto i) { PT_COPY(i.value, t - 1, 0, s.value); });
+    });
+    pt_copies<0, CA>([&](auto i) { PT_COPY(i.value, -1, NX - 1, NW - 1); });
+    PT_SYNC(left(NW) + CA);
 #pragma unroll
-    for (int r = 0; r < TN + TM; ++r) PT_READ(0, 0, a0, b0, r);
-    for (int t = 0; t < T; ++t) {
-        const int b = t & 1;
-        PT_STEP(a0, b0, b, 1, a1, b1, C0, C1, t1, b ^ 1);
-        PT_STEP(a1, b1, b, 2, a0, b0, C1, U, t1, b ^ 1);
-        PT_ASK(t + 2);
-        PT_STEP(a0, b0, b, 3, a1, b1, U, U, 0, 0);
-        if (ASK) PT_SYNC(1); else PT_SYNC(0);
-        // behind the last piece: its copies once more, and operands that nothing multiplies
-        t1 = t + 2 < T ? t + 2 : T - 1;
-        PT_STEP(a1, b1, b ^ 1, 0, a0, b0, 0, C0, t1, b);
-    }
+    for (int r = 0; r < TN + TM; ++r) PT_READ(0, 0, 0, a0, b0, r);
+    int t = 0, bx = 0, bw = 0;                                   // the stage, its buffers: t modulo NX, NW
+    // stage t, R stages behind it (NW: or more), whose copies alone are asked for: first what is left of the copies
+    // between the last wait and this stage's, then those behind it
+#define PT_STAGE(R) do { \
+        constexpr bool X1 = (R) >= NX - 1, W1 = (R) >= NW - 1, X2 = (R) >= NX, W2 = (R) >= NW; \
+        constexpr int END = W1 ? U : X1 ? UX : 0, E2 = W2 ? U : X2 ? UX : 0; \
+        constexpr int S0 = CA < END ? CA : END, S1 = CB < END ? CB : END; \
+        constexpr int S2 = (CB + U) / 2 < END ? (CB + U) / 2 : END, S3 = CA < E2 ? CA : E2; \
+        const int px = bx == 0 ? NX - 1 : bx - 1, pw = bw == 0 ? NW - 1 : bw - 1; \
+        const int nx = bx == NX - 1 ? 0 : bx + 1, nw = bw == NW - 1 ? 0 : bw + 1; \
+        PT_STEP(a0, b0, true, bx, bw, 1, a1, b1, S0, S1, t - 1, px, pw); \
+        PT_STEP(a1, b1, true, bx, bw, 2, a0, b0, S1, S2, t - 1, px, pw); \
+        PT_STEP(a0, b0, true, bx, bw, 3, a1, b1, S2, END, t - 1, px, pw); \
+        if constexpr ((R) > 0) PT_SYNC(left(R)); \
+        PT_STEP(a1, b1, (R) > 0, nx, nw, 0, a0, b0, 0, S3, t, bx, bw); \
+        bx = nx; \
+        bw = nw; \
+    } while (0)
+    for (; t < T - NW; ++t) PT_STAGE(NW);
+    pt_copies<0, NW>([&](auto i) {                               // the last NW
+        constexpr int R = NW - 1 - i.value;
+        if (R < T) {
+            t = T - 1 - R;
+            PT_STAGE(R);
+        }
+    });
     PT_SYNC(0);
 
     // The tile leaves through shared memory as float32, 32 rows of a wave at a time, so that what follows is a
@@ -323,19 +363,17 @@ __device__ __forceinline__ void pt_tile(const PtArgs& g, char* lds, int e, int m
         __builtin_amdgcn_wave_barrier();
     }
 #undef PT_COPY
-#undef PT_ASK
 #undef PT_READ
 #undef PT_STEP
+#undef PT_STAGE
 #undef PT_SYNC
+#undef PT_SWIZZLE
 }
 
 template <int TM, int TN, int MODE>
 __global__ __launch_bounds__(PT_WAVES * 64, (TM + TN) * 64 * 256 <= 80 * 1024 ? 2 : 1)
 void prompt_tile_kernel(const PtArgs g) {
-    constexpr int BM = 64 * TM, BN = 64 * TN, BUF = (BM + BN) * 128;
-    // asking ahead pays where no second workgroup shares the compute unit (1,777 tokens of 32 experts, W 3,584 x
-    // 4,096: tiles of 256 x 256 374 -> 368 us, 256 x 128 409 -> 384, but 128 x 128 368 -> 432)
-    constexpr bool ASK = (BM + BN) * 256 > 80 * 1024;
+    constexpr int BM = 64 * TM, BN = 64 * TN;
     // Tall tiles are as high as their rows: an expert's rest is often far below 256, and a tile of 64, 128 or 192
     // rows takes fewer copies and products; the highest go first, so that the last round is one of low tiles.
     // Whole prompts, all tiles 256 high, heights by the rows, and highest first: 1,777 tokens of 32 experts of
@@ -343,7 +381,8 @@ void prompt_tile_kernel(const PtArgs g) {
     // 17.6; of gated experts of 3 x 4,096 x 2,048 four of 600 to 1,000 20.55, 20.55, 20.2, one of 2,048 14.1, 13.9, 13.95.
     constexpr bool EVEN = TM == 4;
     constexpr int G = 4;                                         // row tiles that run through the columns together
-    __shared__ __attribute__((aligned(1024))) char lds[2 * BUF + (ASK ? PT_WAVES * 256 : 0)];
+    constexpr int LDS = ((TM + TN) * 64 * 256 <= 80 * 1024 ? 80 : 160) * 1024;     // two workgroups to a compute unit, or one
+    __shared__ __attribute__((aligned(1024))) char lds[LDS];
 
     const int F = g.F;
     constexpr int CN = MODE == PT_GATE ? BN / 2 : BN;            // columns of out that a tile makes
@@ -368,8 +407,12 @@ void prompt_tile_kernel(const PtArgs g) {
     }
     int m0 = 0, m1 = 0, e = 0;
     pt_find_tile<BM, EVEN>(g.offsets, g.E, bm, e, m0, m1);
-    if (EVEN && m1 - m0 <= 64) pt_tile<1, TN, MODE, ASK>(g, lds, e, m0, m1, bn * CN);
-    else if (EVEN && m1 - m0 <= 128) pt_tile<2, TN, MODE, ASK>(g, lds, e, m0, m1, bn * CN);
-    else if (EVEN && m1 - m0 <= 192) pt_tile<3, TN, MODE, ASK>(g, lds, e, m0, m1, bn * CN);
-    else pt_tile<TM, TN, MODE, ASK>(g, lds, e, m0, m1, bn * CN);
+    if constexpr (EVEN) {
+        if (m1 - m0 <= 64) return pt_tile<1, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
+        if (m1 - m0 <= 128) return pt_tile<2, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
+        if (m1 - m0 <= 192) return pt_tile<3, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
+        if constexpr (TM > 4) if (m1 - m0 <= 256) return pt_tile<4, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
+        if constexpr (TM > 5) if (m1 - m0 <= 320) return pt_tile<5, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
+    }
+    pt_tile<TM, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
 }

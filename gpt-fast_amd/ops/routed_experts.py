@@ -337,8 +337,9 @@ def tall_tiles_win(n_experts: int, pairs: int, F: int, K: int, mode: int, units:
     187; 32, 4,096 -> 3,584, x 64 201, 210; x 100 267, 227; x 222 390, 346; 8, 3,584 -> 4,096, x 180 82, 98; x 222, a
     second round of the small ones, 132, 101; 32, 2,816 -> 2,048, x 140 137, 153.  Shares that are not the assumed ones
     can end a round elsewhere: 16, 5,120 -> 2 x 1,536, x 120, counted as a little more than a round of small ones, needed
-    one: 130, 154.  Over 935 such points from 36 rows an expert on what the two rules choose is 0.9 % off the fastest
-    kernel on average and more than 5 % at 62.  Up to K = 1,024 :func:`rows_tile` says, but for sums of K = 1,024 from
+    one: 130, 154.  (The kernel with a ring of its own for W, 14 to 20 % faster in tall tiles, up to 10 % in these: over 2,000
+    random points of 20 to 700 rows what the two rules choose is 2.9 % off the fastest kernel on average; the best
+    other factors, and other lines in K, 2.7 %.)  Up to K = 1,024 :func:`rows_tile` says, but for sums of K = 1,024 from
     400 rows an expert on: 1,024 -> 2,048, x 600 older kernel, 128 x 128, these: 16 experts 78, 65, 68; 32 144, 141,
     119; 128 537, 543, 481."""
     if pairs < 36 * n_experts or K < 1024 or K == 1024 and (mode != 0 or pairs < 400 * n_experts):

@@ -1,0 +1,28 @@
+"""The experts' tile kernel where its rings of buffers begin and end."""
+import pytest
+import torch
+
+from util import rel_err
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("tile", [1, 2, 4])
+@pytest.mark.parametrize("pieces", [1, 2, 3, 4, 5, 6, 7])
+def test_fewer_pieces_of_k_than_buffers_and_a_few_more(monkeypatch, tile, pieces):
+    """Tiles of every height (one to four steps of 64 rows), columns beyond a whole tile and beyond a group of tiles that
+    begin at one piece, and as many pieces of 64 k as make every number of stages behind the last copy; against the same
+    bfloat16 operands in float64.  The result is rounded to bfloat16 once: neighbours lie 2^-7 of their power of two apart
+    (eight bits of significand, the leading one among them), so that a value moves by at most half of that, 2^-8 of itself,
+    after float32 sums of up to 448 products (2^-24 each)."""
+    from gpt_fast_amd.ops import routed_experts as RE
+    monkeypatch.setattr(RE, "_tile_of", lambda *a: tile)
+    counts, K, F = [60, 0, 128, 190, 256, 257], 64 * pieces, 1288
+    g = torch.Generator().manual_seed(pieces)
+    x = torch.randn(sum(counts), K, generator=g).bfloat16()
+    w = (torch.randn(len(counts), F, K, generator=g) * 0.3).bfloat16()
+    offsets = torch.tensor([sum(counts[:i]) for i in range(len(counts) + 1)], dtype=torch.int32)
+    got = RE.expert_tile_product(x.to(DEV), None, 1, w.to(DEV), offsets.to(DEV), None, sum(counts)).double().cpu()
+    want = torch.cat([x[sum(counts[:e]):sum(counts[:e + 1])].double() @ w[e].double().T for e in range(len(counts))])
+    assert rel_err(got, want) < 2.0 ** -8
