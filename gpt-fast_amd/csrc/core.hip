@@ -1105,7 +1105,191 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
     }
 }
 
-// Whether a step asks early; pages: the most that its table has for a sequence.  Not where there are many workgroups (one
+// The same for prompts' rows of head sizes up to 64: a workgroup takes four tokens, as they follow each other in the step, of a
+// head, and a wave that has a page in its registers works off all of them that are of its sequence.  The kernel above
+// brings every page in anew for every token, 32 KB through the caches for 8,000 multiply-adds, and a wave's time on a page
+// is one chain; here four rows' chains run beside each other.  What bounds it still is the way of a wave through its page, loads,
+// scores, maximum, values, some 4 us: 717 tokens of four prompts, 12 heads of 64: 55 -> 28 us; one prompt of 200 19 -> 11, of 2,048
+// 449 -> 221; 32 heads on 4 117 -> 59, 37 -> 21, 1,173 -> 547.  Eight rows hold too many registers (717: 44 to 56).
+// The same arithmetic for a row, so the same bits: its pages are shared out to the waves by their own index; a page that it
+// does not see leaves its maximum, sum and elements as they are, and chunks of keys behind its last one are left out.
+// A group of four may hold rows of several sequences: its workgroup takes the first of them, further ones begin
+// "inside" and are shared out to workgroups behind the groups', AF_SLICES for every 64 tokens.
+#define AF_ROWS 4
+#define AF_SLICES 8
+__global__ __launch_bounds__(256, 3) void attention_f32_rows_kernel(
+        const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
+        const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, const int* __restrict__ table,
+        int table_stride, float* __restrict__ out, int n_tokens, int H, int Hkv, int hd, float scale, int window) {
+    constexpr int ROWS = AF_ROWS;
+    static_assert(ROWS == 4, "a thread for every element of the queries");
+    __shared__ __attribute__((aligned(16))) float qs[ROWS][64];
+    __shared__ __attribute__((aligned(16))) float ps[4][ROWS][GFA_PAGE];
+    __shared__ float merged[4][ROWS][66];
+    const int h = blockIdx.y, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = h / (H / Hkv), groups = (n_tokens + ROWS - 1) / ROWS;
+    int base = blockIdx.x * ROWS;
+    unsigned long long starts = 1;                         // tokens base + bit: where this workgroup's runs begin
+    if ((int)blockIdx.x >= groups) {                       // every AF_SLICES-th of those that begin inside a group
+        const int slice = ((int)blockIdx.x - groups) % AF_SLICES;
+        base = ((int)blockIdx.x - groups) / AF_SLICES * 64;
+        const int n = base + lane;
+        const int there = n < n_tokens ? n : 0;
+        unsigned long long all = __ballot(there % ROWS != 0 && tok_seq[there] != tok_seq[there > 0 ? there - 1 : 0]);
+        starts = 0;
+        for (int i = 0; all; ++i, all &= all - 1)
+            if (i % AF_SLICES == slice) starts |= all & -all;
+    }
+    for (; starts; starts &= starts - 1) {
+        const int n0 = base + __builtin_ctzll(starts);
+        const int seq = tok_seq[n0];
+        int count = 1;
+        while (n0 + count < n_tokens && (n0 + count) % ROWS != 0 && tok_seq[n0 + count] == seq) ++count;
+        {                                                  // rows beyond the last: the last one again, not seen
+            const int row = wave < count ? wave : count - 1;
+            if (lane < hd) qs[wave][lane] = q[((size_t)(n0 + row) * H + h) * hd + lane];
+        }
+        __syncthreads();
+        float m[ROWS], l[ROWS], acc[ROWS];
+#pragma unroll
+        for (int t = 0; t < ROWS; ++t) {
+            m[t] = -INFINITY;
+            l[t] = acc[t] = 0.f;
+        }
+        int pos[ROWS], lo[ROWS];                           // the keys that a row sees; none: another sequence's
+        int last = -1, least = 1 << 30, all_from = 0, all_to = 1 << 30;
+#pragma unroll
+        for (int t = 0; t < ROWS; ++t) {
+            const bool in = t < count;
+            pos[t] = in ? tok_pos[n0 + (in ? t : 0)] : -1;
+            lo[t] = window > 0 && pos[t] - window + 1 > 0 ? pos[t] - window + 1 : 0;
+            if (in && lo[t] < least) least = lo[t];
+            if (pos[t] > last) last = pos[t];
+            if (lo[t] > all_from) all_from = lo[t];
+            if (pos[t] < all_to) all_to = pos[t];
+        }
+        const int* pages = table + (size_t)seq * table_stride;
+        const int first = least / GFA_PAGE;
+        for (int page = first + ((wave - first) & 3); page * GFA_PAGE <= last; page += 4) {
+            const size_t region = cache_region(pages[page], g, Hkv, hd);
+            const float* kr = k_pages + region + (lane >> 5) * 32 * hd + key_slot(lane & 31) * 8;
+            const int vd = lane < hd ? lane : 0;           // lanes beyond the head: others' elements again
+            const float* vr = v_pages + region + (vd >> 4) * 1024 + (vd & 15) * 8;
+            float4 ke[16], ve[16];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const float* at = kr + (c * 8 < hd ? c : 0) * 256;
+                ke[2 * c] = *(const float4*)at;
+                ke[2 * c + 1] = *(const float4*)(at + 4);
+            }
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                ve[2 * c] = *(const float4*)(vr + c * 128);
+                ve[2 * c + 1] = *(const float4*)(vr + c * 128 + 4);
+            }
+            float dot0[ROWS], dot1[ROWS];
+#pragma unroll
+            for (int t = 0; t < ROWS; ++t) dot0[t] = dot1[t] = 0.f;
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+                if (c * 8 < hd) {
+                    const float4 a = ke[2 * c], b = ke[2 * c + 1];
+#pragma unroll
+                    for (int t = 0; t < ROWS; ++t) {
+                        const float4 x = *(const float4*)(qs[t] + c * 8), y = *(const float4*)(qs[t] + c * 8 + 4);
+                        dot0[t] = fmaf(a.w, x.w, fmaf(a.z, x.z, fmaf(a.y, x.y, fmaf(a.x, x.x, dot0[t]))));
+                        dot1[t] = fmaf(b.w, y.w, fmaf(b.z, y.z, fmaf(b.y, y.y, fmaf(b.x, y.x, dot1[t]))));
+                    }
+                }
+            const int key = page * GFA_PAGE + lane;
+#pragma unroll
+            for (int t = 0; t < ROWS; ++t) {
+                const bool seen = key >= lo[t] && key <= pos[t];
+                const float s = seen ? (dot0[t] + dot1[t]) * scale : -INFINITY;
+                const float m_new = fmaxf(m[t], wave_max(s));
+                const float ref = m_new == -INFINITY ? 0.f : m_new;
+                const float alpha = m_new == -INFINITY ? 1.f : expf(m[t] - m_new);
+                const float p = seen ? expf(s - ref) : 0.f;
+                l[t] = l[t] * alpha + wave_sum(p);
+                m[t] = m_new;
+                acc[t] *= alpha;
+                ps[wave][t][lane] = p;                     // read by this wave alone
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {                  // keys 8 c .. + 7
+                const int k0 = page * GFA_PAGE + 8 * c;
+                if (k0 > last) break;
+                const float4 a = ve[2 * c], b = ve[2 * c + 1];
+                auto add = [&](int t, const float4& a, const float4& b) {
+                    const float4 x = *(const float4*)(ps[wave][t] + 8 * c), y = *(const float4*)(ps[wave][t] + 8 * c + 4);
+                    float sum = acc[t];
+                    sum = fmaf(a.w, x.w, fmaf(a.z, x.z, fmaf(a.y, x.y, fmaf(a.x, x.x, sum))));
+                    sum = fmaf(b.w, y.w, fmaf(b.z, y.z, fmaf(b.y, y.y, fmaf(b.x, y.x, sum))));
+                    acc[t] = sum;
+                };
+                if (k0 >= all_from && k0 + 7 <= all_to) {  // seen by all rows
+#pragma unroll
+                    for (int t = 0; t < ROWS; ++t) add(t, a, b);
+                    continue;
+                }
+#pragma unroll
+                for (int t = 0; t < ROWS; ++t) {
+                    if (k0 > pos[t] || k0 + 7 < lo[t]) continue;
+                    float4 u = a, v = b;                   // slots that hold no seen key are not numbers to use
+                    if (k0 + 0 < lo[t]) u.x = 0.f;
+                    if (k0 + 1 < lo[t] || k0 + 1 > pos[t]) u.y = 0.f;
+                    if (k0 + 2 < lo[t] || k0 + 2 > pos[t]) u.z = 0.f;
+                    if (k0 + 3 < lo[t] || k0 + 3 > pos[t]) u.w = 0.f;
+                    if (k0 + 4 < lo[t] || k0 + 4 > pos[t]) v.x = 0.f;
+                    if (k0 + 5 < lo[t] || k0 + 5 > pos[t]) v.y = 0.f;
+                    if (k0 + 6 < lo[t] || k0 + 6 > pos[t]) v.z = 0.f;
+                    if (k0 + 7 > pos[t]) v.w = 0.f;
+                    add(t, u, v);
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+#pragma unroll
+        for (int t = 0; t < ROWS; ++t) {
+            merged[wave][t][lane] = acc[t];
+            if (lane == 0) {
+                merged[wave][t][64] = m[t];
+                merged[wave][t][65] = l[t];
+            }
+        }
+        __syncthreads();
+        for (int t = wave; t < count; t += 4) {
+            float top = merged[0][t][64];
+            for (int w = 1; w < 4; ++w) top = fmaxf(top, merged[w][t][64]);
+            float total = 0.f, part[4];
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                part[w] = merged[w][t][64] == -INFINITY ? 0.f : expf(merged[w][t][64] - top);
+                total = fmaf(merged[w][t][65], part[w], total);
+            }
+            float v = 0.f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) v = fmaf(merged[w][t][lane], part[w], v);
+            if (lane < hd) out[((size_t)(n0 + t) * H + h) * hd + lane] = v / total;
+        }
+        __syncthreads();
+    }
+}
+
+// Whether a step's rows go four at a time; pages: the most that its table has for a sequence.  Not where the groups would
+// be too few to hide a wave's way, nor where many rows have sequences of their own: a wave takes as long on a page for one row as for
+// four.  us, one at a time and four: 12 heads of 64, one prompt of 60 8.0, 7.9; 100 11.5, 8.7; 60 behind 2,000 keys 38, 45; 100 behind
+// 900 30.5, 27.1; several: 4 x 50 behind 900 56, 44; 600 and eight single tokens behind 900 73, 51; 200 and the eight 28.5, 30.9;
+// 40 x 3 14.2, 12.4; 4 x 30 behind 300 19.2, 22.8; 64 single tokens behind 100 12.1, 42.4.
+static bool attention_f32_four(int n_tokens, int n_seqs, int H, int hd, int pages) {
+    if (hd > 64) return false;
+    if (n_seqs <= 1) return (long long)n_tokens * H >= 1024;
+    return n_tokens >= 40ll * n_seqs && (long long)n_tokens * H >= 2048 && pages <= 32;
+}
+
+// Whether a step whose rows go one at a time asks early; pages: as above.  Not where there are many workgroups (one
 // a token and head) and they walk many pages, or share the keys of a group, which then are in the caches.  us, early and
 // not, heads of 64, prompts' keys out of the caches and single tokens' out of memory: 12 heads, a token behind 30
 // keys 5.6, 6.7; 16 behind 1,000 25.7, 26.2; prompts of 8 x 200 123, 132; 600 3.12 ms of a model's step either way; 900 124,
@@ -1120,7 +1304,7 @@ static bool attention_f32_early(int n_tokens, int H, int Hkv, int hd, int pages,
 
 extern "C" int gfa_attention_generic(const void* q, const void* k_pages, const void* v_pages,
                                      const int* tok_seq, const int* tok_pos, const int* table,
-                                     int table_stride, void* out, int n_tokens, int H, int Hkv,
+                                     int table_stride, int n_seqs, void* out, int n_tokens, int H, int Hkv,
                                      int hd, float scale, int window, int is_bf16,
                                      hipStream_t stream) {
     if (n_tokens <= 0) return 0;
@@ -1130,7 +1314,11 @@ extern "C" int gfa_attention_generic(const void* q, const void* k_pages, const v
     if (!is_bf16 && hd % 16 == 0 && hd <= 256 && (uintptr_t)k_pages % 16 == 0 && (uintptr_t)v_pages % 16 == 0) {
 #define AF_GO(HD, EARLY) attention_f32_kernel<HD, EARLY><<<grid, 256, 0, stream>>>((const float*)q, (const float*)k_pages, \
         (const float*)v_pages, tok_seq, tok_pos, table, table_stride, (float*)out, H, Hkv, hd, scale, window)
-        if (attention_f32_early(n_tokens, H, Hkv, hd, table_stride, window)) AF_GO(64, true);
+        if (attention_f32_four(n_tokens, n_seqs, H, hd, table_stride)) {
+            const int groups = (n_tokens + AF_ROWS - 1) / AF_ROWS, slices = n_seqs > 1 ? (n_tokens + 63) / 64 * AF_SLICES : 0;
+            attention_f32_rows_kernel<<<dim3(groups + slices, H), 256, 0, stream>>>((const float*)q, (const float*)k_pages,
+                (const float*)v_pages, tok_seq, tok_pos, table, table_stride, (float*)out, n_tokens, H, Hkv, hd, scale, window);
+        } else if (attention_f32_early(n_tokens, H, Hkv, hd, table_stride, window)) AF_GO(64, true);
         else if (hd <= 64) AF_GO(64, false);
         else if (hd <= 128) AF_GO(128, false);
         else AF_GO(256, false);
@@ -1462,8 +1650,8 @@ extern "C" int gfa_few_row_layers_f32(const FewRowLayer* layers, int n_layers, c
                                       s.n_seqs, s.M, s.H, s.Hkv, s.hd, s.rot, 0, 0, stream);
             if (rc) break;
         }
-        rc = gfa_attention_generic(q, L.k_pages, L.v_pages, s.tok_seq, s.tok_pos, L.table, s.table_stride, y, s.M, s.H,
-                                   s.Hkv, s.hd, s.scale, s.window, 0, stream);
+        rc = gfa_attention_generic(q, L.k_pages, L.v_pages, s.tok_seq, s.tok_pos, L.table, s.table_stride, s.n_seqs, y, s.M,
+                                   s.H, s.Hkv, s.hd, s.scale, s.window, 0, stream);
         if (rc) break;
         rc = gfa_gemm_f32(y, (const float*)L.wo, s.residual, s.M, s.D, inner, inner, s.D, 1, stream);
         if (rc) break;

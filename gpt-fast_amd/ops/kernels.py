@@ -294,7 +294,7 @@ def attention_generic(q: torch.Tensor, k_pages, v_pages, tok_seq, tok_pos, table
         out = torch.empty_like(q)
     check(library("core").gfa_attention_generic(
         ptr(q), ptr(k_pages), ptr(v_pages), ptr(tok_seq), ptr(tok_pos), ptr(table),
-        _i(table.shape[1]), ptr(out), _i(n), _i(H), _i(G), _i(hd), _f(scale), _i(window),
+        _i(table.shape[1]), _i(table.shape[0]), ptr(out), _i(n), _i(H), _i(G), _i(hd), _f(scale), _i(window),
         _i(_is_bf16(q)), stream_handle()), "attention_generic")
     return out
 

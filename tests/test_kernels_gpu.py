@@ -483,6 +483,40 @@ def test_a_float32_row_is_the_same_among_few_and_among_many(H, G, hd, S, window)
         close(out[p], _attention_ref(q[p].cpu(), ks[0], vs[0], p, hd ** -0.5, window), 1e-5)
 
 
+@pytest.mark.parametrize("held,new", [([0], [1030]), ([0, 0, 0, 0], [177, 150, 193, 200]), ([130, 0, 5, 64], [1, 259, 2, 61]),
+                                      ([0, 63, 3, 70, 1, 0], [190, 1, 1, 1, 1, 129]), ([1000, 1], [6, 390])])
+@pytest.mark.parametrize("H,G,hd,window", [(12, 12, 64, 0), (32, 4, 64, 70), (16, 16, 48, 0), (16, 2, 16, 3)])
+def test_float32_rows_that_go_four_at_a_time(H, G, hd, window, held, new):
+    """Groups of four rows that hold the ends and beginnings of sequences, one of a single token, pages that some of a
+    group's rows see and others do not, a value that is no number: the same bits as each row alone."""
+    lens = [a + b for a, b in zip(held, new)]
+    k_pages, v_pages, table, ks, vs = _paged(lens, G, hd, torch.float32, sum(lens) + hd)
+    seq = torch.tensor([b for b, n in enumerate(new) for _ in range(n)], dtype=torch.int32)
+    pos = torch.tensor([held[b] + i for b, n in enumerate(new) for i in range(n)], dtype=torch.int32)
+    N = seq.numel()
+    q = torch.randn(N, H, hd, generator=torch.Generator().manual_seed(hd)).to(DEV)
+    on = seq.to(DEV), pos.to(DEV)
+    ends = [sum(new[:b + 1]) for b in range(len(new))]
+    near = {n + d for n in [0] + ends for d in range(-6, 6)} | set(range(1, N, 37))
+    rows = [n for n in sorted(near) if 0 <= n < N]
+    alone = lambda n: K().attention_generic(q[n:n + 1], k_pages, v_pages, on[0][n:n + 1], on[1][n:n + 1], table, hd ** -0.5, window)[0]
+    out = K().attention_generic(q, k_pages, v_pages, *on, table, hd ** -0.5, window)
+    for n in rows:
+        b = int(seq[n])
+        assert torch.equal(alone(n), out[n]), n
+        close(out[n], _attention_ref(q[n].cpu(), ks[b], vs[b], int(pos[n]), hd ** -0.5, window), 1e-5)
+    last = new.index(max(new))                              # a key in the middle of the longest part
+    bad = held[last] + new[last] // 2
+    k_rows, v_cols = from_cache_order(k_pages.cpu(), v_pages.cpu())
+    v_cols[int(table[last, bad // 64]), :, :, bad % 64] = float("nan")
+    v_pages = to_cache_order(k_rows, v_cols)[1].to(DEV)
+    out = K().attention_generic(q, k_pages, v_pages, *on, table, hd ** -0.5, window)
+    sees = (seq == last) & (pos >= bad) & ((pos < bad + window) if window else (pos >= 0))
+    assert torch.equal(out.isnan().cpu(), sees[:, None, None].expand_as(out))
+    for n in rows:
+        assert torch.equal(alone(n).nan_to_num(7.0), out[n].nan_to_num(7.0)), n
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 1.5e-2)])
 @pytest.mark.parametrize("H,G,hd,window", [
     (4, 4, 16, 0), (6, 2, 48, 0), (8, 1, 128, 0), (3, 3, 80, 0), (4, 2, 64, 37), (2, 1, 256, 100),
