@@ -8,6 +8,7 @@
 // position), never on the number of rows or on the other sequences of the launch, so a
 // float32 result is the same however the tokens were cut into steps or batched.
 #include "few_row_layers.h"
+#include <type_traits>
 
 // --------------------------------------------------------------------------------------
 // embedding gather: out[n, :] = float(table[tokens[n], :])          (model.py:140)
@@ -209,17 +210,13 @@ extern "C" int gfa_add_rmsnorm(float* res, const void* y, const float* w, void* 
 //
 // v_mfma_f32_16x16x4_f32: true float32 products and sums, at the vector units' peak rate but without
 // their operand traffic.  The four waves of a workgroup take the same 16 MT x 16 NT tile and every
-// fourth block of 32 k each, so that even a 16-column tile of one row keeps four waves' loads in flight;
-// a lane's 16-byte loads are four k of one row of a or w and land in operand order (the k within a
-// block are taken in an order that is the same for a and w), so nothing goes through shared memory but
-// the four sums at the end.  An output's sum is therefore four chains, added as (0 + 1) + (2 + 3), whose
-// order depends on K alone: every tile size and every M gives the same bits, and a row's result does not
+// fourth block of 32 k each, so that even a 16-column tile of one row keeps four waves' loads in flight.
+// An output's sum is therefore four chains, added as (0 + 1) + (2 + 3), whose
+// order depends on K alone (the k within a block are taken in an order that is the same for a and w): every kernel here,
+// every tile size and every M gives the same bits, and a row's result does not
 // depend on the other rows (a float32 logit is the same however tokens are cut into steps).
-// gf_product picks the tile.  Measured beside 64 x 64 tiles of vector multiply-adds through shared memory,
-// which this replaces: 1 x 768 x 768 76 -> 5.8 us, 1 x 32,000 x 768 120 -> 29 (3.4 TB/s), 717 x 2,304 x 768
-// 99 -> 44, 717 x 768 x 2,048 274 -> 41, 8 x 28,672 x 4,096 617 -> 116 (4.1 TB/s), 2,048 x 4,096 x 4,096
-// 988 -> 704 (98 of the 155 TFLOP/s that a loop of the instruction alone reaches); few rows are bound by
-// latency and the weights, many by the matrix units.
+// gf_product picks the kernel and the tile.  Few rows are bound by latency and the weights (1 x 32,000 x 768 20 us, 5 TB/s),
+// many by the matrix units (2,048 x 4,096 x 4,096 494 us, 139 of the 155 TFLOP/s that a loop of the instruction alone reaches).
 typedef __attribute__((__vector_size__(4 * sizeof(float)))) float gf_floatx4_t;
 
 // out's tile at (m0, n0) from the waves' sums, ((0 + 1) + (2 + 3)); lane: four columns of a row
@@ -244,7 +241,9 @@ __device__ __forceinline__ void gf_store(const gf_floatx4_t (*sums)[MT * NT][64]
     }
 }
 
-template <int MT, int NT, bool WIDE>
+// Operands of any strides, element by element: a lane's loads are four k of one row of a or w and land in operand order, so nothing
+// goes through shared memory but the four sums at the end.
+template <int MT, int NT>
 __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(
         const float* __restrict__ a, const float* __restrict__ w, float* __restrict__ out,
         int M, int N, int K, long long sab, long long sam, long long swb, long long swn,
@@ -284,21 +283,13 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int k = 32 * b + 16 * h + 4 * lg;
-            if (WIDE) {
-                const int at = k < K ? k : 0;      // K is a multiple of four
 #pragma unroll
-                for (int i = 0; i < MT; ++i) r.a[h][i] = *(const gf_floatx4_t*)(ar[i] + at);
+            for (int q = 0; q < 4; ++q) {
+                const int at = k + q < K ? k + q : 0;
 #pragma unroll
-                for (int j = 0; j < NT; ++j) r.w[h][j] = *(const gf_floatx4_t*)(wr[j] + at);
-            } else {
+                for (int i = 0; i < MT; ++i) r.a[h][i][q] = ar[i][at];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int at = k + q < K ? k + q : 0;
-#pragma unroll
-                    for (int i = 0; i < MT; ++i) r.a[h][i][q] = ar[i][at];
-#pragma unroll
-                    for (int j = 0; j < NT; ++j) r.w[h][j][q] = wr[j][(size_t)at * swk];
-                }
+                for (int j = 0; j < NT; ++j) r.w[h][j][q] = wr[j][(size_t)at * swk];
             }
             if (!whole) {
 #pragma unroll
@@ -351,12 +342,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(
 enum GfLoads { GF_WIDE, GF_ALONG, GF_ACROSS };
 typedef gf_floatx4_t gf_loose4_t __attribute__((aligned(4)));
 
-// The same arithmetic for many rows: a 64 x 64 tile whose waves copy their blocks through shared memory of their
-// own (no barrier while K is walked).  A load instruction then takes whole lines, eight rows of 128 bytes (across:
+// The same arithmetic for many rows whose operands are not both 16-byte rows: a 64 x 64 tile whose waves copy their blocks
+// through shared memory of their own (no barrier while K is walked).  A load instruction then takes whole lines, eight rows of 128 bytes (across:
 // 64 rows of one k), where the operand order above takes sixteen rows of 64 bytes, which the compute unit's cache
-// looks up piece by piece: 2,048 x 4,096 x 4,096 took 1,155 us without it, 2,048 x 4,096 x 1,022 (rows at odd
-// addresses) 616 against 168 now and 261 in vector multiply-adds, 32 x 1,000 x 512 x 128 with the second operand
-// transposed, as latent attention has it, 161 against 65 and 98.
+// looks up piece by piece: 2,048 x 4,096 x 1,022 (rows at odd
+// addresses) took 616 us without it against 168, 32 x 1,000 x 512 x 128 with the second operand
+// transposed, as latent attention has it, 161 against 65.
 #define GS_PITCH 144                              // bytes per staged row of 32 k: 128 + pad against conflicts
 template <GfLoads AL, GfLoads WL>
 __global__ __launch_bounds__(256, 2) void gemm_f32_staged_kernel(
@@ -458,9 +449,186 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_staged_kernel(
     gf_store<4, 4>(sums, out, M, N, m0, n0, som, accumulate);
 }
 
-// Up to 16 rows: one 16 x 16 tile a workgroup, which spreads the weights over the most waves.  More rows:
-// 64 x 64 where these tiles are at least 100 (717 x 768 x 2,048, 144 of them: 41 us, as 32 x 32 54 us), else
-// 32 x 32.
+// The same where all loads are 16 bytes at multiples of 16, the form of a model's products: each wave's blocks go through
+// shared memory of its own, and every load, write and read of it is issued between two products.  A wave issues in order: in the
+// staged kernel above the 16 loads, 16 writes and 16 reads of a block stand in a row, some 1,000 cycles in which the wave
+// starts no product, and two waves of a SIMD fall into step (the matrix units were busy 56 to 63 % of the time).  Here, while
+// a block's first half multiplies, its second half is read; while that multiplies, the next block is written, its first half
+// read, and block + 1 + AHEAD asked for.
+//
+// The wave's whole blocks of `at` (16 MT rows) and `wt` (16 NT rows, the second half of them from `wt2`) into acc; from: the lane's bytes
+// from there to its rows, eight a load.  ready() runs once the first AHEAD blocks are asked for.  NORMED: elements of `at` times
+// their row's rs, then times g.
+template <int MT, int NT, int AHEAD, bool NORMED, class Ready>
+__device__ __forceinline__ void gf_piped(const char* at, const char* wt, const char* wt2, const unsigned (&from)[2 * (MT + NT)],
+                                         const float* g, const float (&rs)[2 * MT], int K, char* own, gf_floatx4_t (&acc)[MT][NT], Ready ready) {
+    constexpr int S = MT + NT, HALF = 4 * MT * NT;         // operands of a half block, its products
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = lane >> 3, chunk = lane & 7;           // of eight rows, their 16-byte chunks
+    const int put = row * GS_PITCH + chunk * 16, get = (lane & 15) * GS_PITCH + (lane >> 4) * 16;
+    gf_floatx4_t v[AHEAD][2 * S], gv[AHEAD], f[2][S];
+    auto base = [&](int i) { return i < 2 * MT ? at : i < 2 * MT + NT ? wt : wt2; };
+    auto ask = [&](int j, int slot) {                      // this wave's whole block j
+        const size_t k = (size_t)(wave + 4 * j) * 128;
+#pragma unroll
+        for (int i = 0; i < 2 * S; ++i) v[slot][i] = *(const gf_floatx4_t*)(base(i) + k + from[i]);
+        if (NORMED) gv[slot] = *(const gf_floatx4_t*)((const char*)g + k + 16 * chunk);
+    };
+    auto write = [&](int slot) {
+#pragma unroll
+        for (int i = 0; i < 2 * S; ++i) {
+            gf_floatx4_t x = v[slot][i];
+            if (NORMED && i < 2 * MT)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) x[q] = x[q] * rs[i < 2 * MT ? i : 0] * gv[slot][q];
+            *(gf_floatx4_t*)(own + put + 8 * i * GS_PITCH) = x;
+        }
+    };
+    auto read = [&](int h) {
+#pragma unroll
+        for (int i = 0; i < S; ++i) f[h][i] = *(const gf_floatx4_t*)(own + get + 16 * i * GS_PITCH + 64 * h);
+    };
+    auto multiply = [&](int h) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f[h][MT + j][q], f[h][i][q], acc[i][j], 0, 0, 0);
+    };
+// `times` of the kind `what`, each in front of `each` products
+#define GP_ORDER(what, times, each)                                                  \
+    _Pragma("unroll") for (int u = 0; u < (times); ++u) {                            \
+        __builtin_amdgcn_sched_group_barrier(what, 1, 0);                            \
+        __builtin_amdgcn_sched_group_barrier(GP_PRODUCT, (each), 0);                 \
+    }
+#define GP_PRODUCT 0x008
+#define GP_ASK 0x020
+#define GP_READ 0x100
+#define GP_WRITE 0x200
+    const int whole = K / 32;
+    const int count = wave < whole ? (whole - wave + 3) / 4 : 0;   // this wave's whole blocks
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+        if (u < count) ask(u, u);
+    ready();
+    if (count > 0) {
+        write(0);
+        read(0);
+        if (AHEAD < count) ask(AHEAD, 0);
+        // block j multiplies, j + 1 is written, j + 1 + AHEAD asked for
+        auto step = [&](int j, int slot, auto more) {
+            read(1);
+            multiply(0);
+            write(slot);
+            read(0);
+            if (decltype(more)::value) ask(j + 1 + AHEAD, slot);
+            multiply(1);
+            if (HALF > 4) {
+                GP_ORDER(GP_READ, S, HALF / 2 / S)
+                __builtin_amdgcn_sched_group_barrier(GP_PRODUCT, HALF - S * (HALF / 2 / S), 0);
+                GP_ORDER(GP_WRITE, 2 * S, HALF / 4 / S)
+                GP_ORDER(GP_READ, S, HALF / 4 / S)
+                if (decltype(more)::value) GP_ORDER(GP_ASK, 2 * S, 1)
+            }
+        };
+        int j = 0;
+        for (; j + 2 * AHEAD < count; j += AHEAD) {
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) step(j + u, (u + 1) % AHEAD, std::true_type());
+        }
+#pragma unroll
+        for (int u = 0; u < 2 * AHEAD; ++u) {              // the last 2 AHEAD blocks at most
+            if (j + u + 1 >= count) break;
+            if (u < AHEAD && j + u + 1 + AHEAD < count) step(j + u, (u + 1) % AHEAD, std::true_type());
+            else step(j + u, (u + 1) % AHEAD, std::false_type());
+        }
+        read(1);
+        multiply(0);
+        multiply(1);
+    }
+#undef GP_ORDER
+#undef GP_PRODUCT
+#undef GP_ASK
+#undef GP_READ
+#undef GP_WRITE
+    if (K % 32 && whole % 4 == wave) {                     // the rest behind the whole blocks, zero beyond K, a multiple of four
+        const bool in = 32 * whole + 4 * chunk < K;
+        const size_t k = (size_t)whole * 128;
+        const int back = in ? 0 : 16 * chunk;
+        if (NORMED) gv[0] = *(const gf_floatx4_t*)((const char*)g + k + 16 * chunk - back);
+#pragma unroll
+        for (int i = 0; i < 2 * S; ++i) {
+            v[0][i] = *(const gf_floatx4_t*)(base(i) + k + from[i] - back);
+            if (!in) v[0][i] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
+        }
+        if (NORMED && !in) gv[0] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
+        write(0);
+        read(0);
+        read(1);
+        multiply(0);
+        multiply(1);
+    }
+}
+
+// The product on it in tiles of 16 MT x 16 NT, us before (the two kernels above) and now: 2,048 x 4,096 x 4,096 704 -> 490
+// (140 TFLOP/s), 717 x 4,096 x 768 71 -> 43, 717 x 768 x 2,048 41 -> 24, 60 x 768 x 2,048 19 -> 12, 4 x 32,000 x 768 32.5 -> 20,
+// 4 x 768 x 2,048 10 -> 7.3, 16 x 28,672 x 4,096 142 -> 96.  A 1 x 1 tile with one block ahead takes 78 us for 4 x 4,096 x 14,336, with
+// two 60, with four 45 (before: 55); 2 x 2 tiles with two ahead hold more registers and are slower (29.7, 31.5 at 717 x 768 x 2,048).
+template <int MT, int NT, int AHEAD>
+__global__ __launch_bounds__(256, 2) void gemm_f32_piped_kernel(
+        const float* __restrict__ a, const float* __restrict__ w, float* __restrict__ out, int M, int N, int K,
+        long long sab, long long sam, long long swb, long long swn, long long sob, long long som, int accumulate) {
+    constexpr int S = MT + NT;
+    __shared__ __attribute__((aligned(16))) char lds[4 * 16 * S * GS_PITCH];
+    static_assert(4 * MT * NT * 1024 <= 4 * 16 * S * GS_PITCH, "the waves' sums take the blocks' place");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int m0 = blockIdx.y * (16 * MT), n0 = blockIdx.x * (16 * NT);
+    unsigned from[2 * S];                          // rows beyond the last read it again, never stored
+#pragma unroll
+    for (int i = 0; i < 2 * S; ++i) {
+        const int r = 8 * (i < 2 * MT ? i : i - 2 * MT) + (lane >> 3), most = (i < 2 * MT ? M - m0 : N - n0) - 1;
+        from[i] = (unsigned)(r < most ? r : most) * (unsigned)(4 * (i < 2 * MT ? sam : swn)) + 16 * (lane & 7);
+    }
+    gf_floatx4_t acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
+    const char* wt = (const char*)(w + (size_t)blockIdx.z * swb + (size_t)n0 * swn);
+    const float none[2 * MT] = {};
+    gf_piped<MT, NT, AHEAD, false>((const char*)(a + (size_t)blockIdx.z * sab + (size_t)m0 * sam), wt, wt, from, nullptr, none, K,
+                                   lds + wave * 16 * S * GS_PITCH, acc, [] {});
+    __syncthreads();
+    gf_floatx4_t (*sums)[MT * NT][64] = (gf_floatx4_t (*)[MT * NT][64])lds;
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) sums[wave][i * NT + j][lane] = acc[i][j];
+    __syncthreads();
+    gf_store<MT, NT>(sums, out + (size_t)blockIdx.z * sob, M, N, m0, n0, som, accumulate);
+}
+
+// Side of a 16-byte product's tile by rows and columns, in sixteens.  Up to 16 rows 1 x 1, which spreads the weights over the
+// most waves.  Else a tile's products take the matrix units of one of 256 compute units for as long as it has pieces of 16 x 16, and
+// smaller tiles read more for each: tiles a unit, times pieces, times 1, 1.08, 1.09, 1.17 (2,048 x 4,096 x 4,096: 494, 549, 569,
+// 600 us at 128, 132, 135, 128 pieces a unit; 717 rows of K = 768, us by 4 x 4, 3 x 4, 3 x 3, 2 x 2: N = 4,096 42, 44, 49, 45; 2,304 29.5, 33, 26.5,
+// 27.4; 768 16.3, 13.7, 12.4, 13.6; 200 rows, N = 768, K = 2,048 35, 29, 23, 12).
+static int gf_piped_tile(int B, int M, int N) {
+    if (M <= 16) return 11;
+    int best = 0;
+    double least = 0;
+    const int tiles[4][3] = {{4, 4, 100}, {3, 4, 108}, {3, 3, 109}, {2, 2, 117}};
+    for (const auto& t : tiles) {
+        const double n = (double)B * ((M + 16 * t[0] - 1) / (16 * t[0])) * ((N + 16 * t[1] - 1) / (16 * t[1]));
+        const double cost = ceil(n / 256) * t[0] * t[1] * t[2];
+        if (!best || cost < least) least = cost, best = 10 * t[0] + t[1];
+    }
+    return best;
+}
+
+// Other forms.  Up to 16 rows: one 16 x 16 tile a workgroup.  More rows: 64 x 64 where these tiles are at least 100, else 32 x 32.
 static int gf_product(const float* a, const float* w, float* out, int B, int M, int N, int K,
                       long long sab, long long sam, long long swb, long long swn, long long swk,
                       long long sob, long long som, int accumulate, hipStream_t stream) {
@@ -468,23 +636,29 @@ static int gf_product(const float* a, const float* w, float* out, int B, int M, 
     // 16-byte loads: whole groups of four k, at addresses that are multiples of 16
     const bool a_wide = K % 4 == 0 && sam % 4 == 0 && sab % 4 == 0 && (uintptr_t)a % 16 == 0;
     const bool w_wide = swk == 1 && K % 4 == 0 && swn % 4 == 0 && swb % 4 == 0 && (uintptr_t)w % 16 == 0;
+    const long long far = 1 << 23;                 // of 64 rows: their bytes have 32 bits
+    if (a_wide && w_wide && sam >= 0 && swn >= 0 && sam < far && swn < far) {
+        const int tile = gf_piped_tile(B, M, N), mt = tile / 10 * 16, nt = tile % 10 * 16;
+        if ((M + mt - 1) / mt > 65535 || B > 65535) return (int)hipErrorInvalidValue;
+        const dim3 grid((N + nt - 1) / nt, (M + mt - 1) / mt, B);
+#define GP_GO(MT, NT, AHEAD) gemm_f32_piped_kernel<MT, NT, AHEAD><<<grid, 256, 0, stream>>>(a, w, out, M, N, K, sab, sam, swb, swn, sob, som, accumulate)
+        if (tile == 11) GP_GO(1, 1, 4);
+        else if (tile == 22) GP_GO(2, 2, 1);
+        else if (tile == 33) GP_GO(3, 3, 1);
+        else if (tile == 34) GP_GO(3, 4, 1);
+        else GP_GO(4, 4, 1);
+#undef GP_GO
+        return GFA_LAUNCH_RESULT();
+    }
     const int tile = M <= 16 ? 16 : (long long)((M + 63) / 64) * ((N + 63) / 64) * B < 100 ? 32 : 64;
     if ((M + tile - 1) / tile > 65535 || B > 65535) return (int)hipErrorInvalidValue;
     const dim3 grid((N + tile - 1) / tile, (M + tile - 1) / tile, B);
 #define GF_GO(...) __VA_ARGS__<<<grid, 256, 0, stream>>>(a, w, out, M, N, K, sab, sam, swb, swn, swk, sob, som, accumulate)
-    if (tile == 16) {
-        if (a_wide && w_wide) GF_GO(gemm_f32_kernel<1, 1, true>);
-        else GF_GO(gemm_f32_kernel<1, 1, false>);
-    } else if (tile == 32) {
-        if (a_wide && w_wide) GF_GO(gemm_f32_kernel<2, 2, true>);
-        else GF_GO(gemm_f32_kernel<2, 2, false>);
-    } else if (swk != 1) {
-        if (a_wide) GF_GO(gemm_f32_staged_kernel<GF_WIDE, GF_ACROSS>);
-        else GF_GO(gemm_f32_staged_kernel<GF_ALONG, GF_ACROSS>);
-    } else {
-        if (a_wide && w_wide) GF_GO(gemm_f32_staged_kernel<GF_WIDE, GF_WIDE>);
-        else GF_GO(gemm_f32_staged_kernel<GF_ALONG, GF_ALONG>);
-    }
+    if (tile == 16) GF_GO(gemm_f32_kernel<1, 1>);
+    else if (tile == 32) GF_GO(gemm_f32_kernel<2, 2>);
+    else if (swk != 1 && a_wide) GF_GO(gemm_f32_staged_kernel<GF_WIDE, GF_ACROSS>);
+    else if (swk != 1) GF_GO(gemm_f32_staged_kernel<GF_ALONG, GF_ACROSS>);
+    else GF_GO(gemm_f32_staged_kernel<GF_ALONG, GF_ALONG>);
 #undef GF_GO
     return GFA_LAUNCH_RESULT();
 }
@@ -1424,11 +1598,10 @@ extern "C" int gfa_silu_mul(const void* gu, void* out, int n_rows, int I, int is
 // w = rows of Wg, then of Wu), or q, k, v = n W^T rotated and stored (EPI 2, interleaved pairs, as
 // rope_cache_kernel); n = x * rsqrt(mean(x^2) + eps) * g.
 //
-// What bounds a layer of few rows is its chain of kernels, 5 to 10 us each whatever they do: a norm 5, the rotation
-// 5.5, the gate 5 beside products of 7 to 10 (four rows, 768 columns).  Every workgroup reads all of x
+// What bounds a layer of few rows is its chain of kernels, 4 to 8 us each whatever they do: a norm, the rotation
+// and the gate take 4 to 5 beside products of 5 to 8 (four rows, 768 columns).  Every workgroup reads all of x
 // anyway, so each works the rows' factors out for itself, while its first weights are on the way: five kernels a
-// layer and not nine, four requests of 20 to 200 tokens and then 12 steps on 12 layers of 768 columns 12.5 -> 11.0 ms
-// (few_row_f32_fused: up to where).
+// layer and not nine, four rows of 768 columns 40 -> 33 us (few_row_f32_fused: up to where).
 //
 // The same bits as rmsnorm_vec_kernel, gemm_f32_kernel and the kernels behind them: the squares are added by as
 // many lanes and in the order of that norm kernel's (256 or 1,024 threads by the width), the products as four chains of
@@ -1445,89 +1618,74 @@ template <int EPI>
 __global__ __launch_bounds__(256, 2) void normed_gemm_f32_kernel(
         const float* __restrict__ x, const float* __restrict__ g, const float* __restrict__ w, int M, int N, int K,
         float eps, NormedEpilogue e) {
-    constexpr int AHEAD = 3;                       // the whole step with 2, 3, 4 blocks: 10.60, 10.57, 10.68 ms
+    constexpr int COLS = EPI == 2 ? 16 : 8;
+    __shared__ __attribute__((aligned(16))) char lds[4 * 32 * GS_PITCH];
     __shared__ gf_floatx4_t sums[4][64];
     __shared__ float squares[16][16], factor[16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, lg = lane >> 4;
-    const int n0 = blockIdx.x * (EPI == 2 ? 16 : 8);
-    const float* xr = x + (size_t)(li < M ? li : M - 1) * K;     // rows beyond the last read it again, never stored
+    const int n0 = blockIdx.x * COLS;
+    // what follows the product, asked for in front of it: the lane's row and four columns, their rotation and their place
+    const int m = li, n = n0 + 4 * lg;
+    const bool mine = wave == 0 && m < M && n < N && 4 * lg < COLS;
+    int pos = 0, seq = 0, page = 0, head = 0, d = 0;
+    float freq[2] = {0.f, 0.f};
+    if (EPI == 2 && mine) {
+        head = n / e.hd;                           // hd is a multiple of 16: the columns of one head
+        d = n - head * e.hd;
+        pos = e.tok_pos[m];
+        seq = e.tok_seq[m];
+        if (head < e.H + e.Hkv) {
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                if (d + 2 * p < e.rot) freq[p] = e.freqs[(d + 2 * p) >> 1];
+        }
+    }
     // a gate's tile: eight rows of Wg and the same eight of Wu, which keeps as many workgroups at work as sixteen
     // columns of a plain product (four rows, 768 -> 2 x 2,048: 9 us; two tiles each in half as many, 11)
-    const int wn = n0 + (EPI == 2 ? li : li & 7);
-    const float* wr = w + (size_t)((wn < N ? wn : N - 1) + (EPI != 2 && li >= 8 ? N : 0)) * K;
-    struct Block {
-        gf_floatx4_t a[2], g[2], w[2];
-    };
-    auto place = [&](int b, int h) {               // the lane's k of block b; the row's first ones again beyond K
-        const int k = 32 * b + 16 * h + 4 * lg;
-        return k < K ? k : 0;
-    };
-    auto load = [&](int b, Block& r) {
+    unsigned from[4];                              // rows beyond the last read it again, never stored
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            r.w[h] = *(const gf_floatx4_t*)(wr + place(b, h));
-            r.a[h] = *(const gf_floatx4_t*)(xr + place(b, h));
-            r.g[h] = *(const gf_floatx4_t*)(g + place(b, h));
-        }
-    };
-    const int blocks = (K + 31) / 32;
-    Block ring[AHEAD + 1];
-#pragma unroll
-    for (int u = 0; u < AHEAD; ++u) load(wave + 4 * u, ring[u]);
-
+    for (int i = 0; i < 4; ++i) {
+        const int r = 8 * (i & 1) + (lane >> 3), wr = EPI == 2 ? r : lane >> 3;
+        const int row = i < 2 ? (r < M ? r : M - 1) : (wr < N - n0 ? wr : N - n0 - 1);
+        from[i] = (unsigned)row * (unsigned)(4 * K) + 16 * (lane & 7);
+    }
+    const char* wt = (const char*)(w + (size_t)n0 * K);
+    float rs[2] = {0.f, 0.f};
+    gf_floatx4_t acc[1][1] = {{gf_floatx4_t{0.f, 0.f, 0.f, 0.f}}};
     // 64 lanes at a time of the norm kernel's threads
     const int groups = K <= 1024 ? 4 : 16, n4 = K >> 2;
-    for (int group = wave; group < groups; group += 4) {
-        const int at = group * 64 + lane;
+    gf_piped<1, 1, 4, true>((const char*)x, wt, EPI == 2 ? wt : (const char*)(w + ((size_t)N + n0) * K), from, g, rs, K,
+                            lds + wave * 32 * GS_PITCH, acc, [&] {
+        if (EPI == 2 && mine && head >= e.H) page = e.table[(size_t)seq * e.table_stride + pos / GFA_PAGE];
+        for (int group = wave; group < groups; group += 4) {
+            const int at = group * 64 + lane;
 #pragma unroll 4
-        for (int m = 0; m < M; ++m) {
-            const float4 v = at < n4 ? ((const float4*)(x + (size_t)m * K))[at] : make_float4(0.f, 0.f, 0.f, 0.f);
-            float ss = 0.f;
-            ss = fmaf(v.x, v.x, ss);
-            ss = fmaf(v.y, v.y, ss);
-            ss = fmaf(v.z, v.z, ss);
-            ss = fmaf(v.w, v.w, ss);
-            ss = wave_sum(ss);
-            if (lane == 0) squares[m][group] = ss;
-        }
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < M) {
-        float ss = 0.f;
-        for (int i = 0; i < groups; ++i) ss += squares[threadIdx.x][i];
-        factor[threadIdx.x] = rsqrtf(ss / (float)K + eps);
-    }
-    __syncthreads();
-    const float rs = factor[li < M ? li : M - 1];
-    gf_floatx4_t acc = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
-    for (int b = wave; b < blocks; b += 4 * (AHEAD + 1)) {
-#pragma unroll
-        for (int u = 0; u <= AHEAD; ++u) {
-            const int at = b + 4 * u;
-            if (at >= blocks) break;
-            load(at + 4 * AHEAD, ring[(u + AHEAD) % (AHEAD + 1)]);
-            Block& r = ring[u];
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) r.a[h][q] = r.a[h][q] * rs * r.g[h][q];
-            if (32 * at + 32 > K) {                // the same for the whole wave: zero beyond K
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    if (32 * at + 16 * h + 4 * lg >= K) {
-                        r.a[h] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
-                        r.w[h] = gf_floatx4_t{0.f, 0.f, 0.f, 0.f};
-                    }
+            for (int r = 0; r < M; ++r) {
+                const float4 v = at < n4 ? ((const float4*)(x + (size_t)r * K))[at] : make_float4(0.f, 0.f, 0.f, 0.f);
+                float ss = 0.f;
+                ss = fmaf(v.x, v.x, ss);
+                ss = fmaf(v.y, v.y, ss);
+                ss = fmaf(v.z, v.z, ss);
+                ss = fmaf(v.w, v.w, ss);
+                ss = wave_sum(ss);
+                if (lane == 0) squares[r][group] = ss;
             }
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(r.w[h][q], r.a[h][q], acc, 0, 0, 0);
         }
-    }
-    sums[wave][lane] = acc;
+        __syncthreads();
+        if ((int)threadIdx.x < M) {
+            float ss = 0.f;
+            for (int i = 0; i < groups; ++i) ss += squares[threadIdx.x][i];
+            factor[threadIdx.x] = rsqrtf(ss / (float)K + eps);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int r = 8 * i + (lane >> 3);
+            rs[i] = factor[r < M ? r : M - 1];
+        }
+    });
+    sums[wave][lane] = acc[0][0];
     __syncthreads();
     if (wave != 0) return;
     const gf_floatx4_t v = (sums[0][lane] + sums[1][lane]) + (sums[2][lane] + sums[3][lane]);
@@ -1536,25 +1694,22 @@ __global__ __launch_bounds__(256, 2) void normed_gemm_f32_kernel(
 #pragma unroll
         for (int q = 0; q < 4; ++q) up[q] = __shfl_xor(v[q], 32, GFA_WAVE);
     }
-    const int m = li, n = n0 + 4 * lg;             // four columns of a row
-    if (m >= M || n >= N) return;
+    if (!mine) return;                             // four columns of a row
     if (EPI != 2) {
-        if (lg >= 2) return;
         float* o = e.out + (size_t)m * N + n;
 #pragma unroll
         for (int q = 0; q < 4; ++q)
             if (n + q < N) o[q] = gate_pair<EPI == 1 ? 1 : 0>(v[q], up[q], 0.f);
         return;
     }
-    const int hd = e.hd, head = n / hd, d = n - head * hd;       // hd is a multiple of 16: the columns of one head
-    const int pos = e.tok_pos[m], off = pos % GFA_PAGE;
+    const int hd = e.hd, off = pos % GFA_PAGE;
     float r[4] = {v[0], v[1], v[2], v[3]};
     if (head < e.H + e.Hkv) {
 #pragma unroll
         for (int p = 0; p < 2; ++p)
             if (d + 2 * p < e.rot) {
                 float s, c;
-                sincosf((float)pos * e.freqs[(d + 2 * p) >> 1], &s, &c);
+                sincosf((float)pos * freq[p], &s, &c);
                 const float a = r[2 * p], b = r[2 * p + 1];
                 r[2 * p] = a * c - b * s;
                 r[2 * p + 1] = b * c + a * s;
@@ -1564,7 +1719,6 @@ __global__ __launch_bounds__(256, 2) void normed_gemm_f32_kernel(
         *(float4*)(e.q + ((size_t)m * e.H + head) * hd + d) = make_float4(r[0], r[1], r[2], r[3]);
         return;
     }
-    const int page = e.table[(size_t)e.tok_seq[m] * e.table_stride + pos / GFA_PAGE];
     if (head < e.H + e.Hkv) {
         float* k = e.k_pages + cache_region(page, head - e.H, e.Hkv, hd);
 #pragma unroll
@@ -1578,12 +1732,11 @@ __global__ __launch_bounds__(256, 2) void normed_gemm_f32_kernel(
 
 // Whether the products work the norms out themselves.  Every workgroup then goes through all rows again, 256 float4 at
 // a time up to 1,024 columns and 1,024 beyond; with more rows or wider ones the separate kernels are the faster way.
-// us a layer, fused and separate (30 keys): 288 columns, 12 rows 36.4, 38.9; 16 40.4, 40.4; 512, 10 42.4, 42.9; 12 45.2,
-// 43.9; 768, 4 39.5, 45.5; 10 47.3, 48.3; 12 50.4, 49.8; 1,024, 10 58.3, 60.4; 12 62.1, 62.2; 1,536, 3 80.3, 81.5; 5 86.7,
-// 84.3; 2,048, 1 79, 84; 3 87.4, 87.3; 4 91, 89; 16 141, 110; 3,072, 2 139, 141; 4 150, 147; 4,096, 1 215, 220; 2 222,
-// 219; 16 363, 306.
+// us a layer, fused and separate (30 keys): 288 columns, 16 rows 28.6, 31.0; 512, 16 31.6, 33.9; 768, 4 33.3, 40.0; 12 40.3, 41.7; 14
+// 42.4, 42.2; 1,024, 12 47.6, 49.0; 16 51.5, 50.4; 1,536, 5 58.3, 58.5; 6 60.3, 58.9; 2,048, 5 69.1, 69.8; 6 71.1, 70.1; 16 94,
+// 77; 3,072, 4 116.9, 117.5; 5 120.2, 117.9; 4,096, 1 185, 197; 3 189, 195; 5 197, 194; 16 256, 207.
 static bool few_row_f32_fused(int M, int D) {
-    return D <= 1024 ? M <= 10 || M * D <= 4608 : D <= 4096 && M * D <= 6144;
+    return D <= 1024 ? M <= 12 || D <= 512 : D <= 4096 && M <= 5 && M * D <= 12288;
 }
 
 struct FewRowWorkF32 {

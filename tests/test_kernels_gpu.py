@@ -110,6 +110,25 @@ def test_gemm_f32_is_the_same_in_every_tile(N, K_):
     assert torch.equal(out.view(80, N), whole[:80])
 
 
+@pytest.mark.parametrize("K_", [4, 36, 160, 292, 1028, 1696])
+@pytest.mark.parametrize("M,N", [(1, 3), (16, 50), (17, 20), (70, 130), (717, 768), (333, 2300), (500, 4090)])
+def test_gemm_f32_in_16_byte_rows(M, N, K_):
+    """Rows of 16-byte loads in each of their tiles, the last of them ragged; blocks of 32 k for none of the waves, for some,
+    more than are asked for ahead, a rest: the bits of the element-by-element form, into a new matrix and onto another."""
+    torch.manual_seed(M + K_)
+    a = torch.randn(M, K_, device=DEV)
+    w = torch.randn(N, K_, device=DEV)
+    odd = torch.empty(M, K_ + 1, device=DEV)[:, 1:].copy_(a)
+    out = K().gemm_f32(a, w)
+    most = a.abs().double() @ w.abs().double().T
+    assert bool(((out.double() - a.double() @ w.double().T).abs() <= most * (K_ + 4) * 2.0 ** -24).all())
+    assert torch.equal(out, K().gemm_f32(odd, w))
+    res = torch.randn(M, N, device=DEV)
+    want = res + out
+    K().gemm_f32(a, w, out=res, accumulate=True)
+    assert torch.equal(res, want)
+
+
 @pytest.mark.parametrize("H,G,hd,rot,lens,starts", [
     (*heads, *tokens) for heads in ((8, 2, 128, 128), (4, 4, 64, 32), (3, 1, 24, 8), (2, 1, 80, 80), (20, 20, 128, 128))
     for tokens in (((401,), (0,)), ((3, 5, 640, 17, 8), (61, 7, 3, 0, 56)), ((9,) * 80, range(80)))] + [
