@@ -617,13 +617,14 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_piped_kernel(
 // 27.4; 768 16.3, 13.7, 12.4, 13.6; 200 rows, N = 768, K = 2,048 35, 29, 23, 12).
 static int gf_piped_tile(int B, int M, int N) {
     if (M <= 16) return 11;
-    int best = 0;
-    double least = 0;
+    int best = 44;
+    double least = INFINITY;
     const int tiles[4][3] = {{4, 4, 100}, {3, 4, 108}, {3, 3, 109}, {2, 2, 117}};
     for (const auto& t : tiles) {
+        if ((M + 16 * t[0] - 1) / (16 * t[0]) > 65535) continue;     // rows of a grid
         const double n = (double)B * ((M + 16 * t[0] - 1) / (16 * t[0])) * ((N + 16 * t[1] - 1) / (16 * t[1]));
         const double cost = ceil(n / 256) * t[0] * t[1] * t[2];
-        if (!best || cost < least) least = cost, best = 10 * t[0] + t[1];
+        if (cost < least) least = cost, best = 10 * t[0] + t[1];
     }
     return best;
 }
