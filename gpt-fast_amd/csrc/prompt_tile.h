@@ -20,8 +20,7 @@
 //  * operands of the next 16 k are read between the products of this one, one read per two products, and
 //    the one barrier of a stage stands before its last 16 k, so that nothing waits behind it;
 //  * copies are spread over a stage's four steps instead of issued in a burst (a burst fills the
-//    address unit and holds the products up), x's first, since copies land in order and x's are due sooner;
-//  * groups of neighbouring columns begin at stages of their own (below).
+//    address unit and holds the products up), x's first, since copies land in order and x's are due sooner.
 // 7,108 rows of 32 experts, a prompt's shares, 4,096 -> 3,584: 322 -> 262 us, 3,584 -> 4,096: 313 -> 252; 8,024 rows,
 // 4,096 -> 2 x 2,048 362 -> 305, 2,048 -> 4,096 197 -> 166; 8,192 rows of one 4,096 x 4,096: 215 -> 205 (1,340 TFLOP/s).
 // The copies are written in asm because the compiler takes any operand read to depend on every copy in
@@ -197,10 +196,11 @@ __device__ __forceinline__ void pt_tile(const PtArgs& g, char* lds, int e, int m
 #define PT_SWIZZLE(r) (((r) >> 1) & 7)
     const int T = K / 64;                                        // stages of the whole product
     // experts begin at different stages: their matrices are often a power of two apart, and walked in step from
-    // the first one they meet in the same memory channels (32 experts of 4,096 x 4,096, 40 tokens: 266 -> 190 us).  So do
-    // groups of an expert's column tiles, as many as an XCD takes together (gated: twice as many; a prompt's shares: 300
-    // -> 288, 190 -> 181; every column tile for itself 333, 209: its neighbours no longer read x at the same time)
-    const int turn = (e + n0 / BN / PT_RUN) * 8 % T;
+    // the first one they meet in the same memory channels (32 experts of 4,096 x 4,096, 40 tokens: 266 -> 190 us).  By the
+    // expert alone, so that a row's sums have one order in every tile of this file.  Groups of an expert's column tiles
+    // with stages of their own, 128 or 256 columns wide as the tile, gained nothing behind the rings: 7,108 rows of 32, 4,096 -> 3,584
+    // 294 us with, 295 without, 3,584 -> 4,096 271, 272; 16 x 250, 4,096 x 4,096 171, 175; 32 x 64, 4,096 -> 3,584 185, 183.
+    const int turn = e * 8 % T;
     const char* xp[UX];
     uint32_t wo[UW];
 #pragma unroll
