@@ -610,16 +610,23 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_piped_kernel(
     gf_store<MT, NT>(sums, out + (size_t)blockIdx.z * sob, M, N, m0, n0, som, accumulate);
 }
 
-// Side of a 16-byte product's tile by rows and columns, in sixteens.  Up to 16 rows 1 x 1, which spreads the weights over the
+// Side of a 16-byte product's tile by rows, columns and inner size, in sixteens.  Up to 16 rows 1 x 1, which spreads the weights over the
 // most waves.  Else a tile's products take the matrix units of one of 256 compute units for as long as it has pieces of 16 x 16, and
 // smaller tiles read more for each: tiles a unit, times pieces, times 1, 1.08, 1.09, 1.17 (2,048 x 4,096 x 4,096: 494, 549, 569,
 // 600 us at 128, 132, 135, 128 pieces a unit; 717 rows of K = 768, us by 4 x 4, 3 x 4, 3 x 3, 2 x 2: N = 4,096 42, 44, 49, 45; 2,304 29.5, 33, 26.5,
-// 27.4; 768 16.3, 13.7, 12.4, 13.6; 200 rows, N = 768, K = 2,048 35, 29, 23, 12).
-static int gf_piped_tile(int B, int M, int N) {
+// 27.4; 768 16.3, 13.7, 12.4, 13.6; 200 rows, N = 768, K = 2,048 35, 29, 23, 12).  Of 2 x 2 tiles
+//  * four share a unit where of the others two do, which counts for more than what they read while a wave has a block or two: times 0.95 up to
+//    K = 192 (2,498 x 14,713 x 16 by 4 x 4 and 2 x 2 130, 110; 705 x 2,220 x 116 12.3, 12.0; 60 times 218 x 1,319 x 16 68, 58);
+//  * what is read again is no longer in the caches where operands are larger than these and rows long: times 1.40 (26 times 361 x 390 x 7,876
+//    852, 1,389; 43 times 289 x 219 x 8,668 608, 1,197; but 2,131 x 565 x 1,380, 15 MB, 56, 41).
+// Over 6,942 products of 17 to 2,500 rows, alone and up to 64 at a time, what it picks is 0.9 % off the fastest tile on average (without these two 3.4 %),
+// and 0.5 % of them are more than 3 % slower than in the two kernels above with 16-byte loads, which this one replaced (1.9 %).
+static int gf_piped_tile(int B, int M, int N, int K) {
     if (M <= 16) return 11;
     int best = 44;
     double least = INFINITY;
-    const int tiles[4][3] = {{4, 4, 100}, {3, 4, 108}, {3, 3, 109}, {2, 2, 117}};
+    const int small = K <= 192 ? 95 : K >= 1024 && ((double)M + N) * K * B * 4 > 32e6 ? 140 : 117;
+    const int tiles[4][3] = {{4, 4, 100}, {3, 4, 108}, {3, 3, 109}, {2, 2, small}};
     for (const auto& t : tiles) {
         if ((M + 16 * t[0] - 1) / (16 * t[0]) > 65535) continue;     // rows of a grid
         const double n = (double)B * ((M + 16 * t[0] - 1) / (16 * t[0])) * ((N + 16 * t[1] - 1) / (16 * t[1]));
@@ -639,7 +646,7 @@ static int gf_product(const float* a, const float* w, float* out, int B, int M, 
     const bool w_wide = swk == 1 && K % 4 == 0 && swn % 4 == 0 && swb % 4 == 0 && (uintptr_t)w % 16 == 0;
     const long long far = 1 << 23;                 // of 64 rows: their bytes have 32 bits
     if (a_wide && w_wide && sam >= 0 && swn >= 0 && sam < far && swn < far) {
-        const int tile = gf_piped_tile(B, M, N), mt = tile / 10 * 16, nt = tile % 10 * 16;
+        const int tile = gf_piped_tile(B, M, N, K), mt = tile / 10 * 16, nt = tile % 10 * 16;
         if ((M + mt - 1) / mt > 65535 || B > 65535) return (int)hipErrorInvalidValue;
         const dim3 grid((N + nt - 1) / nt, (M + mt - 1) / mt, B);
 #define GP_GO(MT, NT, AHEAD) gemm_f32_piped_kernel<MT, NT, AHEAD><<<grid, 256, 0, stream>>>(a, w, out, M, N, K, sab, sam, swb, swn, sob, som, accumulate)

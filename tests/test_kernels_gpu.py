@@ -129,6 +129,23 @@ def test_gemm_f32_in_16_byte_rows(M, N, K_):
     assert torch.equal(res, want)
 
 
+@pytest.mark.parametrize("B,M,N,K_", [(1, 500, 4090, 192), (1, 500, 4090, 196), (1, 717, 768, 196), (3, 65, 700, 64),
+                                      (5, 300, 400, 2300), (4, 300, 400, 2300), (1, 1100, 7000, 1024)])
+def test_gemm_f32_where_its_tiles_change(B, M, N, K_):
+    """Inner sizes of few blocks and of a few more, operands within the caches and beyond them, alone and batched: the bits
+    of the element-by-element form."""
+    torch.manual_seed(M + K_)
+    a = torch.randn(B, M, K_, device=DEV)
+    w = torch.randn(B, N, K_, device=DEV)
+    odd = torch.empty(B, M, K_ + 1, device=DEV)[:, :, 1:].copy_(a)
+    out = K().gemm_f32_batched(a, w, torch.empty(B, M, N, device=DEV))
+    rows = slice(0, M, 7)
+    most = a[:, rows].abs().double() @ w.abs().double().transpose(1, 2).contiguous()
+    want = a[:, rows].double() @ w.double().transpose(1, 2).contiguous()
+    assert bool(((out[:, rows].double() - want).abs() <= most * (K_ + 4) * 2.0 ** -24).all())
+    assert torch.equal(out, K().gemm_f32_batched(odd, w, torch.empty(B, M, N, device=DEV)))
+
+
 @pytest.mark.parametrize("H,G,hd,rot,lens,starts", [
     (*heads, *tokens) for heads in ((8, 2, 128, 128), (4, 4, 64, 32), (3, 1, 24, 8), (2, 1, 80, 80), (20, 20, 128, 128))
     for tokens in (((401,), (0,)), ((3, 5, 640, 17, 8), (61, 7, 3, 0, 56)), ((9,) * 80, range(80)))] + [
