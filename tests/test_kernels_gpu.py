@@ -146,6 +146,17 @@ def test_gemm_f32_where_its_tiles_change(B, M, N, K_):
     assert torch.equal(out, K().gemm_f32_batched(odd, w, torch.empty(B, M, N, device=DEV)))
 
 
+def test_gemm_f32_of_more_rows_than_a_grid_has_of_small_tiles():
+    """A row more than 65,535 tiles of 32 hold: taken by larger ones, its first and last rows as they are alone."""
+    M = 65535 * 32 + 1
+    torch.manual_seed(1)
+    a = torch.randn(M, 4, device=DEV)
+    w = torch.randn(3, 4, device=DEV)
+    out = K().gemm_f32(a, w)
+    for rows in (slice(0, 16), slice(M - 16, M)):
+        assert torch.equal(out[rows], K().gemm_f32(a[rows].clone(), w))
+
+
 @pytest.mark.parametrize("H,G,hd,rot,lens,starts", [
     (*heads, *tokens) for heads in ((8, 2, 128, 128), (4, 4, 64, 32), (3, 1, 24, 8), (2, 1, 80, 80), (20, 20, 128, 128))
     for tokens in (((401,), (0,)), ((3, 5, 640, 17, 8), (61, 7, 3, 0, 56)), ((9,) * 80, range(80)))] + [
