@@ -459,8 +459,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_staged_kernel(
 // The wave's whole blocks of `at` (16 MT rows) and `wt` (16 NT rows, the second half of them from `wt2`) into acc; from: the lane's bytes
 // from there to its rows, eight a load.  ready() runs once the first AHEAD blocks are asked for.  NORMED: elements of `at` times
 // their row's rs, then times g.
-template <int MT, int NT, int AHEAD, bool NORMED, class Ready>
-__device__ __forceinline__ void gf_piped(const char* at, const char* wt, const char* wt2, const unsigned (&from)[2 * (MT + NT)],
+template <int MT, int NT, int AHEAD, bool NORMED, class Offset, class Ready>
+__device__ __forceinline__ void gf_piped(const char* at, const char* wt, const char* wt2, const Offset (&from)[2 * (MT + NT)],
                                          const float* g, const float (&rs)[2 * MT], int K, char* own, gf_floatx4_t (&acc)[MT][NT], Ready ready) {
     constexpr int S = MT + NT, HALF = 4 * MT * NT;         // operands of a half block, its products
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -576,7 +576,8 @@ __device__ __forceinline__ void gf_piped(const char* at, const char* wt, const c
 // (140 TFLOP/s), 717 x 4,096 x 768 71 -> 43, 717 x 768 x 2,048 41 -> 24, 60 x 768 x 2,048 19 -> 12, 4 x 32,000 x 768 32.5 -> 20,
 // 4 x 768 x 2,048 10 -> 7.3, 16 x 28,672 x 4,096 142 -> 96.  A 1 x 1 tile with one block ahead takes 78 us for 4 x 4,096 x 14,336, with
 // two 60, with four 45 (before: 55); 2 x 2 tiles with two ahead hold more registers and are slower (29.7, 31.5 at 717 x 768 x 2,048).
-template <int MT, int NT, int AHEAD>
+// Offset: of the bytes from a tile's first row to its others.
+template <int MT, int NT, int AHEAD, class Offset = unsigned>
 __global__ __launch_bounds__(256, 2) void gemm_f32_piped_kernel(
         const float* __restrict__ a, const float* __restrict__ w, float* __restrict__ out, int M, int N, int K,
         long long sab, long long sam, long long swb, long long swn, long long sob, long long som, int accumulate) {
@@ -585,11 +586,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_piped_kernel(
     static_assert(4 * MT * NT * 1024 <= 4 * 16 * S * GS_PITCH, "the waves' sums take the blocks' place");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int m0 = blockIdx.y * (16 * MT), n0 = blockIdx.x * (16 * NT);
-    unsigned from[2 * S];                          // rows beyond the last read it again, never stored
+    Offset from[2 * S];                            // rows beyond the last read it again, never stored
 #pragma unroll
     for (int i = 0; i < 2 * S; ++i) {
         const int r = 8 * (i < 2 * MT ? i : i - 2 * MT) + (lane >> 3), most = (i < 2 * MT ? M - m0 : N - n0) - 1;
-        from[i] = (unsigned)(r < most ? r : most) * (unsigned)(4 * (i < 2 * MT ? sam : swn)) + 16 * (lane & 7);
+        from[i] = (Offset)(r < most ? r : most) * (Offset)(4 * (i < 2 * MT ? sam : swn)) + 16 * (lane & 7);
     }
     gf_floatx4_t acc[MT][NT];
 #pragma unroll
@@ -644,13 +645,18 @@ static int gf_product(const float* a, const float* w, float* out, int B, int M, 
     // 16-byte loads: whole groups of four k, at addresses that are multiples of 16
     const bool a_wide = K % 4 == 0 && sam % 4 == 0 && sab % 4 == 0 && (uintptr_t)a % 16 == 0;
     const bool w_wide = swk == 1 && K % 4 == 0 && swn % 4 == 0 && swb % 4 == 0 && (uintptr_t)w % 16 == 0;
-    const long long far = 1 << 23;                 // of 64 rows: their bytes have 32 bits
-    if (a_wide && w_wide && sam >= 0 && swn >= 0 && sam < far && swn < far) {
-        const int tile = gf_piped_tile(B, M, N, K), mt = tile / 10 * 16, nt = tile % 10 * 16;
+    if (a_wide && w_wide) {
+        // Rows whose offsets within a tile of 64 have no 32 bits: the same with 64, by the tiles that they had in front of this kernel
+        const bool far = sam < 0 || swn < 0 || sam >= 1 << 23 || swn >= 1 << 23;
+        const long long tiles = (long long)((M + 63) / 64) * ((N + 63) / 64) * B;
+        const int tile = !far ? gf_piped_tile(B, M, N, K) : M <= 16 ? 11 : tiles < 100 ? 22 : 44, mt = tile / 10 * 16, nt = tile % 10 * 16;
         if ((M + mt - 1) / mt > 65535 || B > 65535) return (int)hipErrorInvalidValue;
         const dim3 grid((N + nt - 1) / nt, (M + mt - 1) / mt, B);
-#define GP_GO(MT, NT, AHEAD) gemm_f32_piped_kernel<MT, NT, AHEAD><<<grid, 256, 0, stream>>>(a, w, out, M, N, K, sab, sam, swb, swn, sob, som, accumulate)
-        if (tile == 11) GP_GO(1, 1, 4);
+#define GP_GO(...) gemm_f32_piped_kernel<__VA_ARGS__><<<grid, 256, 0, stream>>>(a, w, out, M, N, K, sab, sam, swb, swn, sob, som, accumulate)
+        if (far && tile == 11) GP_GO(1, 1, 4, long long);
+        else if (far && tile == 22) GP_GO(2, 2, 1, long long);
+        else if (far) GP_GO(4, 4, 1, long long);
+        else if (tile == 11) GP_GO(1, 1, 4);
         else if (tile == 22) GP_GO(2, 2, 1);
         else if (tile == 33) GP_GO(3, 3, 1);
         else if (tile == 34) GP_GO(3, 4, 1);

@@ -146,6 +146,22 @@ def test_gemm_f32_where_its_tiles_change(B, M, N, K_):
     assert torch.equal(out, K().gemm_f32_batched(odd, w, torch.empty(B, M, N, device=DEV)))
 
 
+@pytest.mark.parametrize("apart", [2 ** 23 - 4, 2 ** 23, 2 ** 23 + 4])
+def test_gemm_f32_of_rows_far_apart(apart):
+    """Offsets within a tile that need more than 32 bits, in either operand and every tile: the bits of rows side by side."""
+    K_ = 300
+    buffer = torch.empty(70 * apart, device=DEV)
+    many = torch.randn(3300, K_, device=DEV)
+    for M in (1, 16, 20, 70):
+        far = buffer.as_strided((M, K_), (apart, 1))
+        near = torch.randn(M, K_, device=DEV)
+        far.copy_(near)
+        assert torch.equal(K().gemm_f32(far, many), K().gemm_f32(near, many))
+        for rows in (many[:5], many[:40], many):
+            out = K().gemm_f32_batched(rows[None], far[None], torch.empty(1, len(rows), M, device=DEV))
+            assert torch.equal(out[0], K().gemm_f32(rows, near))
+
+
 def test_gemm_f32_of_more_rows_than_a_grid_has_of_small_tiles():
     """A row more than 65,535 tiles of 32 hold: taken by larger ones, its first and last rows as they are alone."""
     M = 65535 * 32 + 1
