@@ -1355,7 +1355,7 @@ __global__ __launch_bounds__(256, 3) void attention_f32_rows_kernel(
             if (in && lo[t] < least) least = lo[t];
             if (pos[t] > last) last = pos[t];
             if (lo[t] > all_from) all_from = lo[t];
-            if (pos[t] < all_to) all_to = pos[t];
+            if (in && pos[t] < all_to) all_to = pos[t];    // what the others add up is not stored
         }
         const int* pages = table + (size_t)seq * table_stride;
         const int first = least / GFA_PAGE;
