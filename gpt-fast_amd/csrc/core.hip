@@ -1297,43 +1297,48 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
 // head, and a wave that has a page in its registers works off all of them that are of its sequence.  The kernel above
 // brings every page in anew for every token, 32 KB through the caches for 8,000 multiply-adds, and a wave's time on a page
 // is one chain; here four rows' chains run beside each other.  What bounds it still is the way of a wave through its page, loads,
-// scores, maximum, values, some 4 us: 717 tokens of four prompts, 12 heads of 64: 55 -> 28 us; one prompt of 200 19 -> 11, of 2,048
-// 449 -> 221; 32 heads on 4 117 -> 59, 37 -> 21, 1,173 -> 547.  Eight rows hold too many registers (717: 44 to 56).
+// scores, maximum, values, some 4 us: 717 tokens of four prompts, 12 heads of 64: 59 -> 27 us; one prompt of 200 21 -> 12, of 2,048
+// 459 -> 229; 32 heads on 4 128 -> 59, 40 -> 23, 1,196 -> 564.  Eight rows hold too many registers (717: 44 to 56).
 // The same arithmetic for a row, so the same bits: its pages are shared out to the waves by their own index; a page that it
 // does not see leaves its maximum, sum and elements as they are, and chunks of keys behind its last one are left out.
-// A group of four may hold rows of several sequences: its workgroup takes the first of them, further ones begin
-// "inside" and are shared out to workgroups behind the groups', AF_SLICES for every 64 tokens.
+// A group of four may hold rows of several sequences: its workgroup takes the first run of one sequence, further ones begin
+// "inside" and are shared out to workgroups behind the groups', for every 64 tokens as many as the tokens can have, or AF_SLICES.
+// SINGLES: a run of one token, a decode step's beside prompts, has a code of its own, since that for four takes as long for one: 172
+// tokens and one behind 1,800 keys 43 -> 22 us (one at a time 26), 640 and fifteen behind 1,900 119 -> 60 (96).  A single sequence does
+// without it, whose code for four then is 1 to 2 % faster.
 #define AF_ROWS 4
-#define AF_SLICES 8
+#define AF_SLICES 16
+template <bool SINGLES>
 __global__ __launch_bounds__(256, 3) void attention_f32_rows_kernel(
         const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
         const int* __restrict__ tok_seq, const int* __restrict__ tok_pos, const int* __restrict__ table,
-        int table_stride, float* __restrict__ out, int n_tokens, int H, int Hkv, int hd, float scale, int window) {
-    constexpr int ROWS = AF_ROWS;
-    static_assert(ROWS == 4, "a thread for every element of the queries");
-    __shared__ __attribute__((aligned(16))) float qs[ROWS][64];
-    __shared__ __attribute__((aligned(16))) float ps[4][ROWS][GFA_PAGE];
-    __shared__ float merged[4][ROWS][66];
+        int table_stride, float* __restrict__ out, int n_tokens, int slices, int H, int Hkv, int hd, float scale, int window) {
+    static_assert(AF_ROWS == 4, "a thread for every element of the queries");
+    __shared__ __attribute__((aligned(16))) float qs[AF_ROWS][64];
+    __shared__ __attribute__((aligned(16))) float ps[4][AF_ROWS][GFA_PAGE];
+    __shared__ float merged[4][AF_ROWS][66];
     const int h = blockIdx.y, lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int g = h / (H / Hkv), groups = (n_tokens + ROWS - 1) / ROWS;
-    int base = blockIdx.x * ROWS;
+    const int g = h / (H / Hkv), groups = (n_tokens + AF_ROWS - 1) / AF_ROWS;
+    int base = blockIdx.x * AF_ROWS;
     unsigned long long starts = 1;                         // tokens base + bit: where this workgroup's runs begin
-    if ((int)blockIdx.x >= groups) {                       // every AF_SLICES-th of those that begin inside a group
-        const int slice = ((int)blockIdx.x - groups) % AF_SLICES;
-        base = ((int)blockIdx.x - groups) / AF_SLICES * 64;
+    if ((int)blockIdx.x >= groups) {                       // every slices-th of those that begin inside a group
+        const int slice = ((int)blockIdx.x - groups) % slices;
+        base = ((int)blockIdx.x - groups) / slices * 64;
         const int n = base + lane;
         const int there = n < n_tokens ? n : 0;
-        unsigned long long all = __ballot(there % ROWS != 0 && tok_seq[there] != tok_seq[there > 0 ? there - 1 : 0]);
+        unsigned long long all = __ballot(there % AF_ROWS != 0 && tok_seq[there] != tok_seq[there > 0 ? there - 1 : 0]);
         starts = 0;
         for (int i = 0; all; ++i, all &= all - 1)
-            if (i % AF_SLICES == slice) starts |= all & -all;
+            if (i % slices == slice) starts |= all & -all;
     }
-    for (; starts; starts &= starts - 1) {
-        const int n0 = base + __builtin_ctzll(starts);
-        const int seq = tok_seq[n0];
-        int count = 1;
-        while (n0 + count < n_tokens && (n0 + count) % ROWS != 0 && tok_seq[n0 + count] == seq) ++count;
+    // the run of `count` tokens from n0 on, worked off by a code for ROWS
+    auto walk = [&](auto rows, int n0, int count, int seq) {
+        constexpr int ROWS = decltype(rows)::value;
+        int lane = threadIdx.x & 63;
+        if (SINGLES) asm("" : "+v"(lane));                 // what follows from it is not kept through both codes
+        const unsigned vd = lane < hd ? lane : 0;
+        const unsigned k_at = (lane >> 5) * 32 * hd + key_slot(lane & 31) * 8, v_at = (vd >> 4) * 1024 + (vd & 15) * 8;
         {                                                  // rows beyond the last: the last one again, not seen
             const int row = wave < count ? wave : count - 1;
             if (lane < hd) qs[wave][lane] = q[((size_t)(n0 + row) * H + h) * hd + lane];
@@ -1361,20 +1366,18 @@ __global__ __launch_bounds__(256, 3) void attention_f32_rows_kernel(
         const int first = least / GFA_PAGE;
         for (int page = first + ((wave - first) & 3); page * GFA_PAGE <= last; page += 4) {
             const size_t region = cache_region(pages[page], g, Hkv, hd);
-            const float* kr = k_pages + region + (lane >> 5) * 32 * hd + key_slot(lane & 31) * 8;
-            const int vd = lane < hd ? lane : 0;           // lanes beyond the head: others' elements again
-            const float* vr = v_pages + region + (vd >> 4) * 1024 + (vd & 15) * 8;
+            const float *kr = k_pages + region, *vr = v_pages + region;
             float4 ke[16], ve[16];
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
                 const float* at = kr + (c * 8 < hd ? c : 0) * 256;
-                ke[2 * c] = *(const float4*)at;
-                ke[2 * c + 1] = *(const float4*)(at + 4);
+                ke[2 * c] = *(const float4*)(at + k_at);
+                ke[2 * c + 1] = *(const float4*)(at + k_at + 4);
             }
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
-                ve[2 * c] = *(const float4*)(vr + c * 128);
-                ve[2 * c + 1] = *(const float4*)(vr + c * 128 + 4);
+                ve[2 * c] = *(const float4*)(vr + c * 128 + v_at);
+                ve[2 * c + 1] = *(const float4*)(vr + c * 128 + v_at + 4);
             }
             float dot0[ROWS], dot1[ROWS];
 #pragma unroll
@@ -1463,14 +1466,23 @@ __global__ __launch_bounds__(256, 3) void attention_f32_rows_kernel(
             if (lane < hd) out[((size_t)(n0 + t) * H + h) * hd + lane] = v / total;
         }
         __syncthreads();
+    };
+    for (; starts; starts &= starts - 1) {
+        const int n0 = base + __builtin_ctzll(starts);
+        const int seq = tok_seq[n0];
+        int count = 1;
+        while (n0 + count < n_tokens && (n0 + count) % AF_ROWS != 0 && tok_seq[n0 + count] == seq) ++count;
+        if (SINGLES && count == 1) walk(std::integral_constant<int, 1>(), n0, count, seq);
+        else walk(std::integral_constant<int, AF_ROWS>(), n0, count, seq);
     }
 }
 
 // Whether a step's rows go four at a time; pages: the most that its table has for a sequence.  Not where the groups would
-// be too few to hide a wave's way, nor where many rows have sequences of their own: a wave takes as long on a page for one row as for
-// four.  us, one at a time and four: 12 heads of 64, one prompt of 60 8.0, 7.9; 100 11.5, 8.7; 60 behind 2,000 keys 38, 45; 100 behind
-// 900 30.5, 27.1; several: 4 x 50 behind 900 56, 44; 600 and eight single tokens behind 900 73, 51; 200 and the eight 28.5, 30.9;
-// 40 x 3 14.2, 12.4; 4 x 30 behind 300 19.2, 22.8; 64 single tokens behind 100 12.1, 42.4.
+// be too few to hide a wave's way; of several sequences, whose shares of the tokens and keys the host does not know, where it was the faster way
+// for all that were measured.  us, one at a time and four, 12 heads of 64: one prompt of 60 8.4, 8.6; 100 12.4, 9.6; 60 behind 2,000 keys
+// 39, 47; 100 behind 900 31, 28; several: 4 x 50 behind 900 56, 39; 600 and eight single tokens behind 900 74, 43; 640 and fifteen
+// behind 1,900 92, 60.  On the other side 64 single tokens behind 100 12.8, 18.6; 16 behind 900 19.7, 20.6 (32 heads on 4 16.3, 42.3); 4 x 30
+// behind 300 20.3, 20.4 (6 heads of 48 10.3, 13.4); but also 20 x 7 17.0, 9.4, behind 200 35, 19, and 30 x 9 behind 100 32, 21.
 static bool attention_f32_four(int n_tokens, int n_seqs, int H, int hd, int pages) {
     if (hd > 64) return false;
     if (n_seqs <= 1) return (long long)n_tokens * H >= 1024;
@@ -1503,9 +1515,14 @@ extern "C" int gfa_attention_generic(const void* q, const void* k_pages, const v
 #define AF_GO(HD, EARLY) attention_f32_kernel<HD, EARLY><<<grid, 256, 0, stream>>>((const float*)q, (const float*)k_pages, \
         (const float*)v_pages, tok_seq, tok_pos, table, table_stride, (float*)out, H, Hkv, hd, scale, window)
         if (attention_f32_four(n_tokens, n_seqs, H, hd, table_stride)) {
-            const int groups = (n_tokens + AF_ROWS - 1) / AF_ROWS, slices = n_seqs > 1 ? (n_tokens + 63) / 64 * AF_SLICES : 0;
-            attention_f32_rows_kernel<<<dim3(groups + slices, H), 256, 0, stream>>>((const float*)q, (const float*)k_pages,
-                (const float*)v_pages, tok_seq, tok_pos, table, table_stride, (float*)out, n_tokens, H, Hkv, hd, scale, window);
+            const int groups = (n_tokens + AF_ROWS - 1) / AF_ROWS;
+            const int slices = n_seqs <= 1 ? 0 : n_seqs - 1 < AF_SLICES ? n_seqs - 1 : AF_SLICES;
+#define AF_ROWS_GO(SINGLES) attention_f32_rows_kernel<SINGLES><<<dim3(groups + (n_tokens + 63) / 64 * slices, H), 256, 0, stream>>>( \
+        (const float*)q, (const float*)k_pages, (const float*)v_pages, tok_seq, tok_pos, table, table_stride, (float*)out, n_tokens, slices, \
+        H, Hkv, hd, scale, window)
+            if (n_seqs > 1) AF_ROWS_GO(true);
+            else AF_ROWS_GO(false);
+#undef AF_ROWS_GO
         } else if (attention_f32_early(n_tokens, H, Hkv, hd, table_stride, window)) AF_GO(64, true);
         else if (hd <= 64) AF_GO(64, false);
         else if (hd <= 128) AF_GO(128, false);

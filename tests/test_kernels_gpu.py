@@ -547,10 +547,11 @@ def test_a_float32_row_is_the_same_among_few_and_among_many(H, G, hd, S, window)
 
 
 @pytest.mark.parametrize("held,new", [([0], [1030]), ([0, 0, 0, 0], [177, 150, 193, 200]), ([130, 0, 5, 64], [1, 259, 2, 61]),
-                                      ([0, 63, 3, 70, 1, 0], [190, 1, 1, 1, 1, 129]), ([1000, 1], [6, 390])])
+                                      ([0, 63, 3, 70, 1, 0], [190, 1, 1, 1, 1, 129]), ([1000, 1], [6, 390]),
+                                      ([70] * 24 + [0], [1] * 24 + [980])])
 @pytest.mark.parametrize("H,G,hd,window", [(12, 12, 64, 0), (32, 4, 64, 70), (16, 16, 48, 0), (16, 2, 16, 3)])
 def test_float32_rows_that_go_four_at_a_time(H, G, hd, window, held, new):
-    """Groups of four rows that hold the ends and beginnings of sequences, one of a single token, pages that some of a
+    """Groups of four rows that hold the ends and beginnings of sequences, one of a single token, many of single tokens, pages that some of a
     group's rows see and others do not, a value that is no number: the same bits as each row alone."""
     lens = [a + b for a, b in zip(held, new)]
     k_pages, v_pages, table, ks, vs = _paged(lens, G, hd, torch.float32, sum(lens) + hd)
