@@ -1491,11 +1491,11 @@ static bool attention_f32_four(int n_tokens, int n_seqs, int H, int hd, int page
 
 // Whether a step whose rows go one at a time asks early; pages: as above.  Not where there are many workgroups (one
 // a token and head) and they walk many pages, or share the keys of a group, which then are in the caches.  us, early and
-// not, heads of 64, prompts' keys out of the caches and single tokens' out of memory: 12 heads, a token behind 30
-// keys 5.6, 6.7; 16 behind 1,000 25.7, 26.2; prompts of 8 x 200 123, 132; 600 3.12 ms of a model's step either way; 900 124,
-// 119; 2,048 484, 459, with a window of 256 231, 257; 300 behind 2,000 151, 142.  32 heads on 4: a token behind
-// 1,000 15.6, 17.2; prompts of 100 23.7, 20.4; 4 x 150 116, 109; 2,048 1,267, 1,192, with a window 596, 635.
-// Heads of 48, whose loads are not whole lines: 900 64, 75; 2,048 237, 241.
+// not, heads of 64, keys out of memory: 12 heads, a token behind 30 keys 5.6, 6.7; 16 behind 1,000 25.7, 26.2; 32 heads on 4, a token
+// behind 1,000 15.6, 17.2; out of the caches: 12 heads, 64 tokens behind 900 65, 68; 64 sequences of 4 behind 100 33, 38; 40 of 30
+// 90, 103, behind 500 with a window of 128 101, 123; 3 of 100 behind 3,000 213, 210; 32 heads on 4, 64 of 4 behind 100 55, 54; 32 of 4 behind
+// 900 145, 128; 40 of 30 222, 202 (but behind 500 504, 550), with the window 249, 310.  Heads of 48, whose loads are not whole lines: 6 heads, 64 of 4
+// behind 100 17, 20; 40 of 30 47, 68.
 static bool attention_f32_early(int n_tokens, int H, int Hkv, int hd, int pages, int window) {
     if (window > 0 && window / GFA_PAGE + 2 < pages) pages = window / GFA_PAGE + 2;
     if ((long long)n_tokens * H < 2048 || hd == 48) return hd <= 64;

@@ -15,14 +15,19 @@
 // two buffers of 64 KB had some 35 KB under way at a time, 1 us of latency long.  Hence:
 //  * x and W have rings of buffers of their own in the 160 KB: two of x, whose rows other workgroups of the XCD
 //    read too, and three of W, which comes from memory and so is asked for two stages ahead (low tiles: three and
-//    three, four and four).  One round of the chip, 16 experts of 256, 192, 128, 64 rows, 4,096 x 4,096: 127, 112,
-//    104, 96 us; with two buffers of both, and lines of W asked for ahead, 146, 133, 119, 107;
+//    three, four and four; of two workgroups to a compute unit 128 x 128 two and three, 64 x 256 two and two, which are all that it
+//    holds).  One round of the chip, 16 experts of 256, 192, 128, 64 rows, 4,096 x 4,096: 155, 120, 109, 102 us; with two buffers of
+//    both, and lines of W asked for ahead, 163, 141, 123, 108; 128 x 128: 8 x 60, 4,096 -> 3,584 71 -> 51, 64 x 60, 2,048 -> 2,048 138 -> 125, though
+//    where W alone bounds it now and then the slower way, by up to 4 % (32 x 40, 4,096 -> 3,584 186 to 197, 182 to 200);
 //  * operands of the next 16 k are read between the products of this one, one read per two products, and
 //    the one barrier of a stage stands before its last 16 k, so that nothing waits behind it;
 //  * copies are spread over a stage's four steps instead of issued in a burst (a burst fills the
 //    address unit and holds the products up), x's first, since copies land in order and x's are due sooner.
-// 7,108 rows of 32 experts, a prompt's shares, 4,096 -> 3,584: 322 -> 262 us, 3,584 -> 4,096: 313 -> 252; 8,024 rows,
-// 4,096 -> 2 x 2,048 362 -> 305, 2,048 -> 4,096 197 -> 166; 8,192 rows of one 4,096 x 4,096: 215 -> 205 (1,340 TFLOP/s).
+// 7,108 rows of 32 experts, sums, shares spread as exp(0.4 normal) and nearly equal: 4,096 -> 3,584 326 -> 271 us, 288 -> 256; 3,584 -> 4,096
+// 318 -> 272, 270 -> 242.  With an activation in the epilogue, which nobody else's products hide, less or nothing: silu 349 -> 295, 289 -> 287;
+// gelu, equal shares, 312 -> 310.  (The rows' gather through `order` costs nothing: 288 in order, 285 gathered.)  In a prompt of 1,777 tokens these two products
+// took 341 on average and take 329, with gelu, and 261.  8,000 rows, 4,096 -> 2 x 2,048 363 -> 319, 2,048 -> 4,096 194 -> 172; 8,192 rows of one
+// 4,096 x 4,096 228 -> 220 (1,250 TFLOP/s).
 // The copies are written in asm because the compiler takes any operand read to depend on every copy in
 // flight and waits for all of them; they have no output registers, and the waits below count them.
 #pragma once
@@ -411,8 +416,6 @@ void prompt_tile_kernel(const PtArgs g) {
         if (m1 - m0 <= 64) return pt_tile<1, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
         if (m1 - m0 <= 128) return pt_tile<2, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
         if (m1 - m0 <= 192) return pt_tile<3, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
-        if constexpr (TM > 4) if (m1 - m0 <= 256) return pt_tile<4, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
-        if constexpr (TM > 5) if (m1 - m0 <= 320) return pt_tile<5, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
     }
     pt_tile<TM, TN, MODE, LDS>(g, lds, e, m0, m1, bn * CN);
 }

@@ -1,8 +1,8 @@
 """Attention over the paged cache: which kernel runs a step's attention.
 
-float32 engine: one workgroup per token and head, float arithmetic in an order fixed by the
-token's position (``attention_generic``, which has a kernel of its own for float32 heads of a
-multiple of 16).  bfloat16 engine: the split-context kernel
+float32 engine: float arithmetic in an order fixed by the token's position (``attention_generic``: one
+workgroup per token and head, with a kernel of its own for float32 heads of a multiple of 16, and one that
+takes the rows of prompts four at a time to the same bits).  bfloat16 engine: the split-context kernel
 for one-token steps, the MFMA kernel for prompts (csrc/attention_bf16.hip), and the
 plain kernel for shapes those refuse.
 """

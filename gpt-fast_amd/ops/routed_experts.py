@@ -330,18 +330,18 @@ def tall_tiles_win(n_experts: int, pairs: int, F: int, K: int, mode: int, units:
     """Whether 256 x 256 tiles, which read each operand half as often and are only as high as their rows (steps of 64),
     make the products of :func:`rows_tile`'s arguments fastest.
 
-    What decides is the rounds of the chip that either needs.  Fitted to the times: one of these tiles to a unit takes
+    What decides is the rounds of the chip that either needs.  Fitted to the times of these kernels with two buffers of
+    both operands: one of these tiles to a unit takes
     1.15 times as long as two of 128 x 128 that share it, nearly whatever its height, and a last round of one small
-    tile to a unit 0.65 of one of two.  Microseconds, 128 x 128 and these (means of two draws of shares spread as
-    :func:`_shares`): 16 experts, 3,584 -> 4,096, x 120 rows 159, 123; x 140, a second round of these, 162, 172; x 222 215,
-    187; 32, 4,096 -> 3,584, x 64 201, 210; x 100 267, 227; x 222 390, 346; 8, 3,584 -> 4,096, x 180 82, 98; x 222, a
-    second round of the small ones, 132, 101; 32, 2,816 -> 2,048, x 140 137, 153.  Shares that are not the assumed ones
-    can end a round elsewhere: 16, 5,120 -> 2 x 1,536, x 120, counted as a little more than a round of small ones, needed
-    one: 130, 154.  (The kernel with a ring of its own for W, 14 to 20 % faster in tall tiles, up to 10 % in these: over 2,000
-    random points of 20 to 700 rows what the two rules choose is 2.9 % off the fastest kernel on average; the best
-    other factors, and other lines in K, 2.7 %.)  Up to K = 1,024 :func:`rows_tile` says, but for sums of K = 1,024 from
-    400 rows an expert on: 1,024 -> 2,048, x 600 older kernel, 128 x 128, these: 16 experts 78, 65, 68; 32 144, 141,
-    119; 128 537, 543, 481."""
+    tile to a unit 0.65 of one of two.  With rings of their own for x and W both are faster, over 7,415 random points of 30 to
+    700 rows by 9 % on average, at 0.8 % of them more than 3 % slower; what the two rules choose is 2.1 % off the faster tile on
+    average, and no other factors (0.95 to 1.15) are better by more than 0.03 %.  Microseconds, 128 x 128 and these (means of two draws of
+    shares spread as :func:`_shares`), these chosen: 16 experts, 3,584 -> 4,096, x 120 rows 146, 114; x 222 184, 159; 32, 4,096 -> 3,584, x 100
+    232, 194; x 222 371, 274; 8, 3,584 -> 4,096, x 222 108, 86; 16, 5,120 -> 2 x 1,536, x 120 176, 141; 128 x 128 chosen: 8,
+    3,584 -> 4,096, x 180 85, 88; but also 16, 3,584 -> 4,096, x 140, a second round of these, 154, 137; 32, 4,096 -> 3,584, x 64
+    201, 187; 32, 2,816 -> 2,048, x 140 123, 118.  Up to K = 1,024 :func:`rows_tile` says, but for sums of K = 1,024 from
+    400 rows an expert on: 1,024 -> 2,048, x 600 older kernel, 128 x 128, these: 16 experts 76, 65, 67; 32 135, 122,
+    107; 128 515, 468, 400."""
     if pairs < 36 * n_experts or K < 1024 or K == 1024 and (mode != 0 or pairs < 400 * n_experts):
         return False
     gated = mode == 2
@@ -364,14 +364,14 @@ def rows_tile(n_experts: int, pairs: int, F: int, K: int, mode: int, units: int)
     on average:
 
     * From 36 rows on shares above 64 become frequent, whose matrices the 64 x 256 tile reads twice: 64 x 34,
-      1,280 -> 2,048 tile 1 68, tile 2 76; 32 x 39, 3,584 -> 4,096 219, 179.  Below, where its workgroups
-      are fewer than the units, tile 2 has twice as many: 8 x 10, 4,096 -> 2 x 2,048 74, 68.
-    * Where tile 2 does not need a second round it is the best: 8 x 400, 1,024 -> 2 x 512 older 23, tile 2 19; 8 x 170,
-      4,096 -> 2 x 2,048 101, 90.
+      1,280 -> 2,048 of equal shares tile 1 68, tile 2 76 (of shares spread as above 95, 79); 32 x 39, 3,584 -> 4,096 232, 191.  Below, where its
+      workgroups are fewer than the units, tile 2 has twice as many: 8 x 10, 4,096 -> 2 x 2,048 84, 55.
+    * Where tile 2 does not need a second round it is the best: 8 x 400, 1,024 -> 2 x 512 older 26, tile 2 17; 8 x 170,
+      4,096 -> 2 x 2,048 121, 93.
     * Up to K = 1,024 a tile is over so soon that its first loads and its last stores show; over some rounds the older
-      kernel, three to a unit, hides them best: 64 x 62, 1,024 -> 2 x 1,024 69, tile 2 77; 128 x 62, 768 -> 2,048 100,
-      110; 256 x 140, 512 -> 2 x 1,024 207, 253.  Over fewer it is not worth the list (3 to 8 us): 64 x 62, 768 ->
-      2,048 64, 58; 128 x 127, 512 -> 2 x 256 37, 31."""
+      kernel, three to a unit, hides them best: 64 x 62, 1,024 -> 2 x 1,024 80, tile 2 83; 256 x 140, 512 -> 2 x 1,024 198,
+      213 (but 128 x 62, 768 -> 2,048 113, 108).  Over fewer it is not worth the list (3 to 8 us): 64 x 62, 768 ->
+      2,048 64, 57; 128 x 127, 512 -> 2 x 256 46, 33."""
     gated = mode == 2
     if pairs < 36 * n_experts:
         columns = 128 if gated else 256
