@@ -26,7 +26,7 @@
 // 7,108 rows of 32 experts, sums, shares spread as exp(0.4 normal) and nearly equal: 4,096 -> 3,584 326 -> 271 us, 288 -> 256; 3,584 -> 4,096
 // 318 -> 272, 270 -> 242.  With an activation in the epilogue, which nobody else's products hide, less or nothing: silu 349 -> 295, 289 -> 287;
 // gelu, equal shares, 312 -> 310.  (The rows' gather through `order` costs nothing: 288 in order, 285 gathered.)  In a prompt of 1,777 tokens these two products
-// took 341 on average and take 329, with gelu, and 261.  8,000 rows, 4,096 -> 2 x 2,048 363 -> 319, 2,048 -> 4,096 194 -> 172; 8,192 rows of one
+// took 341 on average and take 329, with gelu, and 268.  8,000 rows, 4,096 -> 2 x 2,048 363 -> 319, 2,048 -> 4,096 194 -> 172; 8,192 rows of one
 // 4,096 x 4,096 228 -> 220 (1,250 TFLOP/s).
 // The copies are written in asm because the compiler takes any operand read to depend on every copy in
 // flight and waits for all of them; they have no output registers, and the waits below count them.
