@@ -1302,9 +1302,10 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
 // The same arithmetic for a row, so the same bits: its pages are shared out to the waves by their own index; a page that it
 // does not see leaves its maximum, sum and elements as they are, and chunks of keys behind its last one are left out.
 // A group of four may hold rows of several sequences: its workgroup takes the first run of one sequence, further ones begin
-// "inside" and are shared out to workgroups behind the groups', for every 64 tokens as many as the tokens can have, or AF_SLICES.
+// "inside" and are shared out to workgroups behind the groups', 8 to AF_SLICES for every 64 tokens by the number of sequences: one for
+// each but the first were enough where a sequence's tokens follow each other, but 2 x 200 in turn then take 164 us and not 43.
 // SINGLES: a run of one token, a decode step's beside prompts, has a code of its own, since that for four takes as long for one: 172
-// tokens and one behind 1,800 keys 43 -> 22 us (one at a time 26), 640 and fifteen behind 1,900 119 -> 60 (96).  A single sequence does
+// tokens and one behind 1,800 keys 43 -> 24 us (one at a time 26), 640 and fifteen behind 1,900 119 -> 60 (96).  A single sequence does
 // without it, whose code for four then is 1 to 2 % faster.
 #define AF_ROWS 4
 #define AF_SLICES 16
@@ -1516,7 +1517,7 @@ extern "C" int gfa_attention_generic(const void* q, const void* k_pages, const v
         (const float*)v_pages, tok_seq, tok_pos, table, table_stride, (float*)out, H, Hkv, hd, scale, window)
         if (attention_f32_four(n_tokens, n_seqs, H, hd, table_stride)) {
             const int groups = (n_tokens + AF_ROWS - 1) / AF_ROWS;
-            const int slices = n_seqs <= 1 ? 0 : n_seqs - 1 < AF_SLICES ? n_seqs - 1 : AF_SLICES;
+            const int slices = n_seqs <= 1 ? 0 : n_seqs <= 8 ? 8 : n_seqs < AF_SLICES ? n_seqs : AF_SLICES;
 #define AF_ROWS_GO(SINGLES) attention_f32_rows_kernel<SINGLES><<<dim3(groups + (n_tokens + 63) / 64 * slices, H), 256, 0, stream>>>( \
         (const float*)q, (const float*)k_pages, (const float*)v_pages, tok_seq, tok_pos, table, table_stride, (float*)out, n_tokens, slices, \
         H, Hkv, hd, scale, window)

@@ -581,6 +581,20 @@ def test_float32_rows_that_go_four_at_a_time(H, G, hd, window, held, new):
         assert torch.equal(alone(n).nan_to_num(7.0), out[n].nan_to_num(7.0)), n
 
 
+def test_float32_rows_of_sequences_in_turn():
+    """Tokens that change their sequence from one to the next, all runs of one: the bits of each row alone."""
+    lens, H, hd = [260, 231, 7], 12, 64
+    k_pages, v_pages, table, ks, vs = _paged(lens, H, hd, torch.float32, 5)
+    order = sorted((p, b) for b, n in enumerate(lens) for p in range(n))
+    seq = torch.tensor([b for _, b in order], dtype=torch.int32).to(DEV)
+    pos = torch.tensor([p for p, _ in order], dtype=torch.int32).to(DEV)
+    q = torch.randn(len(order), H, hd, generator=torch.Generator().manual_seed(6)).to(DEV)
+    out = K().attention_generic(q, k_pages, v_pages, seq, pos, table, hd ** -0.5, 0)
+    for n in list(range(40)) + list(range(40, len(order), 23)):
+        alone = K().attention_generic(q[n:n + 1], k_pages, v_pages, seq[n:n + 1], pos[n:n + 1], table, hd ** -0.5, 0)
+        assert torch.equal(alone[0], out[n]), n
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-5), (torch.bfloat16, 1.5e-2)])
 @pytest.mark.parametrize("H,G,hd,window", [
     (4, 4, 16, 0), (6, 2, 48, 0), (8, 1, 128, 0), (3, 3, 80, 0), (4, 2, 64, 37), (2, 1, 256, 100),
