@@ -1305,7 +1305,7 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
 // "inside" and are shared out to workgroups behind the groups', 8 to AF_SLICES for every 64 tokens by the number of sequences: one for
 // each but the first were enough where a sequence's tokens follow each other, but 2 x 200 in turn then take 164 us and not 43.
 // SINGLES: a run of one token, a decode step's beside prompts, has a code of its own, since that for four takes as long for one: 172
-// tokens and one behind 1,800 keys 43 -> 24 us (one at a time 26), 640 and fifteen behind 1,900 119 -> 60 (96).  A single sequence does
+// tokens and one behind 1,800 keys 43 -> 24 us (one at a time 26), 640 and fifteen behind 1,900 126 -> 65 (98).  A single sequence does
 // without it, whose code for four then is 1 to 2 % faster.
 #define AF_ROWS 4
 #define AF_SLICES 16
@@ -1482,7 +1482,7 @@ __global__ __launch_bounds__(256, 3) void attention_f32_rows_kernel(
 // be too few to hide a wave's way; of several sequences, whose shares of the tokens and keys the host does not know, where it was the faster way
 // for all that were measured.  us, one at a time and four, 12 heads of 64: one prompt of 60 8.4, 8.6; 100 12.4, 9.6; 60 behind 2,000 keys
 // 39, 47; 100 behind 900 31, 28; several: 4 x 50 behind 900 56, 39; 600 and eight single tokens behind 900 74, 43; 640 and fifteen
-// behind 1,900 92, 60.  On the other side 64 single tokens behind 100 12.8, 18.6; 16 behind 900 19.7, 20.6 (32 heads on 4 16.3, 42.3); 4 x 30
+// behind 1,900 94, 65.  On the other side 64 single tokens behind 100 12.8, 18.6; 16 behind 900 19.7, 20.6 (32 heads on 4 16.3, 42.3); 4 x 30
 // behind 300 20.3, 20.4 (6 heads of 48 10.3, 13.4); but also 20 x 7 17.0, 9.4, behind 200 35, 19, and 30 x 9 behind 100 32, 21.
 static bool attention_f32_four(int n_tokens, int n_seqs, int H, int hd, int pages) {
     if (hd > 64) return false;
